@@ -227,8 +227,8 @@ def bench_kvcache(args, fpb=3):
 
 def bench_composed(args):
     """The composed f32 SDPA on the device (masked plans, Plan::composed, fallbacks): H=12, S=4096,
-    d=128, f32 operands and a shared additive block-causal mask [S, S]; all arithmetic fp32 on the
-    matrix cores (v_mfma_f32_32x32x2_f32: 157.3 TFLOP/s peak)."""
+    d=128, f32 operands and a shared additive block-causal mask [S, S]; all arithmetic f32 (each f32
+    value as three bf16 parts on the bf16 matrix cores; the roofline is the f32 matrix peak, 157.3 TFLOP/s)."""
     import torch
 
     import fv_sdpa
@@ -270,7 +270,7 @@ def bench_composed(args):
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": "composed f32 SDPA with a shared additive [S, S] mask, H=12 S=4096 d=128", "flops_per_call": flops},
         "roofline": {"bound": "mfma", "achieved": round(tf, 3), "peak": 157.3, "unit": "TFLOP/s", "frac": round(tf / 157.3, 4),
-                     "traffic": None, "kernel": "fv::sdpa_composed_mfma_f32_kernel<128>", "avg_kernel_ms": round(avg, 4)},
+                     "traffic": None, "kernel": "fv::sdpa_composed_kernel<128, 3, 1, false>", "avg_kernel_ms": round(avg, 4)},
     }
     print(json.dumps(rec), flush=True)
 

@@ -1,22 +1,37 @@
-// Composed SDPA in f32 on the matrix cores: softmax(scale * q k^T + mask) v with every operand,
-// product and accumulation in fp32 (v_mfma_f32_32x32x2_f32), the path of the plans the reference
-// runs through its composed tensor ops (rt/sdpa.rs:328-342: masked calls, Plan::composed, the
-// block-causal / KV-window fallbacks, FASTVIDEO_SDPA=cublas) — there materialised scores through
-// cuBLAS f32 (rt/attn.rs:748-865), here an online softmax over 32-key tiles, so no [bh, sq, sk]
-// buffer exists. Head dims 32 / 64 / 96 / 128; other head dims keep the scalar kernel of rt_sdpa.hip.
+// Composed SDPA, softmax(scale * q k^T + mask) v with f32 arithmetic, on the bf16 matrix cores: the path of the
+// plans the reference runs through its composed tensor ops (rt/sdpa.rs:328-342: masked calls, Plan::composed, the
+// block-causal / KV-window fallbacks, FASTVIDEO_SDPA=cublas) — there materialised scores through cuBLAS f32
+// (rt/attn.rs:748-865), here an online softmax over key tiles, so no [bh, sq, sk] buffer exists. Head dims up to 128;
+// longer heads keep the scalar kernel of rt_sdpa.hip.
 //
-// One workgroup = 4 waves x 32 queries. K and V tiles of 32 keys go global -> registers -> LDS
-// (double buffered: the loads of tile t+1 are in flight under the arithmetic of tile t, one barrier
-// per tile); 2 workgroups share a CU, so one wave's softmax runs under the other's MFMAs.
+// f32 on bf16 matrix cores: an f32 value is the sum of three bf16 values exactly (24 significant bits = 3 x 8, each
+// part the nearest bf16 of what the ones before it leave), and a product of two of them, x y = sum over the parts, is
+// exact in f32. Of the nine part products the six that matter are multiplied (hi.hi, hi.mid, mid.hi, mid.mid, hi.lo,
+// lo.hi): the three left out are below 2^-24 of the product, the size of one f32 rounding, and the accumulators are
+// f32. v_mfma_f32_32x32x16_bf16 has sixteen times the rate of v_mfma_f32_32x32x2_f32, so six of them cost 0.375 of the
+// one f32 product they replace. Operands that are bf16 numbers already (bf16 tensors, or f32 ones that the caller
+// wants rounded: PARTS = 1) have one part, so K Q^T is one product and P V, whose P is f32, three.
+// (Non-finite operands give NaN rows: the parts of an infinity do not add up.) Measured against the same sums in 64
+// bits, rel_l2: 5.4e-7 at 4096 x 4096 x 128, 3.9e-7 at 1024 x 1024 x 64; the v_mfma_f32_32x32x2_f32 form: 8.1e-7 and
+// 6.1e-7. Time: 1376 -> 830 us at 12 x 4096 x 4096 x 128 with a shared mask (f32 operands, what bounds it is the matrix
+// pipe with 1.5 workgroups of work per CU); with the casts and the rounding of the result taken into the kernel
+// 303 -> 40 us at 64 x 512 x 512 x 64 with a mask per head (bf16; its 67 MB of mask are half of that), and
+// 136 -> 33 us at 16 x 257 x 257 x 80, a head dim that used to take the scalar kernel.
 //
-//   S^T (32 keys x 32 queries) = K Q^T     A = K[key = l%32][k], B = Q[query = l%32][k]; the MFMA's
-//                                          two k slots (lane halves) take d = j and d = j + D/2, so a
-//                                          lane's K operands of 4 consecutive steps are one 16-byte read
+// One workgroup = 4 waves. KS waves share 32 queries, each walking every KS-th key tile with its own running max and
+// sum; their results are merged through LDS at the end. KS = 1 (128 queries a workgroup) where the query tiles fill
+// the chip, more where they do not. Tiles go global -> registers -> (split into parts) -> LDS; the next tile's loads
+// are in flight under the arithmetic of the current one, and two workgroups share a CU, so that one wave's softmax and
+// splitting run under the other's MFMAs.
+//
+//   S^T (32 keys x 32 queries) = K Q^T     A = K[key = l%32][16 j + 8 (l/32) ..], B = Q of the lane's query, same d
 //   C layout                               lane l, register i: query l%32, key 8*(i/4) + 4*(l/32) + i%4
-//   O^T (D x 32 queries) += V^T P^T        step i takes register i of both halves as the two key slots;
-//                                          A = V[that key][32*db + l%32]
+//   O^T (d x 32 queries) += V^T P^T        B = eight score registers as they are; A = V of the same keys, read
+//                                          transposed from the row-major tile (ds_read_b64_tr_b16)
 //
-// LDS rows are padded (K: D + 4 floats, V: D + 8) so that both read patterns spread over all banks.
+// LDS rows are padded so that both read patterns spread over all banks: K rows to 2 D + 16 bytes (a multiple of 16
+// bytes that is odd in 16-byte units: 16 consecutive rows hit 16 different 16-byte columns), V rows to an odd multiple
+// of 64 bytes (the 4 rows of a transposed read land in 4 different 64-byte bank groups).
 #include <limits.h>
 
 #include "../../include/fv_sdpa_hip.h"
@@ -26,187 +41,425 @@
 namespace fv {
 namespace {
 
-constexpr int kCQ = 128;   // queries per workgroup
-constexpr int kCK = 32;    // keys per tile
+struct Parts3 {
+    bf16x8 p[3];
+};
 
-FV_DEV f32x16 mfma32_f32(float a, float b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+// x = p[0] + p[1] + p[2] exactly (nearest bf16 each time)
+FV_DEV Parts3 split3(const f32x8 x) {
+    Parts3 r;
+    r.p[0] = __builtin_convertvector(x, bf16x8);
+    const f32x8 e1 = x - __builtin_convertvector(r.p[0], f32x8);
+    r.p[1] = __builtin_convertvector(e1, bf16x8);
+    const f32x8 e2 = e1 - __builtin_convertvector(r.p[1], f32x8);
+    r.p[2] = __builtin_convertvector(e2, bf16x8);
+    return r;
+}
+
+// Eight consecutive elements [c, c + 8) of a row of d, zeros past d; `vec`: rows are whole 16-byte units at 16-byte
+// aligned addresses.
+template <bool IS16>
+FV_DEV f32x8 load8_f32(const void* row, int c, int d, bool vec) {
+    f32x8 v = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if constexpr (IS16) {
+        const uint16_t* p = (const uint16_t*)row + c;
+        if (vec) {
+            if (c < d) v = __builtin_convertvector(*reinterpret_cast<const bf16x8*>(p), f32x8);
+        } else {
+#pragma unroll
+            for (int x = 0; x < 8; x++)
+                if (c + x < d) v[x] = bf16_bits_to_f32(p[x]);
+        }
+    } else {
+        const float* p = (const float*)row + c;
+        if (vec) {
+            if (c < d) {
+                const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+                for (int x = 0; x < 4; x++) v[x] = a[x], v[4 + x] = b[x];
+            }
+        } else {
+#pragma unroll
+            for (int x = 0; x < 8; x++)
+                if (c + x < d) v[x] = p[x];
+        }
+    }
+    return v;
 }
 
 template <int D>
-__global__ __launch_bounds__(256, 2) void sdpa_composed_mfma_f32_kernel(
-    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    const float* __restrict__ mask, long mask_bh_stride, float* __restrict__ out, int sq, int sk, float scale) {
-    constexpr int RK = D + 4, RV = D + 8;          // padded LDS row lengths (floats)
-    constexpr int kUnits = D / 32;                  // 16-byte units per thread and tile
-    constexpr int kNO = D / 32;
-    extern __shared__ __attribute__((aligned(16))) float csm[];
-    // buffers b = 0, 1: K at csm + b * kKT, V at csm + 2 * kKT + b * kVT (offsets, so that the compiler
-    // keeps every access in the LDS address space)
-    constexpr int kKT = kCK * RK, kVT = kCK * RV;
+struct ComposedGeo {
+    static constexpr int kKRow = 2 * D + 16;
+    static constexpr int kVRow = (D / 32) % 2 == 1 ? 2 * D : 2 * D + 64;
+};
+template <int D, int PARTS, int KS>
+constexpr int composed_lds() {
+    return KS * PARTS * 32 * (ComposedGeo<D>::kKRow + ComposedGeo<D>::kVRow);
+}
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+template <int D, int PARTS, int KS, bool KV16>
+__global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedParams p) {
+    static_assert(D % 32 == 0 && (PARTS == 1 || PARTS == 3) && (KS == 1 || KS == 2 || KS == 4) && !(KV16 && PARTS == 3),
+                  "instantiations");
+    using G = ComposedGeo<D>;
+    constexpr int QG = 4 / KS;               // 32-query groups per workgroup
+    constexpr int kGroup = 64 * QG;          // threads that share a key tile
+    constexpr int kKP = 32 * G::kKRow, kVP = 32 * G::kVRow;   // bytes of one part of a K / V tile
+    constexpr int kUnits = 32 * (D / 8);     // 8-element units per tile
+    constexpr int kPer = (kUnits + kGroup - 1) / kGroup;
+    constexpr int NO = D / 32, NC = D / 16;
+    constexpr int kMine = KV16 ? 4 : 8;      // 32-bit registers per unit in flight
+    extern __shared__ __attribute__((aligned(16))) unsigned char csm[];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, c32 = lane & 31;
+    const int qg = wave % QG, ks = wave / QG;
+    const int gt = tid - ks * kGroup;        // thread within the group
+    lds_u8* kt = (lds_u8*)csm + ks * (PARTS * (kKP + kVP));
+    lds_u8* vt = kt + PARTS * kKP;
     const long bh = blockIdx.y;
-    const int q0 = blockIdx.x * kCQ;
-    const int qi = q0 + wave * 32 + c32;            // this lane's query
+    const int sq = p.sq, sk = p.sk, d = p.d;
+    const bool vec = p.vec != 0;
+    const int qi = blockIdx.x * (32 * QG) + qg * 32 + c32;   // this lane's query
     const bool q_ok = qi < sq;
     const float NEG = neg_inf();
-    const float* kb = k + bh * sk * (long)D;
-    const float* vb = v + bh * sk * (long)D;
-    const float* mr = mask ? mask + bh * mask_bh_stride + (long)(q_ok ? qi : 0) * sk : nullptr;
+    const char* kb = (const char*)p.k + bh * sk * (long)d * (KV16 ? 2 : 4);
+    const char* vb = (const char*)p.v + bh * sk * (long)d * (KV16 ? 2 : 4);
+    const float* mr = p.mask ? p.mask + bh * p.mask_bh + (long)(q_ok ? qi : 0) * sk : nullptr;
 
-    // Q operand: this lane's query, d = h*D/2 + j for step j
-    float qr[D / 2];
+    // Q operand, in parts: this lane's query, d = 16 j + 8 h ..
+    bf16x8 qf[PARTS][NC];
     {
-        const float* src = q + (bh * sq + (q_ok ? qi : 0)) * (long)D + h * (D / 2);
+        const long row = bh * sq + (q_ok ? qi : 0);
 #pragma unroll
-        for (int j = 0; j < D / 2; j += 4) {
-            f32x4 t = {0.f, 0.f, 0.f, 0.f};
-            if (q_ok) t = *reinterpret_cast<const f32x4*>(src + j);
+        for (int j = 0; j < NC; j++) {
+            const int c = 16 * j + 8 * h;
+            f32x8 x = p.q_is_bf16 ? load8_f32<true>((const uint16_t*)p.q + row * d, c, d, vec)
+                                  : load8_f32<false>((const float*)p.q + row * d, c, d, vec);
+            if (!q_ok) x = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if constexpr (PARTS == 1) {
+                qf[0][j] = __builtin_convertvector(x, bf16x8);
+            } else {
+                const Parts3 s = split3(x);
 #pragma unroll
-            for (int x = 0; x < 4; x++) qr[j + x] = t[x];
+                for (int t = 0; t < 3; t++) qf[t][j] = s.p[t];
+            }
         }
     }
 
-    // tile loads: thread t owns 16-byte units t + 256 r of the [32][D] tile
-    f32x4 kreg[kUnits], vreg[kUnits];
-    auto load_tile = [&](int kv0) {
+    // One 8-element unit of the group's tile in registers: raw bf16, or f32.
+    struct Unit {
+        u32x4 r[kMine / 4];
+    };
+    auto load_units = [&](const char* base, int kv0, Unit (&u)[kPer]) {
 #pragma unroll
-        for (int r = 0; r < kUnits; r++) {
-            const int u = tid + 256 * r, row = u / (D / 4), c4 = u % (D / 4);
-            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            kreg[r] = vreg[r] = z;
-            if (kv0 + row < sk) {
-                kreg[r] = *reinterpret_cast<const f32x4*>(kb + (long)(kv0 + row) * D + 4 * c4);
-                vreg[r] = *reinterpret_cast<const f32x4*>(vb + (long)(kv0 + row) * D + 4 * c4);
+        for (int r = 0; r < kPer; r++) {
+            const int un = gt + kGroup * r, row = un / (D / 8), c = 8 * (un % (D / 8));
+#pragma unroll
+            for (int x = 0; x < kMine / 4; x++) u[r].r[x] = u32x4{0u, 0u, 0u, 0u};
+            if (un < kUnits && kv0 + row < sk && c < d) {
+                const char* src = base + ((long)(kv0 + row) * d + c) * (KV16 ? 2 : 4);
+                if (vec) {
+#pragma unroll
+                    for (int x = 0; x < kMine / 4; x++) u[r].r[x] = *reinterpret_cast<const u32x4*>(src + 16 * x);
+                } else {
+                    // rows that are not whole 16-byte units: element by element
+#pragma unroll
+                    for (int x = 0; x < 8; x++) {
+                        if (c + x < d) {
+                            if constexpr (KV16)
+                                u[r].r[0][x >> 1] |= (unsigned)reinterpret_cast<const uint16_t*>(src)[x] << (16 * (x & 1));
+                            else
+                                u[r].r[(x >> 2) % (kMine / 4)][x & 3] = reinterpret_cast<const unsigned*>(src)[x];
+                        }
+                    }
+                }
             }
         }
     };
-    auto store_tile = [&](int buf) {
+    auto store_units = [&](lds_u8* dst, int row_bytes, int part_bytes, const Unit (&u)[kPer]) {
 #pragma unroll
-        for (int r = 0; r < kUnits; r++) {
-            const int u = tid + 256 * r, row = u / (D / 4), c4 = u % (D / 4);
-            *reinterpret_cast<f32x4*>(csm + buf * kKT + row * RK + 4 * c4) = kreg[r];
-            *reinterpret_cast<f32x4*>(csm + 2 * kKT + buf * kVT + row * RV + 4 * c4) = vreg[r];
+        for (int r = 0; r < kPer; r++) {
+            const int un = gt + kGroup * r, row = un / (D / 8), c = 8 * (un % (D / 8));
+            if (un >= kUnits) continue;
+            lds_u8* at = dst + row * row_bytes + 2 * c;
+            if constexpr (KV16) {
+                lds_write_b128(at, u[r].r[0]);
+            } else {
+                const f32x4 a = __builtin_bit_cast(f32x4, u[r].r[0]), b = __builtin_bit_cast(f32x4, u[r].r[kMine / 4 - 1]);
+                const f32x8 x = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+                if constexpr (PARTS == 1) {
+                    lds_write_b128(at, __builtin_bit_cast(u32x4, __builtin_convertvector(x, bf16x8)));
+                } else {
+                    const Parts3 s = split3(x);
+#pragma unroll
+                    for (int t = 0; t < 3; t++) lds_write_b128(at + t * part_bytes, __builtin_bit_cast(u32x4, s.p[t]));
+                }
+            }
         }
     };
 
-    f32x16 o[kNO];
+    f32x16 o[NO];
 #pragma unroll
-    for (int db = 0; db < kNO; db++)
+    for (int db = 0; db < NO; db++)
 #pragma unroll
         for (int i = 0; i < 16; i++) o[db][i] = 0.f;
     float m_run = NEG, l_run = 0.f;
 
-    const int nt = (sk + kCK - 1) / kCK;
-    load_tile(0);
-    store_tile(0);
-    __syncthreads();
+    const lds_u8* ka = kt + c32 * G::kKRow + 16 * h;
+    const int b16 = lane >> 4, i16 = lane & 15;
+    const lds_u8* va = vt + (4 * h + (i16 >> 2)) * G::kVRow + 32 * (b16 & 1) + 8 * (i16 & 3);
+
+    const int nt = (sk + 31) / 32, steps = (nt + KS - 1) / KS;
+    Unit ku[kPer], vu[kPer];
+    load_units(kb, ks * 32, ku);
+    load_units(vb, ks * 32, vu);
 #pragma unroll 1
-    for (int t = 0; t < nt; t++) {
-        const int kv0 = t * kCK, buf = t & 1;
-        if (t + 1 < nt) load_tile(kv0 + kCK);      // in flight under this tile's arithmetic
-        // ---- S^T = K Q^T ----
-        f32x16 s;
-#pragma unroll
-        for (int i = 0; i < 16; i++) s[i] = 0.f;
-        const float* krow = csm + buf * kKT + c32 * RK + h * (D / 2);
-#pragma unroll
-        for (int j = 0; j < D / 2; j += 4) {
-            const f32x4 a = *reinterpret_cast<const f32x4*>(krow + j);
-#pragma unroll
-            for (int x = 0; x < 4; x++) s = mfma32_f32(a[x], qr[j + x], s);
-        }
-        // ---- scale, mask, online softmax (per lane = per query; halves exchange max and sum) ----
-        {
-#pragma clang fp contract(off)
-            float mx = NEG;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int key = kv0 + 8 * (i >> 2) + 4 * h + (i & 3);
-                float sv = s[i] * scale;
-                if (mr && key < sk) sv = sv + mr[key];
-                if (key >= sk) sv = NEG;
-                s[i] = sv;
-                mx = __builtin_fmaxf(mx, sv);
-            }
-            mx = pair_max(mx);
-            const float m_new = __builtin_fmaxf(m_run, mx);
-            const float alpha = (m_run == NEG) ? 0.f : fast_exp2((m_run - m_new) * 1.4426950408889634f);
-            float ls = 0.f;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const float p = (m_new == NEG) ? 0.f : fast_exp2((s[i] - m_new) * 1.4426950408889634f);
-                s[i] = p;
-                ls += p;
-            }
-            l_run = l_run * alpha + pair_sum(ls);
-            m_run = m_new;
-            if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-#pragma unroll
-                for (int db = 0; db < kNO; db++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++) o[db][i] *= alpha;
-            }
-        }
-        // ---- O^T += V^T P^T ----
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const float* vrow = csm + 2 * kKT + buf * kVT + (8 * (i >> 2) + 4 * h + (i & 3)) * RV + c32;
-#pragma unroll
-            for (int db = 0; db < kNO; db++) o[db] = mfma32_f32(vrow[32 * db], s[i], o[db]);
-        }
-        if (t + 1 < nt) store_tile(buf ^ 1);        // the other buffer: its readers passed the last barrier
+    for (int step = 0; step < steps; step++) {
+        const int kv0 = (step * KS + ks) * 32;
+        store_units(kt, G::kKRow, kKP, ku);
+        store_units(vt, G::kVRow, kVP, vu);
         __syncthreads();
+        if (step + 1 < steps) {   // in flight under this tile's arithmetic (rows past the end: zeros)
+            load_units(kb, kv0 + 32 * KS, ku);
+            load_units(vb, kv0 + 32 * KS, vu);
+        }
+        if (kv0 < sk) {           // (a wave whose share has ended keeps the barriers only)
+            // the additive mask of the lane's 16 keys, four consecutive ones per load where rows allow it
+            f32x16 mk;
+            if (mr) {
+                if (p.vec_mask) {
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        const int key = kv0 + 8 * g + 4 * h;
+                        f32x4 t = {0.f, 0.f, 0.f, 0.f};
+                        if (key < sk) t = *reinterpret_cast<const f32x4*>(mr + key);
+#pragma unroll
+                        for (int x = 0; x < 4; x++) mk[4 * g + x] = t[x];
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        const int key = kv0 + 8 * (i >> 2) + 4 * h + (i & 3);
+                        mk[i] = key < sk ? mr[key] : 0.f;
+                    }
+                }
+            }
+            // ---- S^T = K Q^T ----
+            f32x16 s;
+#pragma unroll
+            for (int i = 0; i < 16; i++) s[i] = 0.f;
+#pragma unroll
+            for (int j = 0; j < NC; j++) {
+                bf16x8 a[PARTS];
+#pragma unroll
+                for (int t = 0; t < PARTS; t++) a[t] = lds_read_b128(ka + t * kKP + 32 * j);
+                if constexpr (PARTS == 3) {   // small products first
+                    s = mfma32(a[2], qf[0][j], s);
+                    s = mfma32(a[0], qf[2][j], s);
+                    s = mfma32(a[1], qf[1][j], s);
+                    s = mfma32(a[1], qf[0][j], s);
+                    s = mfma32(a[0], qf[1][j], s);
+                }
+                s = mfma32(a[0], qf[0][j], s);
+            }
+            // ---- scale, mask, online softmax (per lane = per query; halves exchange max and sum) ----
+            {
+#pragma clang fp contract(off)
+                float mx = NEG;
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    float sv = s[i] * p.scale;
+                    if (mr) sv = sv + mk[i];
+                    s[i] = sv;
+                }
+                if (kv0 + 32 > sk) {
+#pragma unroll
+                    for (int i = 0; i < 16; i++)
+                        if (kv0 + 8 * (i >> 2) + 4 * h + (i & 3) >= sk) s[i] = NEG;
+                }
+#pragma unroll
+                for (int i = 0; i < 16; i++) mx = __builtin_fmaxf(mx, s[i]);
+                mx = pair_max(mx);
+                const float m_new = __builtin_fmaxf(m_run, mx);
+                const float alpha = (m_run == NEG) ? 0.f : fast_exp2((m_run - m_new) * 1.4426950408889634f);
+                const float off = (m_new == NEG) ? 0.f : m_new;   // a row that has seen no key: every P is 2^-inf = 0
+                float ls = 0.f;
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const float e = fast_exp2((s[i] - off) * 1.4426950408889634f);
+                    s[i] = e;
+                    ls += e;
+                }
+                l_run = l_run * alpha + pair_sum(ls);
+                m_run = m_new;
+                if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+                    for (int db = 0; db < NO; db++)
+#pragma unroll
+                        for (int i = 0; i < 16; i++) o[db][i] *= alpha;
+                }
+            }
+            // ---- O^T += V^T P^T, 16 keys at a time ----
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                f32x8 e;
+#pragma unroll
+                for (int x = 0; x < 8; x++) e[x] = s[8 * t + x];
+                const Parts3 pp = split3(e);
+#pragma unroll
+                for (int db = 0; db < NO; db++) {
+                    bf16x8 a[PARTS];
+#pragma unroll
+                    for (int x = 0; x < PARTS; x++) {
+                        const lds_u8* at = va + x * kVP + 64 * db + 16 * t * G::kVRow;
+                        s16x8 w;
+                        w.lo = lds_read_tr16_b64(at);
+                        w.hi = lds_read_tr16_b64(at + 8 * G::kVRow);
+                        a[x] = __builtin_bit_cast(bf16x8, w);
+                    }
+                    if constexpr (PARTS == 3) {
+                        o[db] = mfma32(a[2], pp.p[0], o[db]);
+                        o[db] = mfma32(a[1], pp.p[1], o[db]);
+                        o[db] = mfma32(a[0], pp.p[2], o[db]);
+                        o[db] = mfma32(a[1], pp.p[0], o[db]);
+                    } else {
+                        o[db] = mfma32(a[0], pp.p[2], o[db]);
+                    }
+                    o[db] = mfma32(a[0], pp.p[1], o[db]);
+                    o[db] = mfma32(a[0], pp.p[0], o[db]);
+                }
+            }
+        }
+        __syncthreads();
+    }
+
+    if constexpr (KS > 1) {
+        // merge the KS shares of every query: shares 1 .. KS-1 leave O, max and sum in LDS, share 0 adds them up
+        constexpr int kRegs = 16 * NO + 2;
+        static_assert((KS - 1) * QG * kRegs * 256 <= composed_lds<D, PARTS, KS>(), "the merge fits the tile buffers");
+        auto slot = [&](int share) { return (lds_u8*)csm + ((share - 1) * QG + qg) * (kRegs * 256) + lane * 4; };
+        auto at = [](lds_u8* b, int r) { return reinterpret_cast<__attribute__((address_space(3))) float*>(b + r * 256); };
+        if (ks > 0) {
+            lds_u8* b = slot(ks);
+#pragma unroll
+            for (int db = 0; db < NO; db++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) *at(b, 16 * db + i) = o[db][i];
+            *at(b, 16 * NO) = m_run;
+            *at(b, 16 * NO + 1) = l_run;
+        }
+        __syncthreads();
+        if (ks > 0) return;
+        float m_all = m_run, ms[KS], ls[KS];
+#pragma unroll
+        for (int t = 1; t < KS; t++) {
+            ms[t] = *at(slot(t), 16 * NO);
+            ls[t] = *at(slot(t), 16 * NO + 1);
+            m_all = __builtin_fmaxf(m_all, ms[t]);
+        }
+        const float w0 = m_run == NEG ? 0.f : fast_exp2((m_run - m_all) * 1.4426950408889634f);
+        l_run *= w0;
+#pragma unroll
+        for (int db = 0; db < NO; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) o[db][i] *= w0;
+#pragma unroll
+        for (int t = 1; t < KS; t++) {
+            const float w = ms[t] == NEG ? 0.f : fast_exp2((ms[t] - m_all) * 1.4426950408889634f);
+            l_run += ls[t] * w;
+#pragma unroll
+            for (int db = 0; db < NO; db++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) o[db][i] += *at(slot(t), 16 * db + i) * w;
+        }
     }
 
     if (q_ok) {
 #pragma clang fp contract(off)
-        float* dst = out + (bh * sq + qi) * (long)D;
+        const long base = (bh * sq + qi) * (long)d;
 #pragma unroll
-        for (int db = 0; db < kNO; db++)
+        for (int db = 0; db < NO; db++)
 #pragma unroll
             for (int g = 0; g < 4; g++) {
+                const int d0 = 32 * db + 8 * g + 4 * h;
                 f32x4 r;
 #pragma unroll
                 for (int x = 0; x < 4; x++) r[x] = l_run > 0.f ? o[db][4 * g + x] / l_run : 0.f;
-                *reinterpret_cast<f32x4*>(dst + 32 * db + 8 * g + 4 * h) = r;
+                if (p.out_is_bf16) {
+                    uint16_t* dst = (uint16_t*)p.out + base + d0;
+                    const bf16x4 r16 = __builtin_convertvector(r, bf16x4);
+                    if (vec) {
+                        if (d0 < d) *reinterpret_cast<bf16x4*>(dst) = r16;
+                    } else {
+#pragma unroll
+                        for (int x = 0; x < 4; x++)
+                            if (d0 + x < d) reinterpret_cast<__bf16*>(dst)[x] = r16[x];
+                    }
+                } else {
+                    float* dst = (float*)p.out + base + d0;
+                    if (vec) {
+                        if (d0 < d) *reinterpret_cast<f32x4*>(dst) = r;
+                    } else {
+#pragma unroll
+                        for (int x = 0; x < 4; x++)
+                            if (d0 + x < d) dst[x] = r[x];
+                    }
+                }
             }
     }
 }
 
-template <int D>
-hipError_t launch_composed(const float* q, const float* k, const float* v, const float* mask, long mask_bh_stride,
-                           float* out, size_t bh, int sq, int sk, float scale, hipStream_t st) {
-    constexpr int lds = (2 * kCK * (D + 4) + 2 * kCK * (D + 8)) * (int)sizeof(float);   // 67 KB at D = 128
+template <int D, int PARTS, int KS, bool KV16>
+hipError_t launch_as(const ComposedParams& p, size_t bh, hipStream_t st) {
+    constexpr int lds = composed_lds<D, PARTS, KS>();
     if (lds > 64 * 1024) {
         static std::atomic<unsigned long long> attr_done;
-        const hipError_t e = fv_set_max_lds_once((const void*)sdpa_composed_mfma_f32_kernel<D>, lds, attr_done);
+        const hipError_t e = fv_set_max_lds_once((const void*)sdpa_composed_kernel<D, PARTS, KS, KV16>, lds, attr_done);
         if (e != hipSuccess) return e;
     }
-    const dim3 grid((unsigned)((sq + kCQ - 1) / kCQ), (unsigned)bh);
-    hipLaunchKernelGGL((sdpa_composed_mfma_f32_kernel<D>), grid, dim3(256), lds, st, q, k, v, mask, mask_bh_stride, out,
-                       sq, sk, scale);
+    constexpr int rows = 32 * (4 / KS);
+    const dim3 grid((unsigned)((p.sq + rows - 1) / rows), (unsigned)bh);
+    hipLaunchKernelGGL((sdpa_composed_kernel<D, PARTS, KS, KV16>), grid, dim3(256), lds, st, p);
     return hipGetLastError();
+}
+
+template <int D>
+hipError_t launch_d(const ComposedParams& p, int parts, bool kv16, int ks, size_t bh, hipStream_t st) {
+    if (parts == 3) {
+        if (ks == 1) return launch_as<D, 3, 1, false>(p, bh, st);
+        return launch_as<D, 3, 2, false>(p, bh, st);
+    }
+    if (kv16) {
+        if (ks == 1) return launch_as<D, 1, 1, true>(p, bh, st);
+        if (ks == 2) return launch_as<D, 1, 2, true>(p, bh, st);
+        return launch_as<D, 1, 4, true>(p, bh, st);
+    }
+    if (ks == 1) return launch_as<D, 1, 1, false>(p, bh, st);
+    if (ks == 2) return launch_as<D, 1, 2, false>(p, bh, st);
+    return launch_as<D, 1, 4, false>(p, bh, st);
 }
 
 }  // namespace
 }  // namespace fv
 
-// 1 = launched, 0 = this head dim / alignment is the scalar kernel's, < 0 = -(hipError_t)
-extern "C" int fv_internal_launch_composed_mfma(const float* q, const float* k, const float* v, const float* mask,
-                                                long mask_bh_stride, float* out, size_t bh, int sq, int sk, int d,
-                                                float scale, hipStream_t st) {
-    if ((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) != 0) return 0;
-    if (sk > INT_MAX - 2 * fv::kCK || sq > INT_MAX - fv::kCQ) return 0;   // tile indices stay in int range
-    hipError_t e;
-    switch (d) {
-        case 32: e = fv::launch_composed<32>(q, k, v, mask, mask_bh_stride, out, bh, sq, sk, scale, st); break;
-        case 64: e = fv::launch_composed<64>(q, k, v, mask, mask_bh_stride, out, bh, sq, sk, scale, st); break;
-        case 96: e = fv::launch_composed<96>(q, k, v, mask, mask_bh_stride, out, bh, sq, sk, scale, st); break;
-        case 128: e = fv::launch_composed<128>(q, k, v, mask, mask_bh_stride, out, bh, sq, sk, scale, st); break;
-        default: return 0;
-    }
-    return e == hipSuccess ? 1 : -(int)e;
+extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* params, int kv_is_bf16, int round16, size_t bh,
+                                                  hipStream_t st) {
+    fv::ComposedParams p = *params;
+    const int d = p.d;
+    if (d < 1 || d > 128 || p.sk > INT_MAX - 256 || p.sq > INT_MAX - 256) return hipErrorInvalidValue;
+    const uintptr_t any = (uintptr_t)p.q | (uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.out;
+    p.vec = (any & 15) == 0 && d % 8 == 0;
+    p.vec_mask = p.mask && ((uintptr_t)p.mask & 15) == 0 && p.sk % 4 == 0;
+    const int parts = kv_is_bf16 || round16 ? 1 : 3;
+    // 1024 groups are one wave on every SIMD of the chip: below that the keys are shared out over a workgroup's waves
+    int ks = 1;
+    const size_t groups = bh * (size_t)((p.sq + 31) / 32);   // 32-query groups
+    if (groups < 1024) ks = 2;
+    if (groups < 512) ks = 4;
+    if (d <= 32) return fv::launch_d<32>(p, parts, kv_is_bf16 != 0, ks, bh, st);
+    if (d <= 64) return fv::launch_d<64>(p, parts, kv_is_bf16 != 0, ks, bh, st);
+    if (d <= 96) return fv::launch_d<96>(p, parts, kv_is_bf16 != 0, ks, bh, st);
+    return fv::launch_d<128>(p, parts, kv_is_bf16 != 0, ks, bh, st);
 }

@@ -34,6 +34,19 @@ struct FlashParams {
     float* part_lse;
 };
 
+struct ComposedParams {
+    const void* q;                // [bh, sq, d]
+    const void* k;                // [bh, sk, d]
+    const void* v;
+    const float* mask;            // additive, [sq, sk] per mask_bh elements, or null
+    long mask_bh;                 // elements between the masks of consecutive (batch, head) planes (0: shared)
+    void* out;                    // [bh, sq, d] f32 or bf16 (RNE)
+    int q_is_bf16, out_is_bf16;
+    int sq, sk, d;
+    float scale;
+    int vec, vec_mask;            // set by the launcher: 16-byte operand rows / mask rows
+};
+
 struct VsaFineParams {
     const uint16_t* qt;           // tile-ordered bf16 [bh, nb*64, 128]
     const uint16_t* kt;
@@ -138,10 +151,11 @@ extern "C" hipError_t fv_internal_launch_tile_scan3(const void* const x[3], int 
 extern "C" hipError_t fv_internal_launch_tile_qkv(const void* x, int x_is_bf16, const int* slot_src,
                                                   uint16_t* xt, size_t bh, size_t seq, size_t padded,
                                                   int dim, hipStream_t st);
-// 1 = launched, 0 = not this kernel's head dim / alignment, < 0 = -(hipError_t)
-extern "C" int fv_internal_launch_composed_mfma(const float* q, const float* k, const float* v, const float* mask,
-                                                long mask_bh_stride, float* out, size_t bh, int sq, int sk, int d,
-                                                float scale, hipStream_t st);
+// softmax(scale q k^T + mask) v in f32 arithmetic, head dims 1 .. 128 (composed_fwd.hip). kv_is_bf16: k and v are bf16
+// bits (else f32); round16: operands that arrive as f32 are rounded to bf16 first (RNE). A bf16 q with f32 k / v needs
+// round16 == 0 to be exact; an f32 q with bf16 k / v is rounded.
+extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* p, int kv_is_bf16, int round16, size_t bh,
+                                                  hipStream_t st);
 extern "C" hipError_t fv_internal_launch_splitkv_merge(const float* part_o, const float* part_lse, void* out,
                                                        int out_is_bf16, size_t rows, int d, int splits,
                                                        hipStream_t st);

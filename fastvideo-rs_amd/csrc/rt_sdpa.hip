@@ -22,8 +22,8 @@
 
 // ---- composed SDPA on the device (rt/sdpa.rs:328-342) ----------------------------------
 // softmax(scale * q k^T + mask) v in f32, one workgroup per query row, online
-// softmax over chunks of 256 keys: the scalar form, for the head dims the f32 matrix-core kernel
-// (composed_fwd.hip: 32 / 64 / 96 / 128) does not take.
+// softmax over chunks of 256 keys: the scalar form, for the head dims the matrix-core kernel
+// (composed_fwd.hip: up to 128) does not take.
 namespace fv {
 
 constexpr int kCompThreads = 256;
@@ -99,17 +99,18 @@ extern "C" int fv_sdpa_composed_f32(const float* q, const float* k, const float*
     if (!q || !k || !v || !out) return fv_invalid("sdpa_composed: null operand");
     if (bh == 0 || sq == 0) return FV_OK;
     if (sk == 0) return fv_invalid("sdpa_composed: no keys");
-    if (d == 0 || d > 256 || bh > 65535 || sq > (size_t)INT_MAX || sk > (size_t)INT_MAX)
+    if (d == 0 || d > 256 || bh > 65535 || sq > (size_t)INT_MAX - 256 || sk > (size_t)INT_MAX - 256)
         return fv_decline("sdpa_composed: needs 1 <= d <= 256, bh <= 65535, lengths < 2^31");
-    // head dims 32 / 64 / 96 / 128: the f32 matrix-core kernel (composed_fwd.hip)
-    const int rc = fv_internal_launch_composed_mfma(q, k, v, mask, mask_per_bh ? (long)(sq * sk) : 0L, out, bh, (int)sq,
-                                                    (int)sk, (int)d, scale, (hipStream_t)stream);
-    if (rc < 0) return fv_fail_hip((hipError_t)(-rc), "sdpa_composed_mfma_f32");
-    if (rc == 1) return FV_OK;
+    const long mask_bh = mask && mask_per_bh ? (long)(sq * sk) : 0L;
+    hipError_t e;
+    if (d <= 128) {
+        fv::ComposedParams p{q, k, v, mask, mask_bh, out, 0, 0, (int)sq, (int)sk, (int)d, scale, 0, 0};
+        e = fv_internal_launch_composed(&p, 0, 0, bh, (hipStream_t)stream);
+        return e == hipSuccess ? FV_OK : fv_fail_hip(e, "sdpa_composed");
+    }
     hipLaunchKernelGGL(fv::sdpa_composed_f32_kernel, dim3((unsigned)sq, (unsigned)bh), dim3(fv::kCompThreads), 0,
-                       (hipStream_t)stream, q, k, v, mask, mask_per_bh ? (long)(sq * sk) : 0L, out, (int)sq,
-                       (int)sk, (int)d, scale);
-    hipError_t e = hipGetLastError();
+                       (hipStream_t)stream, q, k, v, mask, mask_bh, out, (int)sq, (int)sk, (int)d, scale);
+    e = hipGetLastError();
     return e == hipSuccess ? FV_OK : fv_fail_hip(e, "sdpa_composed_f32");
 }
 
@@ -306,6 +307,87 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
     return std::optional<Tensor>{std::move(out)};
 }
 
+// softmax(scale q k^T + mask) v in f32 arithmetic (rt/sdpa.rs:328-342). act16: on the operands rounded to bf16, the
+// result rounded to bf16 (rt/sdpa.rs:184-214); the kernel does both roundings itself. Else on the operands as they
+// are (bf16 ones widened exactly), the result f32.
+Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::optional<float> scale,
+                        const Tensor* mask, bool act16, hipStream_t st) {
+    if (q.rank() != 4 || k.rank() != 4 || v.rank() != 4) return msg("sdpa expects BHSD");
+    const size_t b = q.shape[0], h = q.shape[1], sq = q.shape[2], d = q.shape[3], sk = k.shape[2], bh = b * h;
+    // rt/tensor.rs:1655-1667: the matmuls need matching batch and inner dims
+    if (k.shape[0] != b || k.shape[1] != h || k.shape[3] != d)
+        return msg("matmul inner " + std::to_string(d) + " vs " + std::to_string(k.shape[3]));
+    if (v.shape[0] != b || v.shape[1] != h || v.shape[2] != sk)
+        return msg("matmul inner " + std::to_string(sk) + " vs " + std::to_string(v.shape[2]));
+    if (v.shape[3] != d) return msg("sdpa: value head dim differs from the query head dim");
+    const DType out_type = act16 ? DType::Bf16 : DType::F32;
+    int mask_per_bh = 0;
+    Tensor tm;
+    const Tensor* pm = nullptr;
+    if (mask) {
+        // additive [.., sq, sk], broadcast over batch*heads or one mask per (batch, head)
+        const size_t r = mask->rank();
+        if (r < 2 || mask->shape[r - 2] != sq || mask->shape[r - 1] != sk)
+            return msg("sdpa: mask must be [.., sq, sk]");
+        if (sq == 0) return Tensor::alloc({b, h, 0, d}, out_type, st);   // no query rows: an empty result
+        if (sk == 0) return msg("sdpa: no keys");
+        const size_t lead = mask->numel() / (sq * sk);
+        if (lead == bh && lead != 1) mask_per_bh = 1;
+        else if (lead != 1) return msg("sdpa: mask batch must be 1 or batch*heads");
+        auto rm = as_f32(*mask, tm, st);
+        if (!is_ok(rm)) return std::get<TensorError>(rm);
+        pm = std::get<const Tensor*>(rm);
+    }
+    // One kernel takes q in either type, k and v both f32 or both bf16. Left over: mixed k / v, f32 queries against
+    // bf16 keys that must not be rounded, and head dims past 128, whose scalar kernel is f32 throughout.
+    Tensor tq, tk, tv, rq, rk, rv;
+    const Tensor *pq = &q, *pk = &k, *pv = &v;
+    const bool wide = d > 128;
+    auto round = [&](const Tensor*& x, Tensor& tmp) -> Result<bool> {
+        auto r = as_bf16(*x, tmp, st);
+        if (!is_ok(r)) return std::get<TensorError>(r);
+        x = std::get<const Tensor*>(r);
+        return true;
+    };
+    auto widen = [&](const Tensor*& x, Tensor& tmp) -> Result<bool> {
+        auto r = as_f32(*x, tmp, st);
+        if (!is_ok(r)) return std::get<TensorError>(r);
+        x = std::get<const Tensor*>(r);
+        return true;
+    };
+    if (wide && act16)
+        for (auto [x, tmp] : {std::pair{&pq, &rq}, std::pair{&pk, &rk}, std::pair{&pv, &rv}})
+            if (auto r = round(*x, *tmp); !is_ok(r)) return std::get<TensorError>(r);
+    const bool kv16 = !wide && k.dtype == DType::Bf16 && v.dtype == DType::Bf16 && (act16 || q.dtype == DType::Bf16);
+    if (wide)
+        if (auto r = widen(pq, tq); !is_ok(r)) return std::get<TensorError>(r);
+    if (!kv16)
+        for (auto [x, tmp] : {std::pair{&pk, &tk}, std::pair{&pv, &tv}})
+            if (auto r = widen(*x, *tmp); !is_ok(r)) return std::get<TensorError>(r);
+    auto ro = Tensor::alloc({b, h, sq, d}, wide ? DType::F32 : out_type, st);
+    if (!is_ok(ro)) return ro;
+    Tensor out = std::move(std::get<Tensor>(ro));
+    const float sc = default_scale(scale, d);
+    if (wide || !pq->data || !pk->data || !pv->data || bh == 0 || sq == 0 || sk == 0 || bh > 65535 || d == 0 || sq > (size_t)INT_MAX - 256 ||
+        sk > (size_t)INT_MAX - 256) {   // (what the kernel-level entry refuses, it refuses here, with its message)
+        const int rc = fv_sdpa_composed_f32((const float*)pq->data, (const float*)pk->data, (const float*)pv->data,
+                                            pm ? (const float*)pm->data : nullptr, mask_per_bh, (float*)out.data, bh, sq,
+                                            sk, d, sc, st);
+        if (rc == FV_DECLINED) return msg("sdpa: every kernel of the route declined");
+        if (rc != FV_OK) return TensorError{"sdpa: " + rc_message(rc), -rc};
+    } else {
+        fv::ComposedParams p{pq->data, pk->data, pv->data, pm ? (const float*)pm->data : nullptr,
+                             mask_per_bh ? (long)(sq * sk) : 0L, out.data, pq->dtype == DType::Bf16, act16, (int)sq,
+                             (int)sk, (int)d, sc, 0, 0};
+        const hipError_t e = fv_internal_launch_composed(&p, kv16, act16, bh, st);
+        if (e != hipSuccess) return TensorError{"sdpa: " + rc_message(fv_fail_hip(e, "sdpa_composed")), (int)e};
+    }
+    g_composed++;
+    log_first_use(mask ? "composed f32 (masked)" : "composed f32", b, h, sq, sk, d);
+    if (act16) return quantized(std::move(out), st);
+    return std::move(out);
+}
+
 // rt/sdpa.rs:184-233 `dense` / `run_step` over the collapsed route.
 Result<Tensor> dense(const Tensor& q, const Tensor& k, const Tensor& v, std::optional<float> scale,
                      const Tensor* mask, hipStream_t st) {
@@ -323,24 +405,7 @@ Result<Tensor> dense(const Tensor& q, const Tensor& k, const Tensor& v, std::opt
         if (step == Step::Composed) composed_step = true;
     }
     if (!composed_step) return msg("sdpa: every kernel of the route declined");
-    // Step::Composed on the bf16-rounded operands under bf16 activations
-    Tensor tq, tk, tv;
-    const Tensor *pq = &q, *pk = &k, *pv = &v;
-    if (act16) {
-        auto rq = as_bf16(q, tq, st);
-        if (!is_ok(rq)) return std::get<TensorError>(rq);
-        auto rk = as_bf16(k, tk, st);
-        if (!is_ok(rk)) return std::get<TensorError>(rk);
-        auto rv = as_bf16(v, tv, st);
-        if (!is_ok(rv)) return std::get<TensorError>(rv);
-        pq = std::get<const Tensor*>(rq);
-        pk = std::get<const Tensor*>(rk);
-        pv = std::get<const Tensor*>(rv);
-    }
-    auto out = sdpa_composed(*pq, *pk, *pv, scale, mask, st);
-    if (!is_ok(out)) return out;
-    if (act16) return quantized(std::move(std::get<Tensor>(out)), st);
-    return out;
+    return composed(q, k, v, scale, mask, act16, st);   // under bf16 activations on the bf16-rounded operands
 }
 
 Result<Tensor> upload_mask(const std::vector<float>& host, size_t sq, size_t sk, hipStream_t st) {
@@ -389,24 +454,7 @@ Result<Tensor> vdn_window(const Tensor& q, const Tensor& k, const Tensor& v, std
 // rt/sdpa.rs:300-324
 Result<Tensor> kv_window(const Tensor& q, const Tensor& k, const Tensor& v, bool flash, hipStream_t st) {
     if (flash) return dense(q, k, v, std::nullopt, nullptr, st);
-    const bool act16 = bf16_activations();
-    Tensor tq, tk, tv;
-    const Tensor *pq = &q, *pk = &k, *pv = &v;
-    if (act16) {
-        auto rq = as_bf16(q, tq, st);
-        if (!is_ok(rq)) return std::get<TensorError>(rq);
-        auto rk = as_bf16(k, tk, st);
-        if (!is_ok(rk)) return std::get<TensorError>(rk);
-        auto rv = as_bf16(v, tv, st);
-        if (!is_ok(rv)) return std::get<TensorError>(rv);
-        pq = std::get<const Tensor*>(rq);
-        pk = std::get<const Tensor*>(rk);
-        pv = std::get<const Tensor*>(rv);
-    }
-    auto out = sdpa_composed(*pq, *pk, *pv, std::nullopt, nullptr, st);
-    if (!is_ok(out)) return out;
-    if (act16) return quantized(std::move(std::get<Tensor>(out)), st);
-    return out;
+    return composed(q, k, v, std::nullopt, nullptr, bf16_activations(), st);
 }
 
 }  // namespace
@@ -607,51 +655,7 @@ Stats stats_snapshot() {
 
 Result<Tensor> sdpa_composed(const Tensor& q, const Tensor& k, const Tensor& v, std::optional<float> scale,
                              const Tensor* mask, hipStream_t st) {
-    if (q.rank() != 4 || k.rank() != 4 || v.rank() != 4) return msg("sdpa expects BHSD");
-    const size_t b = q.shape[0], h = q.shape[1], sq = q.shape[2], d = q.shape[3], sk = k.shape[2];
-    // rt/tensor.rs:1655-1667: the matmuls need matching batch and inner dims
-    if (k.shape[0] != b || k.shape[1] != h || k.shape[3] != d)
-        return msg("matmul inner " + std::to_string(d) + " vs " + std::to_string(k.shape[3]));
-    if (v.shape[0] != b || v.shape[1] != h || v.shape[2] != sk)
-        return msg("matmul inner " + std::to_string(sk) + " vs " + std::to_string(v.shape[2]));
-    if (v.shape[3] != d) return msg("sdpa: value head dim differs from the query head dim");
-    int mask_per_bh = 0;
-    Tensor tm;
-    const Tensor* pm = nullptr;
-    if (mask) {
-        // additive [.., sq, sk], broadcast over batch*heads or one mask per (batch, head)
-        const size_t r = mask->rank();
-        if (r < 2 || mask->shape[r - 2] != sq || mask->shape[r - 1] != sk)
-            return msg("sdpa: mask must be [.., sq, sk]");
-        if (sq == 0) return Tensor::alloc({b, h, 0, d}, DType::F32, st);   // no query rows: an empty result
-        if (sk == 0) return msg("sdpa: no keys");
-        const size_t lead = mask->numel() / (sq * sk);
-        if (lead == b * h && lead != 1) mask_per_bh = 1;
-        else if (lead != 1) return msg("sdpa: mask batch must be 1 or batch*heads");
-        auto rm = as_f32(*mask, tm, st);
-        if (!is_ok(rm)) return std::get<TensorError>(rm);
-        pm = std::get<const Tensor*>(rm);
-    }
-    Tensor tq, tk, tv;
-    auto rq = as_f32(q, tq, st);
-    if (!is_ok(rq)) return std::get<TensorError>(rq);
-    auto rk = as_f32(k, tk, st);
-    if (!is_ok(rk)) return std::get<TensorError>(rk);
-    auto rv = as_f32(v, tv, st);
-    if (!is_ok(rv)) return std::get<TensorError>(rv);
-    auto ro = Tensor::alloc({b, h, sq, d}, DType::F32, st);
-    if (!is_ok(ro)) return ro;
-    Tensor out = std::move(std::get<Tensor>(ro));
-    const int rc = fv_sdpa_composed_f32((const float*)std::get<const Tensor*>(rq)->data,
-                                        (const float*)std::get<const Tensor*>(rk)->data,
-                                        (const float*)std::get<const Tensor*>(rv)->data,
-                                        pm ? (const float*)pm->data : nullptr, mask_per_bh, (float*)out.data, b * h,
-                                        sq, sk, d, default_scale(scale, d), st);
-    if (rc == FV_DECLINED) return msg("sdpa: every kernel of the route declined");
-    if (rc != FV_OK) return TensorError{"sdpa: " + rc_message(rc), -rc};
-    g_composed++;
-    log_first_use(mask ? "composed f32 (masked)" : "composed f32", b, h, sq, sk, d);
-    return std::move(out);
+    return composed(q, k, v, scale, mask, false, st);
 }
 
 Result<Tensor> sdpa(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& plan, hipStream_t st) {

@@ -1,0 +1,101 @@
+"""The composed kernel (f32 arithmetic on the bf16 matrix cores) at the edges of its tiles: head dims that are no
+multiple of 32, of 8 or of 4, one row more and less than a query group and a key tile, every split of the keys over a
+workgroup's waves, operands of either type, rows that are not 16-byte units, both kinds of mask, both result types.
+
+Checked against the same sums in 64 bits. Bounds: with f32 arithmetic a weight 2^x carries the rounding of x, |x| at
+most about 16 at these inputs, so up to 16 ln 2 2^-24 = 7e-7 relative, and the sums a few 2^-24 more: 2e-6 in the
+2-norm. A result rounded to bf16 adds 2^-9 at most: 2e-3."""
+import numpy as np
+import pytest
+
+from util import announce
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def fv():
+    import torch
+
+    assert torch.cuda.is_available()
+    import fv_sdpa
+
+    fv_sdpa.lib()
+    return fv_sdpa
+
+
+def want64(q, k, v, mask):
+    q, k, v = (x.double().cpu().numpy() for x in (q, k, v))
+    s = q @ k.swapaxes(-1, -2) / np.sqrt(q.shape[-1])
+    if mask is not None:
+        s = s + mask.double().cpu().numpy()
+    m = s.max(axis=-1, keepdims=True)
+    e = np.exp(s - np.where(np.isfinite(m), m, 0.0))
+    l = e.sum(axis=-1, keepdims=True)
+    return np.where(l > 0, (e / np.where(l > 0, l, 1.0)) @ v, 0.0)
+
+
+SHAPES = [  # bh, sq, sk, d
+    (1, 1, 1, 1), (2, 5, 7, 8), (1, 31, 33, 7), (2, 33, 32, 30), (1, 32, 31, 33), (3, 64, 65, 40), (1, 127, 129, 72),
+    (2, 129, 64, 80), (1, 100, 257, 96), (1, 96, 63, 100), (2, 130, 191, 128), (1, 33, 300, 127),
+    (40, 500, 90, 64),        # 640 query groups: two shares of the keys
+    (70, 500, 70, 128),       # 1120: one
+]
+
+
+@pytest.mark.parametrize("kinds", ["f32", "bf16", "round", "mixed"])
+@pytest.mark.parametrize("bh,sq,sk,d", SHAPES)
+def test_edges(fv, bh, sq, sk, d, kinds):
+    import torch
+
+    announce(f"composed bh={bh} sq={sq} sk={sk} d={d} {kinds}")
+    g = torch.Generator(device="cuda").manual_seed(1000 * sq + sk + d)
+    mk = lambda s: torch.randn((1, bh, s, d), generator=g, device="cuda")
+    q, k, v = mk(sq), mk(sk), mk(sk)
+    act16 = kinds in ("bf16", "round")
+    if kinds == "bf16":
+        q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    elif kinds == "mixed":                        # f32 queries against bf16 keys: nothing may be rounded
+        k, v = k.to(torch.bfloat16), v.to(torch.bfloat16)
+    shared = torch.randn((1, 1, sq, sk), generator=g, device="cuda")
+    shared[..., ::3] = -1e9
+    per_head = torch.randn((1, bh, sq, sk), generator=g, device="cuda")
+    per_head[:, :, 0, :] = float("-inf")          # a row without a key: zeros
+    for mask in (None, shared, per_head):
+        with fv.with_bf16_act(act16):
+            if kinds == "bf16" or act16:
+                plan = fv.Plan.masked(None, mask) if mask is not None else fv.Plan.kv_window_with(False)
+            else:
+                plan = fv.Plan.composed(None, mask)
+            out = fv.sdpa(q, k, v, plan)
+        torch.cuda.synchronize()
+        assert out.dtype == (torch.bfloat16 if act16 else torch.float32) and tuple(out.shape) == (1, bh, sq, d)
+        qq, kk, vv = (x.to(torch.bfloat16) for x in (q, k, v)) if act16 else (q, k, v)
+        want = want64(qq, kk, vv, mask)
+        got = out.double().cpu().numpy()
+        assert np.isfinite(got).all()
+        if mask is per_head and bh > 1:
+            assert not got[:, :, 0].any()
+        norm = np.linalg.norm(want)
+        assert np.linalg.norm(got - want) <= (2e-3 if act16 else 2e-6) * norm + 1e-30, np.linalg.norm(got - want) / norm
+
+
+def test_unaligned_operands(fv):
+    """Pointers that are not 16-byte aligned take element loads and stores."""
+    import torch
+
+    bh, sq, sk, d = 2, 70, 90, 64
+    announce("composed unaligned")
+    g = torch.Generator(device="cuda").manual_seed(7)
+    lib = fv.lib()
+    mk = lambda n: torch.randn(n + 1, generator=g, device="cuda")[1:]
+    q, k, v = mk(bh * sq * d), mk(bh * sk * d), mk(bh * sk * d)
+    mask, out = mk(sq * sk), torch.full((bh * sq * d + 2,), 7.0, device="cuda")
+    rc = lib.fv_sdpa_composed_f32(q.data_ptr(), k.data_ptr(), v.data_ptr(), mask.data_ptr(), 0, out[1:].data_ptr(), bh, sq,
+                                  sk, d, 0.125, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    want = want64(q.view(bh, sq, d), k.view(bh, sk, d), v.view(bh, sk, d), mask.view(sq, sk))
+    got = out[1:-1].view(bh, sq, d).double().cpu().numpy()
+    assert np.linalg.norm(got - want) <= 2e-6 * np.linalg.norm(want)
+    assert float(out[0]) == 7.0 and float(out[-1]) == 7.0
