@@ -180,9 +180,9 @@ std::string rc_message(int rc) {
 
 // A bf16 view of `x`: `x` itself when it already is bf16, else a rounded copy in `tmp` (of x * mul: the
 // product in f32, one rounding).
-Result<const Tensor*> as_bf16(const Tensor& x, Tensor& tmp, hipStream_t st, float mul = 1.0f) {
+Result<const Tensor*> as_bf16(const Tensor& x, Tensor& tmp, Mem& st, float mul = 1.0f) {
     if (x.dtype == DType::Bf16) return &x;
-    auto r = Tensor::alloc(x.shape, DType::Bf16, st);
+    auto r = st.temp(x.shape, DType::Bf16);
     if (!is_ok(r)) return std::get<TensorError>(r);
     tmp = std::move(std::get<Tensor>(r));
     const int rc = fv_cast_f32_bf16_scaled((const float*)x.data, (uint16_t*)tmp.data, x.numel(), mul, st);
@@ -191,9 +191,9 @@ Result<const Tensor*> as_bf16(const Tensor& x, Tensor& tmp, hipStream_t st, floa
     return &tmp;
 }
 
-Result<const Tensor*> as_f32(const Tensor& x, Tensor& tmp, hipStream_t st) {
+Result<const Tensor*> as_f32(const Tensor& x, Tensor& tmp, Mem& st) {
     if (x.dtype == DType::F32) return &x;
-    auto r = Tensor::alloc(x.shape, DType::F32, st);
+    auto r = st.temp(x.shape, DType::F32);
     if (!is_ok(r)) return std::get<TensorError>(r);
     tmp = std::move(std::get<Tensor>(r));
     const int rc = fv_cast_bf16_f32((const uint16_t*)x.data, (float*)tmp.data, x.numel(), st);
@@ -203,12 +203,14 @@ Result<const Tensor*> as_f32(const Tensor& x, Tensor& tmp, hipStream_t st) {
 }
 
 // rt/tensor.rs:428-443 `quantize_bf16` on a result.
-Result<Tensor> quantized(Tensor&& x, hipStream_t st) {
+Result<Tensor> quantized(Tensor&& x, Mem& st) {
     if (x.dtype == DType::Bf16) return std::move(x);
-    Tensor tmp;
-    auto r = as_bf16(x, tmp, st);
-    if (!is_ok(r)) return std::get<TensorError>(r);
-    return std::move(tmp);
+    auto r = st.result(x.shape, DType::Bf16);
+    if (!is_ok(r)) return r;
+    const int rc = fv_cast_f32_bf16((const float*)x.data, (uint16_t*)std::get<Tensor>(r).data, x.numel(), st);
+    if (rc != FV_OK) return TensorError{"cast_f32_bf16: " + rc_message(rc), rc < 0 ? -rc : 0};
+    g_cast++;
+    return r;
 }
 
 struct Bhsd {
@@ -228,8 +230,8 @@ float default_scale(std::optional<float> scale, size_t d) {
 }
 
 // A contiguous copy of a row window (what the reference's `narrow` always makes).
-Result<Tensor> compact(const Tensor& x, hipStream_t st) {
-    auto r = Tensor::alloc(x.shape, x.dtype, st);
+Result<Tensor> compact(const Tensor& x, Mem& st) {
+    auto r = st.temp(x.shape, x.dtype);
     if (!is_ok(r)) return r;
     Tensor t = std::move(std::get<Tensor>(r));
     const size_t row = x.shape[3] * elem_size(x.dtype), planes = x.shape[0] * x.shape[1];
@@ -245,7 +247,7 @@ Result<Tensor> compact(const Tensor& x, hipStream_t st) {
 // One fused launch (dense, block-causal or VDN window); nullopt = the kernel declined.
 Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tensor& v,
                                     std::optional<float> scale, bool out_bf16,
-                                    const BlockCausal* causal, hipStream_t st,
+                                    const BlockCausal* causal, Mem& st,
                                     const VdnWindow* window = nullptr) {
     const auto s = bhsd(q, k, v);
     if (!s || !fv_sdpa_supported(s->b, s->h, s->sq, s->sk, s->d)) return std::optional<Tensor>{};
@@ -268,7 +270,7 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
     if (!is_ok(rk)) return std::get<TensorError>(rk);
     auto rv = as_bf16(v, tv, st);
     if (!is_ok(rv)) return std::get<TensorError>(rv);
-    auto ro = Tensor::alloc({s->b, s->h, s->sq, s->d}, out_bf16 ? DType::Bf16 : DType::F32, st);
+    auto ro = st.result({s->b, s->h, s->sq, s->d}, out_bf16 ? DType::Bf16 : DType::F32);
     if (!is_ok(ro)) return std::get<TensorError>(ro);
     Tensor out = std::move(std::get<Tensor>(ro));
     const auto* pq = (const uint16_t*)std::get<const Tensor*>(rq)->data;
@@ -287,7 +289,7 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
         const size_t splits = fv_sdpa_splitkv_choose(s->b * s->h, s->sq, s->sk);
         Tensor ws;
         if (splits > 1) {
-            auto rw = Tensor::alloc({fv_sdpa_splitkv_workspace_bytes(s->b * s->h, s->sq, s->d, splits) / 4}, DType::F32, st);
+            auto rw = st.temp({fv_sdpa_splitkv_workspace_bytes(s->b * s->h, s->sq, s->d, splits) / 4}, DType::F32);
             if (!is_ok(rw)) return std::get<TensorError>(rw);
             ws = std::move(std::get<Tensor>(rw));
             rc = fv_sdpa_dense_bf16_splitkv(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc,
@@ -311,7 +313,7 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
 // result rounded to bf16 (rt/sdpa.rs:184-214); the kernel does both roundings itself. Else on the operands as they
 // are (bf16 ones widened exactly), the result f32.
 Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::optional<float> scale,
-                        const Tensor* mask, bool act16, hipStream_t st) {
+                        const Tensor* mask, bool act16, Mem& st) {
     if (q.rank() != 4 || k.rank() != 4 || v.rank() != 4) return msg("sdpa expects BHSD");
     const size_t b = q.shape[0], h = q.shape[1], sq = q.shape[2], d = q.shape[3], sk = k.shape[2], bh = b * h;
     // rt/tensor.rs:1655-1667: the matmuls need matching batch and inner dims
@@ -329,7 +331,7 @@ Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::
         const size_t r = mask->rank();
         if (r < 2 || mask->shape[r - 2] != sq || mask->shape[r - 1] != sk)
             return msg("sdpa: mask must be [.., sq, sk]");
-        if (sq == 0) return Tensor::alloc({b, h, 0, d}, out_type, st);   // no query rows: an empty result
+        if (sq == 0) return st.result({b, h, 0, d}, out_type);   // no query rows: an empty result
         if (sk == 0) return msg("sdpa: no keys");
         const size_t lead = mask->numel() / (sq * sk);
         if (lead == bh && lead != 1) mask_per_bh = 1;
@@ -364,7 +366,7 @@ Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::
     if (!kv16)
         for (auto [x, tmp] : {std::pair{&pk, &tk}, std::pair{&pv, &tv}})
             if (auto r = widen(*x, *tmp); !is_ok(r)) return std::get<TensorError>(r);
-    auto ro = Tensor::alloc({b, h, sq, d}, wide ? DType::F32 : out_type, st);
+    auto ro = wide && act16 ? st.temp({b, h, sq, d}, DType::F32) : st.result({b, h, sq, d}, out_type);
     if (!is_ok(ro)) return ro;
     Tensor out = std::move(std::get<Tensor>(ro));
     const float sc = default_scale(scale, d);
@@ -390,7 +392,7 @@ Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::
 
 // rt/sdpa.rs:184-233 `dense` / `run_step` over the collapsed route.
 Result<Tensor> dense(const Tensor& q, const Tensor& k, const Tensor& v, std::optional<float> scale,
-                     const Tensor* mask, hipStream_t st) {
+                     const Tensor* mask, Mem& st) {
     const bool act16 = bf16_activations();
     const Backend be = backend();
     bool composed_step = false;
@@ -408,8 +410,8 @@ Result<Tensor> dense(const Tensor& q, const Tensor& k, const Tensor& v, std::opt
     return composed(q, k, v, scale, mask, act16, st);   // under bf16 activations on the bf16-rounded operands
 }
 
-Result<Tensor> upload_mask(const std::vector<float>& host, size_t sq, size_t sk, hipStream_t st) {
-    auto r = Tensor::alloc({1, 1, sq, sk}, DType::F32, st);
+Result<Tensor> upload_mask(const std::vector<float>& host, size_t sq, size_t sk, Mem& st) {
+    auto r = st.temp({1, 1, sq, sk}, DType::F32);
     if (!is_ok(r)) return r;
     Tensor t = std::move(std::get<Tensor>(r));
     hipError_t e = hipMemcpyAsync(t.data, host.data(), host.size() * 4, hipMemcpyHostToDevice, st);
@@ -421,7 +423,7 @@ Result<Tensor> upload_mask(const std::vector<float>& host, size_t sq, size_t sk,
 
 // rt/sdpa.rs:248-269
 Result<Tensor> block_causal(const Tensor& q, const Tensor& k, const Tensor& v, std::optional<float> scale,
-                            BlockCausal mask, hipStream_t st) {
+                            BlockCausal mask, Mem& st) {
     const size_t sq = q.shape[2], sk = k.shape[2];
     if (causal_flash_enabled()) {
         auto r = fused(q, k, v, scale, bf16_activations(), &mask, st);
@@ -436,7 +438,7 @@ Result<Tensor> block_causal(const Tensor& q, const Tensor& k, const Tensor& v, s
 
 // rt/sdpa.rs:271-298
 Result<Tensor> vdn_window(const Tensor& q, const Tensor& k, const Tensor& v, std::optional<float> scale,
-                          VdnWindow mask, hipStream_t st) {
+                          VdnWindow mask, Mem& st) {
     const size_t sq = q.shape[2], sk = k.shape[2];
     auto r = fused(q, k, v, scale, bf16_activations(), nullptr, st, &mask);
     if (!is_ok(r)) return std::get<TensorError>(r);
@@ -452,7 +454,7 @@ Result<Tensor> vdn_window(const Tensor& q, const Tensor& k, const Tensor& v, std
 }
 
 // rt/sdpa.rs:300-324
-Result<Tensor> kv_window(const Tensor& q, const Tensor& k, const Tensor& v, bool flash, hipStream_t st) {
+Result<Tensor> kv_window(const Tensor& q, const Tensor& k, const Tensor& v, bool flash, Mem& st) {
     if (flash) return dense(q, k, v, std::nullopt, nullptr, st);
     return composed(q, k, v, std::nullopt, nullptr, bf16_activations(), st);
 }
@@ -504,6 +506,23 @@ Result<Tensor> Tensor::alloc(std::vector<size_t> shape, DType dtype, hipStream_t
     t.owned_ = true;
     t.stream_ = stream;
     return std::move(t);
+}
+Result<Tensor> Mem::temp(std::vector<size_t> shape, DType dtype) {
+    size_t n = elem_size(dtype);
+    for (size_t x : shape) n *= x;
+    const size_t need = (n + 255) & ~(size_t)255;
+    if (n == 0 || need > left_) return Tensor::alloc(std::move(shape), dtype, stream);
+    void* at = ws_;
+    ws_ += need;
+    left_ -= need;
+    return Tensor::borrowed(at, std::move(shape), dtype);
+}
+Result<Tensor> Mem::result(std::vector<size_t> shape, DType dtype) {
+    if (!out_) return Tensor::alloc(std::move(shape), dtype, stream);
+    size_t n = elem_size(dtype);
+    for (size_t x : shape) n *= x;
+    if (n != out_bytes_) return msg("sdpa: the result buffer holds " + std::to_string(out_bytes_) + " bytes, the result " + std::to_string(n));
+    return Tensor::borrowed(out_, std::move(shape), dtype);
 }
 size_t Tensor::numel() const {
     size_t n = 1;
@@ -654,11 +673,27 @@ Stats stats_snapshot() {
 // ---- entry points ----------------------------------------------------------------------------
 
 Result<Tensor> sdpa_composed(const Tensor& q, const Tensor& k, const Tensor& v, std::optional<float> scale,
-                             const Tensor* mask, hipStream_t st) {
-    return composed(q, k, v, scale, mask, false, st);
+                             const Tensor* mask, Mem mem) {
+    return composed(q, k, v, scale, mask, false, mem);
 }
 
-Result<Tensor> sdpa(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& plan, hipStream_t st) {
+Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& plan) {
+    Need n;
+    const bool act16 = bf16_activations();
+    n.out = plan.kind != Plan::Kind::Composed && act16 ? DType::Bf16 : DType::F32;
+    const auto s = bhsd(q, k, v);
+    const bool masked = plan.kind == Plan::Kind::Dense && plan.mask;
+    if (!s || plan.kind == Plan::Kind::Composed || masked || !fv_sdpa_supported(s->b, s->h, s->sq, s->sk, s->d)) return n;
+    for (const Tensor* t : {&q, &k, &v})
+        if (t->dtype == DType::F32) n.workspace += (t->numel() * 2 + 255) & ~(size_t)255;
+    if (plan.kind == Plan::Kind::Dense || plan.kind == Plan::Kind::KvWindow) {
+        const size_t splits = fv_sdpa_splitkv_choose(s->b * s->h, s->sq, s->sk);
+        if (splits > 1) n.workspace += (fv_sdpa_splitkv_workspace_bytes(s->b * s->h, s->sq, s->d, splits) + 255) & ~(size_t)255;
+    }
+    return n;
+}
+
+Result<Tensor> sdpa(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& plan, Mem st) {
     if (q.rank() != 4 || k.rank() != 4 || v.rank() != 4) return msg("sdpa expects BHSD");
     if (q.strided() || k.strided() || v.strided()) {
         // Row windows of longer planes (a KV cache read in place). The fused dense kernel takes bf16
@@ -705,50 +740,63 @@ Result<Tensor> sdpa(const Tensor& q, const Tensor& k, const Tensor& v, const Pla
 
 extern "C" {
 
+namespace {
+// One call's operands and plan, unflattened.
+struct FlatCall {
+    fv::rt::Tensor q, k, v, mask;
+    fv::rt::Plan plan;
+    int open(const fv_tensor* fq, const fv_tensor* fk, const fv_tensor* fv_, const fv_plan* p) {
+        using namespace fv::rt;
+        if (!fq || !fk || !fv_ || !p) return fv_invalid("fv_rt_sdpa: null argument");
+        auto wrap = [](const fv_tensor* t) {
+            std::vector<size_t> shape(t->shape, t->shape + (t->rank < 0 ? 0 : (t->rank > 8 ? 8 : t->rank)));
+            return Tensor::window(t->data, std::move(shape), t->dtype ? DType::Bf16 : DType::F32, t->plane_rows);
+        };
+        for (const fv_tensor* t : {fq, fk, fv_})
+            if (t->plane_rows != 0 && (t->rank != 4 || t->plane_rows < t->shape[2]))
+                return fv_invalid("fv_rt_sdpa: plane_rows needs a rank-4 operand and plane_rows >= shape[2]");
+        q = wrap(fq), k = wrap(fk), v = wrap(fv_);
+        if (p->mask) mask = wrap(p->mask);
+        const Tensor* pm = p->mask ? &mask : nullptr;
+        const std::optional<float> scale = p->has_scale ? std::optional<float>(p->scale) : std::nullopt;
+        switch (p->kind) {
+            case FV_PLAN_DENSE:
+                plan = Plan::masked(scale, pm);
+                if (p->fp8_first) plan = plan.fp8_first();
+                break;
+            case FV_PLAN_COMPOSED:
+                plan = Plan::composed(scale, pm);
+                break;
+            case FV_PLAN_BLOCK_CAUSAL:
+                plan = Plan::block_causal(scale, BlockCausal{p->block_tokens, p->window, p->sink});
+                break;
+            case FV_PLAN_VDN_WINDOW:
+                plan = Plan::vdn_window(scale, VdnWindow{p->video_start, p->frame_tokens, p->frames, p->chunk, p->radius});
+                break;
+            case FV_PLAN_KV_WINDOW:
+                plan = p->kv_flash < 0 ? Plan::kv_window() : Plan::kv_window_with(p->kv_flash != 0);
+                break;
+            default:
+                return fv_invalid("fv_rt_sdpa: unknown plan kind");
+        }
+        return FV_OK;
+    }
+};
+// a refused argument is -hipErrorInvalidValue; an allocation or launch failure keeps its own code
+int flat_error(const fv::rt::TensorError& err) {
+    const int rc = fv_invalid(err.message.c_str());
+    return err.hip_code > 0 ? -err.hip_code : rc;
+}
+}  // namespace
+
 int fv_rt_sdpa(const fv_tensor* q, const fv_tensor* k, const fv_tensor* v, const fv_plan* plan, fv_tensor* out,
                void* stream) {
     using namespace fv::rt;
-    if (!q || !k || !v || !plan || !out) return fv_invalid("fv_rt_sdpa: null argument");
-    auto wrap = [](const fv_tensor* t) {
-        std::vector<size_t> shape(t->shape, t->shape + (t->rank < 0 ? 0 : (t->rank > 8 ? 8 : t->rank)));
-        return Tensor::window(t->data, std::move(shape), t->dtype ? DType::Bf16 : DType::F32, t->plane_rows);
-    };
-    for (const fv_tensor* t : {q, k, v})
-        if (t->plane_rows != 0 && (t->rank != 4 || t->plane_rows < t->shape[2]))
-            return fv_invalid("fv_rt_sdpa: plane_rows needs a rank-4 operand and plane_rows >= shape[2]");
-    const Tensor tq = wrap(q), tk = wrap(k), tv = wrap(v);
-    Tensor tmask;
-    if (plan->mask) tmask = wrap(plan->mask);
-    const std::optional<float> scale = plan->has_scale ? std::optional<float>(plan->scale) : std::nullopt;
-    Plan p;
-    switch (plan->kind) {
-        case FV_PLAN_DENSE:
-            p = Plan::masked(scale, plan->mask ? &tmask : nullptr);
-            if (plan->fp8_first) p = p.fp8_first();
-            break;
-        case FV_PLAN_COMPOSED:
-            p = Plan::composed(scale, plan->mask ? &tmask : nullptr);
-            break;
-        case FV_PLAN_BLOCK_CAUSAL:
-            p = Plan::block_causal(scale, BlockCausal{plan->block_tokens, plan->window, plan->sink});
-            break;
-        case FV_PLAN_VDN_WINDOW:
-            p = Plan::vdn_window(scale, VdnWindow{plan->video_start, plan->frame_tokens, plan->frames, plan->chunk,
-                                                  plan->radius});
-            break;
-        case FV_PLAN_KV_WINDOW:
-            p = plan->kv_flash < 0 ? Plan::kv_window() : Plan::kv_window_with(plan->kv_flash != 0);
-            break;
-        default:
-            return fv_invalid("fv_rt_sdpa: unknown plan kind");
-    }
-    auto r = sdpa(tq, tk, tv, p, (hipStream_t)stream);
-    if (!is_ok(r)) {
-        // a refused argument is -hipErrorInvalidValue; an allocation or launch failure keeps its own code
-        const TensorError& err = std::get<TensorError>(r);
-        const int rc = fv_invalid(err.message.c_str());
-        return err.hip_code > 0 ? -err.hip_code : rc;
-    }
+    if (!out) return fv_invalid("fv_rt_sdpa: null argument");
+    FlatCall c;
+    if (const int rc = c.open(q, k, v, plan); rc != FV_OK) return rc;
+    auto r = sdpa(c.q, c.k, c.v, c.plan, Mem((hipStream_t)stream));
+    if (!is_ok(r)) return flat_error(std::get<TensorError>(r));
     Tensor& t = std::get<Tensor>(r);
     out->rank = (int)t.rank();
     for (size_t i = 0; i < t.rank() && i < 8; i++) out->shape[i] = t.shape[i];
@@ -756,6 +804,31 @@ int fv_rt_sdpa(const fv_tensor* q, const fv_tensor* k, const fv_tensor* v, const
     out->plane_rows = 0;
     out->data = t.release();
     return FV_OK;
+}
+
+int fv_rt_sdpa_need(const fv_tensor* q, const fv_tensor* k, const fv_tensor* v, const fv_plan* plan, size_t need_out[2]) {
+    using namespace fv::rt;
+    if (!need_out) return fv_invalid("fv_rt_sdpa: null argument");
+    FlatCall c;
+    if (const int rc = c.open(q, k, v, plan); rc != FV_OK) return rc;
+    const Need n = sdpa_need(c.q, c.k, c.v, c.plan);
+    need_out[0] = n.out == DType::Bf16 ? 1 : 0;
+    need_out[1] = n.workspace;
+    return FV_OK;
+}
+
+int fv_rt_sdpa_into(const fv_tensor* q, const fv_tensor* k, const fv_tensor* v, const fv_plan* plan, void* out,
+                    size_t out_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace fv::rt;
+    if (!out && out_bytes) return fv_invalid("fv_rt_sdpa: null argument");
+    if (workspace_bytes && (!workspace || ((uintptr_t)workspace & 255) != 0))
+        return fv_invalid("fv_rt_sdpa_into: the workspace must be 256-byte aligned");
+    FlatCall c;
+    if (const int rc = c.open(q, k, v, plan); rc != FV_OK) return rc;
+    // (an empty result is written nowhere, but its buffer must still be the caller's)
+    static char nothing;
+    auto r = sdpa(c.q, c.k, c.v, c.plan, Mem((hipStream_t)stream, out ? out : &nothing, out_bytes, workspace, workspace_bytes));
+    return is_ok(r) ? FV_OK : flat_error(std::get<TensorError>(r));
 }
 
 int fv_rt_free(void* p, void* stream) {

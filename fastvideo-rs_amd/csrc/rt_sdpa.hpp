@@ -66,6 +66,28 @@ class Tensor {
     hipStream_t stream_ = nullptr;
 };
 
+// Where one call's device memory comes from, and the stream it runs on. By itself: stream-ordered allocations. A
+// caller that has buffers in hand gives them: `out` for the result (of exactly that many bytes) and a workspace for the
+// rounded copies of f32 operands and the split-KV partials; what does not fit is allocated as before. (A stream-ordered
+// allocation of a result costs more than it looks: the pool gives its memory back whenever the device is waited for,
+// and mapping 100 MB anew takes 0.3 ms of host time.)
+class Mem {
+  public:
+    Mem(hipStream_t s) : stream(s) {}   // (implicit: a stream alone is a Mem)
+    Mem(hipStream_t s, void* result, size_t result_bytes, void* workspace, size_t workspace_bytes)
+        : stream(s), out_(result), out_bytes_(result_bytes), ws_((char*)workspace), left_(workspace_bytes) {}
+    operator hipStream_t() const { return stream; }
+    Result<Tensor> temp(std::vector<size_t> shape, DType dtype);
+    Result<Tensor> result(std::vector<size_t> shape, DType dtype);
+    hipStream_t stream;
+
+  private:
+    void* out_ = nullptr;
+    size_t out_bytes_ = 0;
+    char* ws_ = nullptr;
+    size_t left_ = 0;
+};
+
 // rt/attn.rs:441-467
 struct BlockCausal {
     size_t block_tokens = 0, window = 0, sink = 0;
@@ -140,13 +162,20 @@ enum class Step : int { Retired = 0, Fused = 1, Composed = 2 };
 std::vector<Step> dense_route(const Shape& shape, bool masked, Backend backend);
 
 // rt/sdpa.rs:141-164. Work is enqueued on `stream`; the result owns its buffer.
-Result<Tensor> sdpa(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& plan,
-                    hipStream_t stream);
+Result<Tensor> sdpa(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& plan, Mem mem);
+
+// What `sdpa` will need for these operands and this plan: the result's type and the bytes of workspace that keep the
+// ordinary routes from allocating (host arithmetic).
+struct Need {
+    DType out = DType::F32;
+    size_t workspace = 0;
+};
+Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& plan);
 
 // rt/sdpa.rs:328-342 on the device: softmax(scale q k^T + mask) v in f32 from the
 // operands as given (bf16 operands are widened exactly).
 Result<Tensor> sdpa_composed(const Tensor& q, const Tensor& k, const Tensor& v,
-                             std::optional<float> scale, const Tensor* mask, hipStream_t stream);
+                             std::optional<float> scale, const Tensor* mask, Mem mem);
 
 // Launch counters (rt/stats.rs:27-72 keeps h2d/d2h/launch/fallback counts).
 struct Stats {

@@ -63,6 +63,8 @@ SIGNATURES = {
     "fv_sdpa_init": (C.c_int, []),
     "fv_rt_sdpa": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp]),
     "fv_rt_free": (C.c_int, [_vp, _vp]),
+    "fv_rt_sdpa_need": (C.c_int, [_vp, _vp, _vp, _vp, _vp]),
+    "fv_rt_sdpa_into": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _sz, _vp, _sz, _vp]),
     "fv_rt_set_bf16_activations": (None, [C.c_int]),
     "fv_rt_bf16_activations": (C.c_int, []),
     "fv_rt_set_fold_scale": (None, [C.c_int]),
@@ -141,6 +143,14 @@ def lib():
             fn.argtypes = args
         _lib = l
     return _lib
+
+
+def stream():
+    """The current torch stream of the current device as a hipStream_t (without the Stream object around it, whose
+    construction costs several times this call)."""
+    import torch
+
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def last_error():

@@ -9,7 +9,7 @@ import ctypes as C
 import torch
 
 from . import _lib
-from .sdpa import TensorError, _desc, _FvTensor
+from .sdpa import TensorError, _desc_bytes, _FvTensor
 
 __all__ = ["KvSpec", "KvMove", "KvBlockKey", "KvRope", "CausalKvCache", "kv_copy_tokens", "kv_shift_tokens_down", "rope_bhsd"]
 
@@ -90,6 +90,20 @@ class _DevView:
             "strides": (h * plane_rows * d * esz, plane_rows * d * esz, d * esz, esz)}
 
 
+class _Handle:
+    """Owns the library's cache: freed when neither the CausalKvCache nor any window of its buffers is left."""
+
+    def __init__(self, ptr):
+        self.ptr = ptr
+
+    def __del__(self):
+        try:
+            torch.cuda.synchronize()
+            _lib.lib().fv_kv_cache_free(self.ptr)
+        except Exception:
+            pass
+
+
 class CausalKvCache:
     """wan/causal.rs:341-723. static (`new_static`, the default here): persistent [b, h, capacity, d]
     buffers per layer, written in place; static=False (`new`): every write builds the layer's K / V anew."""
@@ -102,33 +116,38 @@ class CausalKvCache:
                                              int(spec.rolling), spec.rope, num_layers)
         if not self._h:
             raise TensorError("causal kv: could not create the cache")
+        self._owner = _Handle(self._h)
+        # (layer, 0 = K / 1 = V) -> the layer's whole persistent buffer as a tensor: a window of it is one as_strided,
+        # where importing a pointer takes ten times as long. A static cache's buffers never move; a cache that builds
+        # its tensors anew keeps none here.
+        self._buffers = {}
+        self._static = static
 
-    def __del__(self):
-        h, self._h = getattr(self, "_h", None), None
-        if h:
-            try:
-                torch.cuda.synchronize()
-                _lib.lib().fv_kv_cache_free(h)
-            except Exception:
-                pass
+    def _window(self, layer, which, t, device):
+        b, h, n, d = (int(t.shape[i]) for i in range(4))
+        rows, bf16 = int(t.plane_rows) or n, bool(t.dtype)
+        row_bytes = d * (2 if bf16 else 4)
+        base = self._buffers.get((layer, which))
+        if base is None:
+            start = self.pointers(layer)[1] - n if self._static else 0    # the window ends at the layer's last token
+            view = _DevView(t.data - start * row_bytes, (b, h, rows if self._static else n, d), rows, bf16, self._owner)
+            base = torch.as_tensor(view, device=device)
+            base = base.view(torch.bfloat16) if bf16 else base
+            if not self._static:
+                return base
+            self._buffers[layer, which] = base
+        start = (t.data - base.data_ptr()) // row_bytes
+        return base.as_strided((b, h, n, d), (h * rows * d, rows * d, d, 1), start * d)
 
     def update(self, layer, k, v, current_start):
         """Writes the block's k / v [b, h, n, d]; returns the (K, V) windows its queries read."""
         lib = _lib.lib()
-        dk, dv = _desc(k, "k"), _desc(v, "v")
+        dk, dv = _desc_bytes(k, "k"), _desc_bytes(v, "v")
         kw, vw = _FvTensor(), _FvTensor()
-        rc = lib.fv_kv_cache_update(self._h, layer, C.byref(dk), C.byref(dv), current_start, C.byref(kw), C.byref(vw),
-                                    torch.cuda.current_stream().cuda_stream)
+        rc = lib.fv_kv_cache_update(self._h, layer, dk, dv, current_start, C.byref(kw), C.byref(vw), _lib.stream())
         if rc != 0:
             raise TensorError(lib.fv_sdpa_last_error().decode())
-
-        def view(t):
-            shape = tuple(int(t.shape[i]) for i in range(t.rank))
-            rows = int(t.plane_rows) or shape[2]
-            x = torch.as_tensor(_DevView(t.data, shape, rows, bool(t.dtype), self), device=k.device)
-            return x.view(torch.bfloat16) if t.dtype else x
-
-        return view(kw), view(vw)
+        return self._window(layer, 0, kw, k.device), self._window(layer, 1, vw, k.device)
 
     def reset(self):
         _lib.lib().fv_kv_cache_reset(self._h)
@@ -180,7 +199,7 @@ class CausalKvCache:
                 raise ValueError("rebase_sink: tables must be contiguous f32 [sink_tokens, d] CUDA tensors")
         lib = _lib.lib()
         rc = lib.fv_kv_cache_rebase_sink(self._h, target, orig[0].data_ptr(), orig[1].data_ptr(), new[0].data_ptr(),
-                                         new[1].data_ptr(), torch.cuda.current_stream().cuda_stream)
+                                         new[1].data_ptr(), _lib.stream())
         if rc != 0:
             raise TensorError(lib.fv_sdpa_last_error().decode())
 
@@ -202,7 +221,7 @@ def kv_copy_tokens(dst, dst_off, src, src_off, length):
         raise ValueError("kv copy: dst and src differ in dtype, planes or head dim")
     _lib.check(_lib.lib().fv_kv_copy_tokens(dst.data_ptr(), dst.shape[1], dst_off, src.data_ptr(), src.shape[1], src_off,
                                             length, dst.shape[0], dst.shape[2], int(dst.dtype == torch.bfloat16),
-                                            torch.cuda.current_stream().cuda_stream))
+                                            _lib.stream()))
 
 
 def kv_shift_tokens_down(t, frm, to, length):
@@ -210,7 +229,7 @@ def kv_shift_tokens_down(t, frm, to, length):
     _flat(t, "t")
     _lib.check(_lib.lib().fv_kv_shift_tokens_down(t.data_ptr(), t.shape[1], frm, to, length, t.shape[0], t.shape[2],
                                                   int(t.dtype == torch.bfloat16),
-                                                  torch.cuda.current_stream().cuda_stream))
+                                                  _lib.stream()))
 
 
 def rope_bhsd(x, cos, sin, negate_sin=False, out_bf16=None):
@@ -226,5 +245,5 @@ def rope_bhsd(x, cos, sin, negate_sin=False, out_bf16=None):
     out = torch.empty((b, h, s, d), device=x.device, dtype=torch.bfloat16 if o16 else torch.float32)
     _lib.check(_lib.lib().fv_rope_bhsd(x.data_ptr(), int(x.dtype == torch.bfloat16), s, cos.data_ptr(), sin.data_ptr(),
                                        int(bool(negate_sin)), out.data_ptr(), int(o16), s, b * h, s, d,
-                                       torch.cuda.current_stream().cuda_stream))
+                                       _lib.stream()))
     return out

@@ -12,10 +12,6 @@ from . import _lib
 __all__ = ["sdpa_dense_bf16", "sdpa_dense_bf16_windows", "sdpa_dense_bf16_splitkv", "splitkv_choose", "sdpa_block_causal_bf16", "sdpa_vdn_window_bf16", "cast_f32_bf16", "cast_bf16_f32", "softmax_last", "sdpa_supported"]
 
 
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
-
-
 def _need(t, dtype, name):
     if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype and t.is_contiguous()):
         raise ValueError(f"{name}: want a contiguous CUDA tensor of {dtype}")
@@ -41,7 +37,7 @@ def sdpa_dense_bf16(q, k, v, scale=None, out_bf16=False):
     scale = 1.0 / math.sqrt(d) if scale is None else scale
     out = torch.empty((bh, sq, d), device=q.device, dtype=torch.bfloat16 if out_bf16 else torch.float32)
     _lib.check(_lib.lib().fv_sdpa_dense_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                                             int(out_bf16), bh, sq, sk, d, scale, _stream()))
+                                             int(out_bf16), bh, sq, sk, d, scale, _lib.stream()))
     return out
 
 
@@ -68,7 +64,7 @@ def sdpa_dense_bf16_windows(q, k, v, scale=None, out_bf16=False):
     out = torch.empty((bh, sq, d), device=q.device, dtype=torch.bfloat16 if out_bf16 else torch.float32)
     _lib.check(_lib.lib().fv_sdpa_dense_bf16_strided(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                                                      int(out_bf16), bh, sq, sk, d, scale, rows[0], rows[1], rows[2],
-                                                     _stream()))
+                                                     _lib.stream()))
     return out
 
 
@@ -93,7 +89,7 @@ def sdpa_dense_bf16_splitkv(q, k, v, splits=None, scale=None, out_bf16=False):
     ws = torch.empty(max(nbytes, 256), device=q.device, dtype=torch.uint8)
     _lib.check(lib.fv_sdpa_dense_bf16_splitkv(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), int(out_bf16), bh,
                                               sq, sk, d, scale, rows[0], rows[1], rows[2], splits, ws.data_ptr(), nbytes,
-                                              _stream()))
+                                              _lib.stream()))
     return out
 
 
@@ -107,7 +103,7 @@ def sdpa_block_causal_bf16(q, k, v, block_tokens, window=0, sink=0, scale=None, 
         raise ValueError(f"out must be a contiguous {want} tensor of shape {(bh, sq, d)} on {q.device}")
     _lib.check(_lib.lib().fv_sdpa_block_causal_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                                                     int(out_bf16), bh, sq, sk, d, scale, block_tokens, window,
-                                                    sink, _stream()))
+                                                    sink, _lib.stream()))
     return out
 
 
@@ -117,7 +113,7 @@ def sdpa_vdn_window_bf16(q, k, v, video_start, frame_tokens, frames, chunk=0, ra
     out = torch.empty((bh, sq, d), device=q.device, dtype=torch.bfloat16 if out_bf16 else torch.float32)
     _lib.check(_lib.lib().fv_sdpa_vdn_window_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                                                   int(out_bf16), bh, sq, sk, d, scale, video_start, frame_tokens,
-                                                  frames, chunk, radius, _stream()))
+                                                  frames, chunk, radius, _lib.stream()))
     return out
 
 
@@ -126,16 +122,16 @@ def cast_f32_bf16(x, mul=None):
     _need(x, torch.float32, "x")
     y = torch.empty(x.shape, device=x.device, dtype=torch.bfloat16)
     if mul is None:
-        _lib.check(_lib.lib().fv_cast_f32_bf16(x.data_ptr(), y.data_ptr(), x.numel(), _stream()))
+        _lib.check(_lib.lib().fv_cast_f32_bf16(x.data_ptr(), y.data_ptr(), x.numel(), _lib.stream()))
     else:
-        _lib.check(_lib.lib().fv_cast_f32_bf16_scaled(x.data_ptr(), y.data_ptr(), x.numel(), float(mul), _stream()))
+        _lib.check(_lib.lib().fv_cast_f32_bf16_scaled(x.data_ptr(), y.data_ptr(), x.numel(), float(mul), _lib.stream()))
     return y
 
 
 def cast_bf16_f32(x):
     _need(x, torch.bfloat16, "x")
     y = torch.empty(x.shape, device=x.device, dtype=torch.float32)
-    _lib.check(_lib.lib().fv_cast_bf16_f32(x.data_ptr(), y.data_ptr(), x.numel(), _stream()))
+    _lib.check(_lib.lib().fv_cast_bf16_f32(x.data_ptr(), y.data_ptr(), x.numel(), _lib.stream()))
     return y
 
 
@@ -151,5 +147,5 @@ def softmax_last(x, out_bf16=False, out=None):
         _need(out, torch.bfloat16 if out_bf16 else torch.float32, "out")
         if out.shape != x.shape:
             raise ValueError("out: shape differs from x")
-    _lib.check(_lib.lib().fv_softmax_last(x.data_ptr(), out.data_ptr(), int(out_bf16), rows, width, _stream()))
+    _lib.check(_lib.lib().fv_softmax_last(x.data_ptr(), out.data_ptr(), int(out_bf16), rows, width, _lib.stream()))
     return out

@@ -9,10 +9,6 @@ from . import _lib
 __all__ = ["qk_norm_rope_bhsd", "split_heads_bhsd", "merge_heads", "qk_norm_rope_tiles", "split_heads_tiles"]
 
 
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
-
-
 def _is16(t, name):
     if not (t.is_cuda and t.is_contiguous()):
         raise ValueError(f"{name}: want a contiguous CUDA tensor")
@@ -57,14 +53,14 @@ def qk_norm_rope_bhsd(proj, col_off, heads, weight, rope=None, eps=1e-6, out_bf1
                                                     sin.data_ptr() if sin is not None else None, out.data_ptr(),
                                                     int(out_bf16), batch, seq, heads, d, width, col_off, eps,
                                                     float(out_mul), tiles.token_slot.data_ptr(), tiles.padded,
-                                                    _stream()))
+                                                    _lib.stream()))
         return out
     out = torch.empty((batch, heads, seq, d), device=proj.device, dtype=odt)
     _lib.check(_lib.lib().fv_qk_norm_rope_bhsd(proj.data_ptr(), x16, weight.data_ptr(), w16,
                                                cos.data_ptr() if cos is not None else None,
                                                sin.data_ptr() if sin is not None else None, out.data_ptr(),
                                                int(out_bf16), batch, seq, heads, d, width, col_off, eps,
-                                               float(out_mul), _stream()))
+                                               float(out_mul), _lib.stream()))
     return out
 
 
@@ -84,7 +80,7 @@ def split_heads_tiles(proj, col_off, heads, d, ctx, out=None):
     elif tuple(out.shape) != (batch, heads, ctx.padded, d) or out.dtype != proj.dtype or not out.is_contiguous():
         raise ValueError("split heads: out must be a contiguous [batch, heads, padded, d] tensor of proj's type")
     _lib.check(_lib.lib().fv_split_heads_tiles(proj.data_ptr(), out.data_ptr(), is16, batch, seq, heads, d, width,
-                                               col_off, ctx.token_slot.data_ptr(), ctx.padded, _stream()))
+                                               col_off, ctx.token_slot.data_ptr(), ctx.padded, _lib.stream()))
     return out
 
 
@@ -93,7 +89,7 @@ def split_heads_bhsd(proj, col_off, heads, d):
     is16 = _is16(proj, "proj")
     out = torch.empty((batch, heads, seq, d), device=proj.device, dtype=proj.dtype)
     _lib.check(_lib.lib().fv_split_heads_bhsd(proj.data_ptr(), out.data_ptr(), is16, batch, seq, heads, d, width,
-                                              col_off, _stream()))
+                                              col_off, _lib.stream()))
     return out
 
 
@@ -101,5 +97,5 @@ def merge_heads(x):
     batch, heads, seq, d = x.shape
     is16 = _is16(x, "x")
     out = torch.empty((batch, seq, heads * d), device=x.device, dtype=x.dtype)
-    _lib.check(_lib.lib().fv_merge_heads(x.data_ptr(), out.data_ptr(), is16, batch, heads, seq, d, _stream()))
+    _lib.check(_lib.lib().fv_merge_heads(x.data_ptr(), out.data_ptr(), is16, batch, heads, seq, d, _lib.stream()))
     return out

@@ -3,6 +3,7 @@ over the library's C++ host layer (`fv_rt_sdpa`). Same constructors, same error
 messages; tensors are torch CUDA tensors (device memory only).
 """
 import ctypes as C
+import struct
 from contextlib import contextmanager
 
 import torch
@@ -128,90 +129,69 @@ def _window_rows(t):
     return sh // d
 
 
-def _desc(t, name):
+# struct fv_tensor and struct fv_plan as bytes: packing one takes a microsecond where filling a ctypes structure field by
+# field takes ten, as much as a small launch.
+_TENSOR_BYTES = struct.Struct("@Pii9N")
+_PLAN_BYTES = struct.Struct("@iifPi8Ni0P")
+assert _TENSOR_BYTES.size == C.sizeof(_FvTensor) and _PLAN_BYTES.size == C.sizeof(_FvPlan)
+_NO_SHAPE = (0,) * 8
+
+
+def _desc_bytes(t, name):
+    """`t` as the bytes of a struct fv_tensor."""
+    if not (isinstance(t, torch.Tensor) and t.is_cuda):
+        raise ValueError(f"{name}: want a contiguous CUDA tensor")
     rows = 0
-    if isinstance(t, torch.Tensor) and t.is_cuda and not t.is_contiguous():
+    if not t.is_contiguous():
         rows = _window_rows(t) or 0
         if not rows:
             raise ValueError(f"{name}: want a contiguous CUDA tensor or a row window of a BHSD one")
-    elif not (isinstance(t, torch.Tensor) and t.is_cuda):
-        raise ValueError(f"{name}: want a contiguous CUDA tensor")
-    if t.dtype not in (torch.float32, torch.bfloat16):
+    if t.dtype == torch.bfloat16:
+        bf16 = 1
+    elif t.dtype == torch.float32:
+        bf16 = 0
+    else:
         raise ValueError(f"{name}: want f32 or bf16")
-    if t.dim() > 8:
+    shape = t.shape
+    rank = len(shape)
+    if rank > 8:
         raise ValueError(f"{name}: rank > 8")
-    d = _FvTensor()
-    d.data, d.dtype, d.rank = t.data_ptr(), int(t.dtype == torch.bfloat16), t.dim()
-    d.plane_rows = rows
-    for i, s in enumerate(t.shape):
-        d.shape[i] = s
-    return d
+    return _TENSOR_BYTES.pack(t.data_ptr(), bf16, rank, *shape, *_NO_SHAPE[rank:], rows)
 
 
-class _Owned:
-    """Frees the library-allocated result when the wrapping tensor dies."""
-
-    def __init__(self, ptr, stream):
-        self.ptr, self.stream = ptr, stream
-
-    def __del__(self):
-        try:
-            _lib.lib().fv_rt_free(self.ptr, self.stream)
-        except Exception:
-            pass
+def _desc(t, name):
+    return _FvTensor.from_buffer_copy(_desc_bytes(t, name))
 
 
 def sdpa(q, k, v, plan):
     """rt/sdpa.rs:141-164. Returns a new [b, h, sq, d] tensor (bf16 under bf16 activations, else f32)."""
     lib = _lib.lib()
-    dq, dk, dv = _desc(q, "q"), _desc(k, "k"), _desc(v, "v")
-    p = _FvPlan()
-    p.kind = plan.kind
-    p.has_scale, p.scale = (1, float(plan.scale)) if plan.scale is not None else (0, 0.0)
-    dm = None
+    dq, dk, dv = _desc_bytes(q, "q"), _desc_bytes(k, "k"), _desc_bytes(v, "v")
+    scale, causal, window = plan.scale, plan.causal, plan.window
+    mask = None
     if plan.mask is not None:
-        dm = _desc(plan.mask, "mask")
-        p.mask = C.pointer(dm)
-    p.fp8_first = int(plan.fp8)
-    if plan.causal is not None:
-        p.block_tokens, p.window, p.sink = plan.causal.block_tokens, plan.causal.window, plan.causal.sink
-    if plan.window is not None:
-        p.video_start, p.frame_tokens, p.frames, p.chunk, p.radius = plan.window._args()
-    p.kv_flash = -1 if plan.kv_flash is None else int(plan.kv_flash)
-    out = _FvTensor()
-    stream = torch.cuda.current_stream().cuda_stream
-    rc = lib.fv_rt_sdpa(C.byref(dq), C.byref(dk), C.byref(dv), C.byref(p), C.byref(out), stream)
+        mask = C.create_string_buffer(_desc_bytes(plan.mask, "mask"), _TENSOR_BYTES.size)   # alive until the call is made
+    p = _PLAN_BYTES.pack(plan.kind, 0 if scale is None else 1, 0.0 if scale is None else scale,
+                         0 if mask is None else C.addressof(mask), 1 if plan.fp8 else 0,
+                         *((causal.block_tokens, causal.window, causal.sink) if causal is not None else (0, 0, 0)),
+                         *(window._args() if window is not None else (0, 0, 0, 0, 0)),
+                         -1 if plan.kv_flash is None else int(plan.kv_flash))
+    need = (C.c_size_t * 2)()
+    rc = lib.fv_rt_sdpa_need(dq, dk, dv, p, need)
     if rc != 0:
         raise TensorError(lib.fv_sdpa_last_error().decode(), rc)
-    shape = tuple(out.shape[i] for i in range(out.rank))
-    dtype = torch.bfloat16 if out.dtype else torch.float32
-    n = 1
-    for s in shape:
-        n *= s
-    # copy into torch-owned memory, then hand the library's buffer back (stream-ordered)
-    owner = _Owned(out.data, stream)
-    nbytes = n * (2 if out.dtype else 4)
-    res = torch.empty(shape, device=q.device, dtype=dtype)
-    if nbytes:
-        from torch.cuda import current_stream  # noqa: F401
-
-        _hip_copy(res.data_ptr(), out.data, nbytes, stream)
-    del owner
-    return res
-
-
-_hiprt = None
-
-
-def _hip_copy(dst, src, nbytes, stream):
-    global _hiprt
-    if _hiprt is None:
-        _hiprt = C.CDLL("libamdhip64.so")
-        _hiprt.hipMemcpyAsync.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_void_p]
-        _hiprt.hipMemcpyAsync.restype = C.c_int
-    rc = _hiprt.hipMemcpyAsync(dst, src, nbytes, 3, stream)   # hipMemcpyDeviceToDevice
+    bf16, nbytes = need
+    # (the shape of q is the result's: the library refuses anything else before it writes)
+    try:
+        res = torch.empty(q.shape, device=q.device, dtype=torch.bfloat16 if bf16 else torch.float32)
+        work = torch.empty(nbytes, device=q.device, dtype=torch.uint8) if nbytes else None
+    except torch.cuda.OutOfMemoryError as e:
+        raise TensorError(f"sdpa: device allocation failed: {e}", -2) from e   # hipErrorOutOfMemory
+    rc = lib.fv_rt_sdpa_into(dq, dk, dv, p, res.data_ptr(), res.numel() * (2 if bf16 else 4),
+                             work.data_ptr() if nbytes else None, nbytes, _lib.stream())
     if rc != 0:
-        raise TensorError(f"hipMemcpyAsync failed: {rc}")
+        raise TensorError(lib.fv_sdpa_last_error().decode(), rc)
+    return res
 
 
 def bf16_activations():

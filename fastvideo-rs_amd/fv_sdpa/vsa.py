@@ -17,10 +17,6 @@ __all__ = ["TILE", "TILE_ELEMS", "topk_for", "TilePlan", "VsaCtx", "vsa_tile_mea
            "block_causal_dense_mask", "block_causal_for", "shard_ranges"]
 
 
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
-
-
 def topk_for(sparsity, num_tiles):
     return int(_lib.lib().fv_vsa_topk_for(float(sparsity), num_tiles))
 
@@ -90,7 +86,7 @@ def vsa_tile_mean(x, ctx, round16=False, tiled=False):
     out = torch.empty((bh, ctx.num_tiles, dim), device=x.device, dtype=torch.float32)
     _lib.check(_lib.lib().fv_vsa_tile_mean(x.data_ptr(), _is16(x), None if tiled else ctx.slot_src.data_ptr(),
                                            ctx.block_sizes.data_ptr(),
-                                           out.data_ptr(), bh, seq, dim, ctx.num_tiles, int(round16), _stream()))
+                                           out.data_ptr(), bh, seq, dim, ctx.num_tiles, int(round16), _lib.stream()))
     return out
 
 
@@ -102,7 +98,7 @@ def vsa_coarse(qc, kc, vc, scale, want_coarse=True):
     coarse = torch.empty((bh, nb, dim), device=qc.device, dtype=torch.float32) if want_coarse else None
     _lib.check(_lib.lib().fv_vsa_coarse(qc.data_ptr(), kc.data_ptr(), vc.data_ptr() if vc is not None else None,
                                         scores.data_ptr(), coarse.data_ptr() if coarse is not None else None, bh, nb,
-                                        dim, scale, _stream()))
+                                        dim, scale, _lib.stream()))
     return scores, coarse
 
 
@@ -111,7 +107,7 @@ def vsa_topk(scores, k):
     n = scores.shape[-1]
     rows = scores.numel() // n
     out = torch.empty(scores.shape[:-1] + (k,), device=scores.device, dtype=torch.int32)
-    _lib.check(_lib.lib().fv_vsa_topk(scores.data_ptr(), out.data_ptr(), rows, n, k, _stream()))
+    _lib.check(_lib.lib().fv_vsa_topk(scores.data_ptr(), out.data_ptr(), rows, n, k, _lib.stream()))
     return out
 
 
@@ -121,7 +117,7 @@ def vsa_tile_qkv(x, ctx):
     padded = ctx.plan.padded
     out = torch.empty((bh, padded, dim), device=x.device, dtype=torch.bfloat16)
     _lib.check(_lib.lib().fv_vsa_tile_qkv(x.data_ptr(), _is16(x), ctx.slot_src.data_ptr(), out.data_ptr(), bh, seq,
-                                          padded, dim, _stream()))
+                                          padded, dim, _lib.stream()))
     return out
 
 
@@ -138,7 +134,7 @@ def vsa_fine(qt, kt, vt, selected, ctx, scale, q_base=0, q_tiles=None):
     out = torch.empty((bh, q_tiles * TILE_ELEMS, dim), device=qt.device, dtype=torch.float32)
     _lib.check(_lib.lib().fv_vsa_fine(qt.data_ptr(), kt.data_ptr(), vt.data_ptr(), selected.data_ptr(),
                                       ctx.block_sizes.data_ptr(), out.data_ptr(), bh, nb, topk, dim, scale, q_base,
-                                      q_tiles, _stream()))
+                                      q_tiles, _lib.stream()))
     return out
 
 
@@ -158,7 +154,7 @@ def vsa_combine(sparse, coarse, gate, ctx, out=None, q_base=0, q_tiles=None, rou
     entry = _lib.lib().fv_vsa_combine_round16 if round16 else _lib.lib().fv_vsa_combine
     _lib.check(entry(sparse.data_ptr(), coarse.data_ptr(), gate.data_ptr() if gate is not None else None,
                      g16, ctx.slot_src.data_ptr(), out.data_ptr(), bh, ctx.seq, dim, nb, q_base,
-                     q_tiles, _stream()))
+                     q_tiles, _lib.stream()))
     return out
 
 
@@ -186,7 +182,7 @@ def vsa_attention_device(q, k, v, gate, ctx, scale, topk=None, return_selected=F
                                            _is16(gate) if gate is not None else 0, ctx.slot_src.data_ptr(),
                                            ctx.block_sizes.data_ptr(), out.data_ptr(), ws.data_ptr(), nbytes,
                                            sel.data_ptr() if sel is not None else None, bh, seq, nb, topk, dim, scale,
-                                           _stream()))
+                                           _lib.stream()))
     return (out, sel) if return_selected else out
 
 
@@ -215,7 +211,7 @@ def vsa_attention_tiled(qt, kt, vt, gate, ctx, scale, topk=None, return_selected
                                                  _is16(gate) if gate is not None else 0, ctx.slot_src.data_ptr(),
                                                  ctx.block_sizes.data_ptr(), out.data_ptr(), ws.data_ptr(), nbytes,
                                                  sel.data_ptr() if sel is not None else None, bh, ctx.seq, nb, topk,
-                                                 dim, scale, _stream()))
+                                                 dim, scale, _lib.stream()))
     return (out, sel) if return_selected else out
 
 

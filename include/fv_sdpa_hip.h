@@ -217,6 +217,16 @@ typedef struct fv_plan {
 int fv_rt_sdpa(const fv_tensor* q, const fv_tensor* k, const fv_tensor* v, const fv_plan* plan,
                fv_tensor* out, void* stream);
 int fv_rt_free(void* p, void* stream);
+/* fv_rt_sdpa with the caller's memory (no counterpart in the reference): the result is written to `out`, of out_bytes
+ * bytes = those of the [b,h,sq,d] result in the type fv_rt_sdpa_need names (another size is refused), and the rounded
+ * copies of f32 operands and the split-KV partials live in `workspace` (256-byte aligned; NULL / 0: allocated
+ * stream-ordered, as what does not fit is). A result from the stream-ordered allocator costs its caller a copy or a
+ * wrapper and, after every synchronisation of the device, mapping its memory anew (0.2 - 0.35 ms for 100 MB).
+ * fv_rt_sdpa_need: need_out = {result type (0 f32, 1 bf16), workspace bytes} of that call. Host arithmetic, except that
+ * the number of compute units is asked of the current device once. */
+int fv_rt_sdpa_need(const fv_tensor* q, const fv_tensor* k, const fv_tensor* v, const fv_plan* plan, size_t need_out[2]);
+int fv_rt_sdpa_into(const fv_tensor* q, const fv_tensor* k, const fv_tensor* v, const fv_plan* plan, void* out,
+                    size_t out_bytes, void* workspace, size_t workspace_bytes, void* stream);
 /* rt/tensor.rs `with_bf16_act`: per-thread override of FASTVIDEO_BF16_ACT; v < 0 clears it. */
 void fv_rt_set_bf16_activations(int v);
 int fv_rt_bf16_activations(void);
