@@ -146,3 +146,22 @@ def test_declines(fv):
         fv.sdpa_vdn_window_bf16(x, x, x, 0, 10, 31)        # video past the sequence
     with pytest.raises(fv.FvDeclined):
         fv.sdpa_vdn_window_bf16(x, x, x, 0, 0, 3)          # no frame tokens
+
+
+@pytest.mark.parametrize("bh,s,vs,t,frames,chunk,radius", [
+    (3, 3000, 300, 256, 9, 0, 1),      # two front tiles of global rows, the back tiles start inside the last frame
+    (2, 2560, 0, 256, 10, 3, 1),       # frames = query tiles: every boundary of the order falls on a tile edge
+    (2, 1800, 0, 150, 12, 4, 2),       # the first uncut window starts past the inner tiles: upward part short
+    (1, 1030, 1, 257, 4, 1, 1),        # the inner tiles are one or none
+    (2, 1500, 600, 100, 9, 2, 5),      # radius * chunk past the clip: no upward part at all
+])
+def test_every_query_tile_has_its_place_in_the_order_of_work(fv, oracle, bh, s, vs, t, frames, chunk, radius):
+    """The launch hands out (query tile, head) by rank; a tile left out or taken twice leaves rows of another call."""
+    import torch
+
+    announce(f"vdn window order bh={bh} s={s} video={vs}+{frames}x{t} chunk={chunk} radius={radius}")
+    q, k, v = qkv(7100 + s, bh, s, s, 128)
+    want = oracle.sdpa_composed(q, k, v, mask=oracle.vdn_window_dense_mask(vs, t, frames, chunk, radius, s, s))
+    got = fv.sdpa_vdn_window_bf16(*(to_dev_bf16(x) for x in (q, k, v)), vs, t, frames, chunk, radius, out_bf16=True)
+    torch.cuda.synchronize()
+    assert_parity(got.float().cpu().numpy(), want, f"vdn_order_{s}_{vs}_{t}x{frames}")
