@@ -13,10 +13,10 @@
 // wants rounded: PARTS = 1) have one part, so K Q^T is one product and P V, whose P is f32, three.
 // (Non-finite operands give NaN rows: the parts of an infinity do not add up.) Measured against the same sums in 64
 // bits, rel_l2: 5.4e-7 at 4096 x 4096 x 128, 3.9e-7 at 1024 x 1024 x 64; the v_mfma_f32_32x32x2_f32 form: 8.1e-7 and
-// 6.1e-7. Time: 1376 -> 830 us at 12 x 4096 x 4096 x 128 with a shared mask (f32 operands, what bounds it is the matrix
-// pipe with 1.5 workgroups of work per CU); with the casts and the rounding of the result taken into the kernel
-// 303 -> 40 us at 64 x 512 x 512 x 64 with a mask per head (bf16; its 67 MB of mask are half of that), and
-// 136 -> 33 us at 16 x 257 x 257 x 80, a head dim that used to take the scalar kernel.
+// 6.1e-7. Time against that form with its casts, in us: 12 x 4096 x 4096 x 128 with a shared mask (f32 operands)
+// 1376 -> 615, 54 % of the matrix pipe on the CUs that hold two workgroups of the 384; 64 x 512 x 512 x 64 with a mask per
+// head (bf16; 67 MB of mask) 259 -> 25, bound by the softmax's and the splitting of P's vector instructions; 16 x 257 x
+// 257 x 80, which used to take the scalar kernel, 136 -> 12.6, a chain of three tiles with little to hide their latency.
 //
 // One workgroup = 4 waves. KS waves share 32 queries, each walking every KS-th key tile with its own running max and
 // sum; their results are merged through LDS at the end. KS = 1 (128 queries a workgroup) where the query tiles fill
@@ -48,11 +48,19 @@ struct Parts3 {
 // x = p[0] + p[1] + p[2] exactly (nearest bf16 each time)
 FV_DEV Parts3 split3(const f32x8 x) {
     Parts3 r;
-    r.p[0] = __builtin_convertvector(x, bf16x8);
-    const f32x8 e1 = x - __builtin_convertvector(r.p[0], f32x8);
-    r.p[1] = __builtin_convertvector(e1, bf16x8);
-    const f32x8 e2 = e1 - __builtin_convertvector(r.p[1], f32x8);
-    r.p[2] = __builtin_convertvector(e2, bf16x8);
+    f32x8 e = x;
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+        r.p[t] = __builtin_convertvector(e, bf16x8);
+        if (t < 2) {
+            const u32x4 w = __builtin_bit_cast(u32x4, r.p[t]);   // the parts as f32 again, straight from the packed pairs
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                e[2 * i] -= __builtin_bit_cast(float, w[i] << 16);
+                e[2 * i + 1] -= __builtin_bit_cast(float, w[i] & 0xffff0000u);
+            }
+        }
+    }
     return r;
 }
 
@@ -118,61 +126,64 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
     const int gt = tid - ks * kGroup;        // thread within the group
     lds_u8* kt = (lds_u8*)csm + ks * (PARTS * (kKP + kVP));
     lds_u8* vt = kt + PARTS * kKP;
-    const long bh = blockIdx.y;
     const int sq = p.sq, sk = p.sk, d = p.d;
+    // Workgroup i runs on XCD i % 8. A mask of every head's own (or none): XCD x takes a contiguous eighth of the (head,
+    // query tile) items, so that a head's keys and values pass through one L2. A shared mask: the query tiles go round
+    // the XCDs, so that a mask row is read through one L2 for all heads.
+    int item = blockIdx.x;
+    if (p.by_head) item = (item & 7) * p.per_xcd + (item >> 3);
+    if (item >= p.total) return;
+    const long bh = item / p.nqt;
+    const int qt = item - (int)bh * p.nqt;
     const bool vec = p.vec != 0;
-    const int qi = blockIdx.x * (32 * QG) + qg * 32 + c32;   // this lane's query
+    const int qi = qt * (32 * QG) + qg * 32 + c32;   // this lane's query
     const bool q_ok = qi < sq;
     const float NEG = neg_inf();
+    // Unmasked scores are compared unscaled, so the scale's sign goes into Q and its magnitude into the exponent; a
+    // scale of zero makes Q zero.
+    const float q_mul = p.mask || p.scale > 0.f ? 1.f : p.scale < 0.f ? -1.f : p.scale;
+    const float to_log2 = p.mask || p.scale == 0.f ? 1.4426950408889634f : __builtin_fabsf(p.scale) * 1.4426950408889634f;
     const char* kb = (const char*)p.k + bh * sk * (long)d * (KV16 ? 2 : 4);
     const char* vb = (const char*)p.v + bh * sk * (long)d * (KV16 ? 2 : 4);
     const float* mr = p.mask ? p.mask + bh * p.mask_bh + (long)(q_ok ? qi : 0) * sk : nullptr;
-
-    // Q operand, in parts: this lane's query, d = 16 j + 8 h ..
-    bf16x8 qf[PARTS][NC];
-    {
-        const long row = bh * sq + (q_ok ? qi : 0);
-#pragma unroll
-        for (int j = 0; j < NC; j++) {
-            const int c = 16 * j + 8 * h;
-            f32x8 x = p.q_is_bf16 ? load8_f32<true>((const uint16_t*)p.q + row * d, c, d, vec)
-                                  : load8_f32<false>((const float*)p.q + row * d, c, d, vec);
-            if (!q_ok) x = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            if constexpr (PARTS == 1) {
-                qf[0][j] = __builtin_convertvector(x, bf16x8);
-            } else {
-                const Parts3 s = split3(x);
-#pragma unroll
-                for (int t = 0; t < 3; t++) qf[t][j] = s.p[t];
-            }
-        }
-    }
 
     // One 8-element unit of the group's tile in registers: raw bf16, or f32.
     struct Unit {
         u32x4 r[kMine / 4];
     };
+    // Byte offsets of this thread's units from the tile's first row; units past d are never loaded and stay zero.
+    constexpr int kElem = KV16 ? 2 : 4;
+    int uoff[kPer];
+    bool uok[kPer];
+#pragma unroll
+    for (int r = 0; r < kPer; r++) {
+        const int un = gt + kGroup * r, row = un / (D / 8), c = 8 * (un % (D / 8));
+        uoff[r] = (row * d + c) * kElem;
+        uok[r] = un < kUnits && c < d;
+    }
+    // Rows past the end re-read the last one: their scores are masked, and the last row's values times zero.
     auto load_units = [&](const char* base, int kv0, Unit (&u)[kPer]) {
+        const char* tile = base + (long)kv0 * d * kElem;
+        const int last = sk - 1 - kv0;
 #pragma unroll
         for (int r = 0; r < kPer; r++) {
             const int un = gt + kGroup * r, row = un / (D / 8), c = 8 * (un % (D / 8));
+            if (!uok[r]) continue;
+            const char* src = tile + (uoff[r] - max(0, row - last) * d * kElem);
+            if (vec) {
 #pragma unroll
-            for (int x = 0; x < kMine / 4; x++) u[r].r[x] = u32x4{0u, 0u, 0u, 0u};
-            if (un < kUnits && kv0 + row < sk && c < d) {
-                const char* src = base + ((long)(kv0 + row) * d + c) * (KV16 ? 2 : 4);
-                if (vec) {
+                for (int x = 0; x < kMine / 4; x++) u[r].r[x] = *reinterpret_cast<const u32x4*>(src + 16 * x);
+            } else {
+                // rows that are not whole 16-byte units: element by element
 #pragma unroll
-                    for (int x = 0; x < kMine / 4; x++) u[r].r[x] = *reinterpret_cast<const u32x4*>(src + 16 * x);
-                } else {
-                    // rows that are not whole 16-byte units: element by element
+                for (int x = 0; x < kMine / 4; x++) u[r].r[x] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-                    for (int x = 0; x < 8; x++) {
-                        if (c + x < d) {
-                            if constexpr (KV16)
-                                u[r].r[0][x >> 1] |= (unsigned)reinterpret_cast<const uint16_t*>(src)[x] << (16 * (x & 1));
-                            else
-                                u[r].r[(x >> 2) % (kMine / 4)][x & 3] = reinterpret_cast<const unsigned*>(src)[x];
-                        }
+                for (int x = 0; x < 8; x++) {
+                    if (c + x < d) {
+                        if constexpr (KV16)
+                            u[r].r[0][x >> 1] |= (unsigned)reinterpret_cast<const uint16_t*>(src)[x] << (16 * (x & 1));
+                        else
+                            u[r].r[(x >> 2) % (kMine / 4)][x & 3] = reinterpret_cast<const unsigned*>(src)[x];
                     }
                 }
             }
@@ -200,6 +211,28 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
         }
     };
 
+    // The additive mask of the lane's 16 keys, four consecutive ones per load where rows allow it.
+    auto load_mask = [&](int kv0, f32x16& mk) {
+        if (!mr) return;
+        if (p.vec_mask) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const f32x4 t = *reinterpret_cast<const f32x4*>(mr + min(kv0 + 8 * g + 4 * h, sk - 4));
+#pragma unroll
+                for (int x = 0; x < 4; x++) mk[4 * g + x] = t[x];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; i++) mk[i] = mr[min(kv0 + 8 * (i >> 2) + 4 * h + (i & 3), sk - 1)];
+        }
+    };
+
+    // A tile belongs to one wave where every wave walks keys of its own: its LDS writes and reads complete in order.
+    auto tile_barrier = [&]() {
+        if constexpr (KS == 4) __builtin_amdgcn_wave_barrier();
+        else __syncthreads();
+    };
+
     f32x16 o[NO];
 #pragma unroll
     for (int db = 0; db < NO; db++)
@@ -213,39 +246,47 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
 
     const int nt = (sk + 31) / 32, steps = (nt + KS - 1) / KS;
     Unit ku[kPer], vu[kPer];
+#pragma unroll
+    for (int r = 0; r < kPer; r++)
+#pragma unroll
+        for (int x = 0; x < kMine / 4; x++) ku[r].r[x] = vu[r].r[x] = u32x4{0u, 0u, 0u, 0u};
+    f32x16 mk;
     load_units(kb, ks * 32, ku);
     load_units(vb, ks * 32, vu);
+    load_mask(ks * 32, mk);
+
+    // Q operand, in parts: this lane's query, d = 16 j + 8 h ..
+    bf16x8 qf[PARTS][NC];
+    {
+        const long row = bh * sq + (q_ok ? qi : 0);
+#pragma unroll
+        for (int j = 0; j < NC; j++) {
+            const int c = 16 * j + 8 * h;
+            f32x8 x = p.q_is_bf16 ? load8_f32<true>((const uint16_t*)p.q + row * d, c, d, vec)
+                                  : load8_f32<false>((const float*)p.q + row * d, c, d, vec);
+            if (!q_ok) x = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (q_mul != 1.f) x = x * q_mul;
+            if constexpr (PARTS == 1) {
+                qf[0][j] = __builtin_convertvector(x, bf16x8);
+            } else {
+                const Parts3 s = split3(x);
+#pragma unroll
+                for (int t = 0; t < 3; t++) qf[t][j] = s.p[t];
+            }
+        }
+    }
+
 #pragma unroll 1
     for (int step = 0; step < steps; step++) {
         const int kv0 = (step * KS + ks) * 32;
         store_units(kt, G::kKRow, kKP, ku);
         store_units(vt, G::kVRow, kVP, vu);
-        __syncthreads();
+        tile_barrier();
         if (step + 1 < steps) {   // in flight under this tile's arithmetic (rows past the end: zeros)
             load_units(kb, kv0 + 32 * KS, ku);
             load_units(vb, kv0 + 32 * KS, vu);
         }
         if (kv0 < sk) {           // (a wave whose share has ended keeps the barriers only)
-            // the additive mask of the lane's 16 keys, four consecutive ones per load where rows allow it
-            f32x16 mk;
-            if (mr) {
-                if (p.vec_mask) {
-#pragma unroll
-                    for (int g = 0; g < 4; g++) {
-                        const int key = kv0 + 8 * g + 4 * h;
-                        f32x4 t = {0.f, 0.f, 0.f, 0.f};
-                        if (key < sk) t = *reinterpret_cast<const f32x4*>(mr + key);
-#pragma unroll
-                        for (int x = 0; x < 4; x++) mk[4 * g + x] = t[x];
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 16; i++) {
-                        const int key = kv0 + 8 * (i >> 2) + 4 * h + (i & 3);
-                        mk[i] = key < sk ? mr[key] : 0.f;
-                    }
-                }
-            }
             // ---- S^T = K Q^T ----
             f32x16 s;
 #pragma unroll
@@ -264,35 +305,34 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
                 }
                 s = mfma32(a[0], qf[0][j], s);
             }
-            // ---- scale, mask, online softmax (per lane = per query; halves exchange max and sum) ----
+            // ---- mask, online softmax (per lane = per query; the halves share the max, each sums its own keys) ----
+            // Without a mask the scores stay unscaled up to the exponential; with one they are s * scale + mask.
             {
-#pragma clang fp contract(off)
-                float mx = NEG;
+                if (mr) {
 #pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    float sv = s[i] * p.scale;
-                    if (mr) sv = sv + mk[i];
-                    s[i] = sv;
+                    for (int i = 0; i < 16; i++) s[i] = __builtin_fmaf(s[i], p.scale, mk[i]);
                 }
                 if (kv0 + 32 > sk) {
+                    asm volatile("");   // a branch, not sixteen selects on every tile
 #pragma unroll
                     for (int i = 0; i < 16; i++)
                         if (kv0 + 8 * (i >> 2) + 4 * h + (i & 3) >= sk) s[i] = NEG;
                 }
+                float mx = NEG;
 #pragma unroll
                 for (int i = 0; i < 16; i++) mx = __builtin_fmaxf(mx, s[i]);
                 mx = pair_max(mx);
                 const float m_new = __builtin_fmaxf(m_run, mx);
-                const float alpha = (m_run == NEG) ? 0.f : fast_exp2((m_run - m_new) * 1.4426950408889634f);
+                const float alpha = (m_run == NEG) ? 0.f : fast_exp2((m_run - m_new) * to_log2);
                 const float off = (m_new == NEG) ? 0.f : m_new;   // a row that has seen no key: every P is 2^-inf = 0
                 float ls = 0.f;
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
-                    const float e = fast_exp2((s[i] - off) * 1.4426950408889634f);
+                    const float e = fast_exp2((s[i] - off) * to_log2);
                     s[i] = e;
                     ls += e;
                 }
-                l_run = l_run * alpha + pair_sum(ls);
+                l_run = l_run * alpha + ls;
                 m_run = m_new;
                 if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
 #pragma unroll
@@ -301,6 +341,8 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
                         for (int i = 0; i < 16; i++) o[db][i] *= alpha;
                 }
             }
+            // the next tile's mask, in flight under the rest of this tile (rows past the end: nothing)
+            if (step + 1 < steps) load_mask(kv0 + 32 * KS, mk);
             // ---- O^T += V^T P^T, 16 keys at a time ----
 #pragma unroll
             for (int t = 0; t < 2; t++) {
@@ -332,8 +374,10 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
                 }
             }
         }
-        __syncthreads();
+        tile_barrier();
     }
+    l_run = pair_sum(l_run);
+    if constexpr (KS == 4) __syncthreads();   // the merge below reuses every wave's tile
 
     if constexpr (KS > 1) {
         // merge the KS shares of every query: shares 1 .. KS-1 leave O, max and sum in LDS, share 0 adds them up
@@ -359,7 +403,7 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
             ls[t] = *at(slot(t), 16 * NO + 1);
             m_all = __builtin_fmaxf(m_all, ms[t]);
         }
-        const float w0 = m_run == NEG ? 0.f : fast_exp2((m_run - m_all) * 1.4426950408889634f);
+        const float w0 = m_run == NEG ? 0.f : fast_exp2((m_run - m_all) * to_log2);
         l_run *= w0;
 #pragma unroll
         for (int db = 0; db < NO; db++)
@@ -367,7 +411,7 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
             for (int i = 0; i < 16; i++) o[db][i] *= w0;
 #pragma unroll
         for (int t = 1; t < KS; t++) {
-            const float w = ms[t] == NEG ? 0.f : fast_exp2((ms[t] - m_all) * 1.4426950408889634f);
+            const float w = ms[t] == NEG ? 0.f : fast_exp2((ms[t] - m_all) * to_log2);
             l_run += ls[t] * w;
 #pragma unroll
             for (int db = 0; db < NO; db++)
@@ -420,25 +464,26 @@ hipError_t launch_as(const ComposedParams& p, size_t bh, hipStream_t st) {
         if (e != hipSuccess) return e;
     }
     constexpr int rows = 32 * (4 / KS);
-    const dim3 grid((unsigned)((p.sq + rows - 1) / rows), (unsigned)bh);
-    hipLaunchKernelGGL((sdpa_composed_kernel<D, PARTS, KS, KV16>), grid, dim3(256), lds, st, p);
+    ComposedParams a = p;
+    a.nqt = (p.sq + rows - 1) / rows;
+    const size_t total = bh * (size_t)a.nqt;
+    if (total > (size_t)INT_MAX - 8) return hipErrorInvalidValue;
+    a.total = (int)total;
+    a.per_xcd = (int)((total + 7) / 8);
+    a.by_head = !p.mask || p.mask_bh != 0;
+    hipLaunchKernelGGL((sdpa_composed_kernel<D, PARTS, KS, KV16>), dim3((unsigned)(a.per_xcd * 8)), dim3(256), lds, st, a);
     return hipGetLastError();
 }
 
 template <int D>
 hipError_t launch_d(const ComposedParams& p, int parts, bool kv16, int ks, size_t bh, hipStream_t st) {
-    if (parts == 3) {
-        if (ks == 1) return launch_as<D, 3, 1, false>(p, bh, st);
-        return launch_as<D, 3, 2, false>(p, bh, st);
+    if (parts == 3) return ks == 1 ? launch_as<D, 3, 1, false>(p, bh, st) : launch_as<D, 3, 2, false>(p, bh, st);
+    if (!kv16) return ks == 1 ? launch_as<D, 1, 1, false>(p, bh, st) : launch_as<D, 1, 2, false>(p, bh, st);
+    if (ks == 1) return launch_as<D, 1, 1, true>(p, bh, st);
+    if constexpr (D <= 96) {
+        if (ks == 4) return launch_as<D, 1, 4, true>(p, bh, st);
     }
-    if (kv16) {
-        if (ks == 1) return launch_as<D, 1, 1, true>(p, bh, st);
-        if (ks == 2) return launch_as<D, 1, 2, true>(p, bh, st);
-        return launch_as<D, 1, 4, true>(p, bh, st);
-    }
-    if (ks == 1) return launch_as<D, 1, 1, false>(p, bh, st);
-    if (ks == 2) return launch_as<D, 1, 2, false>(p, bh, st);
-    return launch_as<D, 1, 4, false>(p, bh, st);
+    return launch_as<D, 1, 2, true>(p, bh, st);
 }
 
 }  // namespace
@@ -453,10 +498,16 @@ extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* para
     p.vec = (any & 15) == 0 && d % 8 == 0;
     p.vec_mask = p.mask && ((uintptr_t)p.mask & 15) == 0 && p.sk % 4 == 0;
     const int parts = kv_is_bf16 || round16 ? 1 : 3;
-    // 1024 groups are one wave on every SIMD of the chip: below that the keys are shared out over a workgroup's waves
+    // 1024 groups are one wave on every SIMD of the chip: below two waves (one with three parts, whose second share of
+    // the tiles leaves room for one workgroup per CU) the keys are shared out over a workgroup's waves. One part, bf16,
+    // us with one / two / four shares: 64 x 1024 x 300 x 80 (2048 groups) 34.9 / 40.8 / 64.0, 64 x 512 x 512 x 64 (1024)
+    // 28.4 / 24.8 / 29.8, 12 x 2000 x 2000 x 128 (756) 106 / 93 / 102, 24 x 300 x 300 x 80 (240) 20.0 / 15.0 / 13.4.
+    // Three parts: 64 x 3000 x 700 x 80 (6016) 299 / 346, 12 x 4096 x 4096 x 128 (1536) 615 / 1459, 24 x 1024 x 1024 x 64
+    // (768) 72 / 63. Four shares take the registers of four tiles in flight: bf16 keys up to 96 channels only (f32 keys,
+    // 12 x 700 x 700 x 112: 39 / 29 / 61, with spills).
     int ks = 1;
     const size_t groups = bh * (size_t)((p.sq + 31) / 32);   // 32-query groups
-    if (groups < 1024) ks = 2;
+    if (groups < (parts == 3 ? 1024 : 2048)) ks = 2;
     if (groups < 512) ks = 4;
     if (d <= 32) return fv::launch_d<32>(p, parts, kv_is_bf16 != 0, ks, bh, st);
     if (d <= 64) return fv::launch_d<64>(p, parts, kv_is_bf16 != 0, ks, bh, st);

@@ -45,6 +45,7 @@ struct ComposedParams {
     int sq, sk, d;
     float scale;
     int vec, vec_mask;            // set by the launcher: 16-byte operand rows / mask rows
+    int nqt, total, per_xcd, by_head;   // set by the launcher: query tiles per head, items, ceil(total / 8), item order
 };
 
 struct VsaFineParams {

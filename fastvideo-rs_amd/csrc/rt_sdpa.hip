@@ -104,7 +104,7 @@ extern "C" int fv_sdpa_composed_f32(const float* q, const float* k, const float*
     const long mask_bh = mask && mask_per_bh ? (long)(sq * sk) : 0L;
     hipError_t e;
     if (d <= 128) {
-        fv::ComposedParams p{q, k, v, mask, mask_bh, out, 0, 0, (int)sq, (int)sk, (int)d, scale, 0, 0};
+        fv::ComposedParams p{q, k, v, mask, mask_bh, out, 0, 0, (int)sq, (int)sk, (int)d, scale, 0, 0, 0, 0, 0, 0};
         e = fv_internal_launch_composed(&p, 0, 0, bh, (hipStream_t)stream);
         return e == hipSuccess ? FV_OK : fv_fail_hip(e, "sdpa_composed");
     }
@@ -380,7 +380,7 @@ Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::
     } else {
         fv::ComposedParams p{pq->data, pk->data, pv->data, pm ? (const float*)pm->data : nullptr,
                              mask_per_bh ? (long)(sq * sk) : 0L, out.data, pq->dtype == DType::Bf16, act16, (int)sq,
-                             (int)sk, (int)d, sc, 0, 0};
+                             (int)sk, (int)d, sc, 0, 0, 0, 0, 0, 0};
         const hipError_t e = fv_internal_launch_composed(&p, kv16, act16, bh, st);
         if (e != hipSuccess) return TensorError{"sdpa: " + rc_message(fv_fail_hip(e, "sdpa_composed")), (int)e};
     }

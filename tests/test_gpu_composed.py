@@ -99,3 +99,28 @@ def test_unaligned_operands(fv):
     got = out[1:-1].view(bh, sq, d).double().cpu().numpy()
     assert np.linalg.norm(got - want) <= 2e-6 * np.linalg.norm(want)
     assert float(out[0]) == 7.0 and float(out[-1]) == 7.0
+
+
+@pytest.mark.parametrize("scale", [-0.3, 0.0, 0.125, 1.7])
+@pytest.mark.parametrize("bh,sq,sk,d,act16", [(9, 65, 97, 64, True), (9, 65, 97, 64, False), (1, 33, 40, 128, False),
+                                              (70, 960, 33, 96, True)])
+def test_scales(fv, bh, sq, sk, d, act16, scale):
+    """Unmasked scores are scaled inside the exponential (sign and zero go into the queries), masked ones before the
+    mask is added; item counts that eight does not divide."""
+    import torch
+
+    announce(f"composed scale={scale} bh={bh} sq={sq} sk={sk} d={d} {act16}")
+    g = torch.Generator(device="cuda").manual_seed(sq + sk + d)
+    mk = lambda s: torch.randn((1, bh, s, d), generator=g, device="cuda")
+    q, k, v = mk(sq), mk(sk), mk(sk)
+    if act16:
+        q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    for mask in (None, torch.randn((1, 1, sq, sk), generator=g, device="cuda")):
+        out = fv.sdpa(q, k, v, fv.Plan.composed(scale, mask))
+        torch.cuda.synchronize()
+        # 64-bit reference on keys scaled by scale * sqrt(d) (want64 divides by sqrt(d))
+        want = want64(q, k.double() * (scale * np.sqrt(d)), v, mask)
+        # scores up to |scale| * sqrt(d) * 5 in f32: a rounding of each is that times 2^-24 on its weight
+        bound = 2e-6 + abs(scale) * np.sqrt(d) * 5 * 2.0**-24
+        err = np.linalg.norm(out.double().cpu().numpy() - want) / np.linalg.norm(want)
+        assert err <= bound, (err, bound)
