@@ -126,7 +126,8 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
     // sequence): longest first over the whole launch, tile index major and head minor
     // (block-causal: last tile first; VDN window: vdn_tile_order); measured 9 % faster than the
     // dense order, whose per-XCD ranges hold unequal work.
-    int bh, qt, sp = 0;   // sp: this workgroup's key split (dense launches with kv_split > 1)
+    int bh, qt, sp = 0;   // sp: this workgroup's key split
+    bool split = false;   // dense launches: one of the kv_split workgroups of its query tile
     if constexpr (MASKED) {
         const int work = block;
         if (work >= p.total) return true;
@@ -135,13 +136,18 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         const int r = work / nbh;
         qt = p.mask_mode == 2 ? vdn_tile_order(p, r) : p.nqt - 1 - r;
     } else {
-        const int work = (block & 7) * p.per_xcd + (block >> 3);
-        if (work >= p.total) return true;
-        const int per_bh = p.nqt * p.kv_split;
-        bh = work / per_bh;
-        const int rem = work - bh * per_bh;
-        qt = rem / p.kv_split;
-        sp = rem - qt * p.kv_split;
+        // (the unsplit query tiles first, dealt like a launch of their own: p.full is a multiple of 8)
+        const bool whole = block < p.full;
+        const int b = whole ? block : block - p.full;
+        int work = (b & 7) * (whole ? p.full >> 3 : p.per_xcd) + (b >> 3);
+        if (!whole) {
+            if (work >= p.total) return true;
+            split = p.kv_split > 1;
+            sp = work % p.kv_split;
+            work = p.full + work / p.kv_split;
+        }
+        bh = work / p.nqt;
+        qt = work - bh * p.nqt;
     }
     const int q0 = qt * kPpBM;
     const int sq = p.sq, sk = p.sk;
@@ -162,8 +168,8 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
 
     const int nkt_all = (sk + kBN - 1) / kBN;
     // a split walks key tiles [t0, t0 + nkt) of the nkt_all tiles (the whole range without split-KV)
-    const int t0 = MASKED ? 0 : sp * p.split_tiles;
-    const int nkt = MASKED ? nkt_all : min(p.split_tiles, nkt_all - t0);
+    const int t0 = split ? sp * p.split_tiles : 0;
+    const int nkt = split ? min(p.split_tiles, nkt_all - t0) : nkt_all;
     // The key-tile walk of this query tile: up to three ascending tile ranges [a_i, a_i + n_i),
     // n0 + n1 + n2 = ne tiles in all. A lane's query sees key x iff
     //   x < a_hi  ||  x >= c_lo  ||  (w_lo <= x && x < w_hi).
@@ -476,10 +482,10 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     const int row = wave * 32 + c32;
     if constexpr (!MASKED) {
-        if (p.kv_split > 1) {
+        if (split) {
             // partial result of this split: O / l in f32 and log2 of the sum of 2^(s * sl2) it covers
             if (row < qlen) {
-                const size_t prow = ((size_t)sp * (p.total / (p.nqt * p.kv_split)) + bh) * sq + q0 + row;
+                const size_t prow = (size_t)sp * p.part_rows + ((size_t)bh * sq + q0 + row - p.part_row0);
                 float* po = p.part_o + prow * kD;
 #pragma unroll
                 for (int db = 0; db < kNO; db++)
@@ -636,7 +642,7 @@ hipError_t launch_flash_as(const fv::FlashParams* p, hipStream_t stream) {
     constexpr int lds = 2 * fv::kRing2 * fv::TileGeo<D>::kTile + fv::kVoteBytes;
     hipError_t e = flash_attr<MASKED, D, LOG2DOM, FIXED>();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((fv::flash_fwd_pp2<MASKED, D, LOG2DOM, FIXED>), dim3(p->per_xcd * 8), dim3(512), lds, stream, *p);
+    hipLaunchKernelGGL((fv::flash_fwd_pp2<MASKED, D, LOG2DOM, FIXED>), dim3(p->full + p->per_xcd * 8), dim3(512), lds, stream, *p);
     return hipGetLastError();
 }
 // FASTVIDEO_SDPA_RUNNING_MAX=1: every launch keeps the running max (no fixed-offset first pass).

@@ -92,10 +92,22 @@ size_t settle_splits(size_t nkt, size_t splits) {
     return (nkt + per - 1) / per;
 }
 
+int compute_units() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        return n;
+    }();
+    return cus;
+}
+
 struct MaskArgs {
     int mode = kMaskNone;
     size_t q_rows = 0, k_rows = 0, v_rows = 0;   // rows per (batch, head) plane; 0 = contiguous (sq / sk)
-    size_t splits = 1;                            // split-KV (dense only): key splits per query tile
+    size_t splits = 1;                            // split-KV (dense only): key splits per query tile ...
+    size_t full = 0;                              // ... past the first `full` ones
     void* workspace = nullptr;                    // ... and their partial results
     size_t workspace_bytes = 0;
     size_t block_tokens = 0, window = 0, sink = 0;                           // block-causal
@@ -167,35 +179,92 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         if (m.frames <= 2) mode = kMaskNone;   // anchors only: dense
     }
     p.mask_mode = mode;
+    p.full = 0;
     p.kv_split = 1;
     p.split_tiles = INT_MAX;
+    p.part_row0 = p.part_rows = 0;
     p.part_o = nullptr;
     p.part_lse = nullptr;
     const size_t nkt = (sk + 63) / 64;
     size_t splits = mode == kMaskNone ? settle_splits(nkt, m.splits) : 1;
     if (splits > 1) {
         if (total * splits > (size_t)INT_MAX / 2) return decline("sdpa: too many workgroups for one launch");
-        const size_t need = fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits);
+        // the split query tiles are the last rows of [bh * sq]
+        const size_t full = m.full < total ? m.full : 0;
+        const size_t row0 = full / (size_t)p.nqt * sq + full % (size_t)p.nqt * bm, rows = bh * sq - row0;
+        const size_t need = fv_sdpa_splitkv_workspace_bytes(1, rows, d, splits);
         if (!m.workspace || m.workspace_bytes < need || (((uintptr_t)m.workspace) & 255) != 0)
             return fv_invalid("sdpa: split-KV needs a 256-byte aligned workspace of fv_sdpa_splitkv_workspace_bytes");
         p.kv_split = (int)splits;
         p.split_tiles = (int)((nkt + splits - 1) / splits);
         p.part_o = (float*)m.workspace;
-        p.part_lse = (float*)((char*)m.workspace + ((splits * bh * sq * d * 4 + 255) & ~(size_t)255));
-        p.total = (int)(total * splits);
+        p.part_lse = (float*)((char*)m.workspace + ((splits * rows * d * 4 + 255) & ~(size_t)255));
+        p.full = (int)full;
+        p.part_row0 = (long)row0;
+        p.part_rows = (long)rows;
+        p.total = (int)((total - full) * splits);
         p.per_xcd = (p.total + 7) / 8;
     }
     hipError_t e = fv_internal_launch_flash(&p, mode != kMaskNone ? 1 : 0, (int)d, (hipStream_t)stream);
     if (e != hipSuccess) return fail_hip(e, mode != kMaskNone ? "flash_fwd_pp2<masked>" : "flash_fwd_pp2<dense>");
     if (p.kv_split > 1) {
-        e = fv_internal_launch_splitkv_merge(p.part_o, p.part_lse, out, out_is_bf16 ? 1 : 0, bh * sq, (int)d, p.kv_split,
-                                             (hipStream_t)stream);
+        void* dst = (char*)out + (size_t)p.part_row0 * d * (out_is_bf16 ? 2 : 4);
+        e = fv_internal_launch_splitkv_merge(p.part_o, p.part_lse, dst, out_is_bf16 ? 1 : 0, (size_t)p.part_rows, (int)d,
+                                             p.kv_split, (hipStream_t)stream);
         if (e != hipSuccess) return fail_hip(e, "splitkv_merge");
     }
     return FV_OK;
 }
 
 }  // namespace
+
+// Fewer query tiles than CUs: fv_sdpa_splitkv_choose. More: they run in rounds of one per CU, and the last round costs a
+// whole walk of the keys however few tiles are left for it. Where they are few, they are shared out over the chip by key
+// ranges instead; where they are many it does not pay, because a chip that is half busy runs at a higher clock.
+// Measured on MI355X, unsplit and so, us: 24 x 3000 x 3000 x 128 (288 tiles: 256 + 32 x 5) 145 / 120, 40 x 2000 x 2000
+// x 64 (320: 256 + 64 x 4) 69 / 61, 40 x 75600 x 75600 x 128 (11840: 11776 + 64 x 4) 89600 / 88240.
+FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d) {
+    const size_t cus = (size_t)compute_units(), bm = (size_t)fv_internal_flash_block_m();
+    const size_t nqt = (sq + bm - 1) / bm, wgs = bh * nqt, nkt = (sk + 63) / 64;
+    if (wgs < cus || cus % 8 != 0 || wgs > (size_t)INT_MAX / 64) {
+        const size_t splits = fv_sdpa_splitkv_choose(bh, sq, sk);
+        return {0, splits, fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits)};
+    }
+    const size_t full = wgs / cus * cus, rest = wgs - full;
+    if (rest == 0) return {0, 1, 0};
+    const size_t rows = bh * sq - (full / nqt * sq + full % nqt * bm);
+    // us, measured: a workgroup's fixed part, and a 64-key tile while `w` workgroups run (16 x 4000 x 4000 x 128, 256
+    // tiles: 121 us, half of them 79); partials written and read at 4 TB/s and a launch
+    const double fixed = d == 64 ? 5.0 : 8.0;
+    auto run = [&](size_t w, size_t tiles) {
+        const double x = w <= cus / 2 ? 0.0 : ((double)w / (double)cus - 0.5) * 2.0;
+        return fixed + (d == 64 ? 0.8 + 0.25 * x : 1.15 + 0.65 * x) * (double)tiles;
+    };
+    size_t best = 1;
+    double best_cost = 0.95 * run(rest, nkt);
+    for (size_t sp = 2; sp <= 16 && sp * 8 <= nkt; sp++) {   // at least 8 key tiles (4 phases) per split
+        const size_t per = (nkt + sp - 1) / sp, real = settle_splits(nkt, sp), n = rest * real;
+        const double c = (double)(n / cus) * run(cus, per) + (n % cus ? run(n % cus, per) : 0.0) +
+                         (double)(real * rows * d) * 4.0 / 4.0e6 + 6.0;
+        if (c < best_cost) best_cost = c, best = real;
+    }
+    if (best == 1) return {0, 1, 0};
+    return {full, best, fv_sdpa_splitkv_workspace_bytes(1, rows, d, best)};
+}
+
+int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out, int out_is_bf16, size_t bh,
+                     size_t sq, size_t sk, size_t d, float scale, size_t q_rows, size_t k_rows, size_t v_rows,
+                     const FvSplitPlan& plan, void* workspace, size_t workspace_bytes, void* stream) {
+    MaskArgs m;
+    m.q_rows = q_rows;
+    m.k_rows = k_rows;
+    m.v_rows = v_rows;
+    m.splits = plan.splits;
+    m.full = plan.full;
+    m.workspace = workspace;
+    m.workspace_bytes = workspace_bytes;
+    return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
+}
 
 extern "C" {
 
@@ -247,13 +316,7 @@ size_t fv_sdpa_splitkv_workspace_bytes(size_t bh, size_t sq, size_t d, size_t sp
 }
 
 size_t fv_sdpa_splitkv_choose(size_t bh, size_t sq, size_t sk) {
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        return n;
-    }();
+    const int cus = compute_units();
     const size_t bm = (size_t)fv_internal_flash_block_m();
     const size_t wgs = bh * ((sq + bm - 1) / bm), nkt = (sk + 63) / 64;
     if (wgs == 0 || wgs >= (size_t)cus) return 1;               // the query tiles alone fill the CUs

@@ -18,7 +18,7 @@ struct FlashParams {
     int sq, sk;
     float sl2;          // scale * log2(e)
     int nqt;            // query tiles per (batch, head)
-    int total;          // bh * nqt
+    int total;          // workgroups past the first `full`: (bh * nqt - full) * kv_split
     int per_xcd;        // ceil(total / 8)
     int mask_mode;      // 0 none, 1 block-causal, 2 VDN window
     int ft, win, sink;  // block-causal: block tokens, window blocks, sink blocks; VDN window: ft = frame tokens
@@ -26,10 +26,12 @@ struct FlashParams {
     // elements between consecutive (batch, head) planes of q, k and v: s * d when contiguous, larger
     // when the operand is a row window of a longer plane (a KV cache read in place)
     long q_plane, k_plane, v_plane;
-    // Split-KV (dense launches only): kv_split > 1 gives every (head, query tile) kv_split workgroups,
-    // each walking split_tiles key tiles and writing its own normalised partial output (f32
-    // [split][bh][sq][d]) and base-2 log-sum-exp ([split][bh][sq]) for the merge kernel.
-    int kv_split, split_tiles;
+    // Split-KV (dense launches only): the first `full` (a multiple of 8) query tiles of the launch, counted head by
+    // head, have a workgroup each. kv_split > 1 gives every later one kv_split workgroups, each walking split_tiles
+    // key tiles and writing its own normalised partial output (f32 [split][row][d]) and base-2 log-sum-exp
+    // ([split][row]) for the merge kernel, for the part_rows rows of [bh * sq] from part_row0 on.
+    int full, kv_split, split_tiles;
+    long part_row0, part_rows;
     float* part_o;
     float* part_lse;
 };
@@ -131,6 +133,17 @@ __host__ __device__ inline TileWalk mask_tile_walk(const Params& p, int q0, int 
 }
 
 }  // namespace fv
+
+// How a dense launch of this shape is split where the caller has a workspace for it: all of its query tiles into
+// `splits` key ranges (full == 0), the ones past the first `full`, or none (splits == 1).
+struct FvSplitPlan {
+    size_t full, splits, workspace_bytes;
+};
+FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d);
+// fv_sdpa_dense_bf16_splitkv with such a plan
+int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out, int out_is_bf16, size_t bh,
+                     size_t sq, size_t sk, size_t d, float scale, size_t q_rows, size_t k_rows, size_t v_rows,
+                     const FvSplitPlan& plan, void* workspace, size_t workspace_bytes, void* stream);
 
 extern "C" int fv_internal_flash_block_m(void);   // queries per workgroup of the flash kernel in use
 extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d,

@@ -285,15 +285,15 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
                                      window->video_start, window->frame_tokens, window->frames, window->chunk,
                                      window->radius, st);
     else {
-        // few query tiles against many keys: split the keys over more workgroups (fv_sdpa_splitkv_choose)
-        const size_t splits = fv_sdpa_splitkv_choose(s->b * s->h, s->sq, s->sk);
+        // query tiles that do not fill the CUs, or the last round of them: split the keys over more workgroups
+        const FvSplitPlan plan = fv_split_plan(s->b * s->h, s->sq, s->sk, s->d);
         Tensor ws;
-        if (splits > 1) {
-            auto rw = st.temp({fv_sdpa_splitkv_workspace_bytes(s->b * s->h, s->sq, s->d, splits) / 4}, DType::F32);
+        if (plan.splits > 1) {
+            auto rw = st.temp({plan.workspace_bytes / 4}, DType::F32);
             if (!is_ok(rw)) return std::get<TensorError>(rw);
             ws = std::move(std::get<Tensor>(rw));
-            rc = fv_sdpa_dense_bf16_splitkv(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc,
-                                            q.plane_rows, k.plane_rows, v.plane_rows, splits, ws.data, ws.numel() * 4, st);
+            rc = fv_dense_planned(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc, q.plane_rows,
+                                  k.plane_rows, v.plane_rows, plan, ws.data, ws.numel() * 4, st);
         } else if (q.strided() || k.strided() || v.strided()) {
             rc = fv_sdpa_dense_bf16_strided(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc,
                                             q.plane_rows, k.plane_rows, v.plane_rows, st);
@@ -687,8 +687,7 @@ Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& pl
     for (const Tensor* t : {&q, &k, &v})
         if (t->dtype == DType::F32) n.workspace += (t->numel() * 2 + 255) & ~(size_t)255;
     if (plan.kind == Plan::Kind::Dense || plan.kind == Plan::Kind::KvWindow) {
-        const size_t splits = fv_sdpa_splitkv_choose(s->b * s->h, s->sq, s->sk);
-        if (splits > 1) n.workspace += (fv_sdpa_splitkv_workspace_bytes(s->b * s->h, s->sq, s->d, splits) + 255) & ~(size_t)255;
+        n.workspace += (fv_split_plan(s->b * s->h, s->sq, s->sk, s->d).workspace_bytes + 255) & ~(size_t)255;
     }
     return n;
 }

@@ -98,3 +98,34 @@ def test_choice_and_windows(fv, oracle):
         fv._lib.check(fv.lib().fv_sdpa_dense_bf16_splitkv(q.data_ptr(), kw.data_ptr(), vw.data_ptr(), got.data_ptr(), 0, bh, sq,
                                                           sk, d, 0.088, 0, sk + 500, sk + 500, 4, ws.data_ptr(), 256,
                                                           torch.cuda.current_stream().cuda_stream))
+
+
+@pytest.mark.parametrize("bh,sq,sk,d,act16", [(38, 1700, 2100, 128, True), (37, 1650, 1600, 64, True),
+                                              (38, 1537, 4100, 128, False), (261, 33, 1100, 64, True)])
+def test_last_round_of_tiles_split(fv, oracle, bh, sq, sk, d, act16):
+    """A few query tiles more than one per CU: the first 256 are the unsplit launch's bit for bit, the ones past them
+    agree with it to rounding and with the oracle, and every row is written."""
+    import torch
+
+    announce(f"splitkv last round bh={bh} sq={sq} sk={sk} d={d}")
+    q, k, v = qkv(77 + sq, bh, sq, sk, d)
+    tq, tk, tv = (to_dev_bf16(x) for x in (q, k, v))
+    base = fv.sdpa_dense_bf16(tq, tk, tv)          # f32, unsplit
+    with fv.with_bf16_act(act16):
+        got = fv.sdpa(tq[None], tk[None], tv[None], fv.Plan.dense())[0]
+    torch.cuda.synchronize()
+    assert got.dtype == (torch.bfloat16 if act16 else torch.float32)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    nqt = (sq + 255) // 256
+    full = bh * nqt // cus * cus
+    row0 = full // nqt * sq + full % nqt * 256
+    assert 0 < row0 < bh * sq
+    # P and l share an offset; the offset of a split's own first keys rounds P to bf16 elsewhere
+    assert (got.float() - base).abs().max().item() <= (2e-2 if act16 else 2e-3)
+    if not act16:
+        flat = lambda x: x.reshape(-1, d)
+        assert torch.equal(flat(got)[:row0], flat(base)[:row0])
+        assert not torch.equal(flat(got)[row0:], flat(base)[row0:])   # the rest took the split path
+    heads = np.array(sorted({0, row0 // sq, bh - 1}))
+    assert_parity(got[torch.from_numpy(heads).cuda()].float().cpu().numpy(),
+                  oracle.sdpa_composed(q[heads], k[heads], v[heads]), f"splitkv_last_round_{bh}_{sq}_{sk}_{d}")
