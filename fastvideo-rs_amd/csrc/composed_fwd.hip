@@ -16,10 +16,11 @@
 // 6.1e-7. Time against that form with its casts, in us: 12 x 4096 x 4096 x 128 with a shared mask (f32 operands)
 // 1376 -> 615, 54 % of the matrix pipe on the CUs that hold two workgroups of the 384; 64 x 512 x 512 x 64 with a mask per
 // head (bf16; 67 MB of mask) 259 -> 25, bound by the softmax's and the splitting of P's vector instructions; 16 x 257 x
-// 257 x 80, which used to take the scalar kernel, 136 -> 12.6, a chain of three tiles with little to hide their latency.
+// 257 x 80, which used to take the scalar kernel, 136 -> 10, a chain of two tiles with little to hide their latency.
 //
-// One workgroup = 4 waves. KS waves share 32 queries, each walking every KS-th key tile with its own running max and
-// sum; their results are merged through LDS at the end. KS = 1 (128 queries a workgroup) where the query tiles fill
+// One workgroup = 4 waves (8 with eight shares). KS waves share 32 queries, each walking every KS-th key tile with its own
+// running max and sum; their results are merged through LDS at the end, every wave a part of the channels (one wave
+// merging and dividing them all took 2.9 of 11 us at 16 x 257 x 257 x 80, shader-clock stamps). KS = 1 (128 queries a workgroup) where the query tiles fill
 // the chip, more where they do not. Tiles go global -> registers -> (split into parts) -> LDS; the next tile's loads
 // are in flight under the arithmetic of the current one, and two workgroups share a CU, so that one wave's softmax and
 // splitting run under the other's MFMAs.
@@ -100,17 +101,23 @@ struct ComposedGeo {
     static constexpr int kKRow = 2 * D + 16;
     static constexpr int kVRow = (D / 32) % 2 == 1 ? 2 * D : 2 * D + 64;
 };
+constexpr int composed_waves(int ks) { return ks < 4 ? 4 : ks; }
+// O of one wave in the merge: D / 8 groups of four registers, then max and sum
+template <int D>
+constexpr int kMergeShare = D / 8 * 1024 + 512;
 template <int D, int PARTS, int KS>
 constexpr int composed_lds() {
-    return KS * PARTS * 32 * (ComposedGeo<D>::kKRow + ComposedGeo<D>::kVRow);
+    constexpr int tiles = KS * PARTS * 32 * (ComposedGeo<D>::kKRow + ComposedGeo<D>::kVRow);
+    constexpr int merge = KS > 1 ? composed_waves(KS) * kMergeShare<D> : 0;
+    return tiles > merge ? tiles : merge;
 }
 
 template <int D, int PARTS, int KS, bool KV16>
-__global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedParams p) {
-    static_assert(D % 32 == 0 && (PARTS == 1 || PARTS == 3) && (KS == 1 || KS == 2 || KS == 4) && !(KV16 && PARTS == 3),
-                  "instantiations");
+__global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kernel(const ComposedParams p) {
+    static_assert(D % 32 == 0 && (PARTS == 1 || PARTS == 3) && (KS == 1 || KS == 2 || KS == 4 || KS == 8) &&
+                  !(KV16 && PARTS == 3), "instantiations");
     using G = ComposedGeo<D>;
-    constexpr int QG = 4 / KS;               // 32-query groups per workgroup
+    constexpr int QG = composed_waves(KS) / KS;   // 32-query groups per workgroup
     constexpr int kGroup = 64 * QG;          // threads that share a key tile
     constexpr int kKP = 32 * G::kKRow, kVP = 32 * G::kVRow;   // bytes of one part of a K / V tile
     constexpr int kUnits = 32 * (D / 8);     // 8-element units per tile
@@ -229,7 +236,7 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
 
     // A tile belongs to one wave where every wave walks keys of its own: its LDS writes and reads complete in order.
     auto tile_barrier = [&]() {
-        if constexpr (KS == 4) __builtin_amdgcn_wave_barrier();
+        if constexpr (KS >= 4) __builtin_amdgcn_wave_barrier();
         else __syncthreads();
     };
 
@@ -258,12 +265,12 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
     // Q operand, in parts: this lane's query, d = 16 j + 8 h ..
     bf16x8 qf[PARTS][NC];
     {
-        const long row = bh * sq + (q_ok ? qi : 0);
+        const long row = (bh * sq + (q_ok ? qi : 0)) * d;
 #pragma unroll
         for (int j = 0; j < NC; j++) {
             const int c = 16 * j + 8 * h;
-            f32x8 x = p.q_is_bf16 ? load8_f32<true>((const uint16_t*)p.q + row * d, c, d, vec)
-                                  : load8_f32<false>((const float*)p.q + row * d, c, d, vec);
+            f32x8 x = p.q_is_bf16 ? load8_f32<true>((const uint16_t*)p.q + row, c, d, vec)
+                                  : load8_f32<false>((const float*)p.q + row, c, d, vec);
             if (!q_ok) x = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
             if (q_mul != 1.f) x = x * q_mul;
             if constexpr (PARTS == 1) {
@@ -377,81 +384,93 @@ __global__ __launch_bounds__(256, 2) void sdpa_composed_kernel(const ComposedPar
         tile_barrier();
     }
     l_run = pair_sum(l_run);
-    if constexpr (KS == 4) __syncthreads();   // the merge below reuses every wave's tile
 
-    if constexpr (KS > 1) {
-        // merge the KS shares of every query: shares 1 .. KS-1 leave O, max and sum in LDS, share 0 adds them up
-        constexpr int kRegs = 16 * NO + 2;
-        static_assert((KS - 1) * QG * kRegs * 256 <= composed_lds<D, PARTS, KS>(), "the merge fits the tile buffers");
-        auto slot = [&](int share) { return (lds_u8*)csm + ((share - 1) * QG + qg) * (kRegs * 256) + lane * 4; };
-        auto at = [](lds_u8* b, int r) { return reinterpret_cast<__attribute__((address_space(3))) float*>(b + r * 256); };
-        if (ks > 0) {
-            lds_u8* b = slot(ks);
-#pragma unroll
-            for (int db = 0; db < NO; db++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) *at(b, 16 * db + i) = o[db][i];
-            *at(b, 16 * NO) = m_run;
-            *at(b, 16 * NO + 1) = l_run;
-        }
-        __syncthreads();
-        if (ks > 0) return;
-        float m_all = m_run, ms[KS], ls[KS];
-#pragma unroll
-        for (int t = 1; t < KS; t++) {
-            ms[t] = *at(slot(t), 16 * NO);
-            ls[t] = *at(slot(t), 16 * NO + 1);
-            m_all = __builtin_fmaxf(m_all, ms[t]);
-        }
-        const float w0 = m_run == NEG ? 0.f : fast_exp2((m_run - m_all) * to_log2);
-        l_run *= w0;
-#pragma unroll
-        for (int db = 0; db < NO; db++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) o[db][i] *= w0;
-#pragma unroll
-        for (int t = 1; t < KS; t++) {
-            const float w = ms[t] == NEG ? 0.f : fast_exp2((ms[t] - m_all) * to_log2);
-            l_run += ls[t] * w;
-#pragma unroll
-            for (int db = 0; db < NO; db++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) o[db][i] += *at(slot(t), 16 * db + i) * w;
-        }
-    }
-
-    if (q_ok) {
+    // out = o / l for four consecutive channels from d0 on of the lane's query; l == 0 (no key): zeros
+    auto store4 = [&](f32x4 r, float l, float inv, int d0) {
 #pragma clang fp contract(off)
-        const long base = (bh * sq + qi) * (long)d;
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            // one Newton step on the quotient: the rounding of o / l without the division's scaling (1 <= l < 2^32)
+            const float v = r[x] * inv;
+            r[x] = l > 0.f ? __builtin_fmaf(__builtin_fmaf(-v, l, r[x]), inv, v) : 0.f;
+        }
+        const long at = (bh * sq + qi) * (long)d + d0;
+        if (p.out_is_bf16) {
+            uint16_t* dst = (uint16_t*)p.out + at;
+            const bf16x4 r16 = __builtin_convertvector(r, bf16x4);
+            if (vec) {
+                if (d0 < d) *reinterpret_cast<bf16x4*>(dst) = r16;
+            } else {
+#pragma unroll
+                for (int x = 0; x < 4; x++)
+                    if (d0 + x < d) reinterpret_cast<__bf16*>(dst)[x] = r16[x];
+            }
+        } else {
+            float* dst = (float*)p.out + at;
+            if (vec) {
+                if (d0 < d) *reinterpret_cast<f32x4*>(dst) = r;
+            } else {
+#pragma unroll
+                for (int x = 0; x < 4; x++)
+                    if (d0 + x < d) dst[x] = r[x];
+            }
+        }
+    };
+
+    if constexpr (KS == 1) {
+        if (!q_ok) return;
+        const float inv = __builtin_amdgcn_rcpf(l_run);
 #pragma unroll
         for (int db = 0; db < NO; db++)
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                const int d0 = 32 * db + 8 * g + 4 * h;
                 f32x4 r;
 #pragma unroll
-                for (int x = 0; x < 4; x++) r[x] = l_run > 0.f ? o[db][4 * g + x] / l_run : 0.f;
-                if (p.out_is_bf16) {
-                    uint16_t* dst = (uint16_t*)p.out + base + d0;
-                    const bf16x4 r16 = __builtin_convertvector(r, bf16x4);
-                    if (vec) {
-                        if (d0 < d) *reinterpret_cast<bf16x4*>(dst) = r16;
-                    } else {
-#pragma unroll
-                        for (int x = 0; x < 4; x++)
-                            if (d0 + x < d) reinterpret_cast<__bf16*>(dst)[x] = r16[x];
-                    }
-                } else {
-                    float* dst = (float*)p.out + base + d0;
-                    if (vec) {
-                        if (d0 < d) *reinterpret_cast<f32x4*>(dst) = r;
-                    } else {
-#pragma unroll
-                        for (int x = 0; x < 4; x++)
-                            if (d0 + x < d) dst[x] = r[x];
-                    }
-                }
+                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x];
+                store4(r, l_run, inv, 32 * db + 8 * g + 4 * h);
             }
+    } else {
+        // Merge of a query's KS shares, every wave its part of the channels: all leave O, max and sum in LDS (over the
+        // tiles, which every wave is done with), each adds up every KS-th group of four registers over the shares.
+        typedef __attribute__((address_space(3))) f32x4 lds_f4;
+        typedef __attribute__((address_space(3))) f32x2 lds_f2;
+        if constexpr (KS >= 4) __syncthreads();   // (KS = 2: the loop ends with one)
+        auto share = [&](int t) { return (lds_u8*)csm + (t * QG + qg) * kMergeShare<D>; };
+#pragma unroll
+        for (int db = 0; db < NO; db++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                f32x4 r;
+#pragma unroll
+                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x];
+                *(lds_f4*)(share(ks) + ((4 * db + g) * 64 + lane) * 16) = r;
+            }
+        *(lds_f2*)(share(ks) + D / 8 * 1024 + lane * 8) = f32x2{m_run, l_run};
+        __syncthreads();
+        float w[KS], l = 0.f, m_all = NEG;
+        f32x2 ml[KS];
+#pragma unroll
+        for (int t = 0; t < KS; t++) ml[t] = *(const lds_f2*)(share(t) + D / 8 * 1024 + lane * 8);
+#pragma unroll
+        for (int t = 0; t < KS; t++) m_all = __builtin_fmaxf(m_all, ml[t][0]);
+#pragma unroll
+        for (int t = 0; t < KS; t++) {
+            w[t] = ml[t][0] == NEG ? 0.f : fast_exp2((ml[t][0] - m_all) * to_log2);
+            l = __builtin_fmaf(ml[t][1], w[t], l);
+        }
+        if (!q_ok) return;
+        const float inv = __builtin_amdgcn_rcpf(l);
+#pragma unroll 1
+        for (int gi = ks; gi < D / 8; gi += KS) {
+            f32x4 r = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < KS; t++) {
+                const f32x4 x4 = *(const lds_f4*)(share(t) + (gi * 64 + lane) * 16);
+#pragma unroll
+                for (int x = 0; x < 4; x++) r[x] = __builtin_fmaf(x4[x], w[t], r[x]);
+            }
+            store4(r, l, inv, 8 * gi + 4 * h);
+        }
     }
 }
 
@@ -463,7 +482,7 @@ hipError_t launch_as(const ComposedParams& p, size_t bh, hipStream_t st) {
         const hipError_t e = fv_set_max_lds_once((const void*)sdpa_composed_kernel<D, PARTS, KS, KV16>, lds, attr_done);
         if (e != hipSuccess) return e;
     }
-    constexpr int rows = 32 * (4 / KS);
+    constexpr int rows = 32 * (composed_waves(KS) / KS);
     ComposedParams a = p;
     a.nqt = (p.sq + rows - 1) / rows;
     const size_t total = bh * (size_t)a.nqt;
@@ -471,7 +490,7 @@ hipError_t launch_as(const ComposedParams& p, size_t bh, hipStream_t st) {
     a.total = (int)total;
     a.per_xcd = (int)((total + 7) / 8);
     a.by_head = !p.mask || p.mask_bh != 0;
-    hipLaunchKernelGGL((sdpa_composed_kernel<D, PARTS, KS, KV16>), dim3((unsigned)(a.per_xcd * 8)), dim3(256), lds, st, a);
+    hipLaunchKernelGGL((sdpa_composed_kernel<D, PARTS, KS, KV16>), dim3((unsigned)(a.per_xcd * 8)), dim3(64 * composed_waves(KS)), lds, st, a);
     return hipGetLastError();
 }
 
@@ -482,10 +501,10 @@ hipError_t launch_d(const ComposedParams& p, int parts, bool kv16, int ks, size_
     if (ks == 1) return launch_as<D, 1, 1, true>(p, bh, st);
     if constexpr (D <= 96) {
         if (ks == 4) return launch_as<D, 1, 4, true>(p, bh, st);
+        if (ks == 8) return launch_as<D, 1, 8, true>(p, bh, st);
     }
     return launch_as<D, 1, 2, true>(p, bh, st);
 }
-
 }  // namespace
 }  // namespace fv
 
@@ -500,15 +519,17 @@ extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* para
     const int parts = kv_is_bf16 || round16 ? 1 : 3;
     // 1024 groups are one wave on every SIMD of the chip: below two waves (one with three parts, whose second share of
     // the tiles leaves room for one workgroup per CU) the keys are shared out over a workgroup's waves. One part, bf16,
-    // us with one / two / four shares: 64 x 1024 x 300 x 80 (2048 groups) 34.9 / 40.8 / 64.0, 64 x 512 x 512 x 64 (1024)
-    // 28.4 / 24.8 / 29.8, 12 x 2000 x 2000 x 128 (756) 106 / 93 / 102, 24 x 300 x 300 x 80 (240) 20.0 / 15.0 / 13.4.
-    // Three parts: 64 x 3000 x 700 x 80 (6016) 299 / 346, 12 x 4096 x 4096 x 128 (1536) 615 / 1459, 24 x 1024 x 1024 x 64
-    // (768) 72 / 63. Four shares take the registers of four tiles in flight: bf16 keys up to 96 channels only (f32 keys,
-    // 12 x 700 x 700 x 112: 39 / 29 / 61, with spills).
+    // us with 1 / 2 / 4 / 8 shares: 64 x 1024 x 300 x 80 (2048 groups) 33 / 39 / 56 / 83, 64 x 512 x 512 x 64 (1024)
+    // 28 / 24 / 27 / 38, 24 x 300 x 300 x 80 (240) 18.8 / 13.6 / 12.0 / 11.1, 16 x 257 x 257 x 80 (144) 15.6 / 12.4 / 11.0
+    // / 10.2, 12 x 200 x 200 x 64 (84, seven tiles) 12.2 / 10.1 / 10.0 / 10.4. Three parts, 1 / 2 shares: 64 x 3000 x 700 x
+    // 80 (6016) 284 / 331, 12 x 4096 x 4096 x 128 (1536) 606 / 1459, 24 x 1024 x 1024 x 64 (768) 71 / 62. Four and eight
+    // shares take the registers of whole tiles in flight: bf16 keys up to 96 channels only (f32 keys, 12 x 700 x 700 x
+    // 112: 39 / 29 / 61, with spills).
     int ks = 1;
     const size_t groups = bh * (size_t)((p.sq + 31) / 32);   // 32-query groups
     if (groups < (parts == 3 ? 1024 : 2048)) ks = 2;
     if (groups < 512) ks = 4;
+    if (groups <= 256 && p.sk > 256) ks = 8;
     if (d <= 32) return fv::launch_d<32>(p, parts, kv_is_bf16 != 0, ks, bh, st);
     if (d <= 64) return fv::launch_d<64>(p, parts, kv_is_bf16 != 0, ks, bh, st);
     if (d <= 96) return fv::launch_d<96>(p, parts, kv_is_bf16 != 0, ks, bh, st);

@@ -39,7 +39,9 @@ SHAPES = [  # bh, sq, sk, d
     (1, 1, 1, 1), (2, 5, 7, 8), (1, 31, 33, 7), (2, 33, 32, 30), (1, 32, 31, 33), (3, 64, 65, 40), (1, 127, 129, 72),
     (2, 129, 64, 80), (1, 100, 257, 96), (1, 96, 63, 100), (2, 130, 191, 128), (1, 33, 300, 127),
     (40, 500, 90, 64),        # 640 query groups: two shares of the keys
-    (70, 500, 70, 128),       # 1120: one
+    (70, 500, 70, 128),       # 1120: two (one with three parts)
+    (3, 70, 290, 24), (2, 97, 545, 96), (1, 33, 257, 61),   # eight shares, more than one tile each for some
+    (66, 1000, 40, 64),       # 2112: one
 ]
 
 
