@@ -466,7 +466,8 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
             for (int i = 0; i < 16; i++) chk = __builtin_fmaf(o[db][i], 0.f, chk);
         const bool lane_ok = (pair_sum(st.l_acc) < 0x1p+100f) && (chk == 0.f);
         auto* votes = (__attribute__((address_space(3))) unsigned*)(smem + 2 * kRing2 * kTileBytes);
-        if (lane == 0) votes[wave] = __builtin_amdgcn_ballot_w64(!lane_ok) != 0 ? 1u : 0u;
+        const bool wave_ok = __builtin_amdgcn_ballot_w64(!lane_ok) == 0;   // (of all lanes: outside the branch below)
+        if (lane == 0) votes[wave] = wave_ok ? 0u : 1u;
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the vote is written before the barrier
         block_barrier();   // ... behind which every wave is past its last read of both rings
         const u32x4 v0 = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(votes);

@@ -539,3 +539,27 @@ def test_a_row_one_late_key_dominates(fv, oracle):
     assert inside.max() <= 2.0 ** -8 * 1.01                     # offset = the dominant score: as the running max
     print(f"dominated rows: f32 result max|delta| {np.abs(f32 - want).max():.2e}; bf16 result relative error "
           f"{rel.max():.5f} overall, {inside.max():.5f} on rows dominated from inside the first 128 keys")
+
+
+@pytest.mark.parametrize("row", [0, 5, 31, 33, 195, 255, 299])
+@pytest.mark.parametrize("d", [128, 64])
+def test_one_row_that_outgrows_the_fixed_offset(fv, row, d):
+    """One query of a tile, on any lane of any wave, whose scores grow past the range of the first keys' offset: its
+    tile, and no other, makes its pass again, and the result is the f64 softmax's."""
+    import torch
+
+    sq, sk = 300, 700
+    announce(f"dense rerun of row {row} d={d}")
+    g = torch.Generator(device="cuda").manual_seed(11)
+    q, k, v = (torch.randn((1, s, d), generator=g, device="cuda") for s in (sq, sk, sk))
+    q[0, row] = 3.0
+    k[0, 140:] = k[0, 140:].abs() + 4.0
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    n0 = fv.lib().fv_sdpa_exact_pass_reruns()
+    got = fv.sdpa_dense_bf16(q, k, v, out_bf16=True)
+    torch.cuda.synchronize()
+    s = (q.double().cpu() @ k.double().cpu().transpose(1, 2)) / np.sqrt(d)
+    assert float((s[0, row].max() - s[0, row, :128].max()) * np.log2(np.e)) > 130    # past what f32 exponentials hold
+    assert fv.lib().fv_sdpa_exact_pass_reruns() - n0 == 1
+    want = torch.softmax(s, -1) @ v.double().cpu()
+    assert (got.double().cpu() - want).abs().max().item() <= 2e-2
