@@ -220,7 +220,7 @@ def bench_kvcache(args, fpb=3):
         "ms_per_step_with_window_copies_no_split": round(copied, 4), "ms_per_step_in_place_no_split": round(unsplit, 4),
         "ms_per_step_eager_python_loop": round(eager, 4),
         "roofline": {"bound": "mfma", "achieved": round(tf, 3), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(tf / PEAK_BF16_TFLOPS, 4), "traffic": None, "kernel": "fv::flash_fwd_pp2<false, 128, false, true>"},
+                     "frac": round(tf / PEAK_BF16_TFLOPS, 4), "traffic": None, "kernel": "fv::flash_fwd_pp2<2, false, 128, false, true>"},
     }
     print(json.dumps(rec), flush=True)
 
@@ -676,9 +676,9 @@ def main():
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_BF16_TFLOPS, 4),
                      "traffic": traffic, "traffic_source": traffic_source,
-                     # template arguments: masked, head dim, scale folded into Q, fixed-offset first pass (launches
+                     # template arguments: groups of four waves, masked, head dim, scale folded into Q, fixed-offset first pass (launches
                      # that write bf16 and whose queries all see key 0: every workload here)
-                     "kernel": f"fv::flash_fwd_pp2<{'true' if bt else 'false'}, {d}, {'true' if args.fold_scale else 'false'}, "
+                     "kernel": f"fv::flash_fwd_pp2<2, {'true' if bt else 'false'}, {d}, {'true' if args.fold_scale else 'false'}, "
                                f"{'true' if args.out_bf16 and os.environ.get('FASTVIDEO_SDPA_RUNNING_MAX', '0') in ('', '0') else 'false'}>",
                      "avg_kernel_ms": round(avg_kernel_ms, 4), "median_kernel_ms": round(kern_ms[len(kern_ms) // 2], 4),
                      "min_hbm_bytes": bytes_min,

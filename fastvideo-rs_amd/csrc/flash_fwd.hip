@@ -108,12 +108,14 @@ FV_DEV int vdn_tile_order(const Params& p, int r) {
 // remains: the largest P of a row is exactly 1 under the running max and a rounded bf16 number under the fixed
 // offset, so a row that ONE late key dominates can be off by up to 2^-8 relative; the launcher therefore takes
 // this form only for results that are rounded to bf16 anyway.
-template <bool MASKED, int D, bool LOG2DOM, bool FIXED, class Params>
+template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, class Params>
 FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const int block) {
     // (masked launches: only where every query sees key 0, see launch_flash)
     using G = TileGeo<D>;
     constexpr int kD = D;
     constexpr int kTileBytes = G::kTile;
+    constexpr int kBM = 128 * NG;
+    static_assert(NG == 2 || (NG == 1 && !MASKED), "one group: dense launches only");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     lds_u8* smem = (lds_u8*)smem_raw;
 
@@ -149,9 +151,9 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         bh = work / p.nqt;
         qt = work - bh * p.nqt;
     }
-    const int q0 = qt * kPpBM;
+    const int q0 = qt * kBM;
     const int sq = p.sq, sk = p.sk;
-    const int qlen = min(kPpBM, sq - q0);
+    const int qlen = min(kBM, sq - q0);
     const float sl2 = p.sl2;
     const float NEG = neg_inf();
     // Fetch the epilogue's arguments now. Left to the compiler, their scalar loads sit
@@ -232,7 +234,7 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
     auto kbuf = [&](int t) -> lds_u8* { return smem + (t & (kRing2 - 1)) * kTileBytes; };
     auto vbuf = [&](int t) -> lds_u8* { return smem + (kRing2 + (t & (kRing2 - 1))) * kTileBytes; };
 
-    TileDma<8, D> dma;
+    TileDma<4 * NG, D> dma;
     dma.init(wave, lane);
     // tiles past the end repeat the last one
     auto target_k = [&](int t) {
@@ -243,8 +245,8 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         const int kv0 = kv0_of(t);
         return dma.template prepare<true>(vbuf(t), Vh + (size_t)kv0 * kD, sk - kv0, wave);
     };
-    using Dma = TileDma<8, D>;
-    constexpr int kIt = Dma::ITER;   // DMA instructions per wave and tile: 2 (D = 128) or 1 (D = 64)
+    using Dma = TileDma<4 * NG, D>;
+    constexpr int kIt = Dma::ITER;   // DMA instructions per wave and tile: 2 (D = 128) or 1 (D = 64); one group: twice
     {
         const typename Dma::Prepared a0 = target_k(0), a1 = target_k(1);
 #pragma unroll
@@ -387,20 +389,12 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         // spent in the wait below, measured with shader-clock stamps).
         auto hook_dma = [&](int g) {
             g -= g0;
-            if constexpr (kIt == 2) {
-                if (g == 0) Dma::issue_prepared(dv0, 0);
-                if (g == 1) Dma::issue_prepared(dv0, 1);
-                if (g == 2) Dma::issue_prepared(dk0, 0);
-                if (g == 3) Dma::issue_prepared(dk0, 1);
-                if (g == 4) Dma::issue_prepared(dv1, 0);
-                if (g == 5) Dma::issue_prepared(dv1, 1);
-                if (g == 6) Dma::issue_prepared(dk1, 0);
-                if (g == 7) Dma::issue_prepared(dk1, 1);
-            } else {
-                if (g == 0) Dma::issue_prepared(dv0, 0);
-                if (g == 1) Dma::issue_prepared(dk0, 0);
-                if (g == 2) Dma::issue_prepared(dv1, 0);
-                if (g == 3) Dma::issue_prepared(dk1, 0);
+            // per group as many as fit all loads into the D / 16 groups of the first phase, whose walk has no PV part
+            constexpr int kPer = (4 * kIt + D / 16 - 1) / (D / 16);
+#pragma unroll
+            for (int x = g * kPer; x < g * kPer + kPer && x < 4 * kIt; x++) {
+                const int tile = x / kIt, it = x % kIt;
+                Dma::issue_prepared(tile == 0 ? dv0 : tile == 1 ? dk0 : tile == 2 ? dv1 : dk1, it);
             }
         };
         auto hook_none = [](int) {};
@@ -422,9 +416,11 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
             mfma_phase<true, kAhead, decltype(hook_none)&, D>(va, ka, kTileBytes, pb1, o, qf, s1, s_init, hook_none);
         }
         __builtin_amdgcn_s_setprio(0);
-        wait_vmcnt<0>();             // this wave's loads of this phase have landed
-        __builtin_amdgcn_sched_barrier(0);
-        block_barrier();
+        if constexpr (NG == 2) {
+            wait_vmcnt<0>();             // this wave's loads of this phase have landed
+            __builtin_amdgcn_sched_barrier(0);
+            block_barrier();
+        }
         __builtin_amdgcn_sched_barrier(0);
         // ---- VALU phase: group 0 in slot 2m+1, group 1 in slot 2m+2 ----
         mask_tile(s0, 2 * m);
@@ -445,8 +441,10 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         dk1 = target_k(2 * m + 5);
         dv0 = target_v(2 * m + 2);
         dv1 = target_v(2 * m + 3);
-        if (grp == 0 || m + 1 < np) {
+        if (NG == 1 || grp == 0 || m + 1 < np) {
             __builtin_amdgcn_sched_barrier(0);
+            // (one group: the only barrier of a phase, behind which its loads are resident and its tiles read)
+            if constexpr (NG == 1) wait_vmcnt<0>();
             block_barrier();
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -471,8 +469,11 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the vote is written before the barrier
         block_barrier();   // ... behind which every wave is past its last read of both rings
         const u32x4 v0 = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(votes);
-        const u32x4 v1 = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(votes + 4);
-        const unsigned any = v0[0] | v0[1] | v0[2] | v0[3] | v1[0] | v1[1] | v1[2] | v1[3];
+        unsigned any = v0[0] | v0[1] | v0[2] | v0[3];
+        if constexpr (NG == 2) {
+            const u32x4 v1 = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(votes + 4);
+            any |= v1[0] | v1[1] | v1[2] | v1[3];
+        }
         if (__builtin_amdgcn_readfirstlane(any) != 0) {
             if (tid == 0) atomicAdd(&g_exact_pass_reruns, 1ull);
             return false;
@@ -556,14 +557,18 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
 // one exponential and one add. LOG2DOM: the call's scale * log2(e) is exactly 1 (scores are base-2 logarithms as
 // they leave the MFMAs) and the multiply is gone too. FIXED (launches that write bf16 and whose queries all see key 0): the first pass keeps
 // the offset of the first 128 keys (flash_item); the others keep the running max throughout.
-template <bool MASKED, int D, bool LOG2DOM, bool FIXED>
-__global__ __launch_bounds__(512, 2) void flash_fwd_pp2(const FlashParams p) {
+// NG: groups of four waves. Two (256 queries) alternate; one (128) runs its matrix and VALU phases in turn, with one
+// barrier a phase and no slot in which a group waits for the other's first or last phase: for launches whose query tiles
+// of 128 still have a CU each (fv_split_plan). Bit for bit the same rows. A phase takes 2.1 us instead of 2.4, a launch of
+// one phase 7.1 instead of 8.2.
+template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED>
+__global__ __launch_bounds__(256 * NG, 2) void flash_fwd_pp2(const FlashParams p) {
     const int tid = threadIdx.x;
     int wave = __builtin_amdgcn_readfirstlane(tid >> 6), block = blockIdx.x;
     if constexpr (!FIXED) {
-        flash_item<MASKED, D, LOG2DOM, false>(p, wave, tid & 63, block);
+        flash_item<NG, MASKED, D, LOG2DOM, false>(p, wave, tid & 63, block);
     } else {
-        if (flash_item<MASKED, D, LOG2DOM, true>(p, wave, tid & 63, block)) return;
+        if (flash_item<NG, MASKED, D, LOG2DOM, true>(p, wave, tid & 63, block)) return;
         // The second pass shares nothing with the first but two scalars: its inputs are made opaque (the lane
         // index counted anew from the execution mask, the kernel arguments read again from their segment, of which
         // FlashParams is the whole), so that the compiler keeps no value of the first pass alive for it. It runs
@@ -572,7 +577,7 @@ __global__ __launch_bounds__(512, 2) void flash_fwd_pp2(const FlashParams p) {
         ConstParams* again = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
         int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
         asm volatile("" : "+v"(lane), "+s"(wave), "+s"(block), "+s"(again));
-        flash_item<MASKED, D, LOG2DOM, false>(*again, wave, lane, block);
+        flash_item<NG, MASKED, D, LOG2DOM, false>(*again, wave, lane, block);
     }
 }
 
@@ -632,18 +637,18 @@ extern "C" int fv_internal_flash_block_m(void) { return fv::kPpBM; }
 
 namespace {
 // The kernel's dynamic LDS limit (128 KB at D = 128), once per device.
-template <bool MASKED, int D, bool LOG2DOM, bool FIXED>
+template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED>
 hipError_t flash_attr() {
     static std::atomic<unsigned long long> attr_done;
     constexpr int lds = 2 * fv::kRing2 * fv::TileGeo<D>::kTile + fv::kVoteBytes;
-    return fv_set_max_lds_once((const void*)fv::flash_fwd_pp2<MASKED, D, LOG2DOM, FIXED>, lds, attr_done);
+    return fv_set_max_lds_once((const void*)fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED>, lds, attr_done);
 }
-template <bool MASKED, int D, bool LOG2DOM, bool FIXED>
+template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED>
 hipError_t launch_flash_as(const fv::FlashParams* p, hipStream_t stream) {
     constexpr int lds = 2 * fv::kRing2 * fv::TileGeo<D>::kTile + fv::kVoteBytes;
-    hipError_t e = flash_attr<MASKED, D, LOG2DOM, FIXED>();
+    hipError_t e = flash_attr<NG, MASKED, D, LOG2DOM, FIXED>();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((fv::flash_fwd_pp2<MASKED, D, LOG2DOM, FIXED>), dim3(p->full + p->per_xcd * 8), dim3(512), lds, stream, *p);
+    hipLaunchKernelGGL((fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED>), dim3(p->full + p->per_xcd * 8), dim3(256 * NG), lds, stream, *p);
     return hipGetLastError();
 }
 // FASTVIDEO_SDPA_RUNNING_MAX=1: every launch keeps the running max (no fixed-offset first pass).
@@ -657,11 +662,11 @@ bool running_max_forced() {
 // A call whose scale * log2(e) is exactly 1 (scale = ln 2: the caller folded the softmax scale into Q) runs
 // the form without the per-score multiply.
 std::atomic<unsigned long long> g_log2_domain_launches{0};
-template <bool MASKED, int D, bool FIXED>
+template <int NG, bool MASKED, int D, bool FIXED>
 hipError_t launch_flash_fixed(const fv::FlashParams* p, hipStream_t stream) {
-    if (p->sl2 != 1.0f) return launch_flash_as<MASKED, D, false, FIXED>(p, stream);
+    if (p->sl2 != 1.0f) return launch_flash_as<NG, MASKED, D, false, FIXED>(p, stream);
     g_log2_domain_launches.fetch_add(1, std::memory_order_relaxed);
-    return launch_flash_as<MASKED, D, true, FIXED>(p, stream);
+    return launch_flash_as<NG, MASKED, D, true, FIXED>(p, stream);
 }
 // Launches whose result is rounded to bf16 make their first pass with the fixed offset: on a row that one late
 // key dominates, that key's P is then a rounded bf16 number instead of exactly 1 (up to 2^-8 relative on the row),
@@ -669,11 +674,19 @@ hipError_t launch_flash_fixed(const fv::FlashParams* p, hipStream_t stream) {
 // key 0, the first key of every tile's walk, so that its offset is a score of its own: block-causal without a
 // window or with sink blocks, and the VDN mask (rows before the video and frame 0 are visible to every query).
 // Under a window without a sink a query's first visible key may lie anywhere in the walk: running max.
-template <bool MASKED, int D>
+template <int NG, bool MASKED, int D>
 hipError_t launch_flash(const fv::FlashParams* p, hipStream_t stream) {
     const bool offset_is_a_score = !MASKED || p->mask_mode == 2 || (p->mask_mode == 1 && (p->win == 0 || p->sink > 0));
-    if (p->out_is_bf16 && offset_is_a_score && !running_max_forced()) return launch_flash_fixed<MASKED, D, true>(p, stream);
-    return launch_flash_fixed<MASKED, D, false>(p, stream);
+    if (p->out_is_bf16 && offset_is_a_score && !running_max_forced()) return launch_flash_fixed<NG, MASKED, D, true>(p, stream);
+    return launch_flash_fixed<NG, MASKED, D, false>(p, stream);
+}
+template <int NG, bool MASKED, int D>
+hipError_t init_flash() {
+    hipError_t e = flash_attr<NG, MASKED, D, false, false>();
+    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, true, false>();
+    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, false, true>();
+    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, true, true>();
+    return e;
 }
 }  // namespace
 
@@ -684,28 +697,24 @@ extern "C" hipError_t fv_internal_exact_pass_reruns(unsigned long long* out) {
 }
 
 extern "C" hipError_t fv_internal_init_flash(void) {
-    hipError_t e = flash_attr<false, 128, false, false>();
-    if (e == hipSuccess) e = flash_attr<true, 128, false, false>();
-    if (e == hipSuccess) e = flash_attr<false, 64, false, false>();
-    if (e == hipSuccess) e = flash_attr<true, 64, false, false>();
-    if (e == hipSuccess) e = flash_attr<false, 128, true, false>();
-    if (e == hipSuccess) e = flash_attr<true, 128, true, false>();
-    if (e == hipSuccess) e = flash_attr<false, 64, true, false>();
-    if (e == hipSuccess) e = flash_attr<true, 64, true, false>();
-    if (e == hipSuccess) e = flash_attr<false, 128, false, true>();
-    if (e == hipSuccess) e = flash_attr<false, 64, false, true>();
-    if (e == hipSuccess) e = flash_attr<false, 128, true, true>();
-    if (e == hipSuccess) e = flash_attr<false, 64, true, true>();
-    if (e == hipSuccess) e = flash_attr<true, 128, false, true>();
-    if (e == hipSuccess) e = flash_attr<true, 64, false, true>();
-    if (e == hipSuccess) e = flash_attr<true, 128, true, true>();
-    if (e == hipSuccess) e = flash_attr<true, 64, true, true>();
+    hipError_t e = init_flash<2, false, 128>();
+    if (e == hipSuccess) e = init_flash<2, true, 128>();
+    if (e == hipSuccess) e = init_flash<2, false, 64>();
+    if (e == hipSuccess) e = init_flash<2, true, 64>();
+    if (e == hipSuccess) e = init_flash<1, false, 128>();
+    if (e == hipSuccess) e = init_flash<1, false, 64>();
     return e;
 }
 
-extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d,
+extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d, int block_m,
                                                hipStream_t stream) {
-    if (d == 128) return masked ? launch_flash<true, 128>(p, stream) : launch_flash<false, 128>(p, stream);
-    if (d == 64) return masked ? launch_flash<true, 64>(p, stream) : launch_flash<false, 64>(p, stream);
+    const bool half = block_m == fv::kPpBM / 2;
+    if ((block_m != fv::kPpBM && !half) || (half && masked)) return hipErrorInvalidValue;
+    if (d == 128)
+        return masked ? launch_flash<2, true, 128>(p, stream)
+                      : half ? launch_flash<1, false, 128>(p, stream) : launch_flash<2, false, 128>(p, stream);
+    if (d == 64)
+        return masked ? launch_flash<2, true, 64>(p, stream)
+                      : half ? launch_flash<1, false, 64>(p, stream) : launch_flash<2, false, 64>(p, stream);
     return hipErrorInvalidValue;
 }

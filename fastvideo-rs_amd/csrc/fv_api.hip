@@ -108,6 +108,7 @@ struct MaskArgs {
     size_t q_rows = 0, k_rows = 0, v_rows = 0;   // rows per (batch, head) plane; 0 = contiguous (sq / sk)
     size_t splits = 1;                            // split-KV (dense only): key splits per query tile ...
     size_t full = 0;                              // ... past the first `full` ones
+    size_t block_m = 0;                           // queries per workgroup (0: the kernel's own)
     void* workspace = nullptr;                    // ... and their partial results
     size_t workspace_bytes = 0;
     size_t block_tokens = 0, window = 0, sink = 0;                           // block-causal
@@ -141,7 +142,7 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
     p.q_plane = (long)(q_rows * d);
     p.k_plane = (long)(k_rows * d);
     p.v_plane = (long)(v_rows * d);
-    const size_t bm = (size_t)fv_internal_flash_block_m();
+    const size_t bm = m.block_m ? m.block_m : (size_t)fv_internal_flash_block_m();
     p.nqt = (int)((sq + bm - 1) / bm);
     const size_t total = bh * (size_t)p.nqt;
     if (total > (size_t)INT_MAX / 2) return decline("sdpa: too many query tiles for one launch");
@@ -205,7 +206,7 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         p.total = (int)((total - full) * splits);
         p.per_xcd = (p.total + 7) / 8;
     }
-    hipError_t e = fv_internal_launch_flash(&p, mode != kMaskNone ? 1 : 0, (int)d, (hipStream_t)stream);
+    hipError_t e = fv_internal_launch_flash(&p, mode != kMaskNone ? 1 : 0, (int)d, (int)bm, (hipStream_t)stream);
     if (e != hipSuccess) return fail_hip(e, mode != kMaskNone ? "flash_fwd_pp2<masked>" : "flash_fwd_pp2<dense>");
     if (p.kv_split > 1) {
         void* dst = (char*)out + (size_t)p.part_row0 * d * (out_is_bf16 ? 2 : 4);
@@ -228,10 +229,15 @@ FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d) {
     const size_t nqt = (sq + bm - 1) / bm, wgs = bh * nqt, nkt = (sk + 63) / 64;
     if (wgs < cus || cus % 8 != 0 || wgs > (size_t)INT_MAX / 64) {
         const size_t splits = fv_sdpa_splitkv_choose(bh, sq, sk);
-        return {0, splits, fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits)};
+        // Query tiles of 128 where each still has a CU to itself. Measured on MI355X, 256 / 128 queries a workgroup, us:
+        // 12 x 320 x 320 x 128 13.2 / 11.3, 12 x 1000 x 1000 x 128 25.6 / 23.0, 40 x 700 x 700 x 64 17.4 / 14.8, 12 x 1560 x
+        // 512 x 128 17.2 / 14.9, 24 x 390 x 2000 x 128 at 2 splits 34.2 / 29.7; past one per CU, 12 x 4000 x 512 x 128 20.3 /
+        // 29.1, 40 x 1000 x 1000 x 64 (320 tiles) 21.5 / 21.7.
+        const size_t half = bm / 2, small = bh * ((sq + half - 1) / half) * settle_splits(nkt, splits);
+        return {small <= cus ? half : bm, 0, splits, fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits)};
     }
     const size_t full = wgs / cus * cus, rest = wgs - full;
-    if (rest == 0) return {0, 1, 0};
+    if (rest == 0) return {bm, 0, 1, 0};
     const size_t rows = bh * sq - (full / nqt * sq + full % nqt * bm);
     // us, measured: a workgroup's fixed part, and a 64-key tile while `w` workgroups run (16 x 4000 x 4000 x 128, 256
     // tiles: 121 us, half of them 79); partials written and read at 4 TB/s and a launch
@@ -248,8 +254,8 @@ FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d) {
                          (double)(real * rows * d) * 4.0 / 4.0e6 + 6.0;
         if (c < best_cost) best_cost = c, best = real;
     }
-    if (best == 1) return {0, 1, 0};
-    return {full, best, fv_sdpa_splitkv_workspace_bytes(1, rows, d, best)};
+    if (best == 1) return {bm, 0, 1, 0};
+    return {bm, full, best, fv_sdpa_splitkv_workspace_bytes(1, rows, d, best)};
 }
 
 int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out, int out_is_bf16, size_t bh,
@@ -261,6 +267,7 @@ int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, vo
     m.v_rows = v_rows;
     m.splits = plan.splits;
     m.full = plan.full;
+    m.block_m = plan.block_m;
     m.workspace = workspace;
     m.workspace_bytes = workspace_bytes;
     return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);

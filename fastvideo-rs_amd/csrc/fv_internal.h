@@ -137,7 +137,7 @@ __host__ __device__ inline TileWalk mask_tile_walk(const Params& p, int q0, int 
 // How a dense launch of this shape is split where the caller has a workspace for it: all of its query tiles into
 // `splits` key ranges (full == 0), the ones past the first `full`, or none (splits == 1).
 struct FvSplitPlan {
-    size_t full, splits, workspace_bytes;
+    size_t block_m, full, splits, workspace_bytes;   // block_m: queries per workgroup
 };
 FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d);
 // fv_sdpa_dense_bf16_splitkv with such a plan
@@ -146,7 +146,7 @@ int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, vo
                      const FvSplitPlan& plan, void* workspace, size_t workspace_bytes, void* stream);
 
 extern "C" int fv_internal_flash_block_m(void);   // queries per workgroup of the flash kernel in use
-extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d,
+extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d, int block_m,
                                                hipStream_t stream);
 extern "C" hipError_t fv_internal_exact_pass_reruns(unsigned long long* out);
 extern "C" hipError_t fv_internal_launch_tile_mean(const void* x, int x_is_bf16, const int* slot_src,

@@ -292,14 +292,9 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
             auto rw = st.temp({plan.workspace_bytes / 4}, DType::F32);
             if (!is_ok(rw)) return std::get<TensorError>(rw);
             ws = std::move(std::get<Tensor>(rw));
-            rc = fv_dense_planned(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc, q.plane_rows,
-                                  k.plane_rows, v.plane_rows, plan, ws.data, ws.numel() * 4, st);
-        } else if (q.strided() || k.strided() || v.strided()) {
-            rc = fv_sdpa_dense_bf16_strided(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc,
-                                            q.plane_rows, k.plane_rows, v.plane_rows, st);
-        } else {
-            rc = fv_sdpa_dense_bf16(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc, st);
         }
+        rc = fv_dense_planned(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc, q.plane_rows,
+                              k.plane_rows, v.plane_rows, plan, ws.data, ws.data ? ws.numel() * 4 : 0, st);
     }
     if (rc == FV_DECLINED) return std::optional<Tensor>{};
     if (rc != FV_OK) return TensorError{"sdpa: " + rc_message(rc), rc < 0 ? -rc : 0};
