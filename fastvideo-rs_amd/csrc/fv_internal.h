@@ -134,6 +134,17 @@ __host__ __device__ inline TileWalk mask_tile_walk(const Params& p, int q0, int 
 
 }  // namespace fv
 
+// y = bf16(x * mul), RNE, for up to three operands in one launch
+struct FvCastOperands {
+    struct One {
+        const float* x;
+        uint16_t* y;
+        size_t n;
+        float mul;
+    } at[3];
+};
+int fv_cast_operands(const FvCastOperands& ops, int count, void* stream);
+
 // How a dense launch of this shape is split where the caller has a workspace for it: all of its query tiles into
 // `splits` key ranges (full == 0), the ones past the first `full`, or none (splits == 1).
 struct FvSplitPlan {

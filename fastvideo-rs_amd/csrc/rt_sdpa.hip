@@ -263,19 +263,30 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
             sc = FV_SDPA_SCALE_LOG2_DOMAIN;
         }
     }
-    Tensor tq, tk, tv;
-    auto rq = as_bf16(q, tq, st, q_mul);
-    if (!is_ok(rq)) return std::get<TensorError>(rq);
-    auto rk = as_bf16(k, tk, st);
-    if (!is_ok(rk)) return std::get<TensorError>(rk);
-    auto rv = as_bf16(v, tv, st);
-    if (!is_ok(rv)) return std::get<TensorError>(rv);
+    // operands that arrive as f32, rounded in one launch
+    Tensor rounded[3];
+    const Tensor* const given[3] = {&q, &k, &v};
+    const uint16_t* bits[3];
+    FvCastOperands casts{};
+    int n_casts = 0;
+    for (int i = 0; i < 3; i++) {
+        bits[i] = (const uint16_t*)given[i]->data;
+        if (given[i]->dtype == DType::Bf16) continue;
+        auto r = st.temp(given[i]->shape, DType::Bf16);
+        if (!is_ok(r)) return std::get<TensorError>(r);
+        rounded[i] = std::move(std::get<Tensor>(r));
+        casts.at[n_casts++] = {(const float*)given[i]->data, (uint16_t*)rounded[i].data, given[i]->numel(), i == 0 ? q_mul : 1.0f};
+        bits[i] = (const uint16_t*)rounded[i].data;
+    }
+    if (n_casts) {
+        const int rc = fv_cast_operands(casts, n_casts, st);
+        if (rc != FV_OK) return TensorError{"cast_f32_bf16: " + rc_message(rc), rc < 0 ? -rc : 0};
+        g_cast += n_casts;
+    }
     auto ro = st.result({s->b, s->h, s->sq, s->d}, out_bf16 ? DType::Bf16 : DType::F32);
     if (!is_ok(ro)) return std::get<TensorError>(ro);
     Tensor out = std::move(std::get<Tensor>(ro));
-    const auto* pq = (const uint16_t*)std::get<const Tensor*>(rq)->data;
-    const auto* pk = (const uint16_t*)std::get<const Tensor*>(rk)->data;
-    const auto* pv = (const uint16_t*)std::get<const Tensor*>(rv)->data;
+    const uint16_t *pq = bits[0], *pk = bits[1], *pv = bits[2];
     int rc;
     if (causal)
         rc = fv_sdpa_block_causal_bf16(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc,

@@ -462,3 +462,22 @@ def test_small_launches_take_half_tiles(fv, h, sq, sk, d):
             assert (got[0].float() - want.float()).abs().max().item() <= 2e-2
         else:
             assert not differ.any()
+
+
+@pytest.mark.parametrize("kinds", ["fff", "fbf", "bfb", "ffb"])
+@pytest.mark.parametrize("s,d,shift", [(1, 64, 0), (70, 128, 0), (33, 64, 1), (130, 128, 3)])
+def test_f32_operands_are_rounded_in_one_launch(fv, kinds, s, d, shift):
+    """Any mix of f32 and bf16 operands, 16-byte aligned or not: the call on operands torch rounded, bit for bit, and
+    one count per operand rounded."""
+    import torch
+
+    announce(f"rt cast operands {kinds} s={s} d={d} shift={shift}")
+    g = torch.Generator(device="cuda").manual_seed(s + d)
+    f32 = [(torch.randn(3 * s * d + shift, generator=g, device="cuda") * 3)[shift:].view(1, 3, s, d) for _ in range(3)]
+    b16 = [x.to(torch.bfloat16).contiguous() for x in f32]
+    n0 = fv.rt_stats()["casts"]
+    got = fv.sdpa(*(x if c == "f" else y for c, x, y in zip(kinds, f32, b16)), fv.Plan.dense())
+    assert fv.rt_stats()["casts"] == n0 + kinds.count("f")
+    want = fv.sdpa(*b16, fv.Plan.dense())
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
