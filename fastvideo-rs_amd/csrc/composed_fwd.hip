@@ -14,7 +14,7 @@
 // (Non-finite operands give NaN rows: the parts of an infinity do not add up.) Measured against the same sums in 64
 // bits, rel_l2: 5.4e-7 at 4096 x 4096 x 128, 3.9e-7 at 1024 x 1024 x 64; the v_mfma_f32_32x32x2_f32 form: 8.1e-7 and
 // 6.1e-7. Time against that form with its casts, in us: 12 x 4096 x 4096 x 128 with a shared mask (f32 operands)
-// 1376 -> 615, 54 % of the matrix pipe on the CUs that hold two workgroups of the 384; 64 x 512 x 512 x 64 with a mask per
+// 1376 -> 615 in 384 workgroups of two a CU, 531 with their last 128 cut in two (fv_composed_plan); 64 x 512 x 512 x 64 with a mask per
 // head (bf16; 67 MB of mask) 259 -> 25, bound by the softmax's and the splitting of P's vector instructions; 16 x 257 x
 // 257 x 80, which used to take the scalar kernel, 136 -> 10, a chain of two tiles with little to hide their latency.
 //
@@ -137,9 +137,25 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
     // Workgroup i runs on XCD i % 8. A mask of every head's own (or none): XCD x takes a contiguous eighth of the (head,
     // query tile) items, so that a head's keys and values pass through one L2. A shared mask: the query tiles go round
     // the XCDs, so that a mask row is read through one L2 for all heads.
-    int item = blockIdx.x;
-    if (p.by_head) item = (item & 7) * p.per_xcd + (item >> 3);
-    if (item >= p.total) return;
+    int item = blockIdx.x, tile0 = 0, split = -1;
+    int tiles = (p.sk + 31) / 32;
+    if (KS == 1 && item < p.full) {          // (full is a multiple of 8)
+        if (p.by_head) item = (item & 7) * (p.full >> 3) + (item >> 3);
+    } else {
+        if constexpr (KS == 1) item -= p.full;
+        if (p.by_head) item = (item & 7) * p.per_xcd + (item >> 3);
+        if (item >= p.total) return;
+        if constexpr (KS == 1) {
+            if (p.splits > 1) {
+                const int tile = item / p.splits;
+                split = item - tile * p.splits;
+                item = tile;
+                tile0 = split * p.split_tiles;
+                tiles = min(p.split_tiles, tiles - tile0);
+            }
+            item += p.full;
+        }
+    }
     const long bh = item / p.nqt;
     const int qt = item - (int)bh * p.nqt;
     const bool vec = p.vec != 0;
@@ -251,16 +267,16 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
     const int b16 = lane >> 4, i16 = lane & 15;
     const lds_u8* va = vt + (4 * h + (i16 >> 2)) * G::kVRow + 32 * (b16 & 1) + 8 * (i16 & 3);
 
-    const int nt = (sk + 31) / 32, steps = (nt + KS - 1) / KS;
+    const int steps = (tiles + KS - 1) / KS;
     Unit ku[kPer], vu[kPer];
 #pragma unroll
     for (int r = 0; r < kPer; r++)
 #pragma unroll
         for (int x = 0; x < kMine / 4; x++) ku[r].r[x] = vu[r].r[x] = u32x4{0u, 0u, 0u, 0u};
     f32x16 mk;
-    load_units(kb, ks * 32, ku);
-    load_units(vb, ks * 32, vu);
-    load_mask(ks * 32, mk);
+    load_units(kb, (tile0 + ks) * 32, ku);
+    load_units(vb, (tile0 + ks) * 32, vu);
+    load_mask((tile0 + ks) * 32, mk);
 
     // Q operand, in parts: this lane's query, d = 16 j + 8 h ..
     bf16x8 qf[PARTS][NC];
@@ -285,7 +301,7 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
 
 #pragma unroll 1
     for (int step = 0; step < steps; step++) {
-        const int kv0 = (step * KS + ks) * 32;
+        const int kv0 = (tile0 + step * KS + ks) * 32;
         store_units(kt, G::kKRow, kKP, ku);
         store_units(vt, G::kVRow, kVP, vu);
         tile_barrier();
@@ -419,6 +435,21 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
 
     if constexpr (KS == 1) {
         if (!q_ok) return;
+        if (split >= 0) {                    // sums of a part of the keys, for the merge kernel
+            const long row = split * p.part_rows + (bh * sq + qi - p.part_row0);
+            if (h == 0) *reinterpret_cast<f32x2*>(p.part_ml + 2 * row) = f32x2{m_run, l_run};
+#pragma unroll
+            for (int db = 0; db < NO; db++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const int d0 = 32 * db + 8 * g + 4 * h;
+                    f32x4 r;
+#pragma unroll
+                    for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x];
+                    if (d0 < d) *reinterpret_cast<f32x4*>(p.part_o + row * p.dpad + d0) = r;
+                }
+            return;
+        }
         const float inv = __builtin_amdgcn_rcpf(l_run);
 #pragma unroll
         for (int db = 0; db < NO; db++)
@@ -474,6 +505,37 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
     }
 }
 
+// out = sum over the splits of O 2^(m - max) / sum of l 2^(m - max), four channels a thread. HBM-bound: the
+// partial sums are read once and the result is written once.
+__global__ __launch_bounds__(256) void composed_merge_kernel(const ComposedParams p) {
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    const int d4 = p.dpad >> 2;
+    const long row = i / d4;
+    const int c = (int)(i - row * d4) * 4;
+    if (row >= p.part_rows) return;
+    const float to_log2 = p.mask || p.scale == 0.f ? 1.4426950408889634f : __builtin_fabsf(p.scale) * 1.4426950408889634f;
+    float m = neg_inf(), l = 0.f;
+    for (int t = 0; t < p.splits; t++) m = __builtin_fmaxf(m, p.part_ml[2 * (t * p.part_rows + row)]);
+    f32x4 r = {0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < p.splits; t++) {
+        const long at = t * p.part_rows + row;
+        const f32x2 ml = *reinterpret_cast<const f32x2*>(p.part_ml + 2 * at);
+        const float w = ml[0] == neg_inf() ? 0.f : fast_exp2((ml[0] - m) * to_log2);
+        l = __builtin_fmaf(ml[1], w, l);
+        const f32x4 o = *reinterpret_cast<const f32x4*>(p.part_o + at * p.dpad + c);
+#pragma unroll
+        for (int x = 0; x < 4; x++) r[x] = __builtin_fmaf(o[x], w, r[x]);
+    }
+    const long dst = (p.part_row0 + row) * p.d + c;
+#pragma unroll
+    for (int x = 0; x < 4; x++) {
+        if (c + x >= p.d) continue;
+        const float v = l > 0.f ? r[x] / l : 0.f;
+        if (p.out_is_bf16) ((__bf16*)p.out)[dst + x] = (__bf16)v;
+        else ((float*)p.out)[dst + x] = v;
+    }
+}
+
 template <int D, int PARTS, int KS, bool KV16>
 hipError_t launch_as(const ComposedParams& p, size_t bh, hipStream_t st) {
     constexpr int lds = composed_lds<D, PARTS, KS>();
@@ -487,11 +549,28 @@ hipError_t launch_as(const ComposedParams& p, size_t bh, hipStream_t st) {
     a.nqt = (p.sq + rows - 1) / rows;
     const size_t total = bh * (size_t)a.nqt;
     if (total > (size_t)INT_MAX - 8) return hipErrorInvalidValue;
-    a.total = (int)total;
-    a.per_xcd = (int)((total + 7) / 8);
+    size_t items = total;
+    if (KS == 1 && p.splits > 1) {
+        items = (total - (size_t)p.full) * (size_t)p.splits;
+        const int tiles = (p.sk + 31) / 32;
+        a.split_tiles = (tiles + p.splits - 1) / p.splits;
+        a.dpad = (p.d + 3) & ~3;
+        a.part_row0 = (long)(p.full / a.nqt) * p.sq + (long)(p.full % a.nqt) * rows;
+        a.part_rows = (long)bh * p.sq - a.part_row0;
+    } else {
+        a.full = 0, a.splits = 1;
+    }
+    a.total = (int)items;
+    a.per_xcd = (int)((items + 7) / 8);
     a.by_head = !p.mask || p.mask_bh != 0;
-    hipLaunchKernelGGL((sdpa_composed_kernel<D, PARTS, KS, KV16>), dim3((unsigned)(a.per_xcd * 8)), dim3(64 * composed_waves(KS)), lds, st, a);
-    return hipGetLastError();
+    hipLaunchKernelGGL((sdpa_composed_kernel<D, PARTS, KS, KV16>), dim3((unsigned)(a.full + a.per_xcd * 8)), dim3(64 * composed_waves(KS)), lds, st, a);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && a.splits > 1) {
+        const size_t n = (size_t)a.part_rows * (size_t)(a.dpad / 4);
+        hipLaunchKernelGGL(composed_merge_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);
+        e = hipGetLastError();
+    }
+    return e;
 }
 
 template <int D>
@@ -507,6 +586,36 @@ hipError_t launch_d(const ComposedParams& p, int parts, bool kv16, int ks, size_
 }
 }  // namespace
 }  // namespace fv
+
+// Query tiles (128 queries) past a multiple of the CUs hold up the launch for a whole walk of the keys while other CUs
+// have none left: they are shared out by key ranges, in as many as fill the CUs best, where that saves more than writing
+// and merging the partial sums costs (a quarter above the estimate). A 32-key tile of a workgroup that has its CU to
+// itself takes 3.4 us at 128 channels. Measured on MI355X, a shared mask, uncut / cut, us: 12 x 4096 x 4096 x 128 (384 tiles:
+// 256 + 128 x 2) 618 / 531, 24 x 3000 x 700 x 128 (576: 512 + 64 x 4) 187 / 151, 12 x 3000 x 1024 x 128 (288) 159 / 131,
+// 24 x 3000 x 800 x 80 (576) 158 / 124, 12 x 4096 x 1024 x 64 (384) 94 / 84; a mask per head, 64 x 700 x 700 x 128 (384)
+// 122 / 110, 64 x 600 x 900 x 80 (320) 112 / 97. Where the rule leaves a launch whole the key walk is too short for the
+// merge (12 x 4096 x 300 x 128, 60) or the rest fills the CUs (24 x 2600 x 1000 x 128: 248 of 256 tiles). Launches of one
+// part are not cut: a tile costs them a third of that, and the same merge.
+fv::ComposedPlan fv_composed_plan(size_t bh, size_t sq, size_t sk, size_t d) {
+    const size_t cus = (size_t)fv_compute_units(), groups = bh * ((sq + 31) / 32), total = bh * ((sq + 127) / 128);
+    const size_t full = total / cus * cus, rest = total - full, tiles = (sk + 31) / 32;
+    if (d < 1 || d > 128 || bh > 65535 || sq > (size_t)INT_MAX - 256 || sk > (size_t)INT_MAX - 256 ||
+        groups < 1024 || full == 0 || rest == 0 || cus % 8 != 0 || total > (size_t)INT_MAX / 16)
+        return {0, 1, 0};
+    const size_t nqt = (sq + 127) / 128, rows = bh * sq - (full / nqt * sq + full % nqt * 128), dpad = (d + 3) & ~(size_t)3;
+    const double tile_us = 3.4 * (double)((d + 31) / 32) / 4.0;
+    size_t best = 1, best_bytes = 0;
+    double best_gain = 0.0;
+    for (size_t want = 2; want <= 8; want++) {
+        const size_t per = (tiles + want - 1) / want, s = (tiles + per - 1) / per;
+        if (per < 4 || s != want) continue;
+        const size_t bytes = s * rows * (dpad + 2) * 4;
+        const double walk = (double)((rest * s + cus - 1) / cus) * (double)per;
+        const double gain = ((double)tiles - walk) * tile_us - 1.25 * (6.0 + 2.0 * (double)bytes / 4.0e6);
+        if (gain > best_gain) best_gain = gain, best = s, best_bytes = bytes;
+    }
+    return {best > 1 ? full : 0, best, best_bytes};
+}
 
 extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* params, int kv_is_bf16, int round16, size_t bh,
                                                   hipStream_t st) {
@@ -530,6 +639,7 @@ extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* para
     if (groups < (parts == 3 ? 1024 : 2048)) ks = 2;
     if (groups < 512) ks = 4;
     if (groups <= 256 && p.sk > 256) ks = 8;
+    if (parts != 3 || !p.part_o) p.full = 0, p.splits = 1;   // (a plan has at least 1024 groups: ks is 1)
     if (d <= 32) return fv::launch_d<32>(p, parts, kv_is_bf16 != 0, ks, bh, st);
     if (d <= 64) return fv::launch_d<64>(p, parts, kv_is_bf16 != 0, ks, bh, st);
     if (d <= 96) return fv::launch_d<96>(p, parts, kv_is_bf16 != 0, ks, bh, st);

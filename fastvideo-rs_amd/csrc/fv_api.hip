@@ -111,17 +111,6 @@ size_t settle_splits(size_t nkt, size_t splits) {
     return (nkt + per - 1) / per;
 }
 
-int compute_units() {
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        return n;
-    }();
-    return cus;
-}
-
 struct MaskArgs {
     int mode = kMaskNone;
     size_t q_rows = 0, k_rows = 0, v_rows = 0;   // rows per (batch, head) plane; 0 = contiguous (sq / sk)
@@ -238,13 +227,24 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
 
 }  // namespace
 
+int fv_compute_units() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        return n;
+    }();
+    return cus;
+}
+
 // Fewer query tiles than CUs: fv_sdpa_splitkv_choose. More: they run in rounds of one per CU, and the last round costs a
 // whole walk of the keys however few tiles are left for it. Where they are few, they are shared out over the chip by key
 // ranges instead; where they are many it does not pay, because a chip that is half busy runs at a higher clock.
 // Measured on MI355X, unsplit and so, us: 24 x 3000 x 3000 x 128 (288 tiles: 256 + 32 x 5) 145 / 120, 40 x 2000 x 2000
 // x 64 (320: 256 + 64 x 4) 69 / 61, 40 x 75600 x 75600 x 128 (11840: 11776 + 64 x 4) 89600 / 88240.
 FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d) {
-    const size_t cus = (size_t)compute_units(), bm = (size_t)fv_internal_flash_block_m();
+    const size_t cus = (size_t)fv_compute_units(), bm = (size_t)fv_internal_flash_block_m();
     const size_t nqt = (sq + bm - 1) / bm, wgs = bh * nqt, nkt = (sk + 63) / 64;
     if (wgs < cus || cus % 8 != 0 || wgs > (size_t)INT_MAX / 64) {
         const size_t splits = fv_sdpa_splitkv_choose(bh, sq, sk);
@@ -353,7 +353,7 @@ size_t fv_sdpa_splitkv_workspace_bytes(size_t bh, size_t sq, size_t d, size_t sp
 }
 
 size_t fv_sdpa_splitkv_choose(size_t bh, size_t sq, size_t sk) {
-    const int cus = compute_units();
+    const int cus = fv_compute_units();
     const size_t bm = (size_t)fv_internal_flash_block_m();
     const size_t wgs = bh * ((sq + bm - 1) / bm), nkt = (sk + 63) / 64;
     if (wgs == 0 || wgs >= (size_t)cus) return 1;               // the query tiles alone fill the CUs

@@ -47,7 +47,19 @@ struct ComposedParams {
     int sq, sk, d;
     float scale;
     int vec, vec_mask;            // set by the launcher: 16-byte operand rows / mask rows
-    int nqt, total, per_xcd, by_head;   // set by the launcher: query tiles per head, items, ceil(total / 8), item order
+    int nqt, total, per_xcd, by_head;   // set by the launcher: query tiles per head, items past `full`, ceil(total / 8), item order
+    // Split tail (fv_composed_plan): the first `full` query tiles have a workgroup each, every later one `splits`, each
+    // walking split_tiles key tiles and leaving its sums (f32 [split][row][dpad], unnormalised) and its (max, sum)
+    // ([split][row][2]) for the merge kernel, for the part_rows rows of [bh * sq] from part_row0 on. 0 / 0: no tail.
+    int full, splits, split_tiles, dpad;
+    long part_row0, part_rows;
+    float* part_o;
+    float* part_ml;
+};
+
+// How a composed launch is cut (composed_fwd.hip): splits <= 1: one workgroup a query tile throughout.
+struct ComposedPlan {
+    size_t full, splits, workspace_bytes;
 };
 
 struct VsaFineParams {
@@ -176,6 +188,9 @@ extern "C" hipError_t fv_internal_launch_tile_scan3(const void* const x[3], int 
 extern "C" hipError_t fv_internal_launch_tile_qkv(const void* x, int x_is_bf16, const int* slot_src,
                                                   uint16_t* xt, size_t bh, size_t seq, size_t padded,
                                                   int dim, hipStream_t st);
+int fv_compute_units();   // of the first device used
+// How a launch on f32 operands that are not rounded (three parts) is cut where the caller has a workspace for it.
+fv::ComposedPlan fv_composed_plan(size_t bh, size_t sq, size_t sk, size_t d);
 // softmax(scale q k^T + mask) v in f32 arithmetic, head dims 1 .. 128 (composed_fwd.hip). kv_is_bf16: k and v are bf16
 // bits (else f32); round16: operands that arrive as f32 are rounded to bf16 first (RNE). A bf16 q with f32 k / v needs
 // round16 == 0 to be exact; an f32 q with bf16 k / v is rounded.

@@ -104,7 +104,8 @@ extern "C" int fv_sdpa_composed_f32(const float* q, const float* k, const float*
     const long mask_bh = mask && mask_per_bh ? (long)(sq * sk) : 0L;
     hipError_t e;
     if (d <= 128) {
-        fv::ComposedParams p{q, k, v, mask, mask_bh, out, 0, 0, (int)sq, (int)sk, (int)d, scale, 0, 0, 0, 0, 0, 0};
+        fv::ComposedParams p{q, k, v, mask, mask_bh, out, 0, 0, (int)sq, (int)sk, (int)d, scale, 0, 0, 0, 0, 0, 0,
+                             0, 1, 0, 0, 0, 0, nullptr, nullptr};
         e = fv_internal_launch_composed(&p, 0, 0, bh, (hipStream_t)stream);
         return e == hipSuccess ? FV_OK : fv_fail_hip(e, "sdpa_composed");
     }
@@ -386,7 +387,23 @@ Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::
     } else {
         fv::ComposedParams p{pq->data, pk->data, pv->data, pm ? (const float*)pm->data : nullptr,
                              mask_per_bh ? (long)(sq * sk) : 0L, out.data, pq->dtype == DType::Bf16, act16, (int)sq,
-                             (int)sk, (int)d, sc, 0, 0, 0, 0, 0, 0};
+                             (int)sk, (int)d, sc, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, nullptr, nullptr};
+        Tensor ws;
+        if (!kv16 && !act16) {
+            const fv::ComposedPlan cut = fv_composed_plan(bh, sq, sk, d);
+            if (cut.splits > 1) {
+                auto rw = st.temp({cut.workspace_bytes / 4}, DType::F32);
+                if (is_ok(rw)) {
+                    ws = std::move(std::get<Tensor>(rw));
+                    p.full = (int)cut.full, p.splits = (int)cut.splits;
+                    p.part_o = (float*)ws.data;
+                    const size_t dpad = (d + 3) & ~(size_t)3;   // (max, sum) pairs follow the sums
+                    p.part_ml = p.part_o + cut.workspace_bytes / 4 / (dpad + 2) * dpad;
+                } else {
+                    (void)hipGetLastError();   // no memory for the partial sums: one workgroup a query tile throughout
+                }
+            }
+        }
         const hipError_t e = fv_internal_launch_composed(&p, kv16, act16, bh, st);
         if (e != hipSuccess) return TensorError{"sdpa: " + rc_message(fv_fail_hip(e, "sdpa_composed")), (int)e};
     }
@@ -689,7 +706,15 @@ Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& pl
     n.out = plan.kind != Plan::Kind::Composed && act16 ? DType::Bf16 : DType::F32;
     const auto s = bhsd(q, k, v);
     const bool masked = plan.kind == Plan::Kind::Dense && plan.mask;
-    if (!s || plan.kind == Plan::Kind::Composed || masked || !fv_sdpa_supported(s->b, s->h, s->sq, s->sk, s->d)) return n;
+    if (!s) return n;
+    const bool declined = !fv_sdpa_supported(s->b, s->h, s->sq, s->sk, s->d);
+    if (plan.kind == Plan::Kind::Composed || masked || declined) {
+        const bool rounds = plan.kind != Plan::Kind::Composed && act16;
+        const bool all16 = q.dtype == DType::Bf16 && k.dtype == DType::Bf16 && v.dtype == DType::Bf16;
+        if ((plan.kind == Plan::Kind::Composed || plan.kind == Plan::Kind::Dense) && !rounds && !all16)
+            n.workspace += (fv_composed_plan(s->b * s->h, s->sq, s->sk, s->d).workspace_bytes + 255) & ~(size_t)255;
+        return n;
+    }
     for (const Tensor* t : {&q, &k, &v})
         if (t->dtype == DType::F32) n.workspace += (t->numel() * 2 + 255) & ~(size_t)255;
     if (plan.kind == Plan::Kind::Dense || plan.kind == Plan::Kind::KvWindow) {

@@ -68,7 +68,7 @@ class Tensor {
 
 // Where one call's device memory comes from, and the stream it runs on. By itself: stream-ordered allocations. A
 // caller that has buffers in hand gives them: `out` for the result (of exactly that many bytes) and a workspace for the
-// rounded copies of f32 operands and the split-KV partials; what does not fit is allocated as before. (A stream-ordered
+// rounded copies of f32 operands and the partial sums of split key ranges; what does not fit is allocated as before. (A stream-ordered
 // allocation of a result costs more than it looks: the pool gives its memory back whenever the device is waited for,
 // and mapping 100 MB anew takes 0.3 ms of host time.)
 class Mem {

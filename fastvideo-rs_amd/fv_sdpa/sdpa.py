@@ -184,9 +184,12 @@ def sdpa(q, k, v, plan):
     # (the shape of q is the result's: the library refuses anything else before it writes)
     try:
         res = torch.empty(q.shape, device=q.device, dtype=torch.bfloat16 if bf16 else torch.float32)
-        work = torch.empty(nbytes, device=q.device, dtype=torch.uint8) if nbytes else None
     except torch.cuda.OutOfMemoryError as e:
         raise TensorError(f"sdpa: device allocation failed: {e}", -2) from e   # hipErrorOutOfMemory
+    try:
+        work = torch.empty(nbytes, device=q.device, dtype=torch.uint8) if nbytes else None
+    except torch.cuda.OutOfMemoryError:
+        nbytes = 0   # the library allocates what it cannot do without, or refuses
     rc = lib.fv_rt_sdpa_into(dq, dk, dv, p, res.data_ptr(), res.numel() * (2 if bf16 else 4),
                              work.data_ptr() if nbytes else None, nbytes, _lib.stream())
     if rc != 0:

@@ -126,3 +126,47 @@ def test_scales(fv, bh, sq, sk, d, act16, scale):
         bound = 2e-6 + abs(scale) * np.sqrt(d) * 5 * 2.0**-24
         err = np.linalg.norm(out.double().cpu().numpy() - want) / np.linalg.norm(want)
         assert err <= bound, (err, bound)
+
+
+@pytest.mark.parametrize("bh,sq,sk,d", [(35, 1010, 515, 128), (18, 2000, 700, 40), (24, 1400, 900, 63), (257, 128, 1025, 96),
+                                        (12, 4096, 1000, 128)])
+@pytest.mark.parametrize("masked", ["no", "shared", "per_head"])
+def test_split_tail(fv, bh, sq, sk, d, masked):
+    """Query tiles past a multiple of the CUs, shared out by key ranges: the rows before them are those of the launch
+    that is not cut, bit for bit, the others within f32 rounding of the 64-bit sums; ranges that a row sees no key of."""
+    import torch
+    from fv_sdpa.sdpa import Plan, _PLAN_BYTES, _desc_bytes
+
+    announce(f"composed split tail bh={bh} sq={sq} sk={sk} d={d} {masked}")
+    g = torch.Generator(device="cuda").manual_seed(bh + sq + sk + d)
+    q, k, v = (torch.randn((1, bh, s, d), generator=g, device="cuda") for s in (sq, sk, sk))
+    mask = None
+    if masked != "no":
+        mask = torch.randn((1, 1 if masked == "shared" else bh, sq, sk), generator=g, device="cuda")
+        mask[..., sq // 2:, : sk // 2] = -float("inf")   # the first ranges hold no key of these rows
+        mask[..., sq - 1, : sk - 3] = -1e9
+        if masked == "per_head":
+            mask[:, -1, sq - 2] = -float("inf")          # no key at all
+    lib = fv.lib()
+    need = (fv._lib.C.c_size_t * 2)()
+    plain = _PLAN_BYTES.pack(Plan.COMPOSED, 0, 0.0, 0, 0, *(0,) * 8, -1)
+    assert lib.fv_rt_sdpa_need(*(_desc_bytes(x, "x") for x in (q, k, v)), plain, need) == 0 and need[1] > 0
+    scale = float(np.float32(1.0 / np.sqrt(d)))          # the same f32 number for both
+    got = fv.sdpa(q, k, v, Plan.composed(scale, mask))
+    whole = torch.full_like(got, float("nan"))
+    assert lib.fv_sdpa_composed_f32(q.data_ptr(), k.data_ptr(), v.data_ptr(), mask.data_ptr() if mask is not None else None,
+                                    int(masked == "per_head"), whole.data_ptr(), bh, sq, sk, d, scale,
+                                    torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    nqt = (sq + 127) // 128
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    full = bh * nqt // cus * cus
+    row0 = full // nqt * sq + full % nqt * 128
+    assert 0 < row0 < bh * sq
+    a, b = got.view(bh * sq, d), whole.view(bh * sq, d)
+    assert torch.equal(a[:row0], b[:row0])
+    h0 = row0 // sq                                      # the heads the tail touches
+    want = want64(q[:, h0:], k[:, h0:], v[:, h0:], mask[:, h0:] if masked == "per_head" else mask)
+    have = got[:, h0:].double().cpu().numpy()
+    assert np.isfinite(have).all()
+    assert np.linalg.norm(have - want) <= 2e-6 * np.linalg.norm(want)
