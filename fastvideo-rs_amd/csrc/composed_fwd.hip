@@ -401,14 +401,15 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
     }
     l_run = pair_sum(l_run);
 
-    // out = o / l for four consecutive channels from d0 on of the lane's query; l == 0 (no key): zeros
+    // out = o / l for four consecutive channels from d0 on of the lane's query; l == 0 (no key): zeros. A NaN score is not
+    // the largest of its row (max drops it) but makes l NaN, and the row with it.
     auto store4 = [&](f32x4 r, float l, float inv, int d0) {
 #pragma clang fp contract(off)
 #pragma unroll
         for (int x = 0; x < 4; x++) {
             // one Newton step on the quotient: the rounding of o / l without the division's scaling (1 <= l < 2^32)
             const float v = r[x] * inv;
-            r[x] = l > 0.f ? __builtin_fmaf(__builtin_fmaf(-v, l, r[x]), inv, v) : 0.f;
+            r[x] = l == 0.f ? 0.f : __builtin_fmaf(__builtin_fmaf(-v, l, r[x]), inv, v);
         }
         const long at = (bh * sq + qi) * (long)d + d0;
         if (p.out_is_bf16) {
@@ -530,7 +531,7 @@ __global__ __launch_bounds__(256) void composed_merge_kernel(const ComposedParam
 #pragma unroll
     for (int x = 0; x < 4; x++) {
         if (c + x >= p.d) continue;
-        const float v = l > 0.f ? r[x] / l : 0.f;
+        const float v = l == 0.f ? 0.f : r[x] / l;   // (no key: zeros; NaN stays)
         if (p.out_is_bf16) ((__bf16*)p.out)[dst + x] = (__bf16)v;
         else ((float*)p.out)[dst + x] = v;
     }

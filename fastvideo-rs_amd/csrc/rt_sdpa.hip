@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kCompThreads) void sdpa_composed_f32_kernel(
         const float m_new = fmaxf(m, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
         __syncthreads();
         const float alpha = (m == neg_inf()) ? 0.f : expf(m - m_new);
-        const float p = (j < sk && m_new != neg_inf()) ? expf(s - m_new) : 0.f;
+        const float p = j < sk ? expf(s - (m_new == neg_inf() ? 0.f : m_new)) : 0.f;   // (no key yet: e^-inf, or NaN)
         ps[tid] = p;
         float cs = p;
         for (int off = 32; off > 0; off >>= 1) cs += __shfl_xor(cs, off);
@@ -87,7 +87,7 @@ __global__ __launch_bounds__(kCompThreads) void sdpa_composed_f32_kernel(
     if (tid < d) {
         float t = 0.f;
         for (int pt = 0; pt < parts; pt++) t += accs[pt * d + tid];
-        out[(bh * sq + qi) * (long)d + tid] = l > 0.f ? t / l : 0.f;
+        out[(bh * sq + qi) * (long)d + tid] = l == 0.f ? 0.f : t / l;   // (no key: zeros; NaN stays)
     }
 }
 

@@ -170,3 +170,37 @@ def test_split_tail(fv, bh, sq, sk, d, masked):
     have = got[:, h0:].double().cpu().numpy()
     assert np.isfinite(have).all()
     assert np.linalg.norm(have - want) <= 2e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("bh,sq,sk,d,dtype", [
+    (66, 1000, 40, 64, "bf16"), (40, 500, 90, 64, "bf16"), (3, 70, 200, 64, "bf16"), (3, 70, 290, 64, "bf16"),   # 1, 2, 4, 8 shares
+    (3, 70, 200, 64, "f32"), (35, 1010, 515, 128, "f32"),   # three parts: two shares; whole tiles and a tail cut by key ranges
+    (2, 5, 300, 200, "f32")])                               # past 128 channels
+def test_nan_scores_make_nan_rows(fv, bh, sq, sk, d, dtype):
+    """A NaN in a query makes its row NaN and leaves every other row as it was, one in a key makes the rows of its head
+    NaN, and a row whose mask closes every key stays zeros."""
+    import torch
+
+    announce(f"composed NaN bh={bh} sq={sq} sk={sk} d={d} {dtype}")
+    g = torch.Generator(device="cuda").manual_seed(sq + sk)
+    q, k, v = (torch.randn((1, bh, s, d), generator=g, device="cuda").to(torch.bfloat16 if dtype == "bf16" else torch.float32)
+               for s in (sq, sk, sk))
+    mask = torch.zeros((sq, sk), device="cuda")
+    mask[3] = float("-inf")
+    plan = fv.Plan.masked(None, mask)
+    with fv.with_bf16_act(dtype == "bf16"):
+        base = fv.sdpa(q, k, v, plan)
+        rows = [(0, 0), (bh // 2, 1), (bh - 1, sq - 1)]
+        for h, r in rows:
+            q[0, h, r, d - 1] = float("nan")
+        got = fv.sdpa(q, k, v, plan)
+        k[0, bh - 1, sk // 2, 1] = float("nan")
+        keyed = fv.sdpa(q, k, v, plan)
+    torch.cuda.synchronize()
+    assert not bool(base.isnan().any()) and not bool(base[0, :, 3].any())
+    for h, r in rows:
+        assert bool(got[0, h, r].isnan().all()), (h, r)
+        base[0, h, r] = got[0, h, r]
+    assert torch.equal(got.nan_to_num(7.0), base.nan_to_num(7.0))
+    assert bool(keyed[0, bh - 1].isnan().all())
+    assert torch.equal(keyed[0, :bh - 1].nan_to_num(7.0), got[0, :bh - 1].nan_to_num(7.0))
