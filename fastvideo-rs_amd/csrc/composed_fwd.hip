@@ -5,15 +5,15 @@
 // longer heads keep the scalar kernel of rt_sdpa.hip.
 //
 // f32 on bf16 matrix cores: an f32 value is the sum of three bf16 values exactly (24 significant bits = 3 x 8, each
-// part the nearest bf16 of what the ones before it leave), and a product of two of them, x y = sum over the parts, is
+// part the nearest bf16 of what the ones before it leave; magnitudes from 2^-110 to the largest bf16 number, for the others
+// see composed_redo), and a product of two of them, x y = sum over the parts, is
 // exact in f32. Of the nine part products the six that matter are multiplied (hi.hi, hi.mid, mid.hi, mid.mid, hi.lo,
 // lo.hi): the three left out are below 2^-24 of the product, the size of one f32 rounding, and the accumulators are
 // f32. v_mfma_f32_32x32x16_bf16 has sixteen times the rate of v_mfma_f32_32x32x2_f32, so six of them cost 0.375 of the
 // one f32 product they replace. Operands that are bf16 numbers already (bf16 tensors, or f32 ones that the caller
 // wants rounded: PARTS = 1) have one part, so K Q^T is one product and P V, whose P is f32, three.
-// (Non-finite operands give NaN rows: the parts of an infinity do not add up.) Measured against the same sums in 64
-// bits, rel_l2: 5.4e-7 at 4096 x 4096 x 128, 3.9e-7 at 1024 x 1024 x 64; the v_mfma_f32_32x32x2_f32 form: 8.1e-7 and
-// 6.1e-7. Time against that form with its casts, in us: 12 x 4096 x 4096 x 128 with a shared mask (f32 operands)
+// Measured against the same sums in 64 bits, rel_l2: 5.4e-7 at 4096 x 4096 x 128, 3.9e-7 at 1024 x 1024 x 64; the
+// v_mfma_f32_32x32x2_f32 form: 8.1e-7 and 6.1e-7. Time against that form with its casts, in us: 12 x 4096 x 4096 x 128 with a shared mask (f32 operands)
 // 1376 -> 615 in 384 workgroups of two a CU, 531 with their last 128 cut in two (fv_composed_plan); 64 x 512 x 512 x 64 with a mask per
 // head (bf16; 67 MB of mask) 259 -> 25, bound by the softmax's and the splitting of P's vector instructions; 16 x 257 x
 // 257 x 80, which used to take the scalar kernel, 136 -> 10, a chain of two tiles with little to hide their latency.
@@ -112,6 +112,245 @@ constexpr int composed_lds() {
     return tiles > merge ? tiles : merge;
 }
 
+// One workgroup's item: its (batch, head) plane, query tile and key tiles; split < 0: all of them, else that key range of
+// a cut tail. Workgroup i runs on XCD i % 8. A mask of every head's own (or none): XCD x takes a contiguous eighth of the
+// (head, query tile) items, so that a head's keys and values pass through one L2. A shared mask: the query tiles go round
+// the XCDs, so that a mask row is read through one L2 for all heads.
+struct ComposedItem {
+    bool none;
+    long bh;
+    int qt, tile0, tiles, split;
+};
+template <int KS, class Params>
+FV_DEV ComposedItem composed_item(const Params& p, int item) {
+    ComposedItem r = {false, 0, 0, 0, (p.sk + 31) / 32, -1};
+    if (KS == 1 && item < p.full) {          // (full is a multiple of 8)
+        if (p.by_head) item = (item & 7) * (p.full >> 3) + (item >> 3);
+    } else {
+        if constexpr (KS == 1) item -= p.full;
+        if (p.by_head) item = (item & 7) * p.per_xcd + (item >> 3);
+        if (item >= p.total) {
+            r.none = true;
+            return r;
+        }
+        if constexpr (KS == 1) {
+            if (p.splits > 1) {
+                const int tile = item / p.splits;
+                r.split = item - tile * p.splits;
+                item = tile;
+                r.tile0 = r.split * p.split_tiles;
+                r.tiles = min(p.split_tiles, r.tiles - r.tile0);
+            }
+            item += p.full;
+        }
+    }
+    r.bh = item / p.nqt;
+    r.qt = item - (int)r.bh * p.nqt;
+    return r;
+}
+
+// Unmasked scores are compared unscaled, so the scale's sign goes into Q and its magnitude into the exponent; a scale of
+// zero makes Q zero. With a mask the scores are s * scale + mask before they are compared.
+template <class Params>
+FV_DEV float composed_q_mul(const Params& p) {
+    return p.mask || p.scale > 0.f ? 1.f : p.scale < 0.f ? -1.f : p.scale;
+}
+template <class Params>
+FV_DEV float composed_to_log2(const Params& p) {
+    return p.mask || p.scale == 0.f ? 1.4426950408889634f : __builtin_fabsf(p.scale) * 1.4426950408889634f;
+}
+
+// The additive mask of the lane's 16 keys, four consecutive ones per load where rows allow it.
+FV_DEV void load_mask(const float* mr, int vec, int kv0, int h, int sk, f32x16& mk) {
+    if (!mr) return;
+    if (vec) {
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const f32x4 t = *reinterpret_cast<const f32x4*>(mr + min(kv0 + 8 * g + 4 * h, sk - 4));
+#pragma unroll
+            for (int x = 0; x < 4; x++) mk[4 * g + x] = t[x];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; i++) mk[i] = mr[min(kv0 + 8 * (i >> 2) + 4 * h + (i & 3), sk - 1)];
+    }
+}
+
+// out = o / l for four consecutive channels from d0 on of query qi; l == 0 (no key): zeros. A NaN score is not the largest
+// of its row (max drops it) but makes l NaN, and the row with it. PLAIN: o may be infinite (otherwise composed_redo stores
+// over it).
+template <bool PLAIN, class Params>
+FV_DEV void composed_store4(const Params& p, long bh, int qi, f32x4 r, float l, float inv, int d0) {
+#pragma clang fp contract(off)
+    const int d = p.d;
+    const bool vec = p.vec != 0;
+#pragma unroll
+    for (int x = 0; x < 4; x++) {
+        // one Newton step on the quotient: the rounding of o / l without the division's scaling (1 <= l < 2^32); it makes
+        // an infinity NaN
+        const float v = r[x] * inv;
+        const float n = __builtin_fmaf(__builtin_fmaf(-v, l, r[x]), inv, v);
+        r[x] = l == 0.f ? 0.f : !PLAIN || __builtin_fabsf(v) < __builtin_inff() ? n : v;
+    }
+    const long at = (bh * p.sq + qi) * (long)d + d0;
+    if (p.out_is_bf16) {
+        uint16_t* dst = (uint16_t*)p.out + at;
+        const bf16x4 r16 = __builtin_convertvector(r, bf16x4);
+        if (vec) {
+            if (d0 < d) *reinterpret_cast<bf16x4*>(dst) = r16;
+        } else {
+#pragma unroll
+            for (int x = 0; x < 4; x++)
+                if (d0 + x < d) reinterpret_cast<__bf16*>(dst)[x] = r16[x];
+        }
+    } else {
+        float* dst = (float*)p.out + at;
+        if (vec) {
+            if (d0 < d) *reinterpret_cast<f32x4*>(dst) = r;
+        } else {
+#pragma unroll
+            for (int x = 0; x < 4; x++)
+                if (d0 + x < d) dst[x] = r[x];
+        }
+    }
+}
+
+// A wave's rows where it has walked all keys of its item: the result, or (split >= 0: a part of the keys) the sums for the
+// merge kernel. STEP > 1: every STEP-th group of four channels from `first` on.
+template <int NO, int STEP, bool PLAIN, class Params>
+FV_DEV void composed_store_rows(const Params& p, long bh, int qi, int split, int h, float m, float l, const f32x16 (&o)[NO],
+                                int first) {
+    const long row = split * p.part_rows + (bh * p.sq + qi - p.part_row0);
+    if (split >= 0 && h == 0) *reinterpret_cast<f32x2*>(p.part_ml + 2 * row) = f32x2{m, l};
+    const float inv = __builtin_amdgcn_rcpf(l);
+#pragma unroll
+    for (int db = 0; db < NO; db++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            if (STEP > 1 && (4 * db + g) % STEP != first) continue;
+            const int d0 = 32 * db + 8 * g + 4 * h;
+            f32x4 r;
+#pragma unroll
+            for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x];
+            if (split < 0) composed_store4<PLAIN>(p, bh, qi, r, l, inv, d0);
+            else if (d0 < p.d) *reinterpret_cast<f32x4*>(p.part_o + row * p.dpad + d0) = r;
+        }
+}
+
+// Do sums of weighted values, or l, the sum of their weights, ask for the plain products below? Gathered four at a time.
+template <int PARTS>
+struct ComposedSuspect {
+    f32x4 chk = {0.f, 0.f, 0.f, 0.f};   // NaN once an infinity or a NaN has been seen
+    unsigned least = ~0u;               // the least magnitude but zero
+    FV_DEV void add(const f32x4 r) {
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            const float v = r[x];       // (a bit cast of the vector's element itself reads element 0)
+            chk[x] = __builtin_fmaf(v, 0.f, chk[x]);
+            if constexpr (PARTS == 3) least = min(least, (__builtin_bit_cast(unsigned, v) << 1) - 1u);
+        }
+    }
+    FV_DEV bool operator()(float l) const {
+        bool bad = !((chk[0] + chk[1]) + (chk[2] + chk[3]) + l * 0.f == 0.f);
+        if constexpr (PARTS == 3) bad |= least < (__builtin_bit_cast(unsigned, l * 0x1p-104f) << 1) - 1u;
+        return bad;
+    }
+};
+
+// Operands outside the range of the parts. One past the largest bf16 number (infinities, and f32 numbers above 3.396e38)
+// has parts that do not add up to it, and so has an infinity under the signed parts of P: the sums they enter are NaN. An
+// f32 value below 2^-110 has fewer than three whole parts, which costs a result its last bits when it is that small itself
+// (a score's error, 2^-134 times the other operand, stays below f32's own up to operands of 2^96). Where a query's sums
+// end with a NaN, an infinity or so small a result, its wave makes the walk over its item's keys again in plain f32
+// products (v_mfma_f32_32x32x2_f32: the two k slots of a product are the lane halves), operands straight from memory, no
+// LDS, no barrier, and stores that for the queries with `redo`: 0 times a finite number, the weights of -inf scores and
+// NaN rows come out as in the plain sums, and the other queries keep their bits. The last thing a wave does, with a softmax
+// of its own: sharing the first walk's, or keeping its values alive, cost that walk registers (12 x 1024 x 1024 x 128 in
+// f32 107 -> 117 us; so 107, and the check 0 - 2 % of a launch, 0.6 of 21 us at 12 x 300 x 300 x 80). A launch whose every
+// head holds an infinity takes 5 to 14 times as long: 12 x 4096 x 4096 x 128 3.7 ms (f32), 5.0 (bf16).
+template <int D, int PARTS, int KS, bool KV16>
+FV_DEV void composed_redo(const __attribute__((address_space(4))) ComposedParams& p, int block, int wave, int lane, bool redo) {
+    constexpr int QG = composed_waves(KS) / KS, kElem = KV16 ? 2 : 4, NO = D / 32;
+    const int h = lane >> 5, c32 = lane & 31;
+    const ComposedItem it = composed_item<KS>(p, block);
+    const int sq = p.sq, sk = p.sk, d = p.d, qi = it.qt * (32 * QG) + (wave % QG) * 32 + c32;
+    const bool q_ok = qi < sq, vec = p.vec != 0, q16 = p.q_is_bf16 != 0;
+    const long qrow = (it.bh * sq + (q_ok ? qi : 0)) * d;
+    const char* kb = (const char*)p.k + it.bh * sk * (long)d * kElem;
+    const char* vb = (const char*)p.v + it.bh * sk * (long)d * kElem;
+    const char* qr = (const char*)p.q + qrow * (q16 ? 2 : 4);
+    const float* mr = p.mask ? p.mask + it.bh * p.mask_bh + (long)(q_ok ? qi : 0) * sk : nullptr;
+    const float q_mul = composed_q_mul(p), to_log2 = composed_to_log2(p), scale = p.scale;
+    f32x16 o[NO];
+#pragma unroll
+    for (int db = 0; db < NO; db++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[db][i] = 0.f;
+    float m_run = neg_inf(), l_run = 0.f;
+    auto operand = [&](f32x8 x) {
+        if constexpr (PARTS == 1) return __builtin_convertvector(__builtin_convertvector(x, bf16x8), f32x8);
+        else return x;
+    };
+#pragma unroll 1
+    for (int t = 0; t < it.tiles; t++) {
+        const int kv0 = (it.tile0 + t) * 32;
+        f32x16 mk, s;
+        load_mask(mr, p.vec_mask, kv0, h, sk, mk);
+#pragma unroll
+        for (int i = 0; i < 16; i++) s[i] = 0.f;
+        const char* krow = kb + (long)min(kv0 + c32, sk - 1) * d * kElem;
+#pragma unroll 1
+        for (int c = 0; c < D; c += 16) {
+            const f32x8 a = operand(load8_f32<KV16>(krow, c + 8 * h, d, vec));
+            f32x8 b = q16 ? load8_f32<true>(qr, c + 8 * h, d, vec) : load8_f32<false>(qr, c + 8 * h, d, vec);
+            if (!q_ok) b = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            b = operand(b * q_mul);
+#pragma unroll
+            for (int x = 0; x < 8; x++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(a[x], b[x], s, 0, 0, 0);
+        }
+        float mx = neg_inf(), ls = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            if (mr) s[i] = __builtin_fmaf(s[i], scale, mk[i]);
+            if (kv0 + 8 * (i >> 2) + 4 * h + (i & 3) >= sk) s[i] = neg_inf();
+            mx = __builtin_fmaxf(mx, s[i]);
+        }
+        const float m_new = __builtin_fmaxf(m_run, pair_max(mx));
+        const float alpha = m_run == neg_inf() ? 0.f : fast_exp2((m_run - m_new) * to_log2);
+        const float off = m_new == neg_inf() ? 0.f : m_new;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            s[i] = fast_exp2((s[i] - off) * to_log2);
+            ls += s[i];
+        }
+        m_run = m_new;
+        l_run = l_run * alpha + ls;
+#pragma unroll
+        for (int db = 0; db < NO; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) o[db][i] *= alpha;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int key = kv0 + 8 * (i >> 2) + 4 * h + (i & 3);
+            const char* vrow = vb + (long)min(key, sk - 1) * d * kElem;
+#pragma unroll
+            for (int db = 0; db < NO; db++) {
+                const int c = 32 * db + c32;
+                float a = 0.f;
+                if (key < sk && c < d) {
+                    if constexpr (KV16) a = bf16_bits_to_f32(((const uint16_t*)vrow)[c]);
+                    else a = ((const float*)vrow)[c];
+                }
+                if constexpr (PARTS == 1 && !KV16) a = (float)(__bf16)a;
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, s[i], o[db], 0, 0, 0);
+            }
+            asm volatile("" ::: "memory");   // (few loads in flight, few registers)
+        }
+    }
+    l_run = pair_sum(l_run);
+    if (redo) composed_store_rows<NO, KS, true>(p, it.bh, qi, it.split, h, m_run, l_run, o, wave / QG);
+}
+
 template <int D, int PARTS, int KS, bool KV16>
 __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kernel(const ComposedParams p) {
     static_assert(D % 32 == 0 && (PARTS == 1 || PARTS == 3) && (KS == 1 || KS == 2 || KS == 4 || KS == 8) &&
@@ -134,38 +373,15 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
     lds_u8* kt = (lds_u8*)csm + ks * (PARTS * (kKP + kVP));
     lds_u8* vt = kt + PARTS * kKP;
     const int sq = p.sq, sk = p.sk, d = p.d;
-    // Workgroup i runs on XCD i % 8. A mask of every head's own (or none): XCD x takes a contiguous eighth of the (head,
-    // query tile) items, so that a head's keys and values pass through one L2. A shared mask: the query tiles go round
-    // the XCDs, so that a mask row is read through one L2 for all heads.
-    int item = blockIdx.x, tile0 = 0, split = -1;
-    int tiles = (p.sk + 31) / 32;
-    if (KS == 1 && item < p.full) {          // (full is a multiple of 8)
-        if (p.by_head) item = (item & 7) * (p.full >> 3) + (item >> 3);
-    } else {
-        if constexpr (KS == 1) item -= p.full;
-        if (p.by_head) item = (item & 7) * p.per_xcd + (item >> 3);
-        if (item >= p.total) return;
-        if constexpr (KS == 1) {
-            if (p.splits > 1) {
-                const int tile = item / p.splits;
-                split = item - tile * p.splits;
-                item = tile;
-                tile0 = split * p.split_tiles;
-                tiles = min(p.split_tiles, tiles - tile0);
-            }
-            item += p.full;
-        }
-    }
-    const long bh = item / p.nqt;
-    const int qt = item - (int)bh * p.nqt;
+    const ComposedItem it = composed_item<KS>(p, blockIdx.x);
+    if (it.none) return;
+    const long bh = it.bh;
+    const int qt = it.qt, tile0 = it.tile0, tiles = it.tiles, split = it.split;
     const bool vec = p.vec != 0;
     const int qi = qt * (32 * QG) + qg * 32 + c32;   // this lane's query
     const bool q_ok = qi < sq;
     const float NEG = neg_inf();
-    // Unmasked scores are compared unscaled, so the scale's sign goes into Q and its magnitude into the exponent; a
-    // scale of zero makes Q zero.
-    const float q_mul = p.mask || p.scale > 0.f ? 1.f : p.scale < 0.f ? -1.f : p.scale;
-    const float to_log2 = p.mask || p.scale == 0.f ? 1.4426950408889634f : __builtin_fabsf(p.scale) * 1.4426950408889634f;
+    const float q_mul = composed_q_mul(p), to_log2 = composed_to_log2(p);
     const char* kb = (const char*)p.k + bh * sk * (long)d * (KV16 ? 2 : 4);
     const char* vb = (const char*)p.v + bh * sk * (long)d * (KV16 ? 2 : 4);
     const float* mr = p.mask ? p.mask + bh * p.mask_bh + (long)(q_ok ? qi : 0) * sk : nullptr;
@@ -234,22 +450,6 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
         }
     };
 
-    // The additive mask of the lane's 16 keys, four consecutive ones per load where rows allow it.
-    auto load_mask = [&](int kv0, f32x16& mk) {
-        if (!mr) return;
-        if (p.vec_mask) {
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const f32x4 t = *reinterpret_cast<const f32x4*>(mr + min(kv0 + 8 * g + 4 * h, sk - 4));
-#pragma unroll
-                for (int x = 0; x < 4; x++) mk[4 * g + x] = t[x];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16; i++) mk[i] = mr[min(kv0 + 8 * (i >> 2) + 4 * h + (i & 3), sk - 1)];
-        }
-    };
-
     // A tile belongs to one wave where every wave walks keys of its own: its LDS writes and reads complete in order.
     auto tile_barrier = [&]() {
         if constexpr (KS >= 4) __builtin_amdgcn_wave_barrier();
@@ -276,7 +476,7 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
     f32x16 mk;
     load_units(kb, (tile0 + ks) * 32, ku);
     load_units(vb, (tile0 + ks) * 32, vu);
-    load_mask((tile0 + ks) * 32, mk);
+    load_mask(mr, p.vec_mask, (tile0 + ks) * 32, h, sk, mk);
 
     // Q operand, in parts: this lane's query, d = 16 j + 8 h ..
     bf16x8 qf[PARTS][NC];
@@ -365,7 +565,7 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
                 }
             }
             // the next tile's mask, in flight under the rest of this tile (rows past the end: nothing)
-            if (step + 1 < steps) load_mask(kv0 + 32 * KS, mk);
+            if (step + 1 < steps) load_mask(mr, p.vec_mask, kv0 + 32 * KS, h, sk, mk);
             // ---- O^T += V^T P^T, 16 keys at a time ----
 #pragma unroll
             for (int t = 0; t < 2; t++) {
@@ -401,66 +601,15 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
     }
     l_run = pair_sum(l_run);
 
-    // out = o / l for four consecutive channels from d0 on of the lane's query; l == 0 (no key): zeros. A NaN score is not
-    // the largest of its row (max drops it) but makes l NaN, and the row with it.
-    auto store4 = [&](f32x4 r, float l, float inv, int d0) {
-#pragma clang fp contract(off)
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-            // one Newton step on the quotient: the rounding of o / l without the division's scaling (1 <= l < 2^32)
-            const float v = r[x] * inv;
-            r[x] = l == 0.f ? 0.f : __builtin_fmaf(__builtin_fmaf(-v, l, r[x]), inv, v);
-        }
-        const long at = (bh * sq + qi) * (long)d + d0;
-        if (p.out_is_bf16) {
-            uint16_t* dst = (uint16_t*)p.out + at;
-            const bf16x4 r16 = __builtin_convertvector(r, bf16x4);
-            if (vec) {
-                if (d0 < d) *reinterpret_cast<bf16x4*>(dst) = r16;
-            } else {
-#pragma unroll
-                for (int x = 0; x < 4; x++)
-                    if (d0 + x < d) reinterpret_cast<__bf16*>(dst)[x] = r16[x];
-            }
-        } else {
-            float* dst = (float*)p.out + at;
-            if (vec) {
-                if (d0 < d) *reinterpret_cast<f32x4*>(dst) = r;
-            } else {
-#pragma unroll
-                for (int x = 0; x < 4; x++)
-                    if (d0 + x < d) dst[x] = r[x];
-            }
-        }
-    };
-
+    ComposedSuspect<PARTS> suspect;
+    bool redo;
     if constexpr (KS == 1) {
-        if (!q_ok) return;
-        if (split >= 0) {                    // sums of a part of the keys, for the merge kernel
-            const long row = split * p.part_rows + (bh * sq + qi - p.part_row0);
-            if (h == 0) *reinterpret_cast<f32x2*>(p.part_ml + 2 * row) = f32x2{m_run, l_run};
-#pragma unroll
-            for (int db = 0; db < NO; db++)
-#pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int d0 = 32 * db + 8 * g + 4 * h;
-                    f32x4 r;
-#pragma unroll
-                    for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x];
-                    if (d0 < d) *reinterpret_cast<f32x4*>(p.part_o + row * p.dpad + d0) = r;
-                }
-            return;
-        }
-        const float inv = __builtin_amdgcn_rcpf(l_run);
 #pragma unroll
         for (int db = 0; db < NO; db++)
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                f32x4 r;
-#pragma unroll
-                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x];
-                store4(r, l_run, inv, 32 * db + 8 * g + 4 * h);
-            }
+            for (int g = 0; g < 4; g++) suspect.add(f32x4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]});
+        redo = pair_max(suspect(l_run) ? 1.f : 0.f) > 0.f;   // (a query is a pair of lanes)
+        if (q_ok) composed_store_rows<NO, 1, false>(p, bh, qi, split, h, m_run, l_run, o, 0);
     } else {
         // Merge of a query's KS shares, every wave its part of the channels: all leave O, max and sum in LDS (over the
         // tiles, which every wave is done with), each adds up every KS-th group of four registers over the shares.
@@ -490,7 +639,6 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
             w[t] = ml[t][0] == NEG ? 0.f : fast_exp2((ml[t][0] - m_all) * to_log2);
             l = __builtin_fmaf(ml[t][1], w[t], l);
         }
-        if (!q_ok) return;
         const float inv = __builtin_amdgcn_rcpf(l);
 #pragma unroll 1
         for (int gi = ks; gi < D / 8; gi += KS) {
@@ -501,8 +649,20 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
 #pragma unroll
                 for (int x = 0; x < 4; x++) r[x] = __builtin_fmaf(x4[x], w[t], r[x]);
             }
-            store4(r, l, inv, 8 * gi + 4 * h);
+            suspect.add(r);
+            if (q_ok) composed_store4<false>(p, bh, qi, r, l, inv, 8 * gi + 4 * h);
         }
+        redo = suspect(l);
+    }
+    redo &= q_ok;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(redo) != 0, 0)) {
+        __builtin_amdgcn_s_waitcnt(0);   // (behind the stores above; each wave for the channels it has stored)
+        // (nothing of the first walk is kept alive for this: indices counted anew, arguments read again from their segment)
+        using ConstParams = const __attribute__((address_space(4))) ComposedParams;
+        ConstParams* again = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
+        int lane2 = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), wave2 = wave, block = blockIdx.x;
+        asm volatile("" : "+v"(lane2), "+s"(wave2), "+s"(block), "+s"(again));
+        composed_redo<D, PARTS, KS, KV16>(*again, block, wave2, lane2, redo);
     }
 }
 
@@ -514,7 +674,7 @@ __global__ __launch_bounds__(256) void composed_merge_kernel(const ComposedParam
     const long row = i / d4;
     const int c = (int)(i - row * d4) * 4;
     if (row >= p.part_rows) return;
-    const float to_log2 = p.mask || p.scale == 0.f ? 1.4426950408889634f : __builtin_fabsf(p.scale) * 1.4426950408889634f;
+    const float to_log2 = composed_to_log2(p);
     float m = neg_inf(), l = 0.f;
     for (int t = 0; t < p.splits; t++) m = __builtin_fmaxf(m, p.part_ml[2 * (t * p.part_rows + row)]);
     f32x4 r = {0.f, 0.f, 0.f, 0.f};

@@ -204,3 +204,70 @@ def test_nan_scores_make_nan_rows(fv, bh, sq, sk, d, dtype):
     assert torch.equal(got.nan_to_num(7.0), base.nan_to_num(7.0))
     assert bool(keyed[0, bh - 1].isnan().all())
     assert torch.equal(keyed[0, :bh - 1].nan_to_num(7.0), got[0, :bh - 1].nan_to_num(7.0))
+
+
+def plain64(q, k, v, mask):
+    """The plain sums in 64 bits, with what infinities and NaN make of them; a row without a key is zeros."""
+    q, k, v = (x.double().cpu().numpy() for x in (q, k, v))
+    with np.errstate(all="ignore"):
+        s = q @ k.swapaxes(-1, -2) / np.sqrt(q.shape[-1]) + mask.double().cpu().numpy()
+        m = s.max(axis=-1, keepdims=True)
+        e = np.exp(s - np.where(m == -np.inf, 0.0, m))
+        l = e.sum(axis=-1, keepdims=True)
+        return np.where(l == 0, 0.0, (e @ v) / l)
+
+
+MAX = float(np.finfo(np.float32).max)
+OUT_OF_RANGE = {   # name: (what to do to q, k, v of shape [.., s, d]; key 5 is closed)
+    "v_max_closed": lambda q, k, v: v[..., 5, 0].fill_(MAX) and v[..., 5, 1].fill_(-MAX),
+    "v_inf_closed": lambda q, k, v: v[..., 5, 2].fill_(float("inf")),
+    "v_inf_open": lambda q, k, v: v[..., 6, 1].fill_(float("-inf")),
+    "k_max_closed": lambda q, k, v: (q[..., 3].mul_(2.0 ** -10), k[..., 5, 3].fill_(MAX)),
+    "k_inf_open": lambda q, k, v: (q[..., 1].abs_().add_(0.5), k[..., 7, 1].fill_(float("-inf"))),   # scores of -inf: weight 0
+    "q_inf": lambda q, k, v: q[..., 9, 1].fill_(float("inf")),
+    "v_tiny": lambda q, k, v: v.mul_(2.0 ** -118),
+    "v_tiny_channel": lambda q, k, v: v[..., 3].mul_(2.0 ** -118),
+    "v_huge": lambda q, k, v: v.mul_(2.0 ** 115),
+    "qk_apart": lambda q, k, v: (q.mul_(2.0 ** -105), k.mul_(2.0 ** 105)),
+}
+
+
+@pytest.mark.parametrize("case", OUT_OF_RANGE)
+@pytest.mark.parametrize("bh,sq,sk,d,kinds", [
+    (3, 70, 200, 72, "f32"), (2, 40, 70, 33, "f32"), (35, 1010, 515, 128, "f32"),    # three parts; the last: whole tiles and a cut tail
+    (3, 70, 290, 64, "round"), (66, 1000, 40, 96, "round"),
+    (66, 1000, 40, 64, "bf16"), (40, 500, 90, 128, "bf16"), (3, 70, 200, 80, "bf16"), (3, 70, 290, 30, "bf16")])
+def test_operands_outside_the_range_of_the_parts(fv, bh, sq, sk, d, kinds, case):
+    """Infinities, f32 numbers past the largest bf16 number and values below bf16's subnormals: what the plain f32 sums give,
+    in the rows and channels they concern and nowhere else (a closed key's finite values do not count, whatever they are).
+    Twice 2e-6 and 2e-3, the bounds above, as a channel alone has larger relative errors than all together (a tiny bf16
+    result, 2^-122, adds its subnormals' 2^-134: 2e-4)."""
+    import torch
+
+    announce(f"composed out of range bh={bh} sq={sq} sk={sk} d={d} {kinds} {case}")
+    g = torch.Generator(device="cuda").manual_seed(sq + sk + d)
+    q, k, v = (torch.randn((1, bh, s, d), generator=g, device="cuda") for s in (sq, sk, sk))
+    OUT_OF_RANGE[case](*(x[:, bh - 1:] for x in (q, k, v)))     # in the last head only
+    if kinds == "bf16":
+        q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    mask = torch.zeros((sq, sk), device="cuda")
+    mask[:, 5] = float("-inf")
+    act16 = kinds != "f32"
+    with fv.with_bf16_act(act16):
+        got = fv.sdpa(q, k, v, fv.Plan.masked(None, mask))
+    torch.cuda.synchronize()
+    heads = [0, bh - 1]
+    r16 = (lambda x: x.to(torch.bfloat16)) if act16 else (lambda x: x)
+    want = plain64(*(r16(x[0, heads]) for x in (q, k, v)), mask)
+    got = got[0, heads].double().cpu().numpy()
+    for i, name in enumerate(("an untouched head", case)):
+        g_, w = got[i], want[i]
+        assert np.array_equal(np.isnan(g_), np.isnan(w)), name
+        inf = np.isinf(w)
+        assert np.array_equal(g_[inf], w[inf]) and np.array_equal(np.isinf(g_), inf), name
+        fin = np.isfinite(w)
+        for col in range(d):                                  # by channel: a tiny one does not hide behind the others
+            f = fin[:, col]
+            if f.any():
+                err = np.linalg.norm(g_[f, col] - w[f, col]) / np.linalg.norm(w[f, col])
+                assert err < (4e-3 if act16 else 4e-6), (name, col, err)
