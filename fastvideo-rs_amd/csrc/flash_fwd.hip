@@ -499,7 +499,7 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
                         global_store<f32x4>(po + 32 * db + 8 * g + 4 * h, r);
                     }
                 if (h == 0)
-                    p.part_lse[prow] = l_tot > 0.f ? st.template log2_offset<!LOG2DOM>(sl2) + __builtin_log2f(l_tot) : NEG;
+                    p.part_lse[prow] = l_tot == 0.f ? NEG : st.template log2_offset<!LOG2DOM>(sl2) + __builtin_log2f(l_tot);   // (NaN stays)
             }
             return true;
         }
@@ -593,10 +593,15 @@ __global__ __launch_bounds__(256) void splitkv_merge_kernel(const float* __restr
     const size_t row = i / d4;
     const int c = (int)(i - row * d4) * 4;
     float m = neg_inf();
-    for (int s = 0; s < splits; s++) m = __builtin_fmaxf(m, part_lse[(size_t)s * rows + row]);
+    bool nan = false;   // (a split whose sum is NaN: max drops it)
+    for (int s = 0; s < splits; s++) {
+        const float lse = part_lse[(size_t)s * rows + row];
+        m = __builtin_fmaxf(m, lse);
+        nan |= lse != lse;
+    }
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     float wsum = 0.f;
-    if (m != neg_inf()) {
+    if (m != neg_inf() || nan) {
         for (int s = 0; s < splits; s++) {
             const float w = fast_exp2(part_lse[(size_t)s * rows + row] - m);
             const f32x4 o = *reinterpret_cast<const f32x4*>(part_o + ((size_t)s * rows + row) * d + c);
@@ -605,7 +610,7 @@ __global__ __launch_bounds__(256) void splitkv_merge_kernel(const float* __restr
             for (int x = 0; x < 4; x++) acc[x] += w * o[x];
         }
     }
-    const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
+    const float inv = wsum == 0.f ? 0.f : 1.f / wsum;
 #pragma unroll
     for (int x = 0; x < 4; x++) acc[x] *= inv;
     if constexpr (OUT16) {

@@ -129,3 +129,32 @@ def test_last_round_of_tiles_split(fv, oracle, bh, sq, sk, d, act16):
     heads = np.array(sorted({0, row0 // sq, bh - 1}))
     assert_parity(got[torch.from_numpy(heads).cuda()].float().cpu().numpy(),
                   oracle.sdpa_composed(q[heads], k[heads], v[heads]), f"splitkv_last_round_{bh}_{sq}_{sk}_{d}")
+
+
+@pytest.mark.parametrize("bh,sq,sk,d", [(38, 1700, 2100, 128), (37, 1650, 1600, 64),   # the last round of tiles split
+                                        (2, 100, 3000, 128), (3, 257, 2049, 64)])      # every tile split
+@pytest.mark.parametrize("act16", [False, True])
+def test_nan_rows_stay_nan(fv, bh, sq, sk, d, act16):
+    """A NaN in a query makes its row NaN, one in a key the rows of its head, in split and unsplit tiles alike."""
+    import torch
+
+    announce(f"splitkv NaN bh={bh} sq={sq} sk={sk} d={d} act16={act16}")
+    q, k, v = (to_dev_bf16(x) for x in qkv(5 + sq, bh, sq, sk, d))
+    rows = [(0, 3), (bh // 2, sq - 1), (bh - 1, 0), (bh - 1, sq - 2)]
+    for h, r in rows:
+        q[h, r, d - 1] = float("nan")
+    want = torch.zeros((bh, sq, d), dtype=torch.bool, device="cuda")
+    for h, r in rows:
+        want[h, r] = True
+    with fv.with_bf16_act(act16):
+        got = fv.sdpa(q[None], k[None], v[None], fv.Plan.dense())[0]
+        for h in (0, bh - 1):
+            k[h, sk // 2, 1] = float("nan")
+            want[h] = True
+        keyed = fv.sdpa(q[None], k[None], v[None], fv.Plan.dense())[0]
+    torch.cuda.synchronize()
+    first = torch.zeros_like(want)
+    for h, r in rows:
+        first[h, r] = True
+    assert torch.equal(got.isnan(), first)
+    assert torch.equal(keyed.isnan(), want)
