@@ -297,14 +297,15 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
                                      window->video_start, window->frame_tokens, window->frames, window->chunk,
                                      window->radius, st);
     else {
-        // query tiles that do not fill the CUs, or the last round of them: split the keys over more workgroups
-        const FvSplitPlan plan = fv_split_plan(s->b * s->h, s->sq, s->sk, s->d);
+        // query tiles that do not fill the CUs, or the last round of them: split the keys over more workgroups. Where the partial
+        // results get no memory the launch is made unsplit.
+        FvSplitPlan plan = fv_split_plan(s->b * s->h, s->sq, s->sk, s->d);
         Tensor ws;
         if (plan.splits > 1) {
             auto rw = st.temp({plan.workspace_bytes / 4}, DType::F32);
-            if (!is_ok(rw)) return std::get<TensorError>(rw);
-            ws = std::move(std::get<Tensor>(rw));
+            if (is_ok(rw)) ws = std::move(std::get<Tensor>(rw));
         }
+        if (!ws.data) plan.full = 0, plan.splits = 1, plan.workspace_bytes = 0;
         rc = fv_dense_planned(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc, q.plane_rows,
                               k.plane_rows, v.plane_rows, plan, ws.data, ws.data ? ws.numel() * 4 : 0, st);
     }
@@ -393,14 +394,12 @@ Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::
             const fv::ComposedPlan cut = fv_composed_plan(bh, sq, sk, d);
             if (cut.splits > 1) {
                 auto rw = st.temp({cut.workspace_bytes / 4}, DType::F32);
-                if (is_ok(rw)) {
+                if (is_ok(rw)) {   // (no memory for the partial sums: one workgroup a query tile throughout)
                     ws = std::move(std::get<Tensor>(rw));
                     p.full = (int)cut.full, p.splits = (int)cut.splits;
                     p.part_o = (float*)ws.data;
                     const size_t dpad = (d + 3) & ~(size_t)3;   // (max, sum) pairs follow the sums
                     p.part_ml = p.part_o + cut.workspace_bytes / 4 / (dpad + 2) * dpad;
-                } else {
-                    (void)hipGetLastError();   // no memory for the partial sums: one workgroup a query tile throughout
                 }
             }
         }

@@ -223,6 +223,32 @@ def test_rt_sdpa_reports_an_allocation_failure_with_its_own_code():
     assert rc < -1 and msg.startswith("sdpa: device allocation failed: ")
 
 
+@pytest.mark.parametrize("shape,kind,launch", [
+    ((24, 3000, 3000, 128), 0, "flash_fwd_pp2<dense>"),    # the last round of query tiles split
+    ((12, 1560, 32760, 128), 0, "flash_fwd_pp2<dense>"),   # every tile split
+    ((12, 4096, 4096, 128), 1, "sdpa_composed")])          # a tail cut by key ranges
+def test_no_memory_for_partial_results_is_no_error(shape, kind, launch):
+    """Without a device every allocation fails. A call into the caller's result buffer whose split partial results get
+    no memory goes on unsplit, to the launch (which then reports that there is no device). Skipped where a GPU is
+    present: the fake operands must never reach a kernel."""
+    import torch
+    from fv_sdpa.sdpa import _FvPlan
+
+    if torch.cuda.device_count() > 0:
+        pytest.skip("needs a host without a GPU")
+    lib = fv_sdpa.lib()
+    h, sq, sk, d = shape
+    q, k, v = (_fake_tensor((1, h, s, d), kind == 0) for s in (sq, sk, sk))
+    p = _FvPlan()
+    p.kind, p.kv_flash = kind, -1
+    ref = ctypes.byref
+    need = (ctypes.c_size_t * 2)()
+    assert lib.fv_rt_sdpa_need(ref(q), ref(k), ref(v), ref(p), need) == 0 and need[1] > 0
+    rc = lib.fv_rt_sdpa_into(ref(q), ref(k), ref(v), ref(p), 0x1000, h * sq * d * (2 if need[0] else 4), None, 0, None)
+    msg = lib.fv_sdpa_last_error().decode()
+    assert rc < -1 and launch in msg and "allocation" not in msg, msg
+
+
 def test_log_level_parses_like_the_reference():
     # rt/log.rs:17-37
     parse = fv_sdpa.lib().fv_rt_parse_log_level
