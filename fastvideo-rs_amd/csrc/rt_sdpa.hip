@@ -297,11 +297,15 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
                                      window->video_start, window->frame_tokens, window->frames, window->chunk,
                                      window->radius, st);
     else {
-        // query tiles that do not fill the CUs, or the last round of them: split the keys over more workgroups. Where the partial
+        // query tiles that do not fill the CUs, or the last round of them: split the keys over more workgroups. The last
+        // round only in the caller's workspace: a stream-ordered one costs more than the split gives after every
+        // synchronisation of the device, which unmaps it: fv_rt_sdpa and a wait at 24 x 3000 x 3000 x 128 200 us unsplit,
+        // 380 - 460 so, at 12 x 8000 x 8000 x 128 415 and 570 - 750 (calls among others 150 / 140 and 367 / 373). (The
+        // composed launches gain more than that: 690 us whole, 645 cut, at 12 x 4096 x 4096 x 128.) Where the partial
         // results get no memory the launch is made unsplit.
         FvSplitPlan plan = fv_split_plan(s->b * s->h, s->sq, s->sk, s->d);
         Tensor ws;
-        if (plan.splits > 1) {
+        if (plan.splits > 1 && (plan.full == 0 || st.holds(plan.workspace_bytes))) {
             auto rw = st.temp({plan.workspace_bytes / 4}, DType::F32);
             if (is_ok(rw)) ws = std::move(std::get<Tensor>(rw));
         }
@@ -539,6 +543,7 @@ Result<Tensor> Mem::temp(std::vector<size_t> shape, DType dtype) {
     left_ -= need;
     return Tensor::borrowed(at, std::move(shape), dtype);
 }
+bool Mem::holds(size_t bytes) const { return ((bytes + 255) & ~(size_t)255) <= left_; }
 Result<Tensor> Mem::result(std::vector<size_t> shape, DType dtype) {
     if (!out_) return Tensor::alloc(std::move(shape), dtype, stream);
     size_t n = elem_size(dtype);

@@ -68,7 +68,8 @@ class Tensor {
 
 // Where one call's device memory comes from, and the stream it runs on. By itself: stream-ordered allocations. A
 // caller that has buffers in hand gives them: `out` for the result (of exactly that many bytes) and a workspace for the
-// rounded copies of f32 operands and the partial sums of split key ranges; what does not fit is allocated as before. (A stream-ordered
+// rounded copies of f32 operands and the partial sums of split key ranges; what does not fit is allocated as before, or
+// done without (the last round of tiles is split in the caller's workspace only). (A stream-ordered
 // allocation of a result costs more than it looks: the pool gives its memory back whenever the device is waited for,
 // and mapping 100 MB anew takes 0.3 ms of host time.)
 class Mem {
@@ -78,6 +79,7 @@ class Mem {
         : stream(s), out_(result), out_bytes_(result_bytes), ws_((char*)workspace), left_(workspace_bytes) {}
     operator hipStream_t() const { return stream; }
     Result<Tensor> temp(std::vector<size_t> shape, DType dtype);
+    bool holds(size_t bytes) const;   // does the rest of the caller's workspace have room for this?
     Result<Tensor> result(std::vector<size_t> shape, DType dtype);
     hipStream_t stream;
 

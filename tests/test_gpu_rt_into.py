@@ -54,6 +54,35 @@ def test_the_workspace_is_optional(fv, sq, sk, dtype):
         assert torch.equal(out, want), nbytes
 
 
+@pytest.mark.parametrize("h,sq,sk,d,kind", [(24, 3000, 700, 128, 1), (12, 4096, 1024, 64, 1), (38, 1700, 2100, 128, 0)])
+def test_a_split_tail_and_its_workspace(fv, h, sq, sk, d, kind):
+    """A composed launch on f32 operands whose last query tiles are cut by key ranges: the same bits with the whole
+    workspace, half of it and none (then allocated). A dense one whose last round is split: split in the caller's
+    workspace only, without it the unsplit launch's bits."""
+    import torch
+
+    announce(f"rt into tail {h}x{sq}x{sk}x{d} kind={kind}")
+    g = torch.Generator(device="cuda").manual_seed(sq)
+    q, k, v = (torch.randn((1, h, s, d), generator=g, device="cuda") for s in (sq, sk, sk))
+    if kind == 0:
+        q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    dq, dk, dv, p, need = parts(torch, q, k, v, kind)
+    lib, st = fv.lib(), torch.cuda.current_stream().cuda_stream
+    R = ctypes.byref
+    assert lib.fv_rt_sdpa_need(R(dq), R(dk), R(dv), R(p), need) == 0 and need[1] > 0
+    assert need[0] == (1 if kind == 0 else 0)
+    want = fv.sdpa(q, k, v, fv.Plan.dense() if kind == 0 else fv.Plan.composed())
+    whole = fv.sdpa_dense_bf16(q[0], k[0], v[0], out_bf16=True)[None] if kind == 0 else want
+    assert kind == 1 or not torch.equal(whole, want)
+    for nbytes, expect in ((need[1], want), (need[1] // 2 // 256 * 256, whole), (0, whole)):
+        out = torch.full_like(want, float("nan"))
+        work = torch.empty(max(nbytes, 256), device="cuda", dtype=torch.uint8)
+        assert lib.fv_rt_sdpa_into(R(dq), R(dk), R(dv), R(p), out.data_ptr(), out.numel() * out.element_size(),
+                                   work.data_ptr(), nbytes, st) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(out, expect), nbytes
+
+
 def test_refusals(fv):
     import torch
 
