@@ -760,7 +760,7 @@ hipError_t launch_d(const ComposedParams& p, int parts, bool kv16, int ks, size_
 fv::ComposedPlan fv_composed_plan(size_t bh, size_t sq, size_t sk, size_t d) {
     const size_t cus = (size_t)fv_compute_units(), groups = bh * ((sq + 31) / 32), total = bh * ((sq + 127) / 128);
     const size_t full = total / cus * cus, rest = total - full, tiles = (sk + 31) / 32;
-    if (d < 1 || d > 128 || bh > 65535 || sq > (size_t)INT_MAX - 256 || sk > (size_t)INT_MAX - 256 ||
+    if (d < 1 || d > 128 || bh > 65535 || sk == 0 || sq > (size_t)INT_MAX - 256 || sk > (size_t)INT_MAX - 256 ||
         groups < 1024 || full == 0 || rest == 0 || cus % 8 != 0 || total > (size_t)INT_MAX / 16)
         return {0, 1, 0};
     const size_t nqt = (sq + 127) / 128, rows = bh * sq - (full / nqt * sq + full % nqt * 128), dpad = (d + 3) & ~(size_t)3;

@@ -63,6 +63,16 @@ def test_non_bhsd_operands_are_refused(fv):
         fv.sdpa(q, q, q, fv.Plan.dense(None))
 
 
+@pytest.mark.parametrize("kind", ["dense", "composed"])
+def test_many_queries_and_no_keys_are_refused(fv, kind):
+    import torch
+
+    q = torch.zeros((1, 12, 4096, 128), device="cuda")
+    k = torch.zeros((1, 12, 0, 128), device="cuda")
+    with pytest.raises(fv.TensorError, match="no keys|null operand"):   # (torch gives an empty tensor no address)
+        fv.sdpa(q, k, k, fv.Plan.dense() if kind == "dense" else fv.Plan.composed())
+
+
 def test_vdn_window_of_no_frames_is_dense(fv, oracle):
     """A window without video rows masks nothing (rt/attn.rs:497-501): the kernel declines it
     (frames == 0) and the masked fallback runs with an all-visible mask."""

@@ -249,6 +249,30 @@ def test_no_memory_for_partial_results_is_no_error(shape, kind, launch):
     assert rc < -1 and launch in msg and "allocation" not in msg, msg
 
 
+def test_need_is_host_arithmetic_at_any_shape():
+    """fv_rt_sdpa_need answers for shapes the call itself refuses (no keys, no queries, no heads, lengths past every
+    limit), for every kind of plan and either type: no division by a count of zero, and a workspace of zero or of the
+    order of the operands. In a process of its own, which a failure would end."""
+    out = _in_subprocess("sys.path.insert(0, %r)" % os.path.join(ROOT, "tests") + """
+import ctypes, itertools
+from test_host_abi import _fake_tensor
+import fv_sdpa
+from fv_sdpa.sdpa import _FvPlan
+lib, ref, need, n = fv_sdpa.lib(), ctypes.byref, (ctypes.c_size_t * 2)(), 0
+sizes = (0, 1, 31, 128, 4096, 75600, 1 << 31, 1 << 40, 1 << 63)
+for h, sq, sk, d, bf16, kind in itertools.product((0, 1, 12, 70000), sizes, sizes, (0, 1, 64, 128, 200), (False, True), range(5)):
+    q, k = _fake_tensor((1, h, sq, d), bf16), _fake_tensor((1, h, sk, d), bf16)
+    p = _FvPlan()
+    p.kind, p.kv_flash = kind, -1
+    assert lib.fv_rt_sdpa_need(ref(q), ref(k), ref(k), ref(p), need) == 0
+    if h * d * (sq + sk) < 1 << 50:
+        assert need[1] <= 20 * 4 * h * (sq + 2 * sk + 256) * d + 4096, (h, sq, sk, d, bf16, kind, need[1])
+    n += 1
+print(n)
+""", {})
+    assert int(out) == 4 * 9 * 9 * 5 * 2 * 5
+
+
 def test_log_level_parses_like_the_reference():
     # rt/log.rs:17-37
     parse = fv_sdpa.lib().fv_rt_parse_log_level
