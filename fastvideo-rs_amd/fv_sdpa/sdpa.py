@@ -163,19 +163,34 @@ def _desc(t, name):
     return _FvTensor.from_buffer_copy(_desc_bytes(t, name))
 
 
+def _plan_bytes(plan, mask):
+    """`plan` as the bytes of a struct fv_plan; `mask`: the address of its mask's struct fv_tensor, or 0."""
+    scale, causal, window = plan.scale, plan.causal, plan.window
+    causal = (causal.block_tokens, causal.window, causal.sink) if causal is not None else (0, 0, 0)
+    window = window._args() if window is not None else (0, 0, 0, 0, 0)
+    kv_flash = -1 if plan.kv_flash is None else int(plan.kv_flash)
+    try:
+        return _PLAN_BYTES.pack(plan.kind, 0 if scale is None else 1, 0.0 if scale is None else scale, mask,
+                                1 if plan.fp8 else 0, *causal, *window, kv_flash)
+    except (struct.error, OverflowError):
+        # numbers that do not fit their fields (negative, a scale past f32): what C makes of them, for the library to judge
+        p = _FvPlan()
+        p.kind, p.fp8_first, p.kv_flash = plan.kind, 1 if plan.fp8 else 0, kv_flash
+        p.has_scale, p.scale = (0, 0.0) if scale is None else (1, float(scale))
+        p.mask = C.cast(C.c_void_p(mask), C.POINTER(_FvTensor))
+        p.block_tokens, p.window, p.sink = causal
+        p.video_start, p.frame_tokens, p.frames, p.chunk, p.radius = window
+        return bytes(p)
+
+
 def sdpa(q, k, v, plan):
     """rt/sdpa.rs:141-164. Returns a new [b, h, sq, d] tensor (bf16 under bf16 activations, else f32)."""
     lib = _lib.lib()
     dq, dk, dv = _desc_bytes(q, "q"), _desc_bytes(k, "k"), _desc_bytes(v, "v")
-    scale, causal, window = plan.scale, plan.causal, plan.window
     mask = None
     if plan.mask is not None:
         mask = C.create_string_buffer(_desc_bytes(plan.mask, "mask"), _TENSOR_BYTES.size)   # alive until the call is made
-    p = _PLAN_BYTES.pack(plan.kind, 0 if scale is None else 1, 0.0 if scale is None else scale,
-                         0 if mask is None else C.addressof(mask), 1 if plan.fp8 else 0,
-                         *((causal.block_tokens, causal.window, causal.sink) if causal is not None else (0, 0, 0)),
-                         *(window._args() if window is not None else (0, 0, 0, 0, 0)),
-                         -1 if plan.kv_flash is None else int(plan.kv_flash))
+    p = _plan_bytes(plan, 0 if mask is None else C.addressof(mask))
     need = (C.c_size_t * 2)()
     rc = lib.fv_rt_sdpa_need(dq, dk, dv, p, need)
     if rc != 0:

@@ -273,6 +273,29 @@ print(n)
     assert int(out) == 4 * 9 * 9 * 5 * 2 * 5
 
 
+@pytest.mark.parametrize("scale", [None, 0.125, 1e40, -1e300, float("inf"), np.float32(0.5), 3])
+@pytest.mark.parametrize("numbers", [(1560, 0, 1), (-1, 4, 0), (16, -2, 2**64 + 3), (np.int64(7), 2**63, 0)])
+def test_packed_plans_hold_what_the_c_structure_would(scale, numbers):
+    """Numbers that do not fit their fields are no Python errors: they reach the library as C has them."""
+    from fv_sdpa.sdpa import Plan, _FvPlan, _plan_bytes
+
+    for plan in (Plan.block_causal(scale, fv_sdpa.BlockCausal(*numbers)),
+                 Plan.vdn_window(scale, fv_sdpa.VdnWindow(numbers[1], numbers[0], 5, 0, numbers[2])), Plan.kv_window_with(True)):
+        want = _FvPlan()
+        want.kind = plan.kind
+        want.has_scale, want.scale = (0, 0.0) if plan.scale is None else (1, float(plan.scale))
+        if plan.causal is not None:
+            want.block_tokens, want.window, want.sink = numbers
+        if plan.window is not None:
+            want.video_start, want.frame_tokens, want.frames, want.chunk, want.radius = plan.window._args()
+        want.kv_flash = -1 if plan.kv_flash is None else int(plan.kv_flash)
+        got = _FvPlan.from_buffer_copy(_plan_bytes(plan, 0))
+        for name, _ in _FvPlan._fields_[:3] + _FvPlan._fields_[4:]:
+            assert getattr(got, name) == getattr(want, name), name
+    with pytest.raises(TypeError):
+        _plan_bytes(Plan.block_causal(None, fv_sdpa.BlockCausal(1.5)), 0)
+
+
 def test_log_level_parses_like_the_reference():
     # rt/log.rs:17-37
     parse = fv_sdpa.lib().fv_rt_parse_log_level
