@@ -131,10 +131,12 @@ class CausalKvCache:
         if base is None:
             start = self.pointers(layer)[1] - n if self._static else 0    # the window ends at the layer's last token
             view = _DevView(t.data - start * row_bytes, (b, h, rows if self._static else n, d), rows, bf16, self._owner)
-            base = torch.as_tensor(view, device=device)
-            base = base.view(torch.bfloat16) if bf16 else base
             if not self._static:
-                return base
+                base = torch.as_tensor(view, device=device)
+                return base.view(torch.bfloat16) if bf16 else base
+            with torch.inference_mode(False):   # kept for later calls, whatever mode the first is made in
+                base = torch.as_tensor(view, device=device)
+                base = base.view(torch.bfloat16) if bf16 else base
             self._buffers[layer, which] = base
         start = (t.data - base.data_ptr()) // row_bytes
         return base.as_strided((b, h, n, d), (h * rows * d, rows * d, d, 1), start * d)

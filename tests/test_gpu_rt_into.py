@@ -118,3 +118,21 @@ def test_windows_outlive_their_cache(fv):
     gc.collect()
     junk = torch.full((1 << 20,), 9.0, device="cuda")
     assert torch.equal(kw, want) and torch.equal(vw, -want) and float(junk[0]) == 9.0
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_windows_of_a_cache_first_written_in_inference_mode(fv, dtype):
+    """The windows a later call outside inference mode gets are ordinary tensors: autograd may save them."""
+    import torch
+
+    ft, d = 16, 64
+    cache = fv.CausalKvCache(fv.KvSpec.global_window(ft, 4), 1)
+    mk = lambda: torch.randn((1, 2, ft, d), device="cuda").to(torch.bfloat16 if dtype == "bf16" else torch.float32)
+    k = [mk() for _ in range(2)]
+    with torch.inference_mode():
+        cache.update(0, k[0], k[0], 0)
+    kw, vw = cache.update(0, k[1], k[1], ft)
+    assert not kw.is_inference() and not vw.is_inference()
+    w = torch.ones((), device="cuda", requires_grad=True, dtype=kw.dtype)
+    (w * kw).sum().backward()
+    assert torch.equal(kw, torch.cat(k, dim=2)) and w.grad is not None
