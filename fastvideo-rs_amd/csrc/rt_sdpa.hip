@@ -336,7 +336,7 @@ Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::
     if (v.shape[3] != d) return msg("sdpa: value head dim differs from the query head dim");
     const DType out_type = act16 ? DType::Bf16 : DType::F32;
     int mask_per_bh = 0;
-    Tensor tm;
+    Tensor packed, tm;
     const Tensor* pm = nullptr;
     if (mask) {
         // additive [.., sq, sk], broadcast over batch*heads or one mask per (batch, head)
@@ -348,6 +348,12 @@ Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::
         const size_t lead = mask->numel() / (sq * sk);
         if (lead == bh && lead != 1) mask_per_bh = 1;
         else if (lead != 1) return msg("sdpa: mask batch must be 1 or batch*heads");
+        if (mask->strided()) {   // a row window of longer planes: the kernels take whole ones
+            auto rc = compact(*mask, st);
+            if (!is_ok(rc)) return rc;
+            packed = std::move(std::get<Tensor>(rc));
+            mask = &packed;
+        }
         auto rm = as_f32(*mask, tm, st);
         if (!is_ok(rm)) return std::get<TensorError>(rm);
         pm = std::get<const Tensor*>(rm);
@@ -789,6 +795,8 @@ struct FlatCall {
         for (const fv_tensor* t : {fq, fk, fv_})
             if (t->plane_rows != 0 && (t->rank != 4 || t->plane_rows < t->shape[2]))
                 return fv_invalid("fv_rt_sdpa: plane_rows needs a rank-4 operand and plane_rows >= shape[2]");
+        if (p->mask && p->mask->plane_rows != 0 && (p->mask->rank != 4 || p->mask->plane_rows < p->mask->shape[2]))
+            return fv_invalid("fv_rt_sdpa: plane_rows needs a rank-4 operand and plane_rows >= shape[2]");
         q = wrap(fq), k = wrap(fk), v = wrap(fv_);
         if (p->mask) mask = wrap(p->mask);
         const Tensor* pm = p->mask ? &mask : nullptr;

@@ -271,3 +271,21 @@ def test_operands_outside_the_range_of_the_parts(fv, bh, sq, sk, d, kinds, case)
             if f.any():
                 err = np.linalg.norm(g_[f, col] - w[f, col]) / np.linalg.norm(w[f, col])
                 assert err < (4e-3 if act16 else 4e-6), (name, col, err)
+
+
+@pytest.mark.parametrize("mask_dtype", ["f32", "bf16"])
+def test_a_row_window_as_mask(fv, mask_dtype):
+    """A mask of every head's own that is a row window of longer planes (`full[:, :, a:b]`): its own rows, not the memory
+    behind its first one."""
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(8)
+    q, k, v = (torch.randn((1, 3, s, 64), generator=g, device="cuda") for s in (40, 72, 72))
+    full = torch.randn((1, 3, 100, 72), generator=g, device="cuda").to(torch.bfloat16 if mask_dtype == "bf16" else torch.float32)
+    window = full[:, :, 7:47]
+    with fv.with_bf16_act(False):
+        got = fv.sdpa(q, k, v, fv.Plan.masked(None, window))
+        want = fv.sdpa(q, k, v, fv.Plan.masked(None, window.contiguous()))
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    assert np.linalg.norm(got.double().cpu().numpy() - want64(q, k, v, window)) < 2e-6 * np.linalg.norm(want64(q, k, v, window))
