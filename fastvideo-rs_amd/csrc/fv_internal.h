@@ -37,24 +37,24 @@ struct FlashParams {
 };
 
 struct ComposedParams {
-    const void* q;                // [bh, sq, d]
-    const void* k;                // [bh, sk, d]
-    const void* v;
-    const float* mask;            // additive, [sq, sk] per mask_bh elements, or null
-    long mask_bh;                 // elements between the masks of consecutive (batch, head) planes (0: shared)
-    void* out;                    // [bh, sq, d] f32 or bf16 (RNE)
-    int q_is_bf16, out_is_bf16;
-    int sq, sk, d;
-    float scale;
-    int vec, vec_mask;            // set by the launcher: 16-byte operand rows / mask rows
-    int nqt, total, per_xcd, by_head;   // set by the launcher: query tiles per head, items past `full`, ceil(total / 8), item order
+    const void* q = nullptr;      // [bh, sq, d]
+    const void* k = nullptr;      // [bh, sk, d]
+    const void* v = nullptr;
+    const float* mask = nullptr;  // additive, [sq, sk] per mask_bh elements, or null
+    long mask_bh = 0;             // elements between the masks of consecutive (batch, head) planes (0: shared)
+    void* out = nullptr;          // [bh, sq, d] f32 or bf16 (RNE)
+    int q_is_bf16 = 0, out_is_bf16 = 0;
+    int sq = 0, sk = 0, d = 0;
+    float scale = 1.0f;
+    int vec = 0, vec_mask = 0;    // set by the launcher: 16-byte operand rows / mask rows
+    int nqt = 0, total = 0, per_xcd = 0, by_head = 0;   // set by the launcher: query tiles per head, items past `full`, ceil(total / 8), item order
     // Split tail (fv_composed_plan): the first `full` query tiles have a workgroup each, every later one `splits`, each
     // walking split_tiles key tiles and leaving its sums (f32 [split][row][dpad], unnormalised) and its (max, sum)
-    // ([split][row][2]) for the merge kernel, for the part_rows rows of [bh * sq] from part_row0 on. 0 / 0: no tail.
-    int full, splits, split_tiles, dpad;
-    long part_row0, part_rows;
-    float* part_o;
-    float* part_ml;
+    // ([split][row][2]) for the merge kernel, for the part_rows rows of [bh * sq] from part_row0 on. splits <= 1: no tail.
+    int full = 0, splits = 1, split_tiles = 0, dpad = 0;
+    long part_row0 = 0, part_rows = 0;
+    float* part_o = nullptr;
+    float* part_ml = nullptr;
 };
 
 // How a composed launch is cut (composed_fwd.hip): splits <= 1: one workgroup a query tile throughout.

@@ -104,8 +104,9 @@ extern "C" int fv_sdpa_composed_f32(const float* q, const float* k, const float*
     const long mask_bh = mask && mask_per_bh ? (long)(sq * sk) : 0L;
     hipError_t e;
     if (d <= 128) {
-        fv::ComposedParams p{q, k, v, mask, mask_bh, out, 0, 0, (int)sq, (int)sk, (int)d, scale, 0, 0, 0, 0, 0, 0,
-                             0, 1, 0, 0, 0, 0, nullptr, nullptr};
+        fv::ComposedParams p;
+        p.q = q, p.k = k, p.v = v, p.mask = mask, p.mask_bh = mask_bh, p.out = out;
+        p.sq = (int)sq, p.sk = (int)sk, p.d = (int)d, p.scale = scale;
         e = fv_internal_launch_composed(&p, 0, 0, bh, (hipStream_t)stream);
         return e == hipSuccess ? FV_OK : fv_fail_hip(e, "sdpa_composed");
     }
@@ -179,14 +180,13 @@ std::string rc_message(int rc) {
     return std::string(fv_sdpa_last_error()) + " (rc " + std::to_string(rc) + ")";
 }
 
-// A bf16 view of `x`: `x` itself when it already is bf16, else a rounded copy in `tmp` (of x * mul: the
-// product in f32, one rounding).
-Result<const Tensor*> as_bf16(const Tensor& x, Tensor& tmp, Mem& st, float mul = 1.0f) {
+// A bf16 view of `x`: `x` itself when it already is bf16, else a rounded copy in `tmp`.
+Result<const Tensor*> as_bf16(const Tensor& x, Tensor& tmp, Mem& st) {
     if (x.dtype == DType::Bf16) return &x;
     auto r = st.temp(x.shape, DType::Bf16);
     if (!is_ok(r)) return std::get<TensorError>(r);
     tmp = std::move(std::get<Tensor>(r));
-    const int rc = fv_cast_f32_bf16_scaled((const float*)x.data, (uint16_t*)tmp.data, x.numel(), mul, st);
+    const int rc = fv_cast_f32_bf16((const float*)x.data, (uint16_t*)tmp.data, x.numel(), st);
     if (rc != FV_OK) return TensorError{"cast_f32_bf16: " + rc_message(rc), rc < 0 ? -rc : 0};
     g_cast++;
     return &tmp;
@@ -396,9 +396,11 @@ Result<Tensor> composed(const Tensor& q, const Tensor& k, const Tensor& v, std::
         if (rc == FV_DECLINED) return msg("sdpa: every kernel of the route declined");
         if (rc != FV_OK) return TensorError{"sdpa: " + rc_message(rc), -rc};
     } else {
-        fv::ComposedParams p{pq->data, pk->data, pv->data, pm ? (const float*)pm->data : nullptr,
-                             mask_per_bh ? (long)(sq * sk) : 0L, out.data, pq->dtype == DType::Bf16, act16, (int)sq,
-                             (int)sk, (int)d, sc, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, nullptr, nullptr};
+        fv::ComposedParams p;
+        p.q = pq->data, p.k = pk->data, p.v = pv->data, p.q_is_bf16 = pq->dtype == DType::Bf16;
+        if (pm) p.mask = (const float*)pm->data, p.mask_bh = mask_per_bh ? (long)(sq * sk) : 0L;
+        p.out = out.data, p.out_is_bf16 = act16;
+        p.sq = (int)sq, p.sk = (int)sk, p.d = (int)d, p.scale = sc;
         Tensor ws;
         if (!kv16 && !act16) {
             const fv::ComposedPlan cut = fv_composed_plan(bh, sq, sk, d);
