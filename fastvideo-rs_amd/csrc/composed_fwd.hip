@@ -795,6 +795,10 @@ extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* para
     // 80 (6016) 284 / 331, 12 x 4096 x 4096 x 128 (1536) 606 / 1459, 24 x 1024 x 1024 x 64 (768) 71 / 62. Four and eight
     // shares take the registers of whole tiles in flight: bf16 keys up to 96 channels only (f32 keys, 12 x 700 x 700 x
     // 112: 39 / 29 / 61, with spills).
+    // Between 1024 and 2047 groups, bf16, one / two shares: 12 x 4096 x 4096 x 64 (1536) 189 / 158, 64 x 700 x 700 x 64
+    // (1408) 41.5 / 34.5, 40 x 1000 x 300 x 80 (1280) 26.4 / 23.9, 12 x 3000 x 1024 x 64 (1128) 53.2 / 43.6; but at 128
+    // channels (two shares stage every tile for half as many queries) 12 x 4096 x 4096 (1536) 264 / 283, 24 x
+    // 2000 x 2000 (1512) 142 / 151, 12 x 4000 x 300 (1500) 33.4 / 37.2: the line does not follow the head dim.
     int ks = 1;
     const size_t groups = bh * (size_t)((p.sq + 31) / 32);   // 32-query groups
     if (groups < (parts == 3 ? 1024 : 2048)) ks = 2;
