@@ -15,7 +15,7 @@
 // Measured against the same sums in 64 bits, rel_l2: 5.4e-7 at 4096 x 4096 x 128, 3.9e-7 at 1024 x 1024 x 64; the
 // v_mfma_f32_32x32x2_f32 form: 8.1e-7 and 6.1e-7. Time against that form with its casts, in us: 12 x 4096 x 4096 x 128 with a shared mask (f32 operands)
 // 1376 -> 615 in 384 workgroups of two a CU, 531 with their last 128 cut in two (fv_composed_plan); 64 x 512 x 512 x 64 with a mask per
-// head (bf16; 67 MB of mask) 259 -> 25, bound by the softmax's and the splitting of P's vector instructions; 16 x 257 x
+// head (bf16; 67 MB of mask) 306 -> 22, bound by the softmax's and the splitting of P's vector instructions; 16 x 257 x
 // 257 x 80, which used to take the scalar kernel, 136 -> 10, a chain of two tiles with little to hide their latency.
 //
 // One workgroup = 4 waves (8 with eight shares). KS waves share 32 queries, each walking every KS-th key tile with its own

@@ -78,7 +78,7 @@ def test_seeded_case(fv, oracle, kind, seed):
         want = oracle.sdpa_composed(q, np.ascontiguousarray(k[:, off:off + sk2]), np.ascontiguousarray(v[:, off:off + sk2]))
         assert_parity(got.cpu().numpy(), want, f"sweep_splitkv_{seed}")
     elif kind == "composed_masked":
-        d = int(rng.choice([32, 48, 64, 96, 128]))     # 48: the scalar kernel; the rest: fp32 MFMA
+        d = int(rng.choice([32, 48, 64, 96, 128]))     # 48: no whole 32-channel blocks
         announce(f"sweep composed bh={bh} sq={sq} sk={sk} d={d} seed={data_seed}")
         q, k, v = qkv(data_seed, bh, sq, sk, d, round_bf16=False)
         mask = (rng.standard_normal((sq, sk)) * 3).astype(np.float32)
