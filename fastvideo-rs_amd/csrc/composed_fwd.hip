@@ -783,6 +783,23 @@ extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* para
     fv::ComposedParams p = *params;
     const int d = p.d;
     if (d < 1 || d > 128 || p.sk > INT_MAX - 256 || p.sq > INT_MAX - 256) return hipErrorInvalidValue;
+    // A launch holds fewer than 2^32 work-items: heads in several where their query tiles are more (a tail is not cut there).
+    const size_t tiles = ((size_t)p.sq + 127) / 128, most = ((size_t)1 << 24) - 8;
+    if (bh > 1 && bh > most / (tiles ? tiles : 1)) {
+        const size_t heads = most / tiles ? most / tiles : 1;
+        for (size_t h0 = 0; h0 < bh; h0 += heads) {
+            fv::ComposedParams part = *params;
+            const size_t qe = h0 * (size_t)p.sq * d, ke = h0 * (size_t)p.sk * d * (kv_is_bf16 ? 2 : 4);
+            part.q = (const char*)p.q + qe * (p.q_is_bf16 ? 2 : 4);
+            part.k = (const char*)p.k + ke, part.v = (const char*)p.v + ke;
+            part.out = (char*)p.out + qe * (p.out_is_bf16 ? 2 : 4);
+            if (p.mask) part.mask = p.mask + (long)h0 * p.mask_bh;
+            part.full = 0, part.splits = 1, part.part_o = nullptr;
+            const hipError_t e = fv_internal_launch_composed(&part, kv_is_bf16, round16, heads < bh - h0 ? heads : bh - h0, st);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     const uintptr_t any = (uintptr_t)p.q | (uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.out;
     p.vec = (any & 15) == 0 && d % 8 == 0;
     p.vec_mask = p.mask && ((uintptr_t)p.mask & 15) == 0 && p.sk % 4 == 0;

@@ -289,3 +289,20 @@ def test_a_row_window_as_mask(fv, mask_dtype):
     torch.cuda.synchronize()
     assert torch.equal(got, want)
     assert np.linalg.norm(got.double().cpu().numpy() - want64(q, k, v, window)) < 2e-6 * np.linalg.norm(want64(q, k, v, window))
+
+
+def test_more_query_tiles_than_one_launch_holds(fv):
+    """65535 heads of 33000 queries are 2^24 query tiles and more, a launch of 2^32 work-items: made in parts, every head
+    in its place. One key, whose value is the result; one channel."""
+    import torch
+
+    bh, sq = 65535, 33000
+    announce(f"composed bh={bh} sq={sq}")
+    q = torch.zeros((1, bh, sq, 1), device="cuda", dtype=torch.bfloat16)
+    k = torch.ones((1, bh, 1, 1), device="cuda", dtype=torch.bfloat16)
+    v = (torch.arange(bh, device="cuda") % 251 + 1).to(torch.bfloat16).reshape(1, bh, 1, 1)
+    with fv.with_bf16_act(True):
+        got = fv.sdpa(q, k, v, fv.Plan.dense())
+    torch.cuda.synchronize()
+    for lo in range(0, bh, 8192):
+        assert bool((got[:, lo:lo + 8192] == v[:, lo:lo + 8192]).all())
