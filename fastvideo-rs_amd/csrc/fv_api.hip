@@ -298,7 +298,7 @@ int fv_cast_operands(const FvCastOperands& ops, int count, void* stream) {
     for (int i = 0; i < count; i++) most = ops.at[i].n > most ? ops.at[i].n : most;
     if (most == 0) return FV_OK;
     const size_t blocks = (most + 2047) / 2048;
-    if (blocks > (size_t)INT_MAX / 4) return decline("cast: too many elements for one launch");
+    if (blocks >= (size_t)1 << 24) return decline("cast: too many elements for one launch");   // 2^32 work-items
     hipLaunchKernelGGL(cast_operands_kernel, dim3((unsigned)blocks, (unsigned)count), dim3(256), 0, (hipStream_t)stream, ops);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FV_OK : fail_hip(e, "cast_operands");
@@ -460,15 +460,17 @@ int fv_sdpa_vdn_window_bf16(const uint16_t* q, const uint16_t* k, const uint16_t
     return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
 }
 
+// (a launch holds fewer than 2^32 work-items and the runtime does not say so: longer operands in several)
 int fv_cast_f32_bf16_scaled(const float* x, uint16_t* y, size_t n, float mul, void* stream) {
-    if (n == 0) return FV_OK;
-    const size_t threads = (n + 3) / 4;
-    const size_t blocks = (threads + 255) / 256;
-    if (blocks > (size_t)INT_MAX) return decline("cast: too many elements for one launch");
-    hipLaunchKernelGGL(cast_f32_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                       (hipStream_t)stream, x, y, n, mul);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? FV_OK : fail_hip(e, "cast_f32_bf16");
+    constexpr size_t kMost = (size_t)1 << 33;   // elements: four a thread
+    for (size_t at = 0; at < n; at += kMost) {
+        const size_t len = n - at < kMost ? n - at : kMost, blocks = (len + 1023) / 1024;
+        hipLaunchKernelGGL(cast_f32_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0,
+                           (hipStream_t)stream, x + at, y + at, len, mul);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail_hip(e, "cast_f32_bf16");
+    }
+    return FV_OK;
 }
 
 int fv_cast_f32_bf16(const float* x, uint16_t* y, size_t n, void* stream) {
@@ -476,13 +478,15 @@ int fv_cast_f32_bf16(const float* x, uint16_t* y, size_t n, void* stream) {
 }
 
 int fv_cast_bf16_f32(const uint16_t* x, float* y, size_t n, void* stream) {
-    if (n == 0) return FV_OK;
-    const size_t blocks = (n + 255) / 256;
-    if (blocks > (size_t)INT_MAX) return decline("cast: too many elements for one launch");
-    hipLaunchKernelGGL(cast_bf16_f32_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                       (hipStream_t)stream, x, y, n);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? FV_OK : fail_hip(e, "cast_bf16_f32");
+    constexpr size_t kMost = (size_t)1 << 31;   // elements: one a thread
+    for (size_t at = 0; at < n; at += kMost) {
+        const size_t len = n - at < kMost ? n - at : kMost, blocks = (len + 255) / 256;
+        hipLaunchKernelGGL(cast_bf16_f32_kernel, dim3((unsigned)blocks), dim3(256), 0,
+                           (hipStream_t)stream, x + at, y + at, len);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail_hip(e, "cast_bf16_f32");
+    }
+    return FV_OK;
 }
 
 }  // extern "C"

@@ -215,7 +215,7 @@ int kv_rope_bhsd(const void* x, DType x_dtype, size_t x_rows, const float* cos_t
     if ((((uintptr_t)x | (uintptr_t)out | (uintptr_t)cos_t | (uintptr_t)sin_t) & 15) != 0)
         return fv_invalid("rope_bhsd: operands must be 16-byte aligned");
     const size_t total = bh * s * (d / 8), blocks = (total + 255) / 256;
-    if (blocks > (size_t)INT_MAX) return fv_decline("rope_bhsd: too large for one launch");
+    if (blocks >= (size_t)1 << 24) return fv_decline("rope_bhsd: too large for one launch");
     const float sign = negate_sin ? -1.0f : 1.0f;
     const dim3 grid((unsigned)blocks), block(256);
     const bool i16 = x_dtype == DType::Bf16, o16 = out_dtype == DType::Bf16;

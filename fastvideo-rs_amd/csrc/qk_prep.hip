@@ -321,7 +321,7 @@ static int split_heads_common(const void* src, void* out, int is_bf16, size_t ba
     const size_t du = d / per16, n = batch * heads * seq * du;
     if (n == 0) return FV_OK;
     const size_t blocks = (n + 255) / 256;
-    if (blocks > (size_t)INT_MAX) return fv_decline("split_heads: too large for one launch");
+    if (blocks >= (size_t)1 << 24) return fv_decline("split_heads: too large for one launch");
     hipLaunchKernelGGL(fv::split_heads_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
                        (const fv::u32x4*)src, (fv::u32x4*)out, n, seq, heads, du, src_width / per16,
                        col_off / per16, row_map, out_rows);
@@ -351,7 +351,7 @@ int fv_merge_heads(const void* src, void* out, int is_bf16, size_t batch, size_t
     const size_t du = d / per16, n = batch * heads * seq * du;
     if (n == 0) return FV_OK;
     const size_t blocks = (n + 255) / 256;
-    if (blocks > (size_t)INT_MAX) return fv_decline("merge_heads: too large for one launch");
+    if (blocks >= (size_t)1 << 24) return fv_decline("merge_heads: too large for one launch");
     hipLaunchKernelGGL(fv::merge_heads_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
                        (const fv::u32x4*)src, (fv::u32x4*)out, n, seq, heads, du);
     hipError_t e = hipGetLastError();

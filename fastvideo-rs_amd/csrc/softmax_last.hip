@@ -110,14 +110,20 @@ __global__ __launch_bounds__(WAVES == 16 ? 1024 : 256) void softmax_last_kernel(
 
 template <int WAVES, int KEEP>
 hipError_t launch_softmax(const float* x, void* out, int out_is_bf16, size_t rows, size_t width, hipStream_t st) {
-    constexpr int RPB = WAVES == 1 ? 4 : 1;
-    const dim3 block(WAVES == 16 ? 1024 : 256);
-    const dim3 grid((unsigned)((rows + RPB - 1) / RPB));
-    if (out_is_bf16)
-        hipLaunchKernelGGL((softmax_last_kernel<WAVES, KEEP, true>), grid, block, 0, st, x, out, rows, width);
-    else
-        hipLaunchKernelGGL((softmax_last_kernel<WAVES, KEEP, false>), grid, block, 0, st, x, out, rows, width);
-    return hipGetLastError();
+    constexpr int RPB = WAVES == 1 ? 4 : 1, kThreads = WAVES == 16 ? 1024 : 256;
+    constexpr size_t kMost = ((size_t)1 << 31) / kThreads * RPB;   // rows a launch: it holds fewer than 2^32 work-items
+    for (size_t at = 0; at < rows; at += kMost) {
+        const size_t n = rows - at < kMost ? rows - at : kMost;
+        const dim3 block(kThreads), grid((unsigned)((n + RPB - 1) / RPB));
+        const float* src = x + at * width;
+        if (out_is_bf16)
+            hipLaunchKernelGGL((softmax_last_kernel<WAVES, KEEP, true>), grid, block, 0, st, src, (uint16_t*)out + at * width, n, width);
+        else
+            hipLaunchKernelGGL((softmax_last_kernel<WAVES, KEEP, false>), grid, block, 0, st, src, (float*)out + at * width, n, width);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace

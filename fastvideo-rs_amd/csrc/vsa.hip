@@ -775,21 +775,30 @@ extern "C" hipError_t fv_internal_launch_coarse(const float* qc, const float* kc
 extern "C" hipError_t fv_internal_launch_topk(const float* scores, unsigned* out, int rows, int n, int k,
                                               hipStream_t st) {
     if (n < 1 || n > kTopkMaxN) return hipErrorInvalidValue;
-    const dim3 grid((rows + kTopkRowsPerBlock - 1) / kTopkRowsPerBlock), block(64 * kTopkRowsPerBlock);
     // keys per lane: the smallest instantiated count that holds the row (624 tiles: 10)
     const int need = (n + 63) / 64;
-#define FV_TOPK(K) hipLaunchKernelGGL(vsa_topk_kernel<K>, grid, block, 0, st, scores, out, rows, n, k)
-    if (need <= 4) FV_TOPK(4);
-    else if (need <= 8) FV_TOPK(8);
-    else if (need <= 10) FV_TOPK(10);
-    else if (need <= 12) FV_TOPK(12);
-    else if (need <= 16) FV_TOPK(16);
-    else if (need <= 24) FV_TOPK(24);
-    else if (need <= 32) FV_TOPK(32);
-    else if (need <= 48) FV_TOPK(48);
-    else FV_TOPK(64);
+    constexpr int kMost = 1 << 25;   // rows a launch, 64 threads each: it holds fewer than 2^32 work-items
+    for (int at = 0; at < rows;) {
+        const int some = rows - at < kMost ? rows - at : kMost;
+        const dim3 grid((some + kTopkRowsPerBlock - 1) / kTopkRowsPerBlock), block(64 * kTopkRowsPerBlock);
+        const float* src = scores + (size_t)at * n;
+        unsigned* dst = out + (size_t)at * k;
+#define FV_TOPK(K) hipLaunchKernelGGL(vsa_topk_kernel<K>, grid, block, 0, st, src, dst, some, n, k)
+        if (need <= 4) FV_TOPK(4);
+        else if (need <= 8) FV_TOPK(8);
+        else if (need <= 10) FV_TOPK(10);
+        else if (need <= 12) FV_TOPK(12);
+        else if (need <= 16) FV_TOPK(16);
+        else if (need <= 24) FV_TOPK(24);
+        else if (need <= 32) FV_TOPK(32);
+        else if (need <= 48) FV_TOPK(48);
+        else FV_TOPK(64);
 #undef FV_TOPK
-    return hipGetLastError();
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        at += some;
+    }
+    return hipSuccess;
 }
 
 extern "C" hipError_t fv_internal_launch_tile_qkv(const void* x, int x_is_bf16, const int* slot_src,
