@@ -274,7 +274,7 @@ static int qk_norm_rope_common(const void* src, int src_is_bf16, const void* w, 
     // 16-byte lane chunks: 8 elements, never straddling a head, aligned in the source row
     if (d % 8 != 0 || col_off % 8 != 0 || src_width % 8 != 0)
         return fv_decline("qk_norm_rope: d, col_off and src_width must be multiples of 8");
-    if (batch * seq > (size_t)INT_MAX || seq > (size_t)INT_MAX || heads * d > (size_t)INT_MAX / 2 ||
+    if (seq >= (size_t)1 << 26 || batch * seq >= (size_t)1 << 26 || heads * d > (size_t)INT_MAX / 2 ||   // 64 work-items a row, fewer than 2^32 a launch
         out_rows > (size_t)INT_MAX)
         return fv_decline("qk_norm_rope: too large for one launch");
     const long rows = (long)(batch * seq);

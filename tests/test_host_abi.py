@@ -296,6 +296,17 @@ def test_packed_plans_hold_what_the_c_structure_would(scale, numbers):
         _plan_bytes(Plan.block_causal(None, fv_sdpa.BlockCausal(1.5)), 0)
 
 
+def test_scans_longer_than_one_launch_are_refused():
+    """2^32 work-items and more in a launch are cut off by the runtime without an error: these entries decline instead
+    (host arithmetic; the fake operands reach no kernel)."""
+    lib, x = fv_sdpa.lib(), 0x1000
+    seq = 1 << 26
+    assert lib.fv_split_heads_bhsd(x, x, 1, 1, seq, 4, 128, 512, 0, None) == _lib.FV_DECLINED
+    assert lib.fv_merge_heads(x, x, 1, 1, 4, seq, 128, None) == _lib.FV_DECLINED
+    assert lib.fv_rope_bhsd(x, 1, seq, x, x, 0, x, 1, seq, 4, seq, 128, None) == _lib.FV_DECLINED
+    assert lib.fv_qk_norm_rope_bhsd(x, 1, x, 0, None, None, x, 1, 1, seq, 1, 8, 8, 0, 1e-6, 1.0, None) == _lib.FV_DECLINED
+
+
 def test_log_level_parses_like_the_reference():
     # rt/log.rs:17-37
     parse = fv_sdpa.lib().fv_rt_parse_log_level
