@@ -9,7 +9,7 @@ flash kernel from HIP-event timings, and the CPU baseline (the fp32 host-math
 oracle timed on a bounded sample of query rows, extrapolated to the full call).
 
 Other workloads (--workload cross|causal|causal3|c5|c5cross|tiny|self_d64|vdn32|vsa624|vsa512|prep|layer|kvcache|
-kvcache1|composed|softmax) are for the design notes; the driver's line is the default `self`.
+kvcache1|composed|softmax) are for the design notes; the headline is the default `self`.
 """
 import argparse
 import json

@@ -242,7 +242,7 @@ int fv_compute_units() {
 // whole walk of the keys however few tiles are left for it. Where they are few, they are shared out over the chip by key
 // ranges instead; where they are many it does not pay, because a chip that is half busy runs at a higher clock.
 // Measured on MI355X, unsplit and so, us: 24 x 3000 x 3000 x 128 (288 tiles: 256 + 32 x 5) 145 / 120, 40 x 2000 x 2000
-// x 64 (320: 256 + 64 x 4) 69 / 61, 40 x 75600 x 75600 x 128 (11840: 11776 + 64 x 4) 94470 / 92960 on one box, where runs
+// x 64 (320: 256 + 64 x 4) 69 / 61, 40 x 75600 x 75600 x 128 (11840: 11776 + 64 x 4) 94470 / 92960 on one MI355X, where runs
 // of one side differ by 0.2 %, and inside the spread on another.
 FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d) {
     const size_t cus = (size_t)fv_compute_units(), bm = (size_t)fv_internal_flash_block_m();

@@ -10,7 +10,7 @@ for p in (ROOT, PKG):
     if p not in sys.path:
         sys.path.insert(0, p)
 
-# max|delta| <= 1e-2 and cosine >= 0.9999 against the
+# tolerances: max|delta| <= 1e-2 and cosine >= 0.9999 against the
 # reference's fp32 host-math SDPA on identical seeded inputs
 MAX_ABS = 1e-2
 MIN_COS = 0.9999
