@@ -712,6 +712,15 @@ Result<Tensor> sdpa_composed(const Tensor& q, const Tensor& k, const Tensor& v, 
     return composed(q, k, v, scale, mask, false, mem);
 }
 
+// Row windows of longer planes (a KV cache read in place): the fused dense kernel takes bf16 windows as they are, every
+// other path gets contiguous copies.
+static bool takes_windows(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& plan) {
+    const bool dense_like = (plan.kind == Plan::Kind::Dense && !plan.mask) ||
+                            (plan.kind == Plan::Kind::KvWindow && plan.kv_flash.value_or(causal_flash_enabled()));
+    const bool all16 = q.dtype == DType::Bf16 && k.dtype == DType::Bf16 && v.dtype == DType::Bf16;
+    return dense_like && all16 && backend() == Backend::Dense;
+}
+
 Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& plan) {
     Need n;
     const bool act16 = bf16_activations();
@@ -720,6 +729,9 @@ Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& pl
     const bool masked = plan.kind == Plan::Kind::Dense && plan.mask;
     if (!s) return n;
     const bool declined = !fv_sdpa_supported(s->b, s->h, s->sq, s->sk, s->d);
+    const bool read_in_place = takes_windows(q, k, v, plan) && !declined;
+    for (const Tensor* t : {&q, &k, &v})
+        if (t->strided() && !read_in_place) n.workspace += (t->numel() * elem_size(t->dtype) + 255) & ~(size_t)255;
     if (plan.kind == Plan::Kind::Composed || masked || declined) {
         const bool rounds = plan.kind != Plan::Kind::Composed && act16;
         const bool all16 = q.dtype == DType::Bf16 && k.dtype == DType::Bf16 && v.dtype == DType::Bf16;
@@ -738,12 +750,7 @@ Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& pl
 Result<Tensor> sdpa(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& plan, Mem st) {
     if (q.rank() != 4 || k.rank() != 4 || v.rank() != 4) return msg("sdpa expects BHSD");
     if (q.strided() || k.strided() || v.strided()) {
-        // Row windows of longer planes (a KV cache read in place). The fused dense kernel takes bf16
-        // windows as they are; every other path gets contiguous copies.
-        const bool dense_like = (plan.kind == Plan::Kind::Dense && !plan.mask) ||
-                                (plan.kind == Plan::Kind::KvWindow && plan.kv_flash.value_or(causal_flash_enabled()));
-        const bool all16 = q.dtype == DType::Bf16 && k.dtype == DType::Bf16 && v.dtype == DType::Bf16;
-        if (dense_like && all16 && backend() == Backend::Dense) {
+        if (takes_windows(q, k, v, plan)) {
             auto r = fused(q, k, v, plan.scale, bf16_activations(), nullptr, st);
             if (!is_ok(r)) return std::get<TensorError>(r);
             auto& o = std::get<std::optional<Tensor>>(r);

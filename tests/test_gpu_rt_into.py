@@ -83,6 +83,22 @@ def test_a_split_tail_and_its_workspace(fv, h, sq, sk, d, kind):
         assert torch.equal(out, expect), nbytes
 
 
+@pytest.mark.parametrize("h,sq,sk", [(38, 1700, 2100), (2, 100, 3000)])
+def test_f32_row_windows_and_the_workspace(fv, h, sq, sk):
+    """f32 keys and values that are row windows of longer planes are compacted, rounded and split like contiguous ones:
+    the workspace holds all three, the bits are the same."""
+    import torch
+
+    announce(f"rt into f32 windows {h}x{sq}x{sk}")
+    g = torch.Generator(device="cuda").manual_seed(h)
+    q = torch.randn((1, h, sq, 128), generator=g, device="cuda")
+    k, v = (torch.randn((1, h, sk + 64, 128), generator=g, device="cuda") for _ in range(2))
+    want = fv.sdpa(q, k[:, :, 16:16 + sk].contiguous(), v[:, :, :sk].contiguous(), fv.Plan.dense())
+    got = fv.sdpa(q, k[:, :, 16:16 + sk], v[:, :, :sk], fv.Plan.dense())
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
 def test_refusals(fv):
     import torch
 
