@@ -36,7 +36,7 @@
 #include <limits.h>
 
 #include "../../include/fv_sdpa_hip.h"
-#include "fv_common.h"
+#include "attn_core.h"
 #include "fv_internal.h"
 
 namespace fv {
@@ -666,6 +666,237 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
     }
 }
 
+// ---- short launches on bf16 operands --------------------------------------------------------
+// For launches whose time is one chain of latencies and not the matrix pipe. One workgroup = 32 queries of one (batch,
+// head); wave w of its KS = 8 or 4 walks the 32-key tiles w, w + KS, ... with K and V buffers, running max and sums of its
+// own, and the shares are merged through LDS: one barrier when the query rows are there, none until the merge. Tiles and
+// query rows come by LDS-DMA (whole rows: fragments straight from memory touch every row with every instruction), the
+// next K tile while the softmax runs, the next V tile behind the products. PP: parts of P, 3 for the composed plans
+// (masks, head dims in steps of 8, exact P), 1 for the fused kernels' plans (P rounded to bf16, no mask, head dims 64
+// and 128). Shader-clock stamps at 12 x 320 x 320 x 128, 13 k cycles: arguments 0.6, issue of 17 loads a wave
+// 1.6 (136 KB at 64 bytes a clock), query rows and K 2.2, two tiles 4.3, merge 3.8 (128 KB written, 128 KB read), drain
+// 0.5. us, in a graph, the kernels it replaces / this: 12 x 320 x 320 x 128 11.0 / 6.8 (flash_fwd_pp2, 24 k cycles in five phases),
+// 16 x 257 x 257 x 80 10.2 / 7.8, 12 x 668 x 668 x 128 17.8 / 9.7, 12 x 1200 x 1200 x 64 19.5 / 12.9.
+template <int NC>
+struct ShortGeo {
+    static constexpr int D = NC <= 4 ? 64 : 128;      // channels an LDS row has room for
+    using G = TileGeo<D>;
+    static constexpr int kTile = 32 * G::kRow;        // 32 rows
+    static constexpr int kIt = kTile / 1024;          // LDS-DMA instructions a tile
+    static constexpr int NO = (NC + 1) / 2;           // 32-channel blocks of the result
+};
+template <int NC, int KS>
+constexpr int short_lds() {
+    constexpr int tiles = (2 * KS + 1) * ShortGeo<NC>::kTile, merge = KS * kMergeShare<32 * ShortGeo<NC>::NO>;
+    return tiles > merge ? tiles : merge;
+}
+
+template <int NC, int PP, int KS>
+__global__ __launch_bounds__(64 * KS, NC <= 4 ? 4 : 2) void sdpa_short_kernel(const ComposedParams p) {
+    using SG = ShortGeo<NC>;
+    using G = typename SG::G;
+    constexpr int kTile = SG::kTile, kIt = SG::kIt, NO = SG::NO;
+    extern __shared__ __attribute__((aligned(16))) unsigned char csm[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, c32 = lane & 31;
+    const ComposedItem it = composed_item<KS>(p, blockIdx.x);
+    if (it.none) return;
+    const int sq = p.sq, sk = p.sk, d = PP == 1 ? SG::D : p.d, tiles = it.tiles;
+    const int rowb = 2 * d, nch = d >> 3;             // bytes and 16-byte chunks of a row in memory
+    const long bh = it.bh;
+    const int qi = it.qt * 32 + c32;
+    const bool q_ok = qi < sq;
+    const float NEG = neg_inf();
+    const char* qb = (const char*)p.q + (bh * p.q_plane + (long)it.qt * 32 * d) * 2;
+    const char* kb = (const char*)p.k + bh * p.k_plane * 2;
+    const char* vb = (const char*)p.v + bh * p.v_plane * 2;
+    lds_u8* kt = (lds_u8*)csm + wave * (2 * kTile);
+    lds_u8* vt = kt + kTile;
+    lds_u8* qs = (lds_u8*)csm + 2 * KS * kTile;
+    const int lr = lane / G::kChunks, lc = lane % G::kChunks;
+    // One instruction's rows of a tile of `rows` valid ones (the ones past them re-read the last): whole 16-byte chunks of
+    // the row, each to its swizzled place; lanes whose chunk lies past d fetch nothing. Every instruction has lanes that do.
+    auto request_one = [&](lds_u8* dst, const char* base, int rows, int it_, bool is_v) {
+        const int r = it_ * G::kRowsPerDma + lr, c = lc ^ (is_v ? G::vswz(r) : G::kswz(r));
+        const unsigned at = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst) + it_ * 1024;
+        const unsigned off = (unsigned)(min(r, rows - 1) * rowb + (c << 4));
+        if (PP == 1 || c < nch) lds_dma16_s(at, base, off);
+    };
+    auto request = [&](lds_u8* dst, const char* base, int t, bool is_v) {
+        const char* tile = base + (long)t * 32 * rowb;
+#pragma unroll
+        for (int i = 0; i < kIt; i++) request_one(dst, tile, sk - 32 * t, i, is_v);
+    };
+#pragma unroll
+    for (int i = 0; i < (kIt + KS - 1) / KS; i++)
+        if (i * KS + wave < kIt) request_one(qs, qb, sq - it.qt * 32, i * KS + wave, false);
+    if (wave < tiles) {
+        request(kt, kb, wave, false);
+        request(vt, vb, wave, true);
+    }
+    const float* mr = PP == 3 && p.mask ? p.mask + bh * p.mask_bh + (long)(q_ok ? qi : 0) * sk : nullptr;
+    f32x16 mk;
+    if (PP == 3 && wave < tiles) load_mask(mr, p.vec_mask, wave * 32, h, sk, mk);
+    if (PP == 3 && nch < 2 * NC) {   // the channels between d and the products' last: zeros, in K for each wave and in Q
+#pragma unroll
+        for (int i = 0; i < kIt; i++) {
+            const int r = i * G::kRowsPerDma + lr, c = lc ^ G::kswz(r);
+            if (c >= nch && c < 2 * NC) {
+                lds_write_b128(kt + i * 1024 + lane * 16, u32x4{0u, 0u, 0u, 0u});
+                if (wave == 0) lds_write_b128(qs + i * 1024 + lane * 16, u32x4{0u, 0u, 0u, 0u});
+            }
+        }
+    }
+    // (2 kIt loads after the query rows'; a wave without keys has no other)
+    if (wave < tiles) wait_vmcnt<2 * kIt>();
+    else wait_vmcnt<0>();
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the zeros are written
+    block_barrier();
+    const TileReadBases rb = tile_read_bases<SG::D>(lane);
+    const float q_mul = PP == 3 ? composed_q_mul(p) : 1.f, to_log2 = composed_to_log2(p);
+    bf16x8 qf[NC];
+#pragma unroll
+    for (int j = 0; j < NC; j++) {
+        qf[j] = lds_read_b128(qs + (rb.k ^ (j << 5)));
+        if (q_mul != 1.f) qf[j] = __builtin_convertvector(__builtin_convertvector(qf[j], f32x8) * q_mul, bf16x8);
+    }
+    f32x16 o[NO];
+#pragma unroll
+    for (int db = 0; db < NO; db++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[db][i] = 0.f;
+    float m_run = NEG, l_run = 0.f;
+#pragma unroll 1
+    for (int t = wave; t < tiles; t += KS) {
+        const int kv0 = 32 * t;
+        const bool more = t + KS < tiles;
+        wait_vmcnt<kIt>();                // K(t) has landed; V(t) may be in flight
+        f32x16 s;
+#pragma unroll
+        for (int i = 0; i < 16; i++) s[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NC; j++) s = mfma32(lds_read_b128(kt + (rb.k ^ (j << 5))), qf[j], s);
+        __builtin_amdgcn_s_waitcnt(0xC07F);   // (every K read has returned)
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) request(kt, kb, t + KS, false);
+        if (PP == 3 && mr) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) s[i] = __builtin_fmaf(s[i], p.scale, mk[i]);
+        }
+        if (kv0 + 32 > sk) {
+            asm volatile("");
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if (kv0 + 8 * (i >> 2) + 4 * h + (i & 3) >= sk) s[i] = NEG;
+        }
+        float mx = NEG;
+#pragma unroll
+        for (int i = 0; i < 16; i++) mx = __builtin_fmaxf(mx, s[i]);
+        const float m_new = __builtin_fmaxf(m_run, pair_max(mx));
+        const float alpha = (m_run == NEG) ? 0.f : fast_exp2((m_run - m_new) * to_log2);
+        const float off = (m_new == NEG) ? 0.f : m_new;
+        float ls = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            s[i] = fast_exp2((s[i] - off) * to_log2);
+            ls += s[i];
+        }
+        l_run = l_run * alpha + ls;
+        m_run = m_new;
+        if (t >= KS && __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+            for (int db = 0; db < NO; db++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) o[db][i] *= alpha;
+        }
+        if (PP == 3 && more) load_mask(mr, p.vec_mask, kv0 + 32 * KS, h, sk, mk);
+        if (more) wait_vmcnt<kIt>();      // V(t) has landed; K of the next tile may be in flight
+        else wait_vmcnt<0>();
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            f32x8 e;
+#pragma unroll
+            for (int x = 0; x < 8; x++) e[x] = s[8 * g + x];
+            Parts3 pp;
+            if constexpr (PP == 1) pp.p[0] = __builtin_convertvector(e, bf16x8);
+            else pp = split3(e);
+#pragma unroll
+            for (int db = 0; db < NO; db++) {
+                const lds_u8* at = vt + ((rb.v ^ (db << 6)) + 16 * g * G::kRow);
+                s16x8 w;
+                w.lo = lds_read_tr16_b64(at);
+                w.hi = lds_read_tr16_b64(at + 8 * G::kRow);
+                const bf16x8 a = __builtin_bit_cast(bf16x8, w);
+#pragma unroll
+                for (int x = PP - 1; x >= 0; x--) o[db] = mfma32(a, pp.p[x], o[db]);   // small products first
+            }
+        }
+        if (more) {
+            __builtin_amdgcn_s_waitcnt(0xC07F);   // (every V read has returned)
+            __builtin_amdgcn_sched_barrier(0);
+            request(vt, vb, t + KS, true);
+        }
+    }
+    l_run = pair_sum(l_run);
+
+    typedef __attribute__((address_space(3))) f32x4 lds_f4;
+    typedef __attribute__((address_space(3))) f32x2 lds_f2;
+    __syncthreads();   // every wave is done with its tiles
+    constexpr int kShare = kMergeShare<32 * NO>;
+    lds_u8* shares = (lds_u8*)csm;
+#pragma unroll
+    for (int db = 0; db < NO; db++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            *(lds_f4*)(shares + wave * kShare + ((4 * db + g) * 64 + lane) * 16) =
+                f32x4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
+    *(lds_f2*)(shares + wave * kShare + NO * 4096 + lane * 8) = f32x2{m_run, l_run};
+    __syncthreads();
+    float w[KS], l = 0.f, m_all = NEG;
+    f32x2 ml[KS];
+#pragma unroll
+    for (int t = 0; t < KS; t++) ml[t] = *(const lds_f2*)(shares + t * kShare + NO * 4096 + lane * 8);
+    constexpr int kOwn = (4 * NO + KS - 1) / KS;   // groups of four channels a wave adds up
+    f32x4 part[kOwn][KS];
+#pragma unroll
+    for (int i = 0; i < kOwn; i++)
+#pragma unroll
+        for (int t = 0; t < KS; t++)
+            part[i][t] = *(const lds_f4*)(shares + t * kShare + (min(wave + i * KS, 4 * NO - 1) * 64 + lane) * 16);
+#pragma unroll
+    for (int t = 0; t < KS; t++) m_all = __builtin_fmaxf(m_all, ml[t][0]);
+#pragma unroll
+    for (int t = 0; t < KS; t++) {
+        w[t] = ml[t][0] == NEG ? 0.f : fast_exp2((ml[t][0] - m_all) * to_log2);
+        l = __builtin_fmaf(ml[t][1], w[t], l);
+    }
+    const float inv = __builtin_amdgcn_rcpf(l);
+    ComposedSuspect<1> suspect;
+#pragma unroll
+    for (int i = 0; i < kOwn; i++) {
+        const int gi = wave + i * KS;
+        if (gi >= nch) break;
+        f32x4 r = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < KS; t++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) r[x] = __builtin_fmaf(part[i][t][x], w[t], r[x]);
+        if constexpr (PP == 3) suspect.add(r);
+        if (q_ok) composed_store4<PP == 1>(p, bh, qi, r, l, inv, 8 * gi + 4 * h);
+    }
+    if constexpr (PP == 3) {
+        const bool redo = suspect(l) && q_ok;
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(redo) != 0, 0)) {
+            __builtin_amdgcn_s_waitcnt(0);
+            using ConstParams = const __attribute__((address_space(4))) ComposedParams;
+            ConstParams* again = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
+            int lane2 = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), wave2 = wave, block = blockIdx.x;
+            asm volatile("" : "+v"(lane2), "+s"(wave2), "+s"(block), "+s"(again));
+            composed_redo<32 * NO, 1, KS, true>(*again, block, wave2, lane2, redo);
+        }
+    }
+}
+
 // out = sum over the splits of O 2^(m - max) / sum of l 2^(m - max), four channels a thread. HBM-bound: the
 // partial sums are read once and the result is written once.
 __global__ __launch_bounds__(256) void composed_merge_kernel(const ComposedParams p) {
@@ -745,6 +976,37 @@ hipError_t launch_d(const ComposedParams& p, int parts, bool kv16, int ks, size_
     }
     return launch_as<D, 1, 2, true>(p, bh, st);
 }
+template <int NC, int PP, int KS>
+hipError_t launch_short_as(const ComposedParams& p, size_t bh, hipStream_t st) {
+    constexpr int lds = short_lds<NC, KS>();
+    static std::atomic<unsigned long long> attr_done;
+    const hipError_t e = fv_set_max_lds_once((const void*)sdpa_short_kernel<NC, PP, KS>, lds, attr_done);
+    if (e != hipSuccess) return e;
+    ComposedParams a = p;
+    a.nqt = (p.sq + 31) / 32;
+    a.full = 0, a.splits = 1;
+    const size_t total = bh * (size_t)a.nqt;
+    if (total > ((size_t)1 << 22)) return hipErrorInvalidValue;   // (2^32 work-items a launch)
+    a.total = (int)total;
+    a.per_xcd = (int)((total + 7) / 8);
+    a.by_head = !p.mask || p.mask_bh != 0;
+    hipLaunchKernelGGL((sdpa_short_kernel<NC, PP, KS>), dim3((unsigned)(a.per_xcd * 8)), dim3(64 * KS), lds, st, a);
+    return hipGetLastError();
+}
+template <int NC, int PP>
+hipError_t launch_short_nc(const ComposedParams& p, int waves, size_t bh, hipStream_t st) {
+    return waves == 8 ? launch_short_as<NC, PP, 8>(p, bh, st) : launch_short_as<NC, PP, 4>(p, bh, st);
+}
+template <int PP>
+hipError_t launch_short(const ComposedParams& p, int waves, size_t bh, hipStream_t st) {
+    if (p.d <= 64) return launch_short_nc<4, PP>(p, waves, bh, st);
+    if constexpr (PP == 3) {
+        if (p.d <= 80) return launch_short_nc<5, PP>(p, waves, bh, st);
+        if (p.d <= 96) return launch_short_nc<6, PP>(p, waves, bh, st);
+        if (p.d <= 112) return launch_short_nc<7, PP>(p, waves, bh, st);
+    }
+    return launch_short_nc<8, PP>(p, waves, bh, st);
+}
 }  // namespace
 }  // namespace fv
 
@@ -818,6 +1080,18 @@ extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* para
     // 2000 x 2000 (1512) 142 / 151, 12 x 4000 x 300 (1500) 33.4 / 37.2: the line does not follow the head dim.
     int ks = 1;
     const size_t groups = bh * (size_t)((p.sq + 31) / 32);   // 32-query groups
+    // bf16 operands in whole 16-byte units: the short kernel, eight waves a query group while each has a CU to itself, four
+    // while they are about one resident round. us, that / the kernels below: 16 x 257 x 257 x 80 (144 groups) 7.8 / 10.2,
+    // 12 x 111 x 111 x 128 under a mask (48) 7.5 / 12.5, 16 x 1000 x 1000 x 80 (512) 22.9 / 29.5, 24 x 512 x 512 x 128 under
+    // a mask (384) 17.4 / 24.4; past two a CU, up to 64 channels (half the registers and LDS) 24 x 1024 x 1024 x 64 (768)
+    // 27.7 / 37.4, 64 x 512 x 512 x 64 with a mask per head (1024) 22.3 / 24.4, past 96 (whole LDS rows) 12 x 1500 x 1500 x
+    // 112 (564) 52.6 / 64.8, 32 x 1000 x 1000 x 112 (1024) 46.4 / 49.4; between them 24 x 900 x 900 x 80 (696) 34.8 / 34.8,
+    // 64 x 300 x 300 x 80 under a mask (640) 18.6 / 18.1.
+    const size_t cus = (size_t)fv_compute_units(), most_short = (d <= 64 || d > 96 ? 4 : 2) * cus;
+    if (p.vec && kv_is_bf16 && p.q_is_bf16 && groups <= most_short) {
+        p.q_plane = (long)p.sq * d, p.k_plane = p.v_plane = (long)p.sk * d;
+        return fv::launch_short<3>(p, groups <= cus ? 8 : 4, bh, st);
+    }
     if (groups < (parts == 3 ? 1024 : 2048)) ks = 2;
     if (groups < 512) ks = 4;
     if (groups <= 256 && p.sk > 256) ks = 8;
@@ -826,4 +1100,10 @@ extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* para
     if (d <= 64) return fv::launch_d<64>(p, parts, kv_is_bf16 != 0, ks, bh, st);
     if (d <= 96) return fv::launch_d<96>(p, parts, kv_is_bf16 != 0, ks, bh, st);
     return fv::launch_d<128>(p, parts, kv_is_bf16 != 0, ks, bh, st);
+}
+
+// The same for the plans of the fused kernels: P rounded to bf16, no mask (fv_short_waves).
+extern "C" hipError_t fv_internal_launch_short(const fv::ComposedParams* p, int waves, size_t bh, hipStream_t st) {
+    if (p->d != 64 && p->d != 128) return hipErrorInvalidValue;
+    return fv::launch_short<1>(*p, waves, bh, st);
 }

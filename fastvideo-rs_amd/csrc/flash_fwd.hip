@@ -695,6 +695,7 @@ hipError_t init_flash() {
 }
 }  // namespace
 
+extern "C" void fv_internal_count_log2_domain(void) { g_log2_domain_launches.fetch_add(1, std::memory_order_relaxed); }
 extern "C" uint64_t fv_sdpa_log2_domain_launches(void) { return g_log2_domain_launches.load(std::memory_order_relaxed); }
 
 extern "C" hipError_t fv_internal_exact_pass_reruns(unsigned long long* out) {

@@ -115,8 +115,10 @@ struct MaskArgs {
     int mode = kMaskNone;
     size_t q_rows = 0, k_rows = 0, v_rows = 0;   // rows per (batch, head) plane; 0 = contiguous (sq / sk)
     size_t splits = 1;                            // split-KV (dense only): key splits per query tile ...
+    bool split_entry = false;                     // (asked for by the caller of a split-KV entry)
     size_t full = 0;                              // ... past the first `full` ones
     size_t block_m = 0;                           // queries per workgroup (0: the kernel's own)
+    int short_waves = 0;                          // > 0: the short kernel, with as many waves a workgroup
     void* workspace = nullptr;                    // ... and their partial results
     size_t workspace_bytes = 0;
     size_t block_tokens = 0, window = 0, sink = 0;                           // block-causal
@@ -214,6 +216,22 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         p.total = (int)((total - full) * splits);
         p.per_xcd = (p.total + 7) / 8;
     }
+    // Kernel-level calls take the short kernel up to 512 keys, and past them where a split-KV entry is asked for a bf16
+    // result with the library's own count (the result of fv_rt_sdpa on that shape, bit for bit).
+    int short_waves = m.short_waves;
+    if (mode == kMaskNone && !short_waves &&
+        ((splits == 1 && sk <= 512) || (m.split_entry && out_is_bf16 && m.splits == fv_sdpa_splitkv_choose(bh, sq, sk))))
+        short_waves = fv_short_waves(bh, sq, sk, d);
+    if (short_waves) {
+        fv::ComposedParams c;
+        c.q = q, c.k = k, c.v = v, c.out = out, c.q_is_bf16 = 1, c.out_is_bf16 = out_is_bf16;
+        c.sq = p.sq, c.sk = p.sk, c.d = (int)d, c.scale = scale, c.vec = 1;
+        c.q_plane = p.q_plane, c.k_plane = p.k_plane, c.v_plane = p.v_plane;
+        const hipError_t e = fv_internal_launch_short(&c, short_waves, bh, (hipStream_t)stream);
+        if (e != hipSuccess) return fail_hip(e, "sdpa_short");
+        if (p.sl2 == 1.0f) fv_internal_count_log2_domain();
+        return FV_OK;
+    }
     hipError_t e = fv_internal_launch_flash(&p, mode != kMaskNone ? 1 : 0, (int)d, (int)bm, (hipStream_t)stream);
     if (e != hipSuccess) return fail_hip(e, mode != kMaskNone ? "flash_fwd_pp2<masked>" : "flash_fwd_pp2<dense>");
     if (p.kv_split > 1) {
@@ -236,6 +254,22 @@ int fv_compute_units() {
         return n;
     }();
     return cus;
+}
+
+// The short kernel (composed_fwd.hip) takes calls whose 32-query groups are one round of resident workgroups: of eight
+// waves where each has a CU to itself, of four up to two a CU (three at head dim 64, which has room for four), while the walk of the keys is
+// short enough that sharing it out over the chip (split-KV) or reading K and V once for 128 or 256 queries gains less. us in a
+// graph, flash_fwd_pp2 / short: at 128 channels 12 x 320 x 320 11.0 / 6.8, 3 x 390 x 200 9.6 / 6.4, 12 x 600 x 1000 21.1 / 11.9,
+// x 3000 30.9 / 23.7, x 5000 (12 x 320) 33.6 / 31.7, (3 x 390) 25.5 / 30.7; 264 to 512 groups 12 x 680 x 500 13.8 / 11.4,
+// 12 x 1000 x 1000 24.3 / 16.8, x 2000 31.1 / 28.4, x 3000 35.9 / 38.7; 516 groups 12 x 1360 x 500 14.4 / 16.8, x 2000 37 / 43.
+// At 64 channels 12 x 320 x 320 8.0 / 4.9, 3 x 390 x 3000 16.6 / 13.5, x 5000 19.6 / 19.4, 12 x 1000 x 3000 27.5 / 23.0 (four
+// waves 24.5), 12 x 1560 x 1500 24.9 / 19.5, 40 x 560 x 500 10.6 / 9.9, x 3000 36.9 / 35.2; 880 groups 40 x 700 x 700 14.3 / 14.4.
+// (Query tiles of 256 that have a CU each already, of few rows: flash_fwd_pp2 as before.)
+int fv_short_waves(size_t bh, size_t sq, size_t sk, size_t d) {
+    const size_t cus = (size_t)fv_compute_units(), nq = (sq + 31) / 32, bm = (size_t)fv_internal_flash_block_m();
+    if (nq > 3 * cus || bh * nq > (d == 64 ? 3 : 2) * cus || bh * ((sq + bm - 1) / bm) >= cus) return 0;
+    if (bh * nq <= cus) return sk <= (d == 64 ? 4000 : 3072) ? 8 : 0;
+    return sk <= (d == 64 ? 3072 : 2048) ? 4 : 0;
 }
 
 // Fewer query tiles than CUs: fv_sdpa_splitkv_choose. More: they run in rounds of one per CU, and the last round costs a
@@ -288,6 +322,7 @@ int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, vo
     m.splits = plan.splits;
     m.full = plan.full;
     m.block_m = plan.block_m;
+    m.short_waves = plan.short_waves;
     m.workspace = workspace;
     m.workspace_bytes = workspace_bytes;
     return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
@@ -385,6 +420,7 @@ int fv_sdpa_dense_bf16_splitkv(const uint16_t* q, const uint16_t* k, const uint1
     m.k_rows = k_rows;
     m.v_rows = v_rows;
     m.splits = splits ? splits : 1;
+    m.split_entry = true;
     m.workspace = workspace;
     m.workspace_bytes = workspace_bytes;
     return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
@@ -424,6 +460,7 @@ int fv_sdpa_dense_bf16_splitkv_static(const uint16_t* q, const uint16_t* k, cons
     m.k_rows = k_rows;
     m.v_rows = v_rows;
     m.splits = run;
+    m.split_entry = true;
     if (run > 1) {
         void* p = nullptr;
         const hipError_t e = static_scratch(&p);

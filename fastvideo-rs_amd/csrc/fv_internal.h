@@ -55,6 +55,7 @@ struct ComposedParams {
     long part_row0 = 0, part_rows = 0;
     float* part_o = nullptr;
     float* part_ml = nullptr;
+    long q_plane = 0, k_plane = 0, v_plane = 0;   // short launches: elements between consecutive (batch, head) planes
 };
 
 // How a composed launch is cut (composed_fwd.hip): splits <= 1: one workgroup a query tile throughout.
@@ -161,8 +162,11 @@ int fv_cast_operands(const FvCastOperands& ops, int count, void* stream);
 // `splits` key ranges (full == 0), the ones past the first `full`, or none (splits == 1).
 struct FvSplitPlan {
     size_t block_m, full, splits, workspace_bytes;   // block_m: queries per workgroup
+    int short_waves = 0;                             // > 0: the short kernel, with as many waves a workgroup
 };
 FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d);
+// Waves a workgroup of the short kernel where a dense call of this shape that writes bf16 takes it, else 0.
+int fv_short_waves(size_t bh, size_t sq, size_t sk, size_t d);
 // fv_sdpa_dense_bf16_splitkv with such a plan
 int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out, int out_is_bf16, size_t bh,
                      size_t sq, size_t sk, size_t d, float scale, size_t q_rows, size_t k_rows, size_t v_rows,
@@ -196,6 +200,8 @@ fv::ComposedPlan fv_composed_plan(size_t bh, size_t sq, size_t sk, size_t d);
 // round16 == 0 to be exact; an f32 q with bf16 k / v is rounded.
 extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* p, int kv_is_bf16, int round16, size_t bh,
                                                   hipStream_t st);
+extern "C" hipError_t fv_internal_launch_short(const fv::ComposedParams* p, int waves, size_t bh, hipStream_t st);
+extern "C" void fv_internal_count_log2_domain(void);
 extern "C" hipError_t fv_internal_launch_splitkv_merge(const float* part_o, const float* part_lse, void* out,
                                                        int out_is_bf16, size_t rows, int d, int splits,
                                                        hipStream_t st);

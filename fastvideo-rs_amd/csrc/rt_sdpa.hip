@@ -245,6 +245,14 @@ Result<Tensor> compact(const Tensor& x, Mem& st) {
     return std::move(t);
 }
 
+FvSplitPlan dense_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16) {
+    const int waves = out_bf16 ? fv_short_waves(bh, sq, sk, d) : 0;
+    if (!waves) return fv_split_plan(bh, sq, sk, d);
+    FvSplitPlan p{0, 0, 1, 0};
+    p.short_waves = waves;
+    return p;
+}
+
 // One fused launch (dense, block-causal or VDN window); nullopt = the kernel declined.
 Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tensor& v,
                                     std::optional<float> scale, bool out_bf16,
@@ -303,7 +311,7 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
         // 380 - 460 so, at 12 x 8000 x 8000 x 128 415 and 570 - 750 (calls among others 150 / 140 and 367 / 373). (The
         // composed launches gain more than that: 690 us whole, 645 cut, at 12 x 4096 x 4096 x 128.) Where the partial
         // results get no memory the launch is made unsplit.
-        FvSplitPlan plan = fv_split_plan(s->b * s->h, s->sq, s->sk, s->d);
+        FvSplitPlan plan = dense_plan(s->b * s->h, s->sq, s->sk, s->d, out_bf16);
         Tensor ws;
         if (plan.splits > 1 && (plan.full == 0 || st.holds(plan.workspace_bytes))) {
             auto rw = st.temp({plan.workspace_bytes / 4}, DType::F32);
@@ -742,7 +750,7 @@ Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& pl
     for (const Tensor* t : {&q, &k, &v})
         if (t->dtype == DType::F32) n.workspace += (t->numel() * 2 + 255) & ~(size_t)255;
     if (plan.kind == Plan::Kind::Dense || plan.kind == Plan::Kind::KvWindow) {
-        n.workspace += (fv_split_plan(s->b * s->h, s->sq, s->sk, s->d).workspace_bytes + 255) & ~(size_t)255;
+        n.workspace += (dense_plan(s->b * s->h, s->sq, s->sk, s->d, act16).workspace_bytes + 255) & ~(size_t)255;
     }
     return n;
 }
