@@ -160,13 +160,18 @@ FV_DEV float composed_to_log2(const Params& p) {
     return p.mask || p.scale == 0.f ? 1.4426950408889634f : __builtin_fabsf(p.scale) * 1.4426950408889634f;
 }
 
-// The additive mask of the lane's 16 keys, four consecutive ones per load where rows allow it.
-FV_DEV void load_mask(const float* mr, int vec, int kv0, int h, int sk, f32x16& mk) {
+// The additive mask of the lane's 16 keys, four consecutive ones per load: vector loads need no more than the alignment
+// of a float. Element by element only in a tile that a row ends in between two such groups, where a whole group would
+// reach past the mask's last row. (Rows of any other length than whole 16-byte units used to be read element by element
+// throughout: 32 rows touched by each of 16 instructions, 787 -> 476 us at 64 x 2611 x 2611 x 80 with a shared mask,
+// 58.7 -> 41.6 at 64 x 523 x 523 x 80 with a mask per head.)
+FV_DEV void load_mask(const float* mr, int kv0, int h, int sk, f32x16& mk) {
+    typedef f32x4 __attribute__((aligned(4))) f32x4_any;
     if (!mr) return;
-    if (vec) {
+    if ((sk & 3) == 0 || kv0 + 32 <= sk) {
 #pragma unroll
         for (int g = 0; g < 4; g++) {
-            const f32x4 t = *reinterpret_cast<const f32x4*>(mr + min(kv0 + 8 * g + 4 * h, sk - 4));
+            const f32x4 t = *reinterpret_cast<const f32x4_any*>(mr + min(kv0 + 8 * g + 4 * h, sk - 4));
 #pragma unroll
             for (int x = 0; x < 4; x++) mk[4 * g + x] = t[x];
         }
@@ -295,7 +300,7 @@ FV_DEV void composed_redo(const __attribute__((address_space(4))) ComposedParams
     for (int t = 0; t < it.tiles; t++) {
         const int kv0 = (it.tile0 + t) * 32;
         f32x16 mk, s;
-        load_mask(mr, p.vec_mask, kv0, h, sk, mk);
+        load_mask(mr, kv0, h, sk, mk);
 #pragma unroll
         for (int i = 0; i < 16; i++) s[i] = 0.f;
         const char* krow = kb + (long)min(kv0 + c32, sk - 1) * d * kElem;
@@ -476,7 +481,7 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
     f32x16 mk;
     load_units(kb, (tile0 + ks) * 32, ku);
     load_units(vb, (tile0 + ks) * 32, vu);
-    load_mask(mr, p.vec_mask, (tile0 + ks) * 32, h, sk, mk);
+    load_mask(mr, (tile0 + ks) * 32, h, sk, mk);
 
     // Q operand, in parts: this lane's query, d = 16 j + 8 h ..
     bf16x8 qf[PARTS][NC];
@@ -565,7 +570,7 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
                 }
             }
             // the next tile's mask, in flight under the rest of this tile (rows past the end: nothing)
-            if (step + 1 < steps) load_mask(mr, p.vec_mask, kv0 + 32 * KS, h, sk, mk);
+            if (step + 1 < steps) load_mask(mr, kv0 + 32 * KS, h, sk, mk);
             // ---- O^T += V^T P^T, 16 keys at a time ----
 #pragma unroll
             for (int t = 0; t < 2; t++) {
@@ -736,7 +741,7 @@ __global__ __launch_bounds__(64 * KS, NC <= 4 ? 4 : 2) void sdpa_short_kernel(co
     }
     const float* mr = PP == 3 && p.mask ? p.mask + bh * p.mask_bh + (long)(q_ok ? qi : 0) * sk : nullptr;
     f32x16 mk;
-    if (PP == 3 && wave < tiles) load_mask(mr, p.vec_mask, wave * 32, h, sk, mk);
+    if (PP == 3 && wave < tiles) load_mask(mr, wave * 32, h, sk, mk);
     if (PP == 3 && nch < 2 * NC) {   // the channels between d and the products' last: zeros, in K for each wave and in Q
 #pragma unroll
         for (int i = 0; i < kIt; i++) {
@@ -809,7 +814,7 @@ __global__ __launch_bounds__(64 * KS, NC <= 4 ? 4 : 2) void sdpa_short_kernel(co
 #pragma unroll
                 for (int i = 0; i < 16; i++) o[db][i] *= alpha;
         }
-        if (PP == 3 && more) load_mask(mr, p.vec_mask, kv0 + 32 * KS, h, sk, mk);
+        if (PP == 3 && more) load_mask(mr, kv0 + 32 * KS, h, sk, mk);
         if (more) wait_vmcnt<kIt>();      // V(t) has landed; K of the next tile may be in flight
         else wait_vmcnt<0>();
 #pragma unroll
@@ -1064,7 +1069,6 @@ extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* para
     }
     const uintptr_t any = (uintptr_t)p.q | (uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.out;
     p.vec = (any & 15) == 0 && d % 8 == 0;
-    p.vec_mask = p.mask && ((uintptr_t)p.mask & 15) == 0 && p.sk % 4 == 0;
     const int parts = kv_is_bf16 || round16 ? 1 : 3;
     // 1024 groups are one wave on every SIMD of the chip: below two waves (one with three parts, whose second share of
     // the tiles leaves room for one workgroup per CU) the keys are shared out over a workgroup's waves. One part, bf16,

@@ -46,7 +46,7 @@ struct ComposedParams {
     int q_is_bf16 = 0, out_is_bf16 = 0;
     int sq = 0, sk = 0, d = 0;
     float scale = 1.0f;
-    int vec = 0, vec_mask = 0;    // set by the launcher: 16-byte operand rows / mask rows
+    int vec = 0;                  // set by the launcher: 16-byte operand rows
     int nqt = 0, total = 0, per_xcd = 0, by_head = 0;   // set by the launcher: query tiles per head, items past `full`, ceil(total / 8), item order
     // Split tail (fv_composed_plan): the first `full` query tiles have a workgroup each, every later one `splits`, each
     // walking split_tiles key tiles and leaving its sums (f32 [split][row][dpad], unnormalised) and its (max, sum)

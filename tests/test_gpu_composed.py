@@ -306,3 +306,32 @@ def test_more_query_tiles_than_one_launch_holds(fv):
     torch.cuda.synchronize()
     for lo in range(0, bh, 8192):
         assert bool((got[:, lo:lo + 8192] == v[:, lo:lo + 8192]).all())
+
+
+@pytest.mark.parametrize("act16", [True, False])
+@pytest.mark.parametrize("per_head", [True, False])
+@pytest.mark.parametrize("h,sq,sk,d", [(1, 33, 1, 16), (2, 40, 3, 64), (2, 33, 61, 64), (3, 70, 318, 80), (70, 1000, 95, 40), (40, 1000, 65, 128)])
+def test_masks_of_any_row_length_and_start(fv, h, sq, sk, d, per_head, act16):
+    """Mask rows that are no whole 16-byte units, in storage that starts one, two and three floats past one: the bits of
+    the same mask at an aligned start, and the f64 result."""
+    import torch
+
+    announce(f"composed mask rows h={h} sq={sq} sk={sk} d={d} per_head={per_head} act16={act16}")
+    g = torch.Generator(device="cuda").manual_seed(sq + sk)
+    q, k, v = (torch.randn((1, h, s, d), generator=g, device="cuda") for s in (sq, sk, sk))
+    if act16:
+        q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    n = (h if per_head else 1) * sq * sk
+    values = torch.randn(n, generator=g, device="cuda")
+    base = None
+    for shift in range(4):
+        store = torch.full((n + 8,), 1e9, device="cuda")
+        store[shift:shift + n] = values
+        mask = store[shift:shift + n].view(1, h if per_head else 1, sq, sk)
+        with fv.with_bf16_act(act16):
+            got = fv.sdpa(q, k, v, fv.Plan.masked(None, mask) if act16 else fv.Plan.composed(None, mask))
+        if base is None:
+            base = got
+            want = want64(q, k, v, mask)
+            assert np.linalg.norm(got.double().cpu().numpy() - want) <= (2e-3 if act16 else 2e-6) * np.linalg.norm(want)
+        assert torch.equal(got, base), shift
