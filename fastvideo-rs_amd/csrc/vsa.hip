@@ -506,104 +506,267 @@ __global__ __launch_bounds__(256) void vsa_tile_qkv_kernel(const void* __restric
 }
 
 // ---- fine stage (kernels/core.cu:1029-1179) ---------------------------------------------
-// One workgroup (2 waves x 32 queries) per (query tile, batch*head): online
-// softmax over the selected key tiles in list order; key columns >=
-// block_sizes[tile] are -inf. K and V tiles are separate single LDS buffers fed
-// by direct global->LDS loads: K(i+1) streams in under softmax/PV of tile i and
-// V(i) under QK/softmax of tile i. 32 KB of LDS per workgroup, so four
-// workgroups share a CU.
-// The softmax offset rides in the C operand of the K Q^T MFMAs (softmax_tile_side_off). LOG2DOM: the call's
-// scale * log2(e) is exactly 1 (the caller folded the softmax scale into Q) and the per-score multiply is gone too.
-template <bool LOG2DOM>
-__global__ __launch_bounds__(128, 2) void vsa_fine_kernel(const VsaFineParams p) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    lds_u8* kbuf = (lds_u8*)smem_raw;
-    lds_u8* vbuf = kbuf + kTileBytes;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// One workgroup of two waves per (query tile, batch*head): online softmax over the selected key tiles in list order;
+// key columns >= block_sizes[tile] are -inf. Both waves hold all 64 queries and share the keys out, 32 at a time, so
+// each wave has a ring of its own, fed by its own LDS-DMA, and waits for nobody but its own loads until the end, where
+// the two results are merged through LDS, every wave finishing 32 queries. The ring has five slots of 4 KB; 32 keys
+// pass through it as four chunks (K: channels 0 - 63, then 64 - 127; V: keys 0 - 15, then 16 - 31), each requested into
+// the slot its predecessor but four has just left: a whole step ahead of its use.
+// Padding is left out. A selected tile of more than 32 keys is a step of each wave; one of up to 32 a step of one wave,
+// the waves taking turns; two of up to 16 share a step. A query tile of up to 32 queries (whole op only: the stage entry
+// writes the padding rows too) is walked for those 32 alone (NB = 1), and one wave finishes them.
+// Measured on MI355X, 12 heads, 624 tiles, 125 selected, us, the form this replaces (a wave 32 queries, both waves on
+// every key tile behind three barriers) / this one: ragged tiles of 21 x 30 x 52 2400 / 2010, full tiles with a
+// uniformly random selection 2350 / 2430, a banded one 2075 / 1900.
+constexpr int kFineSlot = 4096;
+constexpr int kFineWave = 5 * kFineSlot;
+constexpr int kFineLds = 2 * kFineWave;
+struct FineState {
+    float thr, off, l;   // rescale above thr (-inf: no finite score yet); P = 2^(sl2 s - off); the lane's share of the sum
+};
+// Two blocks of 16 keys: their first rows in the tile-ordered copies and how many of their keys count.
+struct FineStep {
+    int row_a, row_b, valid_a, valid_b;
+    bool none;
+};
+
+template <int NB>
+FV_DEV void fine_item(const VsaFineParams& p, lds_u8* smem, const int wave, const int lane, const int bh, const int qtile) {
+    lds_u8* ring = smem + wave * kFineWave;
     const int h = lane >> 5, c32 = lane & 31;
-    const int work = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
-    if (work >= p.total) return;
-    const int bh = work / p.q_tiles;
-    const int qtile = p.q_base + work % p.q_tiles;
-    if (qtile >= p.num_tiles) return;
     const int nb = p.num_tiles, topk = p.topk;
     const size_t padded = (size_t)nb * kTileElems;
-    const uint16_t* kb = p.kt + (size_t)bh * padded * 128;
-    const uint16_t* vb = p.vt + (size_t)bh * padded * 128;
+    const char* kb = (const char*)(p.kt + (size_t)bh * padded * 128);
+    const char* vb = (const char*)(p.vt + (size_t)bh * padded * 128);
     const unsigned* sel = p.selected + ((size_t)bh * nb + qtile) * topk;
     const float sl2 = p.sl2;
     const float NEG = neg_inf();
 
-    bf16x8 qf[8];
-    load_q_frags(p.qt + ((size_t)bh * padded + (size_t)qtile * kTileElems) * 128, wave * 32 + c32,
-                 true, lane, qf);
-    const TileReadBases rb = tile_read_bases(lane);
+    // query block 0 is the one this wave finishes: queries 32 wave ..; block 1 the other wave's
+    bf16x8 qf[NB][8];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+        load_q_frags(p.qt + ((size_t)bh * padded + (size_t)qtile * kTileElems) * 128, (NB == 2 ? wave ^ b : 0) * 32 + c32,
+                     true, lane, qf[b]);
+    int krd = tile_read_bases<64>(lane).k, vrd = tile_read_bases<128>(lane).v;
 
-    f32x16 o[4];
+    f32x16 o[NB][4];
+    FineState st[NB];
 #pragma unroll
-    for (int db = 0; db < 4; db++)
+    for (int b = 0; b < NB; b++) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) o[db][i] = 0.f;
-    SoftmaxOffState st;
-    st.init();
-    f32x16 s_init;   // the C operand every S block starts from: minus the lane's softmax offset
+        for (int db = 0; db < 4; db++)
 #pragma unroll
-    for (int i = 0; i < 16; i++) s_init[i] = 0.f;
-
-    // Per-lane DMA offsets are loop-invariant (every tile has 64 rows in the tile-ordered layout), so a
-    // tile load is 8 (m0, load) pairs from a scalar base. The tile indices and sizes of the next two
-    // list entries are fetched one iteration ahead: no scalar-load latency sits in front of a DMA issue.
-    TileDma<2, 128> dma;
-    dma.init(wave, lane);
-    auto tile_at = [&](int i) -> int { return min((int)sel[min(i, topk - 1)], nb - 1); };
-    int tile = tile_at(0), tile_next = tile_at(1);
-    int valid = p.block_sizes[tile], valid_next = p.block_sizes[tile_next];
-    dma.template issue<false>(kbuf, kb + (size_t)tile * kTileElems * 128, kTileElems, wave);
-#pragma unroll 1
-    for (int i = 0; i < topk; i++) {
-        wait_vmcnt<0>();     // K(i) landed
-        block_barrier();     // ... for every wave; PV(i-1) finished everywhere: V buffer free
-        const int tile_nn = tile_at(i + 2);          // consumed an iteration from now
-        f32x16 s[2];
-        // the 8 DMA instructions of V(i) go out one behind every second MFMA of QK(i), those of K(i+1)
-        // in three groups through the softmax: issued in one burst they hold the wave (in-order issue)
-        // while the CU's address path drains, 4 % of the kernel's time
-        const uint16_t* vsrc = vb + (size_t)tile * kTileElems * 128;
-        qk_tile_side(kbuf, rb.k, qf, s, s_init, [&](int g) {
-            if (g & 1) dma.template issue_one<true>(vbuf, vsrc, wave, g >> 1);
-        });
-        block_barrier();     // K buffer free
-        const bool more = i + 1 < topk;
-        const uint16_t* ksrc = kb + (size_t)tile_next * kTileElems * 128;
-        if (valid < kTileElems) {
-#pragma unroll
-            for (int b = 0; b < 2; b++)
-#pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    const int col = 32 * b + 8 * (e >> 2) + 4 * h + (e & 3);
-                    if (col >= valid) s[b][e] = NEG;
-                }
-        }
-        bf16x8 pb[4];
-        auto k_loads = [&](int part) {
-            if (more) {
-                const int first = 3 * part, last = part == 2 ? 8 : first + 3;
-#pragma unroll
-                for (int it = first; it < last; it++) dma.template issue_one<false>(kbuf, ksrc, wave, it);
-            }
-        };
-        softmax_tile_side_off<!LOG2DOM>(s, st, o, s_init, sl2, pb, k_loads);
-        if (more) wait_vmcnt<8>(); else wait_vmcnt<0>();   // V(i) landed; K(i+1) may be in flight
-        block_barrier();
-        pv_tile(vbuf, rb.v, pb, o);
-        tile = tile_next;
-        tile_next = tile_nn;
-        valid = valid_next;
-        valid_next = p.block_sizes[tile_nn];
+            for (int i = 0; i < 16; i++) o[b][db][i] = 0.f;
+        st[b] = {NEG, 0.f, 0.f};
     }
 
-    const float l_tot = pair_sum(st.l_acc);
+    // The list, 64 entries at a time: lane l holds entry l (tile, keys); `mine` the entries this wave takes, `small` those
+    // of up to 16 keys.
+    int entry = 0, base = 0, turn_s = 0, turn_t = 0;
+    unsigned long long mine = 0, small = 0;
+    auto refill = [&]() {
+        const int at = base + lane;
+        base += 64;
+        const bool in = at < topk;
+        const int tile = min(max((int)sel[min(at, topk - 1)], 0), nb - 1);
+        const int keys = in ? min(max(p.block_sizes[tile], 0), kTileElems) : kTileElems;
+        entry = (tile << 7) | keys;
+        const bool one = keys <= 32 && keys > 16, two = keys <= 16;
+        const unsigned long long s = __builtin_amdgcn_ballot_w64(one);
+        small = __builtin_amdgcn_ballot_w64(two);
+        const int turn1 = lanes_below(s) + turn_s, turn2 = (lanes_below(small) >> 1) + turn_t, turn = two ? turn2 : turn1;
+        mine = __builtin_amdgcn_ballot_w64(in & ((keys > 32) | ((turn & 1) == wave)));
+        turn_s += __builtin_popcountll(s);
+        turn_t += (__builtin_popcountll(small) + 1) >> 1;
+    };
+    auto next = [&]() -> FineStep {
+        while (mine == 0 && base < topk) refill();
+        FineStep r = {0, 16, 16, 16, mine == 0};   // (past the end: rows that exist, loaded and not used)
+        if (mine == 0) return r;
+        const int i = __builtin_ctzll(mine);
+        mine &= mine - 1;
+        const int e = __builtin_amdgcn_readlane(entry, i), keys = e & 127, half = keys > 32 ? 32 * wave : 0;
+        r.row_a = (e >> 7) * kTileElems + half;
+        r.valid_a = keys - half;
+        r.row_b = r.row_a + 16;
+        r.valid_b = r.valid_a - 16;
+        const unsigned long long pair = mine & small;
+        if (keys <= 16 && pair != 0) {
+            const int j = __builtin_ctzll(pair);
+            mine &= ~(1ull << j);
+            const int f = __builtin_amdgcn_readlane(entry, j);
+            r.row_b = (f >> 7) * kTileElems;
+            r.valid_b = f & 127;
+        }
+        return r;
+    };
+
+    // A DMA instruction moves 1 KB: eight rows of a K chunk (128 bytes each, K swizzle of 64 channels) or four of a V chunk
+    const int dr = lane >> 4;
+    unsigned koff = (lane >> 3) * kRowBytes + (((lane & 7) ^ dr) << 4);   // (row >> 1) & 7 = 4 (it & 1) + l / 16
+    const unsigned voff = dr * kRowBytes + (((lane & 15) ^ (dr << 2)) << 4);
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)ring);
+    auto load_k = [&](unsigned slot, const FineStep s, int half, int it) {
+        const int row = it < 2 ? s.row_a : s.row_b;
+        const char* src = kb + (size_t)(unsigned)row * kRowBytes;
+        lds_dma16_s(lds0 + slot + it * 1024, src + (it & 1) * 8 * kRowBytes + half * 128, koff ^ ((it & 1) << 6));
+    };
+    auto load_v = [&](unsigned slot, const FineStep s, int half, int it) {
+        const int row = half ? s.row_b : s.row_a;
+        const char* src = vb + (size_t)(unsigned)row * kRowBytes;
+        lds_dma16_s(lds0 + slot + it * 1024, src + it * 1024, voff);
+    };
+
+    unsigned sk0 = 0, sk1 = kFineSlot, sv0 = 2 * kFineSlot, sv1 = 3 * kFineSlot, spare = 4 * kFineSlot;
+    FineStep cur = next();
+#pragma unroll
+    for (int x = 0; x < 8; x++) load_k(x < 4 ? sk0 : sk1, cur, x >> 2, x & 3);
+#pragma unroll
+    for (int x = 0; x < 8; x++) load_v(x < 4 ? sv0 : sv1, cur, x >> 2, x & 3);
+    constexpr int kAhead = 2;   // a fragment feeds NB MFMAs and is read kAhead fragments before them
+    while (!cur.none) {
+        const FineStep nx = next();
+        // (addresses are formed where they are used: kept across the loop they would take 16 registers that it has not got)
+        asm volatile("" : "+v"(krd), "+v"(vrd), "+v"(koff));
+        f32x16 s[NB];
+        {
+            bf16x8 f[8];
+            auto read = [&](int dk) { f[dk] = lds_read_b128(ring + (dk < 4 ? sk0 : sk1) + (krd ^ ((dk & 3) << 5))); };
+            wait_vmcnt<12>();   // the first K chunk has landed; the other three may be in flight
+#pragma unroll
+            for (int dk = 0; dk < kAhead; dk++) read(dk);
+#pragma unroll
+            for (int dk = 0; dk < 8; dk++) {
+                if (dk + kAhead == 4) wait_vmcnt<12>();   // the second one (in flight: both V chunks, the next K chunk)
+                if (dk + kAhead < 8) read(dk + kAhead);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    if (dk == 0)
+#pragma unroll
+                        for (int e = 0; e < 16; e++) s[b][e] = 0.f;
+                    s[b] = mfma32(f[dk], qf[b][dk], s[b]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (dk < 2) load_k(spare, nx, 0, 2 * dk), load_k(spare, nx, 0, 2 * dk + 1);
+                if (dk >= 4) load_k(sk0, nx, 1, dk - 4);   // (every read of the slot has been multiplied)
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (cur.valid_a < 16 || cur.valid_b < 16) {
+            const int va = cur.valid_a - 4 * h, vb16 = cur.valid_b - 4 * h;
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const bool out = 8 * ((e >> 2) & 1) + (e & 3) >= (e < 8 ? va : vb16);
+#pragma unroll
+                for (int b = 0; b < NB; b++) s[b][e] = out ? NEG : s[b][e];
+            }
+        }
+        float mx[NB];
+        bool grown = false;
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            mx[b] = s[b][0];
+#pragma unroll
+            for (int e = 1; e < 16; e++) mx[b] = __builtin_fmaxf(mx[b], s[b][e]);
+            mx[b] = pair_max(mx[b]) * sl2;
+            grown |= mx[b] > st[b].thr;
+        }
+        if (__builtin_amdgcn_ballot_w64(grown) != 0) {
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                const bool need = mx[b] > st[b].thr;
+                const float off = need ? mx[b] : st[b].off;
+                const float alpha = st[b].thr == NEG ? 1.f : fast_exp2(st[b].off - off);   // (no finite score yet: zeros)
+                st[b].off = off;
+                if (need) st[b].thr = off + kRescaleLog2;
+                st[b].l *= alpha;
+#pragma unroll
+                for (int db = 0; db < 4; db++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) o[b][db][e] *= alpha;
+            }
+        }
+        bf16x8 pb[NB][2];
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                f32x8 e;
+#pragma unroll
+                for (int x = 0; x < 8; x++) {
+                    e[x] = fast_exp2(__builtin_fmaf(s[b][8 * t + x], sl2, -st[b].off));
+                    st[b].l += e[x];
+                }
+                pb[b][t] = __builtin_convertvector(e, bf16x8);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int it = 0; it < 2 / NB; it++) load_v(sk1, nx, 0, NB == 2 ? 2 * b + t : 2 * t + it);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        wait_vmcnt<16>();   // the first V chunk
+        {
+            bf16x8 f[8];
+            auto read = [&](int g) {
+                const lds_u8* a0 = ring + (g < 4 ? sv0 : sv1) + (vrd ^ ((g & 3) << 6));
+                s16x8 a;
+                a.lo = lds_read_tr16_b64(a0);
+                a.hi = lds_read_tr16_b64(a0 + 8 * kRowBytes);
+                f[g] = __builtin_bit_cast(bf16x8, a);
+            };
+#pragma unroll
+            for (int g = 0; g < kAhead; g++) read(g);
+#pragma unroll
+            for (int g = 0; g < 8; g++) {
+                if (g + kAhead == 4) wait_vmcnt<12>();   // the second one
+                if (g + kAhead < 8) read(g + kAhead);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int b = 0; b < NB; b++) o[b][g & 3] = mfma32(f[g], pb[b][g >> 2], o[b][g & 3]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (g >= 4) load_v(sv0, nx, 1, g - 4);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        const unsigned left_slot = sv1;   // the ring moves on by four of its five slots
+        sv1 = sv0, sv0 = sk1, sk1 = sk0, sk0 = spare, spare = left_slot;
+        cur = nx;
+    }
+
+    wait_vmcnt<0>();   // (the loads past the end)
+    // The merge: each wave hands the other one's queries over in its own ring.
+    typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+    typedef __attribute__((address_space(3))) f32x2 lds_f32x2;
+    constexpr int kMl = 4 * kFineSlot;   // behind the sums: offset and row sum, a pair a lane
+    if (NB == 2 || wave == 1) {
+        constexpr int B = NB - 1;
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            f32x4 r;
+#pragma unroll
+            for (int x = 0; x < 4; x++) r[x] = o[B][j >> 2][4 * (j & 3) + x];
+            *reinterpret_cast<lds_f32x4*>(ring + (j * 64 + lane) * 16) = r;
+        }
+        *reinterpret_cast<lds_f32x2*>(ring + kMl + lane * 8) = f32x2{st[B].thr == NEG ? NEG : st[B].off, pair_sum(st[B].l)};
+    }
+    __syncthreads();
+    if (NB == 1 && wave == 1) return;
+    const lds_u8* other = smem + (wave ^ 1) * kFineWave;
+    const f32x2 om = *reinterpret_cast<const lds_f32x2*>(other + kMl + lane * 8);
+    const float off0 = st[0].thr == NEG ? NEG : st[0].off;
+    const float m = __builtin_fmaxf(off0, om[0]);
+    const float w0 = off0 == NEG ? 0.f : fast_exp2(off0 - m), w1 = om[0] == NEG ? 0.f : fast_exp2(om[0] - m);
+    const float l_tot = pair_sum(st[0].l) * w0 + om[1] * w1;
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    auto merged = [&](int db, int g) {
+        const f32x4 t = *reinterpret_cast<const lds_f32x4*>(other + ((4 * db + g) * 64 + lane) * 16);
+        f32x4 r;
+#pragma unroll
+        for (int x = 0; x < 4; x++) r[x] = (o[0][db][4 * g + x] * w0 + t[x] * w1) * inv;
+        return r;
+    };
     if (p.final_out) {
         // fused combine (kernels/core.cu:803-835): out[token] = coarse[tile] * gate[token] + sparse,
         // the product rounded to f32 before the add as on the host; padding slots write nothing
@@ -630,12 +793,10 @@ __global__ __launch_bounds__(128, 2) void vsa_fine_kernel(const VsaFineParams p)
                         ga = *reinterpret_cast<const f32x4*>((const float*)p.gate + row + d0);
                     }
                 }
+                const f32x4 sp = merged(db, g);
                 f32x4 r;
 #pragma unroll
-                for (int x = 0; x < 4; x++) {
-                    const float sp = o[db][4 * g + x] * inv;
-                    r[x] = c4[x] * ga[x] + sp;
-                }
+                for (int x = 0; x < 4; x++) r[x] = c4[x] * ga[x] + sp[x];
                 *reinterpret_cast<f32x4*>(p.final_out + row + d0) = r;
             }
         return;
@@ -645,11 +806,20 @@ __global__ __launch_bounds__(128, 2) void vsa_fine_kernel(const VsaFineParams p)
     for (int db = 0; db < 4; db++)
 #pragma unroll
         for (int g = 0; g < 4; g++) {
-            f32x4 r;
-#pragma unroll
-            for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
-            *reinterpret_cast<f32x4*>(ob + 32 * db + 8 * g + 4 * h) = r;
+            *reinterpret_cast<f32x4*>(ob + 32 * db + 8 * g + 4 * h) = merged(db, g);
         }
+}
+
+__global__ __launch_bounds__(128, 2) void vsa_fine_kernel(const VsaFineParams p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int work = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
+    if (work >= p.total) return;
+    const int bh = work / p.q_tiles;
+    const int qtile = p.q_base + work % p.q_tiles;
+    if (qtile >= p.num_tiles) return;
+    if (p.final_out && p.block_sizes[qtile] <= 32) fine_item<1>(p, (lds_u8*)smem_raw, wave, lane, bh, qtile);
+    else fine_item<2>(p, (lds_u8*)smem_raw, wave, lane, bh, qtile);
 }
 
 // ---- combine (kernels/core.cu:803-835) -----------------------------------------------------
@@ -816,10 +986,7 @@ extern "C" hipError_t fv_internal_launch_tile_qkv(const void* x, int x_is_bf16, 
 }
 
 extern "C" hipError_t fv_internal_launch_fine(const fv::VsaFineParams* p, hipStream_t st) {
-    if (p->sl2 == 1.0f)   // scale = ln 2: the caller folded the softmax scale into Q
-        hipLaunchKernelGGL(vsa_fine_kernel<true>, dim3(p->per_xcd * 8), dim3(128), 2 * kTileBytes, st, *p);
-    else
-        hipLaunchKernelGGL(vsa_fine_kernel<false>, dim3(p->per_xcd * 8), dim3(128), 2 * kTileBytes, st, *p);
+    hipLaunchKernelGGL(vsa_fine_kernel, dim3(p->per_xcd * 8), dim3(128), kFineLds, st, *p);
     return hipGetLastError();
 }
 

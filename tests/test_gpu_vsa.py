@@ -426,3 +426,37 @@ def test_log2_domain_form_of_the_fine_stage_and_the_whole_op(fv, oracle, grid):
     assert np.array_equal(np.sort(sel, -1), np.sort(want_sel.reshape(sel.shape), -1))
     m = assert_parity(got, want, f"vsa_op_log2_{grid}")
     assert m["rel_l2"] <= 2e-2
+
+
+@pytest.mark.parametrize("topk", [1, 2, 3, 63, 64, 65, 130])
+def test_fine_stage_on_tiles_of_any_size(fv, topk):
+    """Steps of the fine kernel: tiles of more than 32 keys are shared by two waves, smaller ones taken in turn, those
+    of up to 16 two at a time, lists read 64 entries at a time. Every size at the edges of these, in lists shorter and
+    longer than 64, against sums in 64 bits. P is rounded to bf16, 2^-9 / sqrt(3) = 1.1e-3 of a row at most: four times
+    that is the bar."""
+    import torch
+
+    announce(f"vsa fine, tiles of any size, topk={topk}")
+    ctx = fv.VsaCtx((4, 20, 120), 0.8)   # 150 tiles
+    nb, bh, scale = ctx.num_tiles, 2, 1.0 / np.sqrt(D)
+    gen = torch.Generator(device="cuda").manual_seed(topk)
+    edges = torch.tensor([1, 15, 16, 17, 31, 32, 33, 48, 63, 64], device="cuda", dtype=torch.int32)
+    sizes = edges[torch.randint(0, len(edges), (nb,), generator=gen, device="cuda")]
+    ctx.block_sizes = sizes
+    real = torch.arange(64, device="cuda")[None, :] < sizes[:, None]                       # [nb, 64]
+    q, k, v = (torch.randn(bh, nb * 64, D, generator=gen, device="cuda").to(torch.bfloat16) for _ in range(3))
+    k, v = (x.masked_fill(~real.reshape(1, -1, 1), 0) for x in (k, v))                       # padding slots hold zeros
+    sel = torch.rand(bh, nb, nb, generator=gen, device="cuda").topk(topk, -1).indices.sort(-1).values.to(torch.int32)
+    got = fv.vsa_fine(q, k, v, sel.contiguous(), ctx, scale).double().reshape(bh, nb, 64, D)
+    again = fv.vsa_fine(q, k, v, sel.contiguous(), ctx, scale).double().reshape(bh, nb, 64, D)
+    assert torch.equal(got, again)
+    want = torch.empty_like(got)
+    for b in range(bh):
+        kt, vt = (x[b].double().reshape(nb, 64, D) for x in (k, v))
+        for t in range(nb):
+            s = sel[b, t].long()
+            x = (q[b, 64 * t:64 * t + 64].double() @ kt[s].reshape(-1, D).T) * scale
+            x = x.masked_fill(~real[s].reshape(1, -1), float("-inf"))
+            want[b, t] = torch.softmax(x, -1) @ vt[s].reshape(-1, D)
+    rows = ((got - want).norm(dim=-1) / want.norm(dim=-1)).flatten()
+    assert rows.max().item() <= 4.4e-3, rows.max().item()
