@@ -221,7 +221,7 @@ int fv_vsa_topk(const float* scores, uint32_t* out, size_t rows, size_t n, size_
     if (rows == 0 || k == 0) return FV_OK;
     if (n == 0 || n > kTopkMaxN || !fits_int(rows) || !fits_int(k))
         return fv_decline("vsa_topk: needs 1 <= n <= 4096");
-    hipError_t e = fv_internal_launch_topk(scores, out, (int)rows, (int)n, (int)k, (hipStream_t)stream);
+    hipError_t e = fv_internal_launch_topk(scores, out, (int)rows, (int)n, (int)k, nullptr, 0, (hipStream_t)stream);
     return e == hipSuccess ? FV_OK : fv_fail_hip(e, "vsa_topk");
 }
 
@@ -259,6 +259,8 @@ int fv_vsa_fine(const uint16_t* qt, const uint16_t* kt, const uint16_t* vt, cons
     p.q_tiles = (int)q_tiles;
     p.total = (int)(bh * q_tiles);
     p.per_xcd = (p.total + 7) / 8;
+    p.pace = nullptr;
+    p.gang = p.pace_stride = 0;
     p.final_out = nullptr;
     p.coarse = nullptr;
     p.gate = nullptr;
@@ -356,8 +358,6 @@ static int vsa_attention_common(const void* q, const void* k, const void* v, int
     }
     // 2. coarse attention over tiles; raw scores kept for the selection (rt/vsa.rs:385-394)
     if ((rc = fv_vsa_coarse(qc, kc, vc, scores, coarse, bh, num_tiles, dim, scale, stream))) return rc;
-    // 3. top-k tiles per query tile (rt/vsa.rs:398-400)
-    if ((rc = fv_vsa_topk(scores, sel, bh * num_tiles, num_tiles, topk, stream))) return rc;
     // 5. out = coarse * gate + sparse, back in token order: fused into the fine kernel's epilogue
     //    (no f32 sparse buffer: 2 x 200 MB of traffic and 200 MB of workspace less at Wan 480p)
     fv::VsaFineParams p;
@@ -380,6 +380,12 @@ static int vsa_attention_common(const void* q, const void* k, const void* v, int
     p.gate_is_bf16 = gate_is_bf16;
     p.slot_src = slot_src;
     p.seq = (long)seq;
+    // 3. top-k tiles per query tile (rt/vsa.rs:398-400); the same launch clears the fine kernel's counters, which take the
+    //    place of the query means (fewer words than those: a line per 64 key tiles and 128 query tiles)
+    const size_t words = fv_internal_fine_pace(&p);
+    p.pace = words > 0 && words <= bh * num_tiles * dim ? (int*)qc : nullptr;
+    e = fv_internal_launch_topk(scores, sel, (int)(bh * num_tiles), (int)num_tiles, (int)topk, p.pace, p.pace ? (int)words : 0, st);
+    if (e != hipSuccess) return fv_fail_hip(e, "vsa_topk");
     e = fv_internal_launch_fine(&p, st);
     return e == hipSuccess ? FV_OK : fv_fail_hip(e, "vsa_fine (fused combine)");
 }

@@ -74,6 +74,8 @@ struct VsaFineParams {
     float sl2;
     int q_base, q_tiles;          // query tiles [q_base, q_base + q_tiles)
     int total, per_xcd;           // bh * q_tiles, ceil(total / 8)
+    int* pace;                    // zeroed counters (fv_internal_fine_pace) or null
+    int gang, pace_stride;        // workgroups that share a set of counters; words a set
     // Fused combine (whole-op entry): when `final_out` is set the kernel writes
     // final_out[token] = coarse[tile] * gate[token] + sparse instead of `out`, in token order.
     float* final_out;             // [bh, seq, 128] f32 or null
@@ -184,7 +186,7 @@ extern "C" hipError_t fv_internal_launch_coarse(const float* qc, const float* kc
                                                 float* scores, float* coarse, size_t bh, int nb,
                                                 int dim, float scale, hipStream_t st);
 extern "C" hipError_t fv_internal_launch_topk(const float* scores, unsigned* out, int rows, int n, int k,
-                                              hipStream_t st);
+                                              int* zero, int zeros, hipStream_t st);
 extern "C" hipError_t fv_internal_launch_tile_scan3(const void* const x[3], int x_is_bf16, const int* slot_src,
                                                     const int* block_sizes, uint16_t* const tiles[3],
                                                     float* const means[3], const float* copy_mul, size_t bh, size_t seq,
@@ -207,6 +209,7 @@ extern "C" hipError_t fv_internal_launch_splitkv_merge(const float* part_o, cons
                                                        hipStream_t st);
 extern "C" hipError_t fv_internal_init_flash(void);
 extern "C" hipError_t fv_internal_init_vsa(void);
+extern "C" size_t fv_internal_fine_pace(fv::VsaFineParams* p);
 extern "C" hipError_t fv_internal_launch_fine(const fv::VsaFineParams* p, hipStream_t st);
 extern "C" hipError_t fv_internal_launch_combine(const float* sparse, const float* coarse,
                                                  const void* gate, int gate_is_bf16,

@@ -2,6 +2,8 @@
 // softmax x V, bitwise-descent top-k, tile permute, block-sparse fine attention,
 // gated combine. Reference stages: crates/fastvideo-cudarc/src/rt/vsa.rs:358-470
 // and the kernels cited per function below (kernels/core.cu, kernels/attn3.cu).
+#include <algorithm>
+
 #include "attn_core.h"
 #include "fv_internal.h"
 
@@ -429,7 +431,8 @@ FV_DEV int lanes_below(unsigned long long m) {
 template <int KPL>
 __global__ __launch_bounds__(64 * kTopkRowsPerBlock) void vsa_topk_kernel(const float* __restrict__ scores,
                                                                           unsigned* __restrict__ out, int rows,
-                                                                          int n, int k) {
+                                                                          int n, int k, int* zero, int zeros) {
+    for (int i = blockIdx.x * (64 * kTopkRowsPerBlock) + threadIdx.x; i < zeros; i += gridDim.x * (64 * kTopkRowsPerBlock)) zero[i] = 0;
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * kTopkRowsPerBlock + (threadIdx.x >> 6);
     if (row >= rows) return;   // the whole wave leaves; waves never meet at a barrier
@@ -515,9 +518,15 @@ __global__ __launch_bounds__(256) void vsa_tile_qkv_kernel(const void* __restric
 // Padding is left out. A selected tile of more than 32 keys is a step of each wave; one of up to 32 a step of one wave,
 // the waves taking turns; two of up to 16 share a step. A query tile of up to 32 queries (whole op only: the stage entry
 // writes the padding rows too) is walked for those 32 alone (NB = 1), and one wave finishes them.
-// Measured on MI355X, 12 heads, 624 tiles, 125 selected, us, the form this replaces (a wave 32 queries, both waves on
-// every key tile behind three barriers) / this one: ragged tiles of 21 x 30 x 52 2400 / 2010, full tiles with a
-// uniformly random selection 2350 / 2430, a banded one 2075 / 1900.
+// Workgroups in step (FinePace). A selection that is spread over the sequence reads K and V as many times as it
+// has tiles a row (31 GB at 12 heads, 125 of 624 tiles), and what misses the 4 MB of an XCD's L2 comes at 6.8 TB/s
+// however the kernel is scheduled. The workgroups resident on an XCD belong to one or two heads and walk their ascending lists
+// from the front together, but drift apart; so a wave enters the next window of kPaceTiles key tiles (2 MB of K and V)
+// only when half the waves of its gang, the workgroups that one XCD holds at a time, have entered the one before.
+// Measured on MI355X, 12 heads, 624 tiles, 125 selected, us: the form this replaces (a wave 32 queries, both waves on
+// every key tile behind three barriers) / steps as above / in step: ragged tiles of 21 x 30 x 52 2400 / 2010 / 1650, full
+// tiles with a uniformly random selection 2350 / 2430 / 2150, a banded one 2075 / 1900 / 1965. All waves instead of half
+// of them: 2860, 3100 and 2820; windows of 48, 96 tiles with 7/8: 1900, 1720 (ragged).
 constexpr int kFineSlot = 4096;
 constexpr int kFineWave = 5 * kFineSlot;
 constexpr int kFineLds = 2 * kFineWave;
@@ -530,8 +539,35 @@ struct FineStep {
     bool none;
 };
 
+// How far the waves of a gang have got: counters[w] of them have entered window w or a later one. Only a hint: no result
+// depends on it, a wave that has polled kPaceTries times (about 30 us) stops asking, and the atomics are those of one
+// workgroup's scope, which are carried out in the L2 that the gang shares (agent scope, past the L2s: 4.7 ms a launch).
+constexpr int kPaceTiles = 64, kPaceTries = 30;
+struct FinePace {
+    int* counters;   // null: no pace is kept
+    int half;        // of the gang's waves
+    int window;      // the one this wave has entered
+    bool asks;
+    FV_DEV void enter(int w, int lane) {
+        if (lane == 0)
+            for (int x = window + 1; x <= w; x++) __hip_atomic_fetch_add(counters + x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        window = w;
+    }
+    FV_DEV void wait(int lane) {
+        for (int tries = 0; asks; tries++) {
+            int n = 0;
+            asm volatile("" : "+v"(n));   // (an addition of nothing, not a load: that may come from the L1)
+            if (lane == 0) n = __hip_atomic_fetch_add(counters + window - 1, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (__builtin_amdgcn_readfirstlane(n) >= half) break;
+            if (tries == kPaceTries) asks = false;
+            __builtin_amdgcn_s_sleep(16);
+        }
+    }
+};
+
 template <int NB>
-FV_DEV void fine_item(const VsaFineParams& p, lds_u8* smem, const int wave, const int lane, const int bh, const int qtile) {
+FV_DEV void fine_item(const VsaFineParams& p, lds_u8* smem, const int wave, const int lane, const int bh, const int qtile,
+                      FinePace pace) {
     lds_u8* ring = smem + wave * kFineWave;
     const int h = lane >> 5, c32 = lane & 31;
     const int nb = p.num_tiles, topk = p.topk;
@@ -624,9 +660,17 @@ FV_DEV void fine_item(const VsaFineParams& p, lds_u8* smem, const int wave, cons
     for (int x = 0; x < 8; x++) load_k(x < 4 ? sk0 : sk1, cur, x >> 2, x & 3);
 #pragma unroll
     for (int x = 0; x < 8; x++) load_v(x < 4 ? sv0 : sv1, cur, x >> 2, x & 3);
+    if (pace.counters) pace.enter(0, lane);
     constexpr int kAhead = 2;   // a fragment feeds NB MFMAs and is read kAhead fragments before them
     while (!cur.none) {
         const FineStep nx = next();
+        if (pace.counters) {
+            const int w = nx.row_a / (kPaceTiles * kTileElems);
+            if (w > pace.window) {
+                pace.enter(w, lane);
+                pace.wait(lane);
+            }
+        }
         // (addresses are formed where they are used: kept across the loop they would take 16 registers that it has not got)
         asm volatile("" : "+v"(krd), "+v"(vrd), "+v"(koff));
         f32x16 s[NB];
@@ -735,6 +779,7 @@ FV_DEV void fine_item(const VsaFineParams& p, lds_u8* smem, const int wave, cons
         cur = nx;
     }
 
+    if (pace.counters) pace.enter((nb - 1) / kPaceTiles, lane);
     wait_vmcnt<0>();   // (the loads past the end)
     // The merge: each wave hands the other one's queries over in its own ring.
     typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
@@ -818,8 +863,14 @@ __global__ __launch_bounds__(128, 2) void vsa_fine_kernel(const VsaFineParams p)
     const int bh = work / p.q_tiles;
     const int qtile = p.q_base + work % p.q_tiles;
     if (qtile >= p.num_tiles) return;
-    if (p.final_out && p.block_sizes[qtile] <= 32) fine_item<1>(p, (lds_u8*)smem_raw, wave, lane, bh, qtile);
-    else fine_item<2>(p, (lds_u8*)smem_raw, wave, lane, bh, qtile);
+    FinePace pace = {nullptr, 0, -1, true};
+    if (p.pace) {
+        const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3, gang = at / p.gang;
+        pace.counters = p.pace + ((size_t)xcd * ((p.per_xcd + p.gang - 1) / p.gang) + gang) * p.pace_stride;
+        pace.half = min(p.gang, min(p.per_xcd, p.total - xcd * p.per_xcd) - gang * p.gang);   // workgroups, of two waves
+    }
+    if (p.final_out && p.block_sizes[qtile] <= 32) fine_item<1>(p, (lds_u8*)smem_raw, wave, lane, bh, qtile, pace);
+    else fine_item<2>(p, (lds_u8*)smem_raw, wave, lane, bh, qtile, pace);
 }
 
 // ---- combine (kernels/core.cu:803-835) -----------------------------------------------------
@@ -942,8 +993,18 @@ extern "C" hipError_t fv_internal_launch_coarse(const float* qc, const float* kc
     return hipGetLastError();
 }
 
+// Counters of FinePace that a launch of `total` query tiles asks for (none where the key tiles of a head, 32 KB each, fit
+// an XCD's L2), and its layout: gangs of as many workgroups as an XCD holds at a time, each with whole cache lines.
+extern "C" size_t fv_internal_fine_pace(fv::VsaFineParams* p) {
+    p->pace_stride = ((p->num_tiles + kPaceTiles - 1) / kPaceTiles + 31) & ~31;
+    p->gang = std::max(1, fv_compute_units() / 8 * 4);
+    if (p->num_tiles <= 128) return 0;
+    return (size_t)8 * ((p->per_xcd + p->gang - 1) / p->gang) * p->pace_stride;
+}
+
+// zero: so many words set to zero besides (fv_internal_fine_pace)
 extern "C" hipError_t fv_internal_launch_topk(const float* scores, unsigned* out, int rows, int n, int k,
-                                              hipStream_t st) {
+                                              int* zero, int zeros, hipStream_t st) {
     if (n < 1 || n > kTopkMaxN) return hipErrorInvalidValue;
     // keys per lane: the smallest instantiated count that holds the row (624 tiles: 10)
     const int need = (n + 63) / 64;
@@ -953,7 +1014,7 @@ extern "C" hipError_t fv_internal_launch_topk(const float* scores, unsigned* out
         const dim3 grid((some + kTopkRowsPerBlock - 1) / kTopkRowsPerBlock), block(64 * kTopkRowsPerBlock);
         const float* src = scores + (size_t)at * n;
         unsigned* dst = out + (size_t)at * k;
-#define FV_TOPK(K) hipLaunchKernelGGL(vsa_topk_kernel<K>, grid, block, 0, st, src, dst, some, n, k)
+#define FV_TOPK(K) hipLaunchKernelGGL(vsa_topk_kernel<K>, grid, block, 0, st, src, dst, some, n, k, zero, zeros)
         if (need <= 4) FV_TOPK(4);
         else if (need <= 8) FV_TOPK(8);
         else if (need <= 10) FV_TOPK(10);
@@ -985,6 +1046,7 @@ extern "C" hipError_t fv_internal_launch_tile_qkv(const void* x, int x_is_bf16, 
     return hipGetLastError();
 }
 
+// (40 KB of LDS a workgroup: four fill a CU)
 extern "C" hipError_t fv_internal_launch_fine(const fv::VsaFineParams* p, hipStream_t st) {
     hipLaunchKernelGGL(vsa_fine_kernel, dim3(p->per_xcd * 8), dim3(128), kFineLds, st, *p);
     return hipGetLastError();

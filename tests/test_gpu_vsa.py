@@ -460,3 +460,25 @@ def test_fine_stage_on_tiles_of_any_size(fv, topk):
             want[b, t] = torch.softmax(x, -1) @ vt[s].reshape(-1, D)
     rows = ((got - want).norm(dim=-1) / want.norm(dim=-1)).flatten()
     assert rows.max().item() <= 4.4e-3, rows.max().item()
+
+
+@pytest.mark.parametrize("grid, heads", [((9, 21, 50), 3), ((6, 33, 47), 12)])
+def test_whole_op_in_step_equals_the_stages(fv, grid, heads):
+    """Whole op on more than 128 tiles: its fine kernel keeps the workgroups of an XCD in step and walks query tiles of up
+    to 32 rows for those alone. The stages one by one do neither."""
+    import torch
+
+    announce(f"vsa whole op in step grid={grid}")
+    ctx = fv.VsaCtx(grid, 0.8)
+    assert ctx.num_tiles > 128
+    scale = 1.0 / np.sqrt(D)
+    gen = torch.Generator(device="cuda").manual_seed(heads)
+    q, k, v, g = (torch.randn(heads, ctx.seq, D, generator=gen, device="cuda").to(torch.bfloat16) for _ in range(4))
+    whole, sel = fv.vsa_attention_device(q, k, v, g, ctx, scale, return_selected=True)
+    qc, kc, vc = (fv.vsa_tile_mean(x, ctx) for x in (q, k, v))
+    _, coarse = fv.vsa_coarse(qc, kc, vc, scale)
+    qt, kt, vt = (fv.vsa_tile_qkv(x, ctx) for x in (q, k, v))
+    sparse = fv.vsa_fine(qt, kt, vt, sel, ctx, scale)
+    parts = fv.vsa_combine(sparse, coarse, g, ctx)
+    # the same rows, their keys shared out over the waves in the same way: f32 sums of the same terms
+    assert ((whole - parts).norm() / parts.norm()).item() <= 1e-6
