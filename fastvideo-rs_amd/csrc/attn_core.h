@@ -318,8 +318,8 @@ FV_DEV void softmax_tile_pair_fixed(const f32x16 (&s0)[2], const f32x16 (&s1)[2]
 
 // One tile. `side(part)` runs after the rescale (part 0) and after each 32-key half of the exponentials
 // (parts 1, 2): slots for side work, such as tile DMA issue, spread through the VALU stream.
-template <bool SCALED, class Side>
-FV_DEV void softmax_tile_side_off(f32x16 (&s)[2], SoftmaxOffState& st, f32x16 (&o)[4], f32x16& negoff, float sl2,
+template <bool SCALED, class Side, int NO>
+FV_DEV void softmax_tile_side_off(f32x16 (&s)[2], SoftmaxOffState& st, f32x16 (&o)[NO], f32x16& negoff, float sl2,
                                   bf16x8 (&pb)[4], Side&& side) {
     float mx = s[0][0];
 #pragma unroll
@@ -328,7 +328,7 @@ FV_DEV void softmax_tile_side_off(f32x16 (&s)[2], SoftmaxOffState& st, f32x16 (&
     for (int i = 0; i < 16; i++) mx = __builtin_fmaxf(mx, s[1][i]);
     mx = pair_max(mx);
     f32x16* const sc[2] = {&s[0], &s[1]};
-    softmax_off_rescale<SCALED, 4, 2>(mx, st, o, negoff, sl2, sc);
+    softmax_off_rescale<SCALED, NO, 2>(mx, st, o, negoff, sl2, sc);
     side(0);
 #pragma unroll
     for (int b = 0; b < 2; b++) {

@@ -97,6 +97,53 @@ FV_DEV int vdn_tile_order(const Params& p, int r) {
     return back - 1 - r;   // r counts on from back - start: start - 1 down to front
 }
 
+// A wave's 32 rows o * inv, the first of them row `row0` of the result; `rows` (and no more) are stored. `my`: 32 x 2D bytes
+// of LDS of the wave's own.
+template <int D>
+FV_DEV void store_rows(lds_u8* my, const f32x16 (&o)[D / 32], float inv, float* out_f32, uint16_t* out_bf16, int out_is_bf16,
+                       size_t row0, int rows, int lane) {
+    const int h = lane >> 5, c32 = lane & 31;
+    constexpr int kNO = D / 32;
+    if (out_is_bf16) {
+        // bf16 rows: scattered 8-byte pieces in, whole rows out, 16 bytes per lane and 1 KB (D = 128) of consecutive
+        // output per store instruction
+        constexpr int kRowB = 2 * D, kCh = kRowB / 16;
+#pragma unroll
+        for (int db = 0; db < kNO; db++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                f32x4 r;
+#pragma unroll
+                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
+                const bf16x4 rb4 = __builtin_convertvector(r, bf16x4);
+                const int ch = (4 * db + g) ^ (c32 & (kCh - 1));
+                *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>(my + c32 * kRowB + (ch << 4) + 8 * h) = rb4;
+            }
+        // (same-wave LDS writes and reads complete in order; the compiler waits on the reads' data)
+        constexpr int kRowsPer = 64 / kCh;           // rows one store instruction covers
+        const int lr = lane / kCh, lc = lane % kCh;
+        uint16_t* ob = out_bf16 + row0 * D;
+#pragma unroll
+        for (int i = 0; i < 32 / kRowsPer; i++) {
+            const int rr = i * kRowsPer + lr;
+            const u32x4 val = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(
+                my + rr * kRowB + ((lc ^ (rr & (kCh - 1))) << 4));
+            if (rr < rows) global_store<u32x4>(ob + (size_t)rr * D + lc * 8, val);
+        }
+    } else if (c32 < rows) {
+        float* ob = out_f32 + (row0 + c32) * D;
+#pragma unroll
+        for (int db = 0; db < kNO; db++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                f32x4 r;
+#pragma unroll
+                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
+                global_store<f32x4>(ob + 32 * db + 8 * g + 4 * h, r);
+            }
+    }
+}
+
 // One workgroup's item: the whole pass over its key tiles and the store of its rows. Returns false (FIXED only,
 // nothing stored) when the pass has to be made again with the running max.
 // FIXED: once the first phase has put every query's offset at the largest score of its first 128 keys, the offset
@@ -504,52 +551,8 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
             return true;
         }
     }
-    if (out_is_bf16) {
-        // bf16 rows through this wave's own 32 x 2D-byte slice of the K ring (every K read is behind the last
-        // barrier and no load is in flight): scattered 8-byte pieces in, whole rows out, 16 bytes per
-        // lane and 1 KB (D = 128) of consecutive output per store instruction
-        constexpr int kRowB = 2 * kD, kCh = kRowB / 16;
-        lds_u8* my = smem + wave * (32 * kRowB);
-#pragma unroll
-        for (int db = 0; db < kNO; db++)
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                f32x4 r;
-#pragma unroll
-                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
-                const bf16x4 rb4 = __builtin_convertvector(r, bf16x4);
-                const int ch = (4 * db + g) ^ (c32 & (kCh - 1));
-                *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>(my + c32 * kRowB + (ch << 4) + 8 * h) = rb4;
-            }
-        // (same-wave LDS writes and reads complete in order; the compiler waits on the reads' data)
-        constexpr int kRowsPer = 64 / kCh;           // rows one store instruction covers
-        const int lr = lane / kCh, lc = lane % kCh;
-        uint16_t* ob = out_bf16 + ((size_t)bh * sq + q0 + wave * 32) * kD;
-#pragma unroll
-        for (int i = 0; i < 32 / kRowsPer; i++) {
-            const int rr = i * kRowsPer + lr;
-            const u32x4 val = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(
-                my + rr * kRowB + ((lc ^ (rr & (kCh - 1))) << 4));
-            if (wave * 32 + rr < qlen) global_store<u32x4>(ob + (size_t)rr * kD + lc * 8, val);
-        }
-    } else if (row < qlen) {
-        const size_t base = ((size_t)bh * sq + q0 + row) * kD;
-#pragma unroll
-        for (int db = 0; db < kNO; db++)
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int d0 = 32 * db + 8 * g + 4 * h;
-                f32x4 r;
-#pragma unroll
-                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
-                if (out_is_bf16) {
-                    const bf16x4 rb4 = __builtin_convertvector(r, bf16x4);
-                    global_store<bf16x4>(out_bf16 + base + d0, rb4);
-                } else {
-                    global_store<f32x4>(out_f32 + base + d0, r);
-                }
-            }
-    }
+    store_rows<D>(smem + wave * (32 * 2 * kD), o, inv, out_f32, out_bf16, out_is_bf16, (size_t)bh * sq + q0 + wave * 32,
+                  qlen - wave * 32, lane);
     return true;
 }
 
@@ -578,6 +581,173 @@ __global__ __launch_bounds__(256 * NG, 2) void flash_fwd_pp2(const FlashParams p
         int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
         asm volatile("" : "+v"(lane), "+s"(wave), "+s"(block), "+s"(again));
         flash_item<NG, MASKED, D, LOG2DOM, false>(*again, wave, lane, block);
+    }
+}
+
+// Dense launches on few keys (fv_duo): two workgroups a CU. flash_fwd_pp2 gives an item the CU and pays its first loads,
+// its first and last slot and its store in the open, half of the time at eight key tiles. Here an item is four waves x 32
+// queries with two K and two V buffers (64 KB at D = 128), so that two share a CU unsynchronised and one's ends pass under
+// the other's arithmetic. A phase is one key tile: the matrix part (O += P V of the tile before, S = K Q^T, with the loads
+// of the next K and of this V going out behind the first MFMAs), the softmax, one barrier.
+constexpr int kDuoBM = 128;
+template <int D>
+constexpr int kDuoLds = 4 * TileGeo<D>::kTile + kVoteBytes;
+template <int D, bool LOG2DOM, bool FIXED, class Params>
+FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int block) {
+    using G = TileGeo<D>;
+    using Dma = TileDma<4, D>;
+    constexpr int kTileBytes = G::kTile, kNO = D / 32, kIt = Dma::ITER;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    lds_u8* smem = (lds_u8*)smem_raw;
+    const int h = lane >> 5, c32 = lane & 31;
+    const int work = (block & 7) * p.per_xcd + (block >> 3);   // XCD x: a contiguous eighth of the (head, query tile) items
+    if (work >= p.total) return true;
+    const int bh = work / p.nqt, q0 = (work - bh * p.nqt) * kDuoBM;
+    const int sq = p.sq, sk = p.sk, qlen = min(kDuoBM, sq - q0), nkt = (sk + kBN - 1) / kBN;
+    const float sl2 = p.sl2, NEG = neg_inf();
+    float* out_f32 = p.out_f32;
+    uint16_t* out_bf16 = p.out_bf16;
+    int out_is_bf16 = p.out_is_bf16;
+    asm volatile("" : "+s"(out_f32), "+s"(out_bf16), "+s"(out_is_bf16));   // (fetched now, see flash_item)
+    const uint16_t* Qh = p.q + (size_t)bh * p.q_plane + (size_t)q0 * D;
+    const uint16_t* Kh = p.k + (size_t)bh * p.k_plane;
+    const uint16_t* Vh = p.v + (size_t)bh * p.v_plane;
+
+    auto kbuf = [&](int t) -> lds_u8* { return smem + (t & 1) * kTileBytes; };
+    auto vbuf = [&](int t) -> lds_u8* { return smem + (2 + (t & 1)) * kTileBytes; };
+    Dma dma;
+    dma.init(wave, lane);
+    // (tiles past the end repeat the last one)
+    auto target_k = [&](int t) {
+        const int kv0 = min(t, nkt - 1) * kBN;
+        return dma.template prepare<false>(kbuf(t), Kh + (size_t)kv0 * D, sk - kv0, wave);
+    };
+    auto target_v = [&](int t) {
+        const int kv0 = t * kBN;
+        return dma.template prepare<true>(vbuf(t), Vh + (size_t)kv0 * D, sk - kv0, wave);
+    };
+    bf16x8 qf[D / 16];
+    const TileReadBases rb = tile_read_bases<D>(lane);
+    {
+        // the wave's query rows through its slice of the V buffers, as in flash_item; K(0) besides
+        lds_u8* qs = smem + 2 * kTileBytes + wave * (32 * G::kRow);
+        const unsigned qlds = __builtin_amdgcn_readfirstlane((unsigned)(size_t)qs);
+#pragma unroll
+        for (int it = 0; it < 32 * G::kRow / 1024; it++) {
+            const int r = it * G::kRowsPerDma + lane / G::kChunks, pch = lane % G::kChunks;
+            const int rg = min(wave * 32 + r, qlen - 1);   // rows past the end re-read the last one (zeroed below)
+            lds_dma16_s(qlds + it * 1024, Qh, (unsigned)(rg * G::kRow + ((pch ^ G::kswz(r)) << 4)));
+        }
+        const typename Dma::Prepared k0 = target_k(0);
+#pragma unroll
+        for (int it = 0; it < kIt; it++) Dma::issue_prepared(k0, it);
+        wait_vmcnt<kIt>();
+        const bool ok = wave * 32 + c32 < qlen;
+#pragma unroll
+        for (int dk = 0; dk < D / 16; dk++) {
+            bf16x8 t = lds_read_b128(qs + (rb.k ^ (dk << 5)));
+            if (!ok) t = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+            qf[dk] = t;
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the slice is read before the wave passes its next barrier
+    }
+    f32x16 o[kNO], s_init, s[2];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        s_init[i] = 0.f;
+#pragma unroll
+        for (int db = 0; db < kNO; db++) o[db][i] = 0.f;
+    }
+    SoftmaxOffState st;
+    st.init();
+    bf16x8 pb[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int x = 0; x < 8; x++) pb[t][x] = (__bf16)0.0f;
+    auto mask_tail = [&](int m) {
+        const int left = sk - m * kBN - 4 * h;
+        if (sk - m * kBN < kBN) {
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    if (32 * b + 8 * (i >> 2) + (i & 3) >= left) s[b][i] = NEG;
+        }
+    };
+    typename Dma::Prepared dk = target_k(1), dv = target_v(0);
+    wait_vmcnt<0>();
+    block_barrier();   // K(0) resident, every wave has its queries
+    // The first phase has no tile before it to multiply: unrolled apart.
+#pragma unroll
+    for (int part = 0; part < 2; part++) {
+        const bool first = part == 0;
+#pragma unroll 1
+        for (int m = part; m < (first ? 1 : nkt); m++) {
+            __builtin_amdgcn_s_setprio(1);
+            constexpr int kAhead = 3;
+            auto hook_dma = [&](int g) {
+                g -= first ? D / 16 : 0;
+                if (g >= 0 && g < kIt) Dma::issue_prepared(dv, g);
+                else if (g < 2 * kIt) Dma::issue_prepared(dk, g - kIt);
+            };
+            if (first) mfma_phase<false, kAhead, decltype(hook_dma)&, D>(vbuf(1), kbuf(0), rb, pb, o, qf, s, s_init, hook_dma);
+            else mfma_phase<true, kAhead, decltype(hook_dma)&, D>(vbuf(m - 1), kbuf(m), rb, pb, o, qf, s, s_init, hook_dma);
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
+            mask_tail(m);
+            if (FIXED && !first) {
+#pragma unroll
+                for (int b = 0; b < 2; b++) softmax_off_block<!LOG2DOM>(s[b], st, sl2, pb[2 * b], pb[2 * b + 1]);
+            } else {
+                softmax_tile_side_off<!LOG2DOM>(s, st, o, s_init, sl2, pb, [](int) {});
+            }
+            asm volatile("" ::"v"(pb[0]), "v"(pb[1]), "v"(pb[2]), "v"(pb[3]), "v"(st.l_acc));
+            dk = target_k(m + 2);
+            dv = target_v(min(m + 1, nkt - 1));
+            __builtin_amdgcn_sched_barrier(0);
+            wait_vmcnt<0>();
+            block_barrier();   // K(m+1), V(m) resident; this phase's tiles read by every wave
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    pv_tile<D>(vbuf(nkt - 1), rb.v, pb, o);
+
+    if constexpr (FIXED) {   // did the fixed offset hold (flash_item)?
+        float chk = 0.f;
+#pragma unroll
+        for (int db = 0; db < kNO; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) chk = __builtin_fmaf(o[db][i], 0.f, chk);
+        const bool lane_ok = (pair_sum(st.l_acc) < 0x1p+100f) && (chk == 0.f);
+        auto* votes = (__attribute__((address_space(3))) unsigned*)(smem + 4 * kTileBytes);
+        const bool wave_ok = __builtin_amdgcn_ballot_w64(!lane_ok) == 0;
+        if (lane == 0) votes[wave] = wave_ok ? 0u : 1u;
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        block_barrier();
+        const u32x4 v = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(votes);
+        if (__builtin_amdgcn_readfirstlane(v[0] | v[1] | v[2] | v[3]) != 0) {
+            if (wave == 0 && lane == 0) atomicAdd(&g_exact_pass_reruns, 1ull);
+            return false;
+        }
+    }
+    const float l_tot = pair_sum(st.l_acc);
+    store_rows<D>(smem + wave * (32 * 2 * D), o, l_tot > 0.f ? 1.f / l_tot : 0.f, out_f32, out_bf16, out_is_bf16,
+                  (size_t)bh * sq + q0 + wave * 32, qlen - wave * 32, lane);
+    return true;
+}
+template <int D, bool LOG2DOM, bool FIXED>
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_fwd_duo(const FlashParams p) {
+    int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), block = blockIdx.x;
+    if constexpr (!FIXED) {
+        duo_item<D, LOG2DOM, false>(p, wave, threadIdx.x & 63, block);
+    } else {
+        if (duo_item<D, LOG2DOM, true>(p, wave, threadIdx.x & 63, block)) return;
+        using ConstParams = const __attribute__((address_space(4))) FlashParams;   // (as in flash_fwd_pp2)
+        ConstParams* again = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
+        int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+        asm volatile("" : "+v"(lane), "+s"(wave), "+s"(block), "+s"(again));
+        duo_item<D, LOG2DOM, false>(*again, wave, lane, block);
     }
 }
 
@@ -656,6 +826,18 @@ hipError_t launch_flash_as(const fv::FlashParams* p, hipStream_t stream) {
     hipLaunchKernelGGL((fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED>), dim3(p->full + p->per_xcd * 8), dim3(256 * NG), lds, stream, *p);
     return hipGetLastError();
 }
+template <int D, bool LOG2DOM, bool FIXED>
+hipError_t duo_attr() {
+    static std::atomic<unsigned long long> attr_done;
+    return fv_set_max_lds_once((const void*)fv::flash_fwd_duo<D, LOG2DOM, FIXED>, fv::kDuoLds<D>, attr_done);
+}
+template <int D, bool LOG2DOM, bool FIXED>
+hipError_t launch_duo_as(const fv::FlashParams* p, hipStream_t stream) {
+    hipError_t e = duo_attr<D, LOG2DOM, FIXED>();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((fv::flash_fwd_duo<D, LOG2DOM, FIXED>), dim3(p->per_xcd * 8), dim3(256), fv::kDuoLds<D>, stream, *p);
+    return hipGetLastError();
+}
 // FASTVIDEO_SDPA_RUNNING_MAX=1: every launch keeps the running max (no fixed-offset first pass).
 bool running_max_forced() {
     static const bool v = [] {
@@ -685,6 +867,21 @@ hipError_t launch_flash(const fv::FlashParams* p, hipStream_t stream) {
     if (p->out_is_bf16 && offset_is_a_score && !running_max_forced()) return launch_flash_fixed<NG, MASKED, D, true>(p, stream);
     return launch_flash_fixed<NG, MASKED, D, false>(p, stream);
 }
+template <int D>
+hipError_t launch_duo(const fv::FlashParams* p, hipStream_t stream) {
+    const bool fixed = p->out_is_bf16 && !running_max_forced();
+    if (p->sl2 != 1.0f) return fixed ? launch_duo_as<D, false, true>(p, stream) : launch_duo_as<D, false, false>(p, stream);
+    g_log2_domain_launches.fetch_add(1, std::memory_order_relaxed);
+    return fixed ? launch_duo_as<D, true, true>(p, stream) : launch_duo_as<D, true, false>(p, stream);
+}
+template <int D>
+hipError_t init_duo() {
+    hipError_t e = duo_attr<D, false, false>();
+    if (e == hipSuccess) e = duo_attr<D, true, false>();
+    if (e == hipSuccess) e = duo_attr<D, false, true>();
+    if (e == hipSuccess) e = duo_attr<D, true, true>();
+    return e;
+}
 template <int NG, bool MASKED, int D>
 hipError_t init_flash() {
     hipError_t e = flash_attr<NG, MASKED, D, false, false>();
@@ -709,7 +906,13 @@ extern "C" hipError_t fv_internal_init_flash(void) {
     if (e == hipSuccess) e = init_flash<2, true, 64>();
     if (e == hipSuccess) e = init_flash<1, false, 128>();
     if (e == hipSuccess) e = init_flash<1, false, 64>();
+    if (e == hipSuccess) e = init_duo<128>();
+    if (e == hipSuccess) e = init_duo<64>();
     return e;
+}
+
+extern "C" hipError_t fv_internal_launch_duo(const fv::FlashParams* p, int d, hipStream_t stream) {
+    return d == 128 ? launch_duo<128>(p, stream) : d == 64 ? launch_duo<64>(p, stream) : hipErrorInvalidValue;
 }
 
 extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d, int block_m,

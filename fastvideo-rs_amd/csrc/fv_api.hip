@@ -232,6 +232,13 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         if (p.sl2 == 1.0f) fv_internal_count_log2_domain();
         return FV_OK;
     }
+    if (mode == kMaskNone && splits == 1 && fv_duo(bh, sq, sk, d)) {
+        p.nqt = (int)((sq + 127) / 128);
+        p.total = (int)(bh * (size_t)p.nqt);
+        p.per_xcd = (p.total + 7) / 8;
+        const hipError_t e = fv_internal_launch_duo(&p, (int)d, (hipStream_t)stream);
+        return e == hipSuccess ? FV_OK : fail_hip(e, "flash_fwd_duo");
+    }
     hipError_t e = fv_internal_launch_flash(&p, mode != kMaskNone ? 1 : 0, (int)d, (int)bm, (hipStream_t)stream);
     if (e != hipSuccess) return fail_hip(e, mode != kMaskNone ? "flash_fwd_pp2<masked>" : "flash_fwd_pp2<dense>");
     if (p.kv_split > 1) {
@@ -272,6 +279,20 @@ int fv_short_waves(size_t bh, size_t sq, size_t sk, size_t d) {
     return sk <= (d == 64 ? 3072 : 2048) ? 4 : 0;
 }
 
+// flash_fwd_duo (two or, at head dim 64, three workgroups a CU) against flash_fwd_pp2, for walks so short that an item's
+// ends count. Past them the chip runs at its power limit in either form, and 256 queries to a K and V stream cost less. us,
+// flash_fwd_pp2 / flash_fwd_duo: at 128 channels 12 x 32760 x 64 60 / 38, x 200 77 / 65, x 512 120 / 108, x 770 175 / 154, x
+// 1024 193 / 190, x 1200 231 / 222, x 2048 350 / 354, x 4096 670 / 683; 12 x 1560 x 512 16.3 / 12.6, 24 x 3000 x 1000 56 / 50, 24 x
+// 2500 x 1500 45.7 / 46.2, 12 x 6000 x 1500 77 / 71. At 64: 24 x 1300 x 512 11.5 / 10.3, 24 x 4000 x 1500 51 / 43, 24 x
+// 6000 x 3000 145 / 123, 24 x 20000 x 4000 520 / 484, 24 x 7800 x 7800 366 / 373, 24 x 32760 x 32760 6130 / 6155.
+// (Few query tiles have a CU each, of 128 queries where fv_split_plan says so; a few tiles past whole rounds of
+// flash_fwd_pp2 are split there and would cost this one a round too.)
+bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d) {
+    const size_t cus = (size_t)fv_compute_units(), bm = (size_t)fv_internal_flash_block_m(), wgs = bh * ((sq + bm - 1) / bm);
+    const bool crumbs = wgs > cus && wgs % cus > 0 && wgs % cus <= cus / 16;
+    return sk <= (d == 64 ? 6144 : 1536) && !crumbs && bh * ((sq + 127) / 128) > cus / 2;
+}
+
 // Fewer query tiles than CUs: fv_sdpa_splitkv_choose. More: they run in rounds of one per CU, and the last round costs a
 // whole walk of the keys however few tiles are left for it. Where they are few, they are shared out over the chip by key
 // ranges instead; where they are many it does not pay, because a chip that is half busy runs at a higher clock.
@@ -287,11 +308,12 @@ FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d) {
         // 12 x 320 x 320 x 128 13.2 / 11.3, 12 x 1000 x 1000 x 128 25.6 / 23.0, 40 x 700 x 700 x 64 17.4 / 14.8, 12 x 1560 x
         // 512 x 128 17.2 / 14.9, 24 x 390 x 2000 x 128 at 2 splits 34.2 / 29.7; past one per CU, 12 x 4000 x 512 x 128 20.3 /
         // 29.1, 40 x 1000 x 1000 x 64 (320 tiles) 21.5 / 21.7.
+        if (splits == 1 && fv_duo(bh, sq, sk, d)) return {bm, 0, 1, 0};
         const size_t half = bm / 2, small = bh * ((sq + half - 1) / half) * settle_splits(nkt, splits);
         return {small <= cus ? half : bm, 0, splits, fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits)};
     }
     const size_t full = wgs / cus * cus, rest = wgs - full;
-    if (rest == 0) return {bm, 0, 1, 0};
+    if (rest == 0 || fv_duo(bh, sq, sk, d)) return {bm, 0, 1, 0};
     const size_t rows = bh * sq - (full / nqt * sq + full % nqt * bm);
     // us, measured: a workgroup's fixed part, and a 64-key tile while `w` workgroups run (16 x 4000 x 4000 x 128, 256
     // tiles: 121 us, half of them 79); partials written and read at 4 TB/s and a launch

@@ -1,0 +1,89 @@
+"""Unsplit dense calls on few keys, two (head dim 64: three) workgroups a CU: the edges of its key and query tiles, one tile
+and two, the longest walks it takes, f32 and bf16 results, row windows, and rows whose scores outgrow the offset of their
+first tile, so that the pass is made again.
+
+Against the f64 softmax on the same operands. P is rounded to bf16, 2^-9 of each weight at most, and so is a bf16 result:
+2^-9 in the 2-norm for an f32 one, twice that for a bf16 one."""
+import numpy as np
+import pytest
+
+from util import announce
+
+pytestmark = pytest.mark.gpu
+HEADS = 256   # a query tile for every CU: more than the short kernel takes
+
+
+@pytest.fixture(scope="module")
+def fv():
+    import torch
+
+    assert torch.cuda.is_available()
+    import fv_sdpa
+
+    fv_sdpa.lib()
+    return fv_sdpa
+
+
+def operands(torch, seed, sq, sk, d):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return [torch.randn((HEADS, s, d), generator=g, device="cuda").to(torch.bfloat16) for s in (sq, sk, sk)]
+
+
+def want64(torch, q, k, v):
+    out = torch.empty(q.shape, dtype=torch.float64, device=q.device)
+    for b in range(q.shape[0]):
+        s = (q[b].double() @ k[b].double().T) / np.sqrt(q.shape[-1])
+        out[b] = torch.softmax(s, -1) @ v[b].double()
+    return out
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("sq,sk", [(1, 1), (31, 63), (32, 64), (33, 65), (127, 100), (128, 128), (129, 129), (200, 191),
+                                   (257, 192), (40, 513), (20, 1535), (20, 1536), (20, 1537), (20, 6144)])
+def test_edges(fv, sq, sk, d):
+    import torch
+
+    announce(f"duo {HEADS}x{sq}x{sk}x{d}")
+    q, k, v = operands(torch, sq + sk, sq, sk, d)
+    want = want64(torch, q, k, v)
+    for out_bf16, bound in ((True, 2 * 2.0 ** -9), (False, 2.0 ** -9)):
+        got = fv.sdpa_dense_bf16(q, k, v, out_bf16=out_bf16)
+        assert torch.isfinite(got).all()
+        assert ((got.double() - want).norm() / want.norm()).item() <= bound, out_bf16
+        assert torch.equal(got, fv.sdpa(q[None], k[None], v[None], fv.Plan.dense())[0]) or not out_bf16
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_windows_and_reruns(fv, d):
+    import torch
+
+    announce(f"duo windows and reruns d={d}")
+    sq, sk = 70, 300
+    q, k, v = operands(torch, d, sq, sk, d)
+    plain = fv.sdpa_dense_bf16(q, k, v, out_bf16=True)
+    pad = [torch.full((HEADS, x.shape[1] + 9, d), float("nan"), device="cuda", dtype=torch.bfloat16) for x in (q, k, v)]
+    for p, x in zip(pad, (q, k, v)):
+        p[:, 2:2 + x.shape[1]] = x
+    wins = [p[:, 2:2 + x.shape[1]] for p, x in zip(pad, (q, k, v))]
+    assert torch.equal(fv.sdpa_dense_bf16_windows(*wins, out_bf16=True), plain)
+    # scores of head 0 that climb by hundreds of base-2 units past its first tile: that head's workgroup goes again
+    lib = fv.lib()
+    n0 = lib.fv_sdpa_exact_pass_reruns()
+    kc = k.clone()
+    q1 = q.clone()
+    q1[0] = 4.0
+    kc[0] = (torch.arange(sk, device="cuda", dtype=torch.float32)[:, None] * (8.0 / sk)).to(torch.bfloat16).expand(sk, d)
+    got = fv.sdpa_dense_bf16(q1, kc, v, out_bf16=True)
+    torch.cuda.synchronize()
+    assert lib.fv_sdpa_exact_pass_reruns() == n0 + 1
+    want = want64(torch, q1, kc, v)
+    assert ((got.double() - want).norm(dim=(1, 2)) / want.norm(dim=(1, 2))).max().item() <= 2.0 ** -7
+    assert torch.equal(got[1:], plain[1:])
+    # a NaN query is its own row's
+    q2 = q.clone()
+    q2[3, 5, 7] = float("nan")
+    got = fv.sdpa_dense_bf16(q2, k, v, out_bf16=True)
+    assert torch.isnan(got[3, 5]).all()
+    rest = torch.ones(HEADS, sq, dtype=torch.bool, device="cuda")
+    rest[3, 5] = False
+    assert torch.isfinite(got[rest]).all()
