@@ -135,6 +135,7 @@ _TENSOR_BYTES = struct.Struct("@Pii9N")
 _PLAN_BYTES = struct.Struct("@iifPi8Ni0P")
 assert _TENSOR_BYTES.size == C.sizeof(_FvTensor) and _PLAN_BYTES.size == C.sizeof(_FvPlan)
 _NO_SHAPE = (0,) * 8
+_BF16, _F32 = torch.bfloat16, torch.float32
 
 
 def _desc_bytes(t, name):
@@ -146,14 +147,17 @@ def _desc_bytes(t, name):
         rows = _window_rows(t) or 0
         if not rows:
             raise ValueError(f"{name}: want a contiguous CUDA tensor or a row window of a BHSD one")
-    if t.dtype == torch.bfloat16:
+    dtype = t.dtype
+    if dtype is _BF16:
         bf16 = 1
-    elif t.dtype == torch.float32:
+    elif dtype is _F32:
         bf16 = 0
     else:
         raise ValueError(f"{name}: want f32 or bf16")
     shape = t.shape
     rank = len(shape)
+    if rank == 4:
+        return _TENSOR_BYTES.pack(t.data_ptr(), bf16, 4, *shape, 0, 0, 0, 0, rows)
     if rank > 8:
         raise ValueError(f"{name}: rank > 8")
     return _TENSOR_BYTES.pack(t.data_ptr(), bf16, rank, *shape, *_NO_SHAPE[rank:], rows)
@@ -197,8 +201,12 @@ def sdpa(q, k, v, plan):
         raise TensorError(lib.fv_sdpa_last_error().decode(), rc)
     bf16, nbytes = need
     # (the shape of q is the result's: the library refuses anything else before it writes)
+    dtype = _BF16 if bf16 else _F32
     try:
-        res = torch.empty(q.shape, device=q.device, dtype=torch.bfloat16 if bf16 else torch.float32)
+        if type(q) is torch.Tensor and q.dtype is dtype and q.is_contiguous():
+            res = torch.empty_like(q, memory_format=torch.contiguous_format)   # half the time of an empty() by shape
+        else:
+            res = torch.empty(q.shape, device=q.device, dtype=dtype)
     except torch.cuda.OutOfMemoryError as e:
         raise TensorError(f"sdpa: device allocation failed: {e}", -2) from e   # hipErrorOutOfMemory
     try:
