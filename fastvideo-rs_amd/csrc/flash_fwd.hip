@@ -82,19 +82,52 @@ __device__ unsigned long long g_exact_pass_reruns;
 // flight and the longest inner walks came last: 12 heads, 32 frames x 1560, chunk 5, radius 1: 7.45 -> 6.47 ms;
 // 16 frames, chunk 3: 2.43 -> 2.14; 40 heads, 18 frames x 880, chunk 5, radius 2: 4.27 -> 4.10; clips whose windows
 // cover everything: equal. (Heads dealt to XCDs besides, so that an L2 serves few of them: equal to 1 %.)
-template <class Params>
+template <int BM, class Params>
 FV_DEV int vdn_tile_order(const Params& p, int r) {
     const int n = p.nqt, t = p.ft;
-    const int front = min(n, (p.vs + t + kPpBM - 1) / kPpBM);         // tiles [0, front)
-    const int back = min(n, max(front, (p.ve - t) / kPpBM));          // tiles [back, n)
+    const int front = min(n, (p.vs + t + BM - 1) / BM);         // tiles [0, front)
+    const int back = min(n, max(front, (p.ve - t) / BM));          // tiles [back, n)
     const int first_full = max(1, min(p.frames, (int)min(0x7fffffffL, (long)p.radius * max(1, p.chunk))));
-    const int start = min(max((p.vs + first_full * t) / kPpBM, front), back);
+    const int start = min(max((p.vs + first_full * t) / BM, front), back);
     if (r < front) return r;
     r -= front;
     if (r < n - back) return back + r;
     r -= n - back;
     if (r < back - start) return start + r;
     return back - 1 - r;   // r counts on from back - start: start - 1 down to front
+}
+
+// The keys query qi of a masked launch sees: x < a_hi || x >= c_lo || (w_lo <= x && x < w_hi).
+struct LaneMask {
+    int a_hi, c_lo, w_lo, w_hi;
+};
+template <class Params>
+FV_DEV LaneMask lane_mask(const Params& p, int qi) {
+    LaneMask m = {0, 0x7fffffff, 0, 0};
+    if (p.mask_mode == 1) {
+        // block-causal (rt/attn.rs:449-453): keys of blocks (tq - win, tq], plus the sink blocks
+        const int ft = p.ft, win = p.win;
+        const int tq = qi / ft;
+        m.a_hi = (int)min((long)p.sk, (long)p.sink * ft);
+        m.w_hi = (int)min((long)0x7fffffff, (long)(tq + 1) * ft);
+        m.w_lo = win > 0 ? max(0, tq - win + 1) * ft : 0;
+    } else {
+        // VDN window (rt/attn.rs:483-510): rows outside [vs, ve) and the frames 0 and
+        // frames-1 are dense both ways; any other frame sees the frames of its window
+        const int vs = p.vs, ve = p.ve, t = p.ft, last = p.frames - 1, c = p.chunk, r = p.radius;
+        auto lo_frame = [&](int f) { return max(0, c > 0 ? (f / c - r) * c : f - r); };
+        auto hi_frame = [&](int f) { return min(last, c > 0 ? (f / c + r + 1) * c - 1 : f + r); };
+        if (qi >= vs + t && qi < ve - t) {
+            const int qf = (qi - vs) / t;
+            m.a_hi = vs + t;
+            m.c_lo = ve - t;
+            m.w_lo = vs + lo_frame(qf) * t;
+            m.w_hi = vs + (hi_frame(qf) + 1) * t;
+        } else {
+            m.a_hi = 0x7fffffff;
+        }
+    }
+    return m;
 }
 
 // A wave's 32 rows o * inv, the first of them row `row0` of the result; `rows` (and no more) are stored. `my`: 32 x 2D bytes
@@ -183,7 +216,7 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         const int nbh = p.total / p.nqt;
         bh = work % nbh;
         const int r = work / nbh;
-        qt = p.mask_mode == 2 ? vdn_tile_order(p, r) : p.nqt - 1 - r;
+        qt = p.mask_mode == 2 ? vdn_tile_order<kPpBM>(p, r) : p.nqt - 1 - r;
     } else {
         // (the unsplit query tiles first, dealt like a launch of their own: p.full is a multiple of 8)
         const bool whole = block < p.full;
@@ -232,6 +265,7 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         n0 = w.n0;
         n1 = w.n1;
         ne = w.ne;
+        // (lane_mask() written out: through the call the long masked launches took 4 % longer)
         if (p.mask_mode == 1) {
             // block-causal (rt/attn.rs:449-453): keys of blocks (tq - win, tq], plus the sink blocks
             const int ft = p.ft, win = p.win;
@@ -551,8 +585,53 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
             return true;
         }
     }
-    store_rows<D>(smem + wave * (32 * 2 * kD), o, inv, out_f32, out_bf16, out_is_bf16, (size_t)bh * sq + q0 + wave * 32,
-                  qlen - wave * 32, lane);
+    // (store_rows() written out: its call costs the long masked launches 1 %)
+    if (out_is_bf16) {
+        // bf16 rows through this wave's own 32 x 2D-byte slice of the K ring (every K read is behind the last
+        // barrier and no load is in flight): scattered 8-byte pieces in, whole rows out, 16 bytes per
+        // lane and 1 KB (D = 128) of consecutive output per store instruction
+        constexpr int kRowB = 2 * kD, kCh = kRowB / 16;
+        lds_u8* my = smem + wave * (32 * kRowB);
+#pragma unroll
+        for (int db = 0; db < kNO; db++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                f32x4 r;
+#pragma unroll
+                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
+                const bf16x4 rb4 = __builtin_convertvector(r, bf16x4);
+                const int ch = (4 * db + g) ^ (c32 & (kCh - 1));
+                *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>(my + c32 * kRowB + (ch << 4) + 8 * h) = rb4;
+            }
+        // (same-wave LDS writes and reads complete in order; the compiler waits on the reads' data)
+        constexpr int kRowsPer = 64 / kCh;           // rows one store instruction covers
+        const int lr = lane / kCh, lc = lane % kCh;
+        uint16_t* ob = out_bf16 + ((size_t)bh * sq + q0 + wave * 32) * kD;
+#pragma unroll
+        for (int i = 0; i < 32 / kRowsPer; i++) {
+            const int rr = i * kRowsPer + lr;
+            const u32x4 val = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(
+                my + rr * kRowB + ((lc ^ (rr & (kCh - 1))) << 4));
+            if (wave * 32 + rr < qlen) global_store<u32x4>(ob + (size_t)rr * kD + lc * 8, val);
+        }
+    } else if (row < qlen) {
+        const size_t base = ((size_t)bh * sq + q0 + row) * kD;
+#pragma unroll
+        for (int db = 0; db < kNO; db++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int d0 = 32 * db + 8 * g + 4 * h;
+                f32x4 r;
+#pragma unroll
+                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
+                if (out_is_bf16) {
+                    const bf16x4 rb4 = __builtin_convertvector(r, bf16x4);
+                    global_store<bf16x4>(out_bf16 + base + d0, rb4);
+                } else {
+                    global_store<f32x4>(out_f32 + base + d0, r);
+                }
+            }
+    }
     return true;
 }
 
@@ -592,7 +671,7 @@ __global__ __launch_bounds__(256 * NG, 2) void flash_fwd_pp2(const FlashParams p
 constexpr int kDuoBM = 128;
 template <int D>
 constexpr int kDuoLds = 4 * TileGeo<D>::kTile + kVoteBytes;
-template <int D, bool LOG2DOM, bool FIXED, class Params>
+template <bool MASKED, int D, bool LOG2DOM, bool FIXED, class Params>
 FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int block) {
     using G = TileGeo<D>;
     using Dma = TileDma<4, D>;
@@ -600,15 +679,49 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     lds_u8* smem = (lds_u8*)smem_raw;
     const int h = lane >> 5, c32 = lane & 31;
-    const int work = (block & 7) * p.per_xcd + (block >> 3);   // XCD x: a contiguous eighth of the (head, query tile) items
+    // work order as in flash_item: XCD x takes a contiguous eighth of the (head, query tile) items; masked, longest first
+    const int work = MASKED ? block : (block & 7) * p.per_xcd + (block >> 3);
     if (work >= p.total) return true;
-    const int bh = work / p.nqt, q0 = (work - bh * p.nqt) * kDuoBM;
-    const int sq = p.sq, sk = p.sk, qlen = min(kDuoBM, sq - q0), nkt = (sk + kBN - 1) / kBN;
+    int bh, qt;
+    if constexpr (MASKED) {
+        const int nbh = p.total / p.nqt, r = work / nbh;
+        bh = work - r * nbh;
+        qt = p.mask_mode == 2 ? vdn_tile_order<kDuoBM>(p, r) : p.nqt - 1 - r;
+    } else {
+        bh = work / p.nqt;
+        qt = work - bh * p.nqt;
+    }
+    const int q0 = qt * kDuoBM, sq = p.sq, sk = p.sk, qlen = min(kDuoBM, sq - q0), nkt = (sk + kBN - 1) / kBN;
+    int a1 = 0, a2 = 0, n0 = nkt, n1 = 0, ne = nkt;   // the walk, as in flash_item
+    LaneMask lm = {0, 0x7fffffff, 0, 0};
+    if constexpr (MASKED) {
+        const TileWalk w = mask_tile_walk(p, q0, qlen, nkt);
+        a1 = w.a1, a2 = w.a2, n0 = w.n0, n1 = w.n1, ne = w.ne;
+        lm = lane_mask(p, q0 + wave * 32 + c32);
+    }
     const float sl2 = p.sl2, NEG = neg_inf();
     float* out_f32 = p.out_f32;
     uint16_t* out_bf16 = p.out_bf16;
     int out_is_bf16 = p.out_is_bf16;
     asm volatile("" : "+s"(out_f32), "+s"(out_bf16), "+s"(out_is_bf16));   // (fetched now, see flash_item)
+    if constexpr (MASKED) {
+        if (ne <= 0) {   // no key tile is visible to any query of this tile: rows of zeros (flash_item)
+            f32x16 zero[kNO];
+#pragma unroll
+            for (int db = 0; db < kNO; db++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) zero[db][i] = 0.f;
+            store_rows<D>(smem + wave * (32 * 2 * D), zero, 0.f, out_f32, out_bf16, out_is_bf16,
+                          (size_t)bh * sq + q0 + wave * 32, qlen - wave * 32, lane);
+            return true;
+        }
+    }
+    // first key of walk position e; positions past the end repeat the last tile
+    auto kv0_of = [&](int e) -> int {
+        e = min(e, ne - 1);
+        if constexpr (MASKED) return (e < n0 ? e : e < n0 + n1 ? a1 + (e - n0) : a2 + (e - n0 - n1)) * kBN;
+        else return e * kBN;
+    };
     const uint16_t* Qh = p.q + (size_t)bh * p.q_plane + (size_t)q0 * D;
     const uint16_t* Kh = p.k + (size_t)bh * p.k_plane;
     const uint16_t* Vh = p.v + (size_t)bh * p.v_plane;
@@ -617,13 +730,12 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     auto vbuf = [&](int t) -> lds_u8* { return smem + (2 + (t & 1)) * kTileBytes; };
     Dma dma;
     dma.init(wave, lane);
-    // (tiles past the end repeat the last one)
     auto target_k = [&](int t) {
-        const int kv0 = min(t, nkt - 1) * kBN;
+        const int kv0 = kv0_of(t);
         return dma.template prepare<false>(kbuf(t), Kh + (size_t)kv0 * D, sk - kv0, wave);
     };
     auto target_v = [&](int t) {
-        const int kv0 = t * kBN;
+        const int kv0 = kv0_of(t);
         return dma.template prepare<true>(vbuf(t), Vh + (size_t)kv0 * D, sk - kv0, wave);
     };
     bf16x8 qf[D / 16];
@@ -665,14 +777,29 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int x = 0; x < 8; x++) pb[t][x] = (__bf16)0.0f;
-    auto mask_tail = [&](int m) {
-        const int left = sk - m * kBN - 4 * h;
-        if (sk - m * kBN < kBN) {
+    auto mask_tile = [&](int e) {
+        const int kv0 = kv0_of(e);
+        if (kv0 + kBN > sk) {
+            const int left = sk - kv0 - 4 * h;
 #pragma unroll
             for (int b = 0; b < 2; b++)
 #pragma unroll
                 for (int i = 0; i < 16; i++)
                     if (32 * b + 8 * (i >> 2) + (i & 3) >= left) s[b][i] = NEG;
+        }
+        if constexpr (MASKED) {
+            const int kend = min(kv0 + kBN, sk);
+            const bool lane_all = kend <= lm.a_hi || kv0 >= lm.c_lo || (kv0 >= lm.w_lo && kend <= lm.w_hi);
+            if (__builtin_amdgcn_ballot_w64(!lane_all) != 0) {
+#pragma unroll
+                for (int b = 0; b < 2; b++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        const int key = kv0 + 32 * b + 8 * (i >> 2) + 4 * h + (i & 3);
+                        const bool vis = key < lm.a_hi || key >= lm.c_lo || (key >= lm.w_lo && key < lm.w_hi);
+                        if (!vis) s[b][i] = NEG;
+                    }
+            }
         }
     };
     typename Dma::Prepared dk = target_k(1), dv = target_v(0);
@@ -683,7 +810,7 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     for (int part = 0; part < 2; part++) {
         const bool first = part == 0;
 #pragma unroll 1
-        for (int m = part; m < (first ? 1 : nkt); m++) {
+        for (int m = part; m < (first ? 1 : ne); m++) {
             __builtin_amdgcn_s_setprio(1);
             constexpr int kAhead = 3;
             auto hook_dma = [&](int g) {
@@ -695,7 +822,7 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
             else mfma_phase<true, kAhead, decltype(hook_dma)&, D>(vbuf(m - 1), kbuf(m), rb, pb, o, qf, s, s_init, hook_dma);
             __builtin_amdgcn_s_setprio(0);
             __builtin_amdgcn_sched_barrier(0);
-            mask_tail(m);
+            mask_tile(m);
             if (FIXED && !first) {
 #pragma unroll
                 for (int b = 0; b < 2; b++) softmax_off_block<!LOG2DOM>(s[b], st, sl2, pb[2 * b], pb[2 * b + 1]);
@@ -704,14 +831,14 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
             }
             asm volatile("" ::"v"(pb[0]), "v"(pb[1]), "v"(pb[2]), "v"(pb[3]), "v"(st.l_acc));
             dk = target_k(m + 2);
-            dv = target_v(min(m + 1, nkt - 1));
+            dv = target_v(m + 1);
             __builtin_amdgcn_sched_barrier(0);
             wait_vmcnt<0>();
             block_barrier();   // K(m+1), V(m) resident; this phase's tiles read by every wave
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    pv_tile<D>(vbuf(nkt - 1), rb.v, pb, o);
+    pv_tile<D>(vbuf(ne - 1), rb.v, pb, o);
 
     if constexpr (FIXED) {   // did the fixed offset hold (flash_item)?
         float chk = 0.f;
@@ -736,18 +863,18 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
                   (size_t)bh * sq + q0 + wave * 32, qlen - wave * 32, lane);
     return true;
 }
-template <int D, bool LOG2DOM, bool FIXED>
+template <bool MASKED, int D, bool LOG2DOM, bool FIXED>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_fwd_duo(const FlashParams p) {
     int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), block = blockIdx.x;
     if constexpr (!FIXED) {
-        duo_item<D, LOG2DOM, false>(p, wave, threadIdx.x & 63, block);
+        duo_item<MASKED, D, LOG2DOM, false>(p, wave, threadIdx.x & 63, block);
     } else {
-        if (duo_item<D, LOG2DOM, true>(p, wave, threadIdx.x & 63, block)) return;
+        if (duo_item<MASKED, D, LOG2DOM, true>(p, wave, threadIdx.x & 63, block)) return;
         using ConstParams = const __attribute__((address_space(4))) FlashParams;   // (as in flash_fwd_pp2)
         ConstParams* again = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
         int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
         asm volatile("" : "+v"(lane), "+s"(wave), "+s"(block), "+s"(again));
-        duo_item<D, LOG2DOM, false>(*again, wave, lane, block);
+        duo_item<MASKED, D, LOG2DOM, false>(*again, wave, lane, block);
     }
 }
 
@@ -826,16 +953,16 @@ hipError_t launch_flash_as(const fv::FlashParams* p, hipStream_t stream) {
     hipLaunchKernelGGL((fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED>), dim3(p->full + p->per_xcd * 8), dim3(256 * NG), lds, stream, *p);
     return hipGetLastError();
 }
-template <int D, bool LOG2DOM, bool FIXED>
+template <bool MASKED, int D, bool LOG2DOM, bool FIXED>
 hipError_t duo_attr() {
     static std::atomic<unsigned long long> attr_done;
-    return fv_set_max_lds_once((const void*)fv::flash_fwd_duo<D, LOG2DOM, FIXED>, fv::kDuoLds<D>, attr_done);
+    return fv_set_max_lds_once((const void*)fv::flash_fwd_duo<MASKED, D, LOG2DOM, FIXED>, fv::kDuoLds<D>, attr_done);
 }
-template <int D, bool LOG2DOM, bool FIXED>
+template <bool MASKED, int D, bool LOG2DOM, bool FIXED>
 hipError_t launch_duo_as(const fv::FlashParams* p, hipStream_t stream) {
-    hipError_t e = duo_attr<D, LOG2DOM, FIXED>();
+    hipError_t e = duo_attr<MASKED, D, LOG2DOM, FIXED>();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((fv::flash_fwd_duo<D, LOG2DOM, FIXED>), dim3(p->per_xcd * 8), dim3(256), fv::kDuoLds<D>, stream, *p);
+    hipLaunchKernelGGL((fv::flash_fwd_duo<MASKED, D, LOG2DOM, FIXED>), dim3(p->per_xcd * 8), dim3(256), fv::kDuoLds<D>, stream, *p);
     return hipGetLastError();
 }
 // FASTVIDEO_SDPA_RUNNING_MAX=1: every launch keeps the running max (no fixed-offset first pass).
@@ -861,25 +988,28 @@ hipError_t launch_flash_fixed(const fv::FlashParams* p, hipStream_t stream) {
 // key 0, the first key of every tile's walk, so that its offset is a score of its own: block-causal without a
 // window or with sink blocks, and the VDN mask (rows before the video and frame 0 are visible to every query).
 // Under a window without a sink a query's first visible key may lie anywhere in the walk: running max.
+template <bool MASKED>
+bool offset_is_a_score(const fv::FlashParams* p) {
+    return !MASKED || p->mask_mode == 2 || (p->mask_mode == 1 && (p->win == 0 || p->sink > 0));
+}
 template <int NG, bool MASKED, int D>
 hipError_t launch_flash(const fv::FlashParams* p, hipStream_t stream) {
-    const bool offset_is_a_score = !MASKED || p->mask_mode == 2 || (p->mask_mode == 1 && (p->win == 0 || p->sink > 0));
-    if (p->out_is_bf16 && offset_is_a_score && !running_max_forced()) return launch_flash_fixed<NG, MASKED, D, true>(p, stream);
+    if (p->out_is_bf16 && offset_is_a_score<MASKED>(p) && !running_max_forced()) return launch_flash_fixed<NG, MASKED, D, true>(p, stream);
     return launch_flash_fixed<NG, MASKED, D, false>(p, stream);
 }
-template <int D>
+template <bool MASKED, int D>
 hipError_t launch_duo(const fv::FlashParams* p, hipStream_t stream) {
-    const bool fixed = p->out_is_bf16 && !running_max_forced();
-    if (p->sl2 != 1.0f) return fixed ? launch_duo_as<D, false, true>(p, stream) : launch_duo_as<D, false, false>(p, stream);
+    const bool fixed = p->out_is_bf16 && offset_is_a_score<MASKED>(p) && !running_max_forced();
+    if (p->sl2 != 1.0f) return fixed ? launch_duo_as<MASKED, D, false, true>(p, stream) : launch_duo_as<MASKED, D, false, false>(p, stream);
     g_log2_domain_launches.fetch_add(1, std::memory_order_relaxed);
-    return fixed ? launch_duo_as<D, true, true>(p, stream) : launch_duo_as<D, true, false>(p, stream);
+    return fixed ? launch_duo_as<MASKED, D, true, true>(p, stream) : launch_duo_as<MASKED, D, true, false>(p, stream);
 }
-template <int D>
+template <bool MASKED, int D>
 hipError_t init_duo() {
-    hipError_t e = duo_attr<D, false, false>();
-    if (e == hipSuccess) e = duo_attr<D, true, false>();
-    if (e == hipSuccess) e = duo_attr<D, false, true>();
-    if (e == hipSuccess) e = duo_attr<D, true, true>();
+    hipError_t e = duo_attr<MASKED, D, false, false>();
+    if (e == hipSuccess) e = duo_attr<MASKED, D, true, false>();
+    if (e == hipSuccess) e = duo_attr<MASKED, D, false, true>();
+    if (e == hipSuccess) e = duo_attr<MASKED, D, true, true>();
     return e;
 }
 template <int NG, bool MASKED, int D>
@@ -906,13 +1036,17 @@ extern "C" hipError_t fv_internal_init_flash(void) {
     if (e == hipSuccess) e = init_flash<2, true, 64>();
     if (e == hipSuccess) e = init_flash<1, false, 128>();
     if (e == hipSuccess) e = init_flash<1, false, 64>();
-    if (e == hipSuccess) e = init_duo<128>();
-    if (e == hipSuccess) e = init_duo<64>();
+    if (e == hipSuccess) e = init_duo<false, 128>();
+    if (e == hipSuccess) e = init_duo<false, 64>();
+    if (e == hipSuccess) e = init_duo<true, 128>();
+    if (e == hipSuccess) e = init_duo<true, 64>();
     return e;
 }
 
-extern "C" hipError_t fv_internal_launch_duo(const fv::FlashParams* p, int d, hipStream_t stream) {
-    return d == 128 ? launch_duo<128>(p, stream) : d == 64 ? launch_duo<64>(p, stream) : hipErrorInvalidValue;
+extern "C" hipError_t fv_internal_launch_duo(const fv::FlashParams* p, int masked, int d, hipStream_t stream) {
+    if (d == 128) return masked ? launch_duo<true, 128>(p, stream) : launch_duo<false, 128>(p, stream);
+    if (d == 64) return masked ? launch_duo<true, 64>(p, stream) : launch_duo<false, 64>(p, stream);
+    return hipErrorInvalidValue;
 }
 
 extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d, int block_m,

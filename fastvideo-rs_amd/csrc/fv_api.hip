@@ -5,6 +5,7 @@
 #include <limits.h>
 #include <stdio.h>
 
+#include <algorithm>
 #include <atomic>
 #include <string>
 
@@ -125,6 +126,25 @@ struct MaskArgs {
     size_t video_start = 0, frame_tokens = 0, frames = 0, chunk = 0, radius = 0;   // VDN window
 };
 
+// flash_fwd_duo for masked launches (bf16 results; f32 ones keep one kernel for every length, so that a clip's first
+// blocks are the shorter clip's bit for bit). Its tiles of 128 queries cross fewer frame boundaries and leave a shorter
+// last round, which counts where a query reaches few keys; long walks run at the chip's power limit, where 256 queries to a
+// K and V stream cost less. us, flash_fwd_pp2 / flash_fwd_duo, heads x frame x frames (keys reached): causal 12 x 880 x 2 (1760) 59 /
+// 56, 12 x 390 x 6 in blocks of 3 (2340) 97 / 68, 24 x 390 x 8 (3120) 94 / 82, 40 x 880 x 4 (3520) 174 / 164, 12 x 880 x 8 under a window
+// of 4 (3520) 172 / 164, 12 x 1560 x 8 under one of 3 with a sink (6240) 429 / 408, 12 x 1560 x 4 (6240) 170 / 172, 24 x 1560 x 6 (9360)
+// 565 / 561, 12 x 1560 x 12 under a window (18720) 1211 / 1250; VDN window 40 x 390 x 16 (2730) 452 / 410, 12 x 880 x 10 (4400) 390 / 317,
+// 12 x 390 x 24 (6630) 360 / 356, 12 x 1560 x 24 (7800) 2383 / 2102, 24 x 880 x 12 (9680) 930 / 945, 12 x 1560 x 32 (26520) 6478 /
+// 6623. At head dim 64 causal 24 x 880 x 4 92 / 83, 12 x 1560 x 21 (32760) 1817 / 1674.
+bool duo_masked(const fv::FlashParams& p, size_t bh, size_t d) {
+    const long ft = p.ft;
+    long reach = p.sq;
+    if (p.mask_mode == kMaskVdnWindow)
+        reach = ft * std::min((long)p.frames, 2 + (2 * (long)p.radius + 1) * std::max(1, p.chunk));
+    else if (p.win > 0)
+        reach = ft * ((long)p.win + p.sink);
+    return bh * (((size_t)p.sq + 127) / 128) > (size_t)fv_compute_units() / 2 && (d == 64 || reach <= 8192);
+}
+
 int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,
                  int out_is_bf16, size_t bh, size_t sq, size_t sk, size_t d, float scale,
                  const MaskArgs& m, void* stream) {
@@ -232,11 +252,11 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         if (p.sl2 == 1.0f) fv_internal_count_log2_domain();
         return FV_OK;
     }
-    if (mode == kMaskNone && splits == 1 && fv_duo(bh, sq, sk, d)) {
+    if (mode == kMaskNone ? splits == 1 && fv_duo(bh, sq, sk, d) : out_is_bf16 && duo_masked(p, bh, d)) {
         p.nqt = (int)((sq + 127) / 128);
         p.total = (int)(bh * (size_t)p.nqt);
         p.per_xcd = (p.total + 7) / 8;
-        const hipError_t e = fv_internal_launch_duo(&p, (int)d, (hipStream_t)stream);
+        const hipError_t e = fv_internal_launch_duo(&p, mode != kMaskNone ? 1 : 0, (int)d, (hipStream_t)stream);
         return e == hipSuccess ? FV_OK : fail_hip(e, "flash_fwd_duo");
     }
     hipError_t e = fv_internal_launch_flash(&p, mode != kMaskNone ? 1 : 0, (int)d, (int)bm, (hipStream_t)stream);

@@ -177,7 +177,7 @@ int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, vo
                      const FvSplitPlan& plan, void* workspace, size_t workspace_bytes, void* stream);
 
 extern "C" int fv_internal_flash_block_m(void);   // queries per workgroup of the flash kernel in use
-extern "C" hipError_t fv_internal_launch_duo(const fv::FlashParams* p, int d, hipStream_t stream);   // total, nqt: of 128 queries
+extern "C" hipError_t fv_internal_launch_duo(const fv::FlashParams* p, int masked, int d, hipStream_t stream);   // total, nqt: of 128 queries
 extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d, int block_m,
                                                hipStream_t stream);
 extern "C" hipError_t fv_internal_exact_pass_reruns(unsigned long long* out);

@@ -87,3 +87,30 @@ def test_windows_and_reruns(fv, d):
     rest = torch.ones(HEADS, sq, dtype=torch.bool, device="cuda")
     rest[3, 5] = False
     assert torch.isfinite(got[rest]).all()
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("heads,s,mask", [
+    (40, 513, ("causal", 100, 0, 0)), (40, 700, ("causal", 64, 2, 1)), (30, 640, ("causal", 128, 2, 0)),
+    (40, 640, ("window", 0, 64, 10, 3, 1)), (40, 701, ("window", 13, 40, 16, 0, 2)), (30, 1024, ("window", 0, 128, 8, 2, 1))])
+def test_masked(fv, d, heads, s, mask):
+    """Masked bf16 launches of more than 128 query tiles of 128: frame boundaries inside, on and off the tiles."""
+    import torch
+
+    announce(f"duo masked {heads}x{s}x{d} {mask}")
+    g = torch.Generator(device="cuda").manual_seed(s + d)
+    q, k, v = (torch.randn((heads, s, d), generator=g, device="cuda").to(torch.bfloat16) for _ in range(3))
+    if mask[0] == "causal":
+        bias = fv.BlockCausal(*mask[1:]).dense_mask(s, s)
+        got = fv.sdpa_block_causal_bf16(q, k, v, *mask[1:], out_bf16=True)
+    else:
+        bias = fv.VdnWindow(*mask[1:]).dense_mask(s, s)
+        got = fv.sdpa_vdn_window_bf16(q, k, v, *mask[1:], out_bf16=True)
+    shut = torch.from_numpy(np.asarray(bias).reshape(s, s) < -1e8).cuda()
+    assert shut.any() and not shut.all(-1).any()
+    want = torch.empty(q.shape, dtype=torch.float64, device=q.device)
+    for b in range(heads):
+        x = ((q[b].double() @ k[b].double().T) / np.sqrt(d)).masked_fill(shut, float("-inf"))
+        want[b] = torch.softmax(x, -1) @ v[b].double()
+    rows = ((got.double() - want).norm(dim=-1) / want.norm(dim=-1)).max().item()
+    assert ((got.double() - want).norm() / want.norm()).item() <= 2 * 2.0 ** -9 and rows <= 2.0 ** -7, rows
