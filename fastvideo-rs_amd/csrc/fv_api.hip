@@ -129,20 +129,26 @@ struct MaskArgs {
 // flash_fwd_duo for masked launches (bf16 results; f32 ones keep one kernel for every length, so that a clip's first
 // blocks are the shorter clip's bit for bit). Its tiles of 128 queries cross fewer frame boundaries and leave a shorter
 // last round, which counts where a query reaches few keys; long walks run at the chip's power limit, where 256 queries to a
-// K and V stream cost less. us, flash_fwd_pp2 / flash_fwd_duo, heads x frame x frames (keys reached): causal 12 x 880 x 2 (1760) 59 /
-// 56, 12 x 390 x 6 in blocks of 3 (2340) 97 / 68, 24 x 390 x 8 (3120) 94 / 82, 40 x 880 x 4 (3520) 174 / 164, 12 x 880 x 8 under a window
-// of 4 (3520) 172 / 164, 12 x 1560 x 8 under one of 3 with a sink (6240) 429 / 408, 12 x 1560 x 4 (6240) 170 / 172, 24 x 1560 x 6 (9360)
-// 565 / 561, 12 x 1560 x 12 under a window (18720) 1211 / 1250; VDN window 40 x 390 x 16 (2730) 452 / 410, 12 x 880 x 10 (4400) 390 / 317,
-// 12 x 390 x 24 (6630) 360 / 356, 12 x 1560 x 24 (7800) 2383 / 2102, 24 x 880 x 12 (9680) 930 / 945, 12 x 1560 x 32 (26520) 6478 /
-// 6623. At head dim 64 causal 24 x 880 x 4 92 / 83, 12 x 1560 x 21 (32760) 1817 / 1674.
+// K and V stream cost less. Causal launches without a window, whose walks are half their reach on average, and windows that
+// are part of their clip take it up to 8192 keys reached, walks of one length up to 4096. us, flash_fwd_pp2 / flash_fwd_duo,
+// heads x frame x frames (keys reached): causal 12 x 880 x 2 (1760) 59 / 56, 12 x 390 x 6 in blocks of 3 (2340) 97 / 68, 24 x 390 x 8
+// (3120) 94 / 82, 40 x 390 x 12 in blocks of 3 (4680) 303 / 270, 24 x 880 x 8 (7040) 341 / 318, 12 x 1560 x 4 (6240) 180 / 181;
+// under a window 12 x 880 x 8 (3520) 172 / 164, 24 x 880 x 8 with a sink (3520) 266 / 255, 12 x 1560 x 6 (6240) 304 / 314, x 8 438 / 425,
+// 12 x 1560 x 12 (18720) 1211 / 1250; VDN window 40 x 390 x 16 (2730) 452 / 410, 12 x 880 x 10 (4400) 390 / 317, 24 x 390 x 20 (6630)
+// 518 / 508, 12 x 1560 x 24 (7800) 2383 / 2102, 40 x 1560 x 12 (7800) 3199 / 3213, 24 x 880 x 12 (9680) 930 / 945, 12 x 1560 x 32 (26520)
+// 6478 / 6623, over the whole clip 12 x 390 x 8 (3120) 97 / 82, 12 x 390 x 12 (4680) 120 / 125. At head dim 64 causal 24 x 880 x 4
+// 92 / 83, 12 x 1560 x 21 (32760) 1817 / 1674.
 bool duo_masked(const fv::FlashParams& p, size_t bh, size_t d) {
     const long ft = p.ft;
-    long reach = p.sq;
-    if (p.mask_mode == kMaskVdnWindow)
-        reach = ft * std::min((long)p.frames, 2 + (2 * (long)p.radius + 1) * std::max(1, p.chunk));
-    else if (p.win > 0)
-        reach = ft * ((long)p.win + p.sink);
-    return bh * (((size_t)p.sq + 127) / 128) > (size_t)fv_compute_units() / 2 && (d == 64 || reach <= 8192);
+    long reach = p.sq, most = 8192;
+    if (p.mask_mode == kMaskVdnWindow) {
+        const long seen = 2 + (2 * (long)p.radius + 1) * std::max(1, p.chunk);
+        if (seen >= p.frames) most = 4096;
+        else reach = ft * seen;
+    } else if (p.win > 0) {
+        reach = ft * ((long)p.win + p.sink), most = 4096;
+    }
+    return bh * (((size_t)p.sq + 127) / 128) > (size_t)fv_compute_units() / 2 && (d == 64 || reach <= most);
 }
 
 int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,
