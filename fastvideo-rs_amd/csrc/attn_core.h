@@ -103,6 +103,9 @@ struct TileDma {
     }
     // A tile load prepared ahead of its issue: everything the DMA instructions need,
     // so that issuing them from inside a matrix phase costs 3 instructions each.
+    // tile_base (wave-uniform) points at the tile's first row. Rows >= rows_valid re-read
+    // the last valid row: the caller masks their scores to -inf, so their content only has
+    // to be finite data the tensor already holds.
     struct Prepared {
         unsigned long long base;   // wave-uniform global address of the tile's first row
         unsigned lds;              // wave-uniform LDS byte address of this wave's first row
@@ -127,31 +130,6 @@ struct TileDma {
     static FV_DEV void issue_prepared(const Prepared& d, int it) {
         lds_dma16_s(d.lds + it * 1024, (const void*)d.base, d.off[it]);
     }
-    // tile_base (wave-uniform) points at the tile's first row. Rows >= rows_valid
-    // re-read the last valid row: the caller masks their scores to -inf, so their
-    // content only has to be finite data the tensor already holds.
-    // one of the ITER instructions of a full tile's load
-    template <bool IS_V>
-    FV_DEV void issue_one(lds_u8* buf, const uint16_t* tile_base, int wave, int it) const {
-        const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)buf + wave * ITER * 1024);
-        lds_dma16_s(base + it * 1024, tile_base, IS_V ? voff[it] : koff[it]);
-    }
-    template <bool IS_V>
-    FV_DEV void issue(lds_u8* buf, const uint16_t* tile_base, int rows_valid, int wave) const {
-        const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)buf + wave * ITER * 1024);
-        if (rows_valid >= kTileRows) {
-#pragma unroll
-            for (int it = 0; it < ITER; it++)
-                lds_dma16_s(base + it * 1024, tile_base, IS_V ? voff[it] : koff[it]);
-        } else {
-#pragma unroll
-            for (int it = 0; it < ITER; it++) {
-                const unsigned off = IS_V ? voff[it] : koff[it];
-                const int over = max(0, (int)(off / G::kRow) - (rows_valid - 1));
-                lds_dma16_s(base + it * 1024, tile_base, off - over * G::kRow);
-            }
-        }
-    }
 };
 
 // Per-lane read bases into a swizzled tile.
@@ -172,39 +150,6 @@ FV_DEV TileReadBases tile_read_bases(int lane) {
     const int c_lane = 2 * (b16 & 1) + ((i16 & 3) >> 1);
     b.v = r * G::kRow + ((G::vswz(r) ^ c_lane) << 4) + 8 * (i16 & 1);
     return b;
-}
-
-// S^T (64 keys x 32 queries) = K Q^T for one wave: s[b][i] is key
-// 32 b + 8 (i/4) + 4 (lane/32) + i%4 of the tile, query lane%32.
-FV_DEV void qk_tile(const lds_u8* kb, int k_base, const bf16x8 (&qf)[8], f32x16 (&s)[2]) {
-#pragma unroll
-    for (int b = 0; b < 2; b++) {
-#pragma unroll
-        for (int i = 0; i < 16; i++) s[b][i] = 0.f;
-#pragma unroll
-        for (int dk = 0; dk < 8; dk++) {
-            const bf16x8 a = lds_read_b128(kb + (k_base ^ (dk << 5)) + b * 32 * kRowBytes);
-            s[b] = mfma32(a, qf[dk], s[b]);
-        }
-    }
-}
-
-// qk_tile with `side(g)` after MFMA g (0..15): side work that rides under the matrix pipe. Every S block
-// starts from `s_init` (the C operand of its first MFMA): zeros, or minus the softmax offset of the lane's query.
-template <class Side>
-FV_DEV void qk_tile_side(const lds_u8* kb, int k_base, const bf16x8 (&qf)[8], f32x16 (&s)[2], const f32x16& s_init,
-                         Side&& side) {
-#pragma unroll
-    for (int b = 0; b < 2; b++) {
-#pragma unroll
-        for (int dk = 0; dk < 8; dk++) {
-            const bf16x8 a = lds_read_b128(kb + (k_base ^ (dk << 5)) + b * 32 * kRowBytes);
-            s[b] = mfma32(a, qf[dk], dk == 0 ? s_init : s[b]);
-            __builtin_amdgcn_sched_barrier(0);
-            side(b * 8 + dk);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
 }
 
 constexpr float kRescaleLog2 = 6.0f;

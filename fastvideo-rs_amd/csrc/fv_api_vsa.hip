@@ -343,7 +343,7 @@ static int vsa_attention_common(const void* q, const void* k, const void* v, int
         if (!tiled) {
             uint16_t* const tiles[3] = {(uint16_t*)(ws + w.qt), (uint16_t*)(ws + w.kt), (uint16_t*)(ws + w.vt)};
             // f32 queries get their one rounding here: with the fold switch on (fv_rt_fold_scale), of
-            // q * (scale * log2 e), and the fine kernel then runs its form without the per-score multiply
+            // q * (scale * log2 e), and the fine kernel's factor is one
             const float c = scale * 1.4426950408889634f;
             const float copy_mul[3] = {c, 1.0f, 1.0f};
             fold = !qkv_is_bf16 && fv_rt_fold_scale() && c != 1.0f && c < 3.0e38f;
