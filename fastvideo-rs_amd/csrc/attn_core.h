@@ -261,11 +261,45 @@ FV_DEV void softmax_tile_pair_fixed(const f32x16 (&s0)[2], const f32x16 (&s1)[2]
     for (int b = 0; b < 2; b++) softmax_off_block<SCALED>(s1[b], st, sl2, pb1[2 * b], pb1[2 * b + 1]);
 }
 
-// One tile. `side(part)` runs after the rescale (part 0) and after each 32-key half of the exponentials
-// (parts 1, 2): slots for side work, such as tile DMA issue, spread through the VALU stream.
-template <bool SCALED, class Side, int NO>
-FV_DEV void softmax_tile_side_off(f32x16 (&s)[2], SoftmaxOffState& st, f32x16 (&o)[NO], f32x16& negoff, float sl2,
-                                  bf16x8 (&pb)[4], Side&& side) {
+// The first pair of a walk (or its only tile), before anything has been added up: the same offset and the same P.
+template <int NS>
+FV_DEV void softmax_first_offset(f32x16* const (&sc)[NS], SoftmaxOffState& st, f32x16& negoff) {
+    const float NEG = neg_inf();
+    float mx = (*sc[0])[0];
+#pragma unroll
+    for (int b = 0; b < NS; b++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) mx = __builtin_fmaxf(mx, (*sc[b])[i]);
+    const float r = __builtin_fmaxf(NEG, pair_max(mx));   // (a NaN: as no score)
+    st.off = r == NEG ? 0.f : r;
+    st.r = r == NEG ? NEG : 0.f;
+    st.l_acc = 0.f;
+#pragma unroll
+    for (int b = 0; b < NS; b++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) (*sc[b])[i] -= st.off;
+#pragma unroll
+    for (int i = 0; i < 16; i++) negoff[i] = -st.off;
+}
+template <bool SCALED>
+FV_DEV void softmax_first_off(f32x16 (&s0)[2], f32x16 (&s1)[2], SoftmaxOffState& st, f32x16& negoff, float sl2,
+                              bf16x8 (&pb0)[4], bf16x8 (&pb1)[4]) {
+    f32x16* const sc[4] = {&s0[0], &s0[1], &s1[0], &s1[1]};
+    softmax_first_offset<4>(sc, st, negoff);
+    softmax_tile_pair_fixed<SCALED>(s0, s1, st, sl2, pb0, pb1);
+}
+template <bool SCALED>
+FV_DEV void softmax_first_off(f32x16 (&s)[2], SoftmaxOffState& st, f32x16& negoff, float sl2, bf16x8 (&pb)[4]) {
+    f32x16* const sc[2] = {&s[0], &s[1]};
+    softmax_first_offset<2>(sc, st, negoff);
+#pragma unroll
+    for (int b = 0; b < 2; b++) softmax_off_block<SCALED>(s[b], st, sl2, pb[2 * b], pb[2 * b + 1]);
+}
+
+// One tile.
+template <bool SCALED, int NO>
+FV_DEV void softmax_tile_off(f32x16 (&s)[2], SoftmaxOffState& st, f32x16 (&o)[NO], f32x16& negoff, float sl2,
+                             bf16x8 (&pb)[4]) {
     float mx = s[0][0];
 #pragma unroll
     for (int i = 1; i < 16; i++) mx = __builtin_fmaxf(mx, s[0][i]);
@@ -274,12 +308,8 @@ FV_DEV void softmax_tile_side_off(f32x16 (&s)[2], SoftmaxOffState& st, f32x16 (&
     mx = pair_max(mx);
     f32x16* const sc[2] = {&s[0], &s[1]};
     softmax_off_rescale<SCALED, NO, 2>(mx, st, o, negoff, sl2, sc);
-    side(0);
 #pragma unroll
-    for (int b = 0; b < 2; b++) {
-        softmax_off_block<SCALED>(s[b], st, sl2, pb[2 * b], pb[2 * b + 1]);
-        side(1 + b);
-    }
+    for (int b = 0; b < 2; b++) softmax_off_block<SCALED>(s[b], st, sl2, pb[2 * b], pb[2 * b + 1]);
 }
 
 // O^T (128 d x 32 queries) += V^T P^T.

@@ -663,14 +663,17 @@ __global__ __launch_bounds__(256 * NG, 2) void flash_fwd_pp2(const FlashParams p
     }
 }
 
-// Dense launches on few keys (fv_duo): two workgroups a CU. flash_fwd_pp2 gives an item the CU and pays its first loads,
-// its first and last slot and its store in the open, half of the time at eight key tiles. Here an item is four waves x 32
-// queries with two K and two V buffers (64 KB at D = 128), so that two share a CU unsynchronised and one's ends pass under
-// the other's arithmetic. A phase is one key tile: the matrix part (O += P V of the tile before, S = K Q^T, with the loads
-// of the next K and of this V going out behind the first MFMAs), the softmax, one barrier.
+// Walks of few keys under a fixed offset (fv_duo, duo_masked): two workgroups a CU, three at head dim 64. flash_fwd_pp2
+// gives an item the CU and pays its first loads, its first and last slot and its store in the open, half of the time at
+// eight key tiles. Here an item is four waves x 32 queries with five buffers of a tile (80 KB at D = 128), so that two share
+// a CU unsynchronised and one's ends pass under the other's arithmetic. A phase is one key tile: the matrix part (O += P V of
+// the tile before, S = K Q^T, with the loads of the next K and of this V going out behind the first MFMAs), the softmax, one
+// barrier; the first phase has two. Every sum is flash_fwd_pp2's, term by term: the offset of a row is the largest score of the walk's first two
+// tiles, so the two kernels give the same bits and the line between them is drawn by time alone (a workgroup that goes
+// again with the running max is one of 128 queries here and of 256 there: its rows differ by the rounding of P).
 constexpr int kDuoBM = 128;
 template <int D>
-constexpr int kDuoLds = 4 * TileGeo<D>::kTile + kVoteBytes;
+constexpr int kDuoLds = 5 * TileGeo<D>::kTile;
 template <bool MASKED, int D, bool LOG2DOM, bool FIXED, class Params>
 FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int block) {
     using G = TileGeo<D>;
@@ -711,7 +714,7 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
             for (int db = 0; db < kNO; db++)
 #pragma unroll
                 for (int i = 0; i < 16; i++) zero[db][i] = 0.f;
-            store_rows<D>(smem + wave * (32 * 2 * D), zero, 0.f, out_f32, out_bf16, out_is_bf16,
+            store_rows<D>(smem + wave * (kTileBytes / 2), zero, 0.f, out_f32, out_bf16, out_is_bf16,
                           (size_t)bh * sq + q0 + wave * 32, qlen - wave * 32, lane);
             return true;
         }
@@ -726,8 +729,10 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     const uint16_t* Kh = p.k + (size_t)bh * p.k_plane;
     const uint16_t* Vh = p.v + (size_t)bh * p.v_plane;
 
-    auto kbuf = [&](int t) -> lds_u8* { return smem + (t & 1) * kTileBytes; };
-    auto vbuf = [&](int t) -> lds_u8* { return smem + (2 + (t & 1)) * kTileBytes; };
+    // Buffers: K(0), K(1), V(0), V(1), K(2) each in its own; from then on odd phases read V(m - 1) and K(m) from 0 and 1 and
+    // load V(m) and K(m + 1) into 3 and 4, even ones the other way round.
+    auto kbuf = [&](int t) -> lds_u8* { return smem + (t == 0 ? 0 : t & 1 ? 1 : 4) * kTileBytes; };
+    auto vbuf = [&](int t) -> lds_u8* { return smem + (t == 0 ? 2 : t & 1 ? 3 : 0) * kTileBytes; };
     Dma dma;
     dma.init(wave, lane);
     auto target_k = [&](int t) {
@@ -741,7 +746,7 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     bf16x8 qf[D / 16];
     const TileReadBases rb = tile_read_bases<D>(lane);
     {
-        // the wave's query rows through its slice of the V buffers, as in flash_item; K(0) besides
+        // the wave's query rows through its slice of buffers 2 and 3, as in flash_item; K(0) and K(1) besides
         lds_u8* qs = smem + 2 * kTileBytes + wave * (32 * G::kRow);
         const unsigned qlds = __builtin_amdgcn_readfirstlane((unsigned)(size_t)qs);
 #pragma unroll
@@ -750,10 +755,16 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
             const int rg = min(wave * 32 + r, qlen - 1);   // rows past the end re-read the last one (zeroed below)
             lds_dma16_s(qlds + it * 1024, Qh, (unsigned)(rg * G::kRow + ((pch ^ G::kswz(r)) << 4)));
         }
-        const typename Dma::Prepared k0 = target_k(0);
+        const typename Dma::Prepared k0 = target_k(0), k1 = target_k(1);
 #pragma unroll
         for (int it = 0; it < kIt; it++) Dma::issue_prepared(k0, it);
-        wait_vmcnt<kIt>();
+        if (ne > 1) {
+#pragma unroll
+            for (int it = 0; it < kIt; it++) Dma::issue_prepared(k1, it);
+            wait_vmcnt<2 * kIt>();
+        } else {
+            wait_vmcnt<kIt>();
+        }
         const bool ok = wave * 32 + c32 < qlen;
 #pragma unroll
         for (int dk = 0; dk < D / 16; dk++) {
@@ -763,21 +774,7 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the slice is read before the wave passes its next barrier
     }
-    f32x16 o[kNO], s_init, s[2];
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        s_init[i] = 0.f;
-#pragma unroll
-        for (int db = 0; db < kNO; db++) o[db][i] = 0.f;
-    }
-    SoftmaxOffState st;
-    st.init();
-    bf16x8 pb[4];
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-        for (int x = 0; x < 8; x++) pb[t][x] = (__bf16)0.0f;
-    auto mask_tile = [&](int e) {
+    auto mask_tile = [&](f32x16 (&s)[2], int e) {
         const int kv0 = kv0_of(e);
         if (kv0 + kBN > sk) {
             const int left = sk - kv0 - 4 * h;
@@ -802,43 +799,94 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
             }
         }
     };
-    typename Dma::Prepared dk = target_k(1), dv = target_v(0);
-    wait_vmcnt<0>();
-    block_barrier();   // K(0) resident, every wave has its queries
-    // The first phase has no tile before it to multiply: unrolled apart.
+    f32x16 o[kNO], s_init;
 #pragma unroll
-    for (int part = 0; part < 2; part++) {
-        const bool first = part == 0;
-#pragma unroll 1
-        for (int m = part; m < (first ? 1 : ne); m++) {
-            __builtin_amdgcn_s_setprio(1);
-            constexpr int kAhead = 3;
-            auto hook_dma = [&](int g) {
-                g -= first ? D / 16 : 0;
-                if (g >= 0 && g < kIt) Dma::issue_prepared(dv, g);
-                else if (g < 2 * kIt) Dma::issue_prepared(dk, g - kIt);
-            };
-            if (first) mfma_phase<false, kAhead, decltype(hook_dma)&, D>(vbuf(1), kbuf(0), rb, pb, o, qf, s, s_init, hook_dma);
-            else mfma_phase<true, kAhead, decltype(hook_dma)&, D>(vbuf(m - 1), kbuf(m), rb, pb, o, qf, s, s_init, hook_dma);
+    for (int i = 0; i < 16; i++) s_init[i] = 0.f;
+    SoftmaxOffState st;
+    bf16x8 pb[4];
+    constexpr int kAhead = 3;
+    typename Dma::Prepared dv = target_v(0), dk = target_v(1);
+    wait_vmcnt<0>();
+    block_barrier();   // K(0), K(1) resident, every wave has its queries
+    // The first two tiles have one offset, the largest score of their 128 keys: the one flash_fwd_pp2 gives them, and with
+    // it the result's bits.
+    {
+        if (ne > 2) {
+            const typename Dma::Prepared k2 = target_k(2);
+#pragma unroll
+            for (int it = 0; it < kIt; it++) Dma::issue_prepared(k2, it);
+        }
+        f32x16 s0[2], s1[2];
+        constexpr int kPer = (kIt + D / 16 - 1) / (D / 16);
+        auto hook_v0 = [&](int g) {
+#pragma unroll
+            for (int x = (g - D / 16) * kPer; x < (g - D / 16 + 1) * kPer && x < kIt; x++) Dma::issue_prepared(dv, x);
+        };
+        auto hook_v1 = [&](int g) {
+#pragma unroll
+            for (int x = (g - D / 16) * kPer; x < (g - D / 16 + 1) * kPer && x < kIt; x++) Dma::issue_prepared(dk, x);
+        };
+        __builtin_amdgcn_s_setprio(1);
+        mfma_phase<false, kAhead, decltype(hook_v0)&, D>(vbuf(0), kbuf(0), rb, pb, o, qf, s0, s_init, hook_v0);
+        bf16x8 pa[4];
+        if (ne > 1) {
+            mfma_phase<false, kAhead, decltype(hook_v1)&, D>(vbuf(0), kbuf(1), rb, pb, o, qf, s1, s_init, hook_v1);
             __builtin_amdgcn_s_setprio(0);
             __builtin_amdgcn_sched_barrier(0);
-            mask_tile(m);
-            if (FIXED && !first) {
+            mask_tile(s0, 0);
+            mask_tile(s1, 1);
+            softmax_first_off<!LOG2DOM>(s0, s1, st, s_init, sl2, pa, pb);
+        } else {
+            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_sched_barrier(0);
+            mask_tile(s0, 0);
+            softmax_first_off<!LOG2DOM>(s0, st, s_init, sl2, pa);
 #pragma unroll
-                for (int b = 0; b < 2; b++) softmax_off_block<!LOG2DOM>(s[b], st, sl2, pb[2 * b], pb[2 * b + 1]);
-            } else {
-                softmax_tile_side_off<!LOG2DOM>(s, st, o, s_init, sl2, pb, [](int) {});
-            }
-            asm volatile("" ::"v"(pb[0]), "v"(pb[1]), "v"(pb[2]), "v"(pb[3]), "v"(st.l_acc));
-            dk = target_k(m + 2);
-            dv = target_v(m + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            wait_vmcnt<0>();
-            block_barrier();   // K(m+1), V(m) resident; this phase's tiles read by every wave
-            __builtin_amdgcn_sched_barrier(0);
+            for (int t = 0; t < 4; t++) pb[t] = pa[t];
         }
+        asm volatile("" ::"v"(pa[0]), "v"(pa[1]), "v"(pa[2]), "v"(pa[3]), "v"(pb[0]), "v"(pb[1]), "v"(pb[2]), "v"(pb[3]), "v"(st.l_acc));
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<0>();
+        block_barrier();   // V(0), V(1), K(2) resident, K(0) and K(1) read by every wave
+#pragma unroll
+        for (int db = 0; db < kNO; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) o[db][i] = 0.f;
+        __builtin_amdgcn_s_setprio(1);
+        pv_tile<D>(vbuf(0), rb.v, pa, o);
+        dk = target_k(3);
+        dv = target_v(2);
+        __builtin_amdgcn_sched_barrier(0);
     }
-    pv_tile<D>(vbuf(ne - 1), rb.v, pb, o);
+#pragma unroll 1
+    for (int m = 2; m < ne; m++) {
+        f32x16 s[2];
+        auto hook_dma = [&](int g) {
+            if (g < kIt) Dma::issue_prepared(dv, g);
+            else if (g < 2 * kIt) Dma::issue_prepared(dk, g - kIt);
+        };
+        __builtin_amdgcn_s_setprio(1);
+        mfma_phase<true, kAhead, decltype(hook_dma)&, D>(vbuf(m - 1), kbuf(m), rb, pb, o, qf, s, s_init, hook_dma);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        mask_tile(s, m);
+        if constexpr (FIXED) {
+#pragma unroll
+            for (int b = 0; b < 2; b++) softmax_off_block<!LOG2DOM>(s[b], st, sl2, pb[2 * b], pb[2 * b + 1]);
+        } else {
+            softmax_tile_off<!LOG2DOM>(s, st, o, s_init, sl2, pb);
+        }
+        asm volatile("" ::"v"(pb[0]), "v"(pb[1]), "v"(pb[2]), "v"(pb[3]), "v"(st.l_acc));
+        dk = target_k(m + 2);
+        dv = target_v(m + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmcnt<0>();
+        block_barrier();   // K(m+1), V(m) resident; this phase's tiles read by every wave
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(1);
+    if (ne > 1) pv_tile<D>(vbuf(ne - 1), rb.v, pb, o);
+    __builtin_amdgcn_s_setprio(0);
 
     if constexpr (FIXED) {   // did the fixed offset hold (flash_item)?
         float chk = 0.f;
@@ -847,6 +895,7 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
 #pragma unroll
             for (int i = 0; i < 16; i++) chk = __builtin_fmaf(o[db][i], 0.f, chk);
         const bool lane_ok = (pair_sum(st.l_acc) < 0x1p+100f) && (chk == 0.f);
+        // (in buffer 4: its last K is behind the last barrier, and a second pass loads it behind its first)
         auto* votes = (__attribute__((address_space(3))) unsigned*)(smem + 4 * kTileBytes);
         const bool wave_ok = __builtin_amdgcn_ballot_w64(!lane_ok) == 0;
         if (lane == 0) votes[wave] = wave_ok ? 0u : 1u;
@@ -859,23 +908,21 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
         }
     }
     const float l_tot = pair_sum(st.l_acc);
-    store_rows<D>(smem + wave * (32 * 2 * D), o, l_tot > 0.f ? 1.f / l_tot : 0.f, out_f32, out_bf16, out_is_bf16,
-                  (size_t)bh * sq + q0 + wave * 32, qlen - wave * 32, lane);
+    // (through buffers 0 and 1 behind the vote, else 1 and 4, which the last P V does not read: half of one a wave)
+    store_rows<D>((FIXED ? smem + (wave >> 1) * kTileBytes : kbuf(1 + (wave >> 1))) + (wave & 1) * (kTileBytes / 2), o,
+                  l_tot > 0.f ? 1.f / l_tot : 0.f, out_f32, out_bf16, out_is_bf16, (size_t)bh * sq + q0 + wave * 32,
+                  qlen - wave * 32, lane);
     return true;
 }
-template <bool MASKED, int D, bool LOG2DOM, bool FIXED>
+template <bool MASKED, int D, bool LOG2DOM>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_fwd_duo(const FlashParams p) {
     int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), block = blockIdx.x;
-    if constexpr (!FIXED) {
-        duo_item<MASKED, D, LOG2DOM, false>(p, wave, threadIdx.x & 63, block);
-    } else {
-        if (duo_item<MASKED, D, LOG2DOM, true>(p, wave, threadIdx.x & 63, block)) return;
-        using ConstParams = const __attribute__((address_space(4))) FlashParams;   // (as in flash_fwd_pp2)
-        ConstParams* again = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
-        int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-        asm volatile("" : "+v"(lane), "+s"(wave), "+s"(block), "+s"(again));
-        duo_item<MASKED, D, LOG2DOM, false>(*again, wave, lane, block);
-    }
+    if (duo_item<MASKED, D, LOG2DOM, true>(p, wave, threadIdx.x & 63, block)) return;
+    using ConstParams = const __attribute__((address_space(4))) FlashParams;   // (as in flash_fwd_pp2)
+    ConstParams* again = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(lane), "+s"(wave), "+s"(block), "+s"(again));
+    duo_item<MASKED, D, LOG2DOM, false>(*again, wave, lane, block);
 }
 
 // Merge of the split-KV partials: out[row] = sum_s w_s O_s / sum_s w_s with w_s = 2^(lse_s - max lse).
@@ -937,6 +984,15 @@ extern "C" hipError_t fv_internal_launch_splitkv_merge(const float* part_o, cons
 
 extern "C" int fv_internal_flash_block_m(void) { return fv::kPpBM; }
 
+// FASTVIDEO_SDPA_RUNNING_MAX=1: every launch keeps the running max (no fixed-offset first pass).
+extern "C" int fv_internal_fixed_offset(int out_is_bf16) {
+    static const bool forced = [] {
+        const char* e = getenv("FASTVIDEO_SDPA_RUNNING_MAX");
+        return e && *e && strcmp(e, "0") != 0;
+    }();
+    return out_is_bf16 && !forced;
+}
+
 namespace {
 // The kernel's dynamic LDS limit (128 KB at D = 128), once per device.
 template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED>
@@ -953,25 +1009,17 @@ hipError_t launch_flash_as(const fv::FlashParams* p, hipStream_t stream) {
     hipLaunchKernelGGL((fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED>), dim3(p->full + p->per_xcd * 8), dim3(256 * NG), lds, stream, *p);
     return hipGetLastError();
 }
-template <bool MASKED, int D, bool LOG2DOM, bool FIXED>
+template <bool MASKED, int D, bool LOG2DOM>
 hipError_t duo_attr() {
     static std::atomic<unsigned long long> attr_done;
-    return fv_set_max_lds_once((const void*)fv::flash_fwd_duo<MASKED, D, LOG2DOM, FIXED>, fv::kDuoLds<D>, attr_done);
+    return fv_set_max_lds_once((const void*)fv::flash_fwd_duo<MASKED, D, LOG2DOM>, fv::kDuoLds<D>, attr_done);
 }
-template <bool MASKED, int D, bool LOG2DOM, bool FIXED>
+template <bool MASKED, int D, bool LOG2DOM>
 hipError_t launch_duo_as(const fv::FlashParams* p, hipStream_t stream) {
-    hipError_t e = duo_attr<MASKED, D, LOG2DOM, FIXED>();
+    hipError_t e = duo_attr<MASKED, D, LOG2DOM>();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((fv::flash_fwd_duo<MASKED, D, LOG2DOM, FIXED>), dim3(p->per_xcd * 8), dim3(256), fv::kDuoLds<D>, stream, *p);
+    hipLaunchKernelGGL((fv::flash_fwd_duo<MASKED, D, LOG2DOM>), dim3(p->per_xcd * 8), dim3(256), fv::kDuoLds<D>, stream, *p);
     return hipGetLastError();
-}
-// FASTVIDEO_SDPA_RUNNING_MAX=1: every launch keeps the running max (no fixed-offset first pass).
-bool running_max_forced() {
-    static const bool v = [] {
-        const char* e = getenv("FASTVIDEO_SDPA_RUNNING_MAX");
-        return e && *e && strcmp(e, "0") != 0;
-    }();
-    return v;
 }
 // A call whose scale * log2(e) is exactly 1 (scale = ln 2: the caller folded the softmax scale into Q) runs
 // the form without the per-score multiply.
@@ -989,28 +1037,25 @@ hipError_t launch_flash_fixed(const fv::FlashParams* p, hipStream_t stream) {
 // window or with sink blocks, and the VDN mask (rows before the video and frame 0 are visible to every query).
 // Under a window without a sink a query's first visible key may lie anywhere in the walk: running max.
 template <bool MASKED>
-bool offset_is_a_score(const fv::FlashParams* p) {
-    return !MASKED || p->mask_mode == 2 || (p->mask_mode == 1 && (p->win == 0 || p->sink > 0));
+bool takes_fixed_offset(const fv::FlashParams* p) {
+    const bool offset_is_a_score = !MASKED || p->mask_mode == 2 || (p->mask_mode == 1 && (p->win == 0 || p->sink > 0));
+    return fv_internal_fixed_offset(p->out_is_bf16) && offset_is_a_score;
 }
 template <int NG, bool MASKED, int D>
 hipError_t launch_flash(const fv::FlashParams* p, hipStream_t stream) {
-    if (p->out_is_bf16 && offset_is_a_score<MASKED>(p) && !running_max_forced()) return launch_flash_fixed<NG, MASKED, D, true>(p, stream);
-    return launch_flash_fixed<NG, MASKED, D, false>(p, stream);
+    return takes_fixed_offset<MASKED>(p) ? launch_flash_fixed<NG, MASKED, D, true>(p, stream) : launch_flash_fixed<NG, MASKED, D, false>(p, stream);
 }
 template <bool MASKED, int D>
 hipError_t launch_duo(const fv::FlashParams* p, hipStream_t stream) {
-    const bool fixed = p->out_is_bf16 && offset_is_a_score<MASKED>(p) && !running_max_forced();
-    if (p->sl2 != 1.0f) return fixed ? launch_duo_as<MASKED, D, false, true>(p, stream) : launch_duo_as<MASKED, D, false, false>(p, stream);
+    if (!takes_fixed_offset<MASKED>(p)) return hipErrorInvalidValue;
+    if (p->sl2 != 1.0f) return launch_duo_as<MASKED, D, false>(p, stream);
     g_log2_domain_launches.fetch_add(1, std::memory_order_relaxed);
-    return fixed ? launch_duo_as<MASKED, D, true, true>(p, stream) : launch_duo_as<MASKED, D, true, false>(p, stream);
+    return launch_duo_as<MASKED, D, true>(p, stream);
 }
 template <bool MASKED, int D>
 hipError_t init_duo() {
-    hipError_t e = duo_attr<MASKED, D, false, false>();
-    if (e == hipSuccess) e = duo_attr<MASKED, D, true, false>();
-    if (e == hipSuccess) e = duo_attr<MASKED, D, false, true>();
-    if (e == hipSuccess) e = duo_attr<MASKED, D, true, true>();
-    return e;
+    const hipError_t e = duo_attr<MASKED, D, false>();
+    return e == hipSuccess ? duo_attr<MASKED, D, true>() : e;
 }
 template <int NG, bool MASKED, int D>
 hipError_t init_flash() {

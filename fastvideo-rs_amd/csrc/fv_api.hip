@@ -126,8 +126,9 @@ struct MaskArgs {
     size_t video_start = 0, frame_tokens = 0, frames = 0, chunk = 0, radius = 0;   // VDN window
 };
 
-// flash_fwd_duo for masked launches (bf16 results; f32 ones keep one kernel for every length, so that a clip's first
-// blocks are the shorter clip's bit for bit). Its tiles of 128 queries cross fewer frame boundaries and leave a shorter
+// flash_fwd_duo for masked launches, where it gives flash_fwd_pp2's bits, so that neither a clip's length nor the number of
+// heads shows in a row: the offset is fixed (a bf16 result, and key 0 in every query's sight: fv_internal_launch_duo), and
+// the first two tiles of every walk are keys 0 to 127 whatever the query tile's size. Its tiles of 128 queries cross fewer frame boundaries and leave a shorter
 // last round, which counts where a query reaches few keys; long walks run at the chip's power limit, where 256 queries to a
 // K and V stream cost less. Causal launches without a window, whose walks are half their reach on average, and windows that
 // are part of their clip take it up to 8192 keys reached, walks of one length up to 4096. us, flash_fwd_pp2 / flash_fwd_duo,
@@ -140,8 +141,10 @@ struct MaskArgs {
 // 92 / 83, 12 x 1560 x 21 (32760) 1817 / 1674.
 bool duo_masked(const fv::FlashParams& p, size_t bh, size_t d) {
     const long ft = p.ft;
+    const bool causal = p.mask_mode == kMaskBlockCausal;
+    if (!fv_internal_fixed_offset(p.out_is_bf16) || (causal && p.win > 0 && p.sink * ft <= 64) || (!causal && p.vs + ft <= 64)) return false;
     long reach = p.sq, most = 8192;
-    if (p.mask_mode == kMaskVdnWindow) {
+    if (!causal) {
         const long seen = 2 + (2 * (long)p.radius + 1) * std::max(1, p.chunk);
         if (seen >= p.frames) most = 4096;
         else reach = ft * seen;
@@ -258,7 +261,7 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         if (p.sl2 == 1.0f) fv_internal_count_log2_domain();
         return FV_OK;
     }
-    if (mode == kMaskNone ? splits == 1 && fv_duo(bh, sq, sk, d) : out_is_bf16 && duo_masked(p, bh, d)) {
+    if (mode == kMaskNone ? splits == 1 && fv_duo(bh, sq, sk, d, out_is_bf16) : duo_masked(p, bh, d)) {
         p.nqt = (int)((sq + 127) / 128);
         p.total = (int)(bh * (size_t)p.nqt);
         p.per_xcd = (p.total + 7) / 8;
@@ -312,11 +315,12 @@ int fv_short_waves(size_t bh, size_t sq, size_t sk, size_t d) {
 // 2500 x 1500 45.7 / 46.2, 12 x 6000 x 1500 77 / 71. At 64: 24 x 1300 x 512 11.5 / 10.3, 24 x 4000 x 1500 51 / 43, 24 x
 // 6000 x 3000 145 / 123, 24 x 20000 x 4000 520 / 484, 24 x 7800 x 7800 366 / 373, 24 x 32760 x 32760 6130 / 6155.
 // (Few query tiles have a CU each, of 128 queries where fv_split_plan says so; a few tiles past whole rounds of
-// flash_fwd_pp2 are split there and would cost this one a round too.)
-bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d) {
+// flash_fwd_pp2 are split there and would cost this one a round too. f32 results follow the running max, whose rescales
+// go by pairs of tiles in flash_fwd_pp2: they stay there, and a block's result does not depend on the clip's length.)
+bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16) {
     const size_t cus = (size_t)fv_compute_units(), bm = (size_t)fv_internal_flash_block_m(), wgs = bh * ((sq + bm - 1) / bm);
     const bool crumbs = wgs > cus && wgs % cus > 0 && wgs % cus <= cus / 16;
-    return sk <= (d == 64 ? 6144 : 1536) && !crumbs && bh * ((sq + 127) / 128) > cus / 2;
+    return fv_internal_fixed_offset(out_bf16) && sk <= (d == 64 ? 6144 : 1536) && !crumbs && bh * ((sq + 127) / 128) > cus / 2;
 }
 
 // Fewer query tiles than CUs: fv_sdpa_splitkv_choose. More: they run in rounds of one per CU, and the last round costs a
@@ -325,7 +329,7 @@ bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d) {
 // Measured on MI355X, unsplit and so, us: 24 x 3000 x 3000 x 128 (288 tiles: 256 + 32 x 5) 145 / 120, 40 x 2000 x 2000
 // x 64 (320: 256 + 64 x 4) 69 / 61, 40 x 75600 x 75600 x 128 (11840: 11776 + 64 x 4) 94470 / 92960 on one MI355X, where runs
 // of one side differ by 0.2 %, and inside the spread on another.
-FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d) {
+FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16) {
     const size_t cus = (size_t)fv_compute_units(), bm = (size_t)fv_internal_flash_block_m();
     const size_t nqt = (sq + bm - 1) / bm, wgs = bh * nqt, nkt = (sk + 63) / 64;
     if (wgs < cus || cus % 8 != 0 || wgs > (size_t)INT_MAX / 64) {
@@ -334,12 +338,12 @@ FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d) {
         // 12 x 320 x 320 x 128 13.2 / 11.3, 12 x 1000 x 1000 x 128 25.6 / 23.0, 40 x 700 x 700 x 64 17.4 / 14.8, 12 x 1560 x
         // 512 x 128 17.2 / 14.9, 24 x 390 x 2000 x 128 at 2 splits 34.2 / 29.7; past one per CU, 12 x 4000 x 512 x 128 20.3 /
         // 29.1, 40 x 1000 x 1000 x 64 (320 tiles) 21.5 / 21.7.
-        if (splits == 1 && fv_duo(bh, sq, sk, d)) return {bm, 0, 1, 0};
+        if (splits == 1 && fv_duo(bh, sq, sk, d, out_bf16)) return {bm, 0, 1, 0};
         const size_t half = bm / 2, small = bh * ((sq + half - 1) / half) * settle_splits(nkt, splits);
         return {small <= cus ? half : bm, 0, splits, fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits)};
     }
     const size_t full = wgs / cus * cus, rest = wgs - full;
-    if (rest == 0 || fv_duo(bh, sq, sk, d)) return {bm, 0, 1, 0};
+    if (rest == 0 || fv_duo(bh, sq, sk, d, out_bf16)) return {bm, 0, 1, 0};
     const size_t rows = bh * sq - (full / nqt * sq + full % nqt * bm);
     // us, measured: a workgroup's fixed part, and a 64-key tile while `w` workgroups run (16 x 4000 x 4000 x 128, 256
     // tiles: 121 us, half of them 79); partials written and read at 4 TB/s and a launch

@@ -166,16 +166,17 @@ struct FvSplitPlan {
     size_t block_m, full, splits, workspace_bytes;   // block_m: queries per workgroup
     int short_waves = 0;                             // > 0: the short kernel, with as many waves a workgroup
 };
-FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d);
+FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16);
 // Waves a workgroup of the short kernel where a dense call of this shape that writes bf16 takes it, else 0.
 int fv_short_waves(size_t bh, size_t sq, size_t sk, size_t d);
 // whether an unsplit dense launch takes the kernel with two workgroups a CU
-bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d);
+bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16);
 // fv_sdpa_dense_bf16_splitkv with such a plan
 int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out, int out_is_bf16, size_t bh,
                      size_t sq, size_t sk, size_t d, float scale, size_t q_rows, size_t k_rows, size_t v_rows,
                      const FvSplitPlan& plan, void* workspace, size_t workspace_bytes, void* stream);
 
+extern "C" int fv_internal_fixed_offset(int out_is_bf16);   // whether results of that type are made with a fixed offset first
 extern "C" int fv_internal_flash_block_m(void);   // queries per workgroup of the flash kernel in use
 extern "C" hipError_t fv_internal_launch_duo(const fv::FlashParams* p, int masked, int d, hipStream_t stream);   // total, nqt: of 128 queries
 extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d, int block_m,

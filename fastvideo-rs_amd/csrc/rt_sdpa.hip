@@ -247,7 +247,7 @@ Result<Tensor> compact(const Tensor& x, Mem& st) {
 
 FvSplitPlan dense_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16) {
     const int waves = out_bf16 ? fv_short_waves(bh, sq, sk, d) : 0;
-    if (!waves) return fv_split_plan(bh, sq, sk, d);
+    if (!waves) return fv_split_plan(bh, sq, sk, d, out_bf16);
     FvSplitPlan p{0, 0, 1, 0};
     p.short_waves = waves;
     return p;

@@ -61,7 +61,7 @@ uint64_t fv_sdpa_log2_domain_launches(void);
 
 /* No counterpart in the reference (a diagnostic). Launches that write bf16 and in which every query sees key 0
  * (dense; block-causal without a window or with sink blocks; the VDN window) make their pass over the keys with every
- * query's softmax offset fixed at the largest score of its first 128 keys (64 on short walks; no running max in the loop), check the row sums
+ * query's softmax offset fixed at the largest score of its first 128 keys (no running max in the loop), check the row sums
  * and accumulators before anything is stored, and make the pass again with the running max in any workgroup where
  * a row's scores outgrew that offset by more than about 2^90: results are exact either way, the second pass only
  * costs time. This is the number of workgroups that took it on the current device since the library was loaded.
@@ -73,7 +73,7 @@ uint64_t fv_sdpa_exact_pass_reruns(void);
  * q [bh,sq,128], k/v [bh,sk,128] bf16 bits; out is f32 [bh,sq,128] when
  * out_is_bf16 == 0, else bf16 bits (RNE). scale > 0.
  * Rounding: with out_is_bf16 == 0 every row follows its running maximum (its largest P is exactly 1); with
- * out_is_bf16 == 1 the softmax offset of a row is the largest score of its first 128 (short walks: 64) keys (see
+ * out_is_bf16 == 1 the softmax offset of a row is the largest score of its first 128 keys (see
  * fv_sdpa_exact_pass_reruns), so a row that one later key dominates carries that key's bf16-rounded P: up to 2^-8
  * relative on such a row, beside the 2^-8 of the result's own rounding. FASTVIDEO_SDPA_RUNNING_MAX=1 (read once)
  * keeps the running maximum in every launch. */

@@ -1,6 +1,6 @@
 """Unsplit dense calls on few keys, two (head dim 64: three) workgroups a CU: the edges of its key and query tiles, one tile
-and two, the longest walks it takes, f32 and bf16 results, row windows, and rows whose scores outgrow the offset of their
-first tile, so that the pass is made again.
+and two, the longest walks it takes, f32 and bf16 results, row windows, rows whose scores outgrow the offset of their
+first 128 keys, so that the pass is made again, and the bits of the kernel that takes the same rows in calls of few heads.
 
 Against the f64 softmax on the same operands. P is rounded to bf16, 2^-9 of each weight at most, and so is a bf16 result:
 2^-9 in the 2-norm for an f32 one, twice that for a bf16 one."""
@@ -114,3 +114,49 @@ def test_masked(fv, d, heads, s, mask):
         want[b] = torch.softmax(x, -1) @ v[b].double()
     rows = ((got.double() - want).norm(dim=-1) / want.norm(dim=-1)).max().item()
     assert ((got.double() - want).norm() / want.norm()).item() <= 2 * 2.0 ** -9 and rows <= 2.0 ** -7, rows
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("sq,sk", [(129, 513), (257, 576), (40, 640), (300, 1535), (256, 1536)])
+def test_the_bits_do_not_depend_on_the_number_of_heads(fv, sq, sk, d):
+    """A launch of few heads takes flash_fwd_pp2, one of many flash_fwd_duo: the same sums term by term, so each head's
+    result is that of a call on a few of them, bit for bit."""
+    import torch
+
+    announce(f"duo heads {HEADS}x{sq}x{sk}x{d}")
+    q, k, v = operands(torch, 3 * sq + sk, sq, sk, d)
+    many = fv.sdpa_dense_bf16(q, k, v, out_bf16=True)
+    few = 128 // ((sq + 127) // 128)          # as many as leave no more than 128 tiles of 128 queries
+    assert few < HEADS
+    for lo in range(0, HEADS, few):
+        part = fv.sdpa_dense_bf16(*(x[lo:lo + few].contiguous() for x in (q, k, v)), out_bf16=True)
+        assert torch.equal(part, many[lo:lo + few]), lo
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("mask", [("causal", 70, 0, 0), ("causal", 128, 0, 0), ("causal", 66, 3, 1), ("causal", 33, 3, 2), ("causal", 64, 3, 1),
+                                  ("causal", 100, 2, 0), ("window", 0, 70, 11, 3, 1), ("window", 20, 50, 14, 0, 1),
+                                  ("window", 0, 40, 16, 0, 1)])
+def test_masked_bits_do_not_depend_on_heads_or_clip_length(fv, d, mask):
+    """Masked bf16 results: a head's rows are those of a call on two heads, and the first blocks of a causal clip are the
+    shorter clip's, bit for bit, with and without window and sink, whichever kernel the sizes select."""
+    import torch
+
+    heads, s = 60, 770
+    announce(f"duo masked bits {heads}x{s}x{d} {mask}")
+    g = torch.Generator(device="cuda").manual_seed(s + d + mask[1])
+    q, k, v = (torch.randn((heads, s, d), generator=g, device="cuda").to(torch.bfloat16) for _ in range(3))
+
+    def call(h, n):
+        x = [t[:h, :n].contiguous() for t in (q, k, v)]
+        if mask[0] == "causal":
+            return fv.sdpa_block_causal_bf16(*x, *mask[1:], out_bf16=True)
+        return fv.sdpa_vdn_window_bf16(*x, *mask[1:], out_bf16=True)
+
+    whole = call(heads, s)
+    assert torch.equal(call(2, s), whole[:2])
+    if mask[0] == "causal":
+        for blocks in (2, 5, s // mask[1]):
+            n = blocks * mask[1]
+            for h in (2, heads):
+                assert torch.equal(call(h, n), whole[:h, :n]), (blocks, h)
