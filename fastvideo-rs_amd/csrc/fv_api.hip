@@ -310,17 +310,22 @@ int fv_short_waves(size_t bh, size_t sq, size_t sk, size_t d) {
 
 // flash_fwd_duo (two or, at head dim 64, three workgroups a CU) against flash_fwd_pp2, for walks so short that an item's
 // ends count. Past them the chip runs at its power limit in either form, and 256 queries to a K and V stream cost less. us,
-// flash_fwd_pp2 / flash_fwd_duo: at 128 channels 12 x 32760 x 64 60 / 38, x 200 77 / 65, x 512 120 / 108, x 770 175 / 154, x
-// 1024 193 / 190, x 1200 231 / 222, x 2048 350 / 354, x 4096 670 / 683; 12 x 1560 x 512 16.3 / 12.6, 24 x 3000 x 1000 56 / 50, 24 x
-// 2500 x 1500 45.7 / 46.2, 12 x 6000 x 1500 77 / 71. At 64: 24 x 1300 x 512 11.5 / 10.3, 24 x 4000 x 1500 51 / 43, 24 x
-// 6000 x 3000 145 / 123, 24 x 20000 x 4000 520 / 484, 24 x 7800 x 7800 366 / 373, 24 x 32760 x 32760 6130 / 6155.
-// (Few query tiles have a CU each, of 128 queries where fv_split_plan says so; a few tiles past whole rounds of
-// flash_fwd_pp2 are split there and would cost this one a round too. f32 results follow the running max, whose rescales
-// go by pairs of tiles in flash_fwd_pp2: they stay there, and a block's result does not depend on the clip's length.)
+// flash_fwd_pp2 / flash_fwd_duo: at 128 channels 12 x 32760 x 64 57 / 39, x 200 77 / 69, x 512 116 / 111, x 800 168 / 157, x 1000
+// 187 / 188, x 1500 264 / 267; 16 x 2560 x 700 25.2 / 23.1, 16 x 6144 x 1500 84.9 / 80.0, 24 x 10000 x 1000 126 / 124. At 64: 24 x
+// 4001 x 50 14.3 / 8.4, 16 x 4096 x 3000 55 / 53, 16 x 6144 x 4000 119 / 109, 16 x 12288 x 6000 311 / 299, 16 x 7680 x 6000 202 / 198.
+// A last round of a quarter of the CUs or less is shared out by key ranges (fv_split_plan), the sooner the fewer its tiles:
+// at 64 channels 16 x 4608 (32 tiles past a round) x 2000 54 / 52, x 2500 64 / 65, x 6000 129 / 147, 16 x 8704 (32 past two) x 2500
+// 103 / 102, x 6000 213 / 231, 16 x 5120 (64) x 3000 80 / 77, x 4000 99 / 101; at 128 16 x 4608 x 1300 70 / 66, x 1500 71 / 74,
+// 16 x 8960 (48) x 1350 109 / 104, x 1500 113 / 113. (Of a sixteenth or less: at any length, this kernel would pay a round for them.)
+// Few query tiles have a CU each, of 128 queries where fv_split_plan says so. f32 results follow the running max, whose
+// rescales go by pairs of tiles in flash_fwd_pp2: they stay there, and a block's result does not depend on the clip's length.
 bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16) {
     const size_t cus = (size_t)fv_compute_units(), bm = (size_t)fv_internal_flash_block_m(), wgs = bh * ((sq + bm - 1) / bm);
-    const bool crumbs = wgs > cus && wgs % cus > 0 && wgs % cus <= cus / 16;
-    return fv_internal_fixed_offset(out_bf16) && sk <= (d == 64 ? 6144 : 1536) && !crumbs && bh * ((sq + 127) / 128) > cus / 2;
+    const size_t rest = wgs > cus ? wgs % cus : 0;   // tiles of the last round that flash_fwd_pp2 would split
+    size_t most = d == 64 ? 6144 : 1536;
+    if (rest > 0 && rest <= cus / 4) most = d == 128 ? 1408 : rest <= cus / 8 ? 2304 : 3072;
+    if (rest > 0 && rest <= cus / 16) most = 0;
+    return fv_internal_fixed_offset(out_bf16) && sk <= most && bh * ((sq + 127) / 128) > cus / 2;
 }
 
 // Fewer query tiles than CUs: fv_sdpa_splitkv_choose. More: they run in rounds of one per CU, and the last round costs a

@@ -249,6 +249,27 @@ def test_no_memory_for_partial_results_is_no_error(shape, kind, launch):
     assert rc < -1 and launch in msg and "allocation" not in msg, msg
 
 
+@pytest.mark.parametrize("shape,act16,split", [
+    ((24, 3000, 6100, 64), True, True), ((24, 3000, 2300, 64), True, False), ((24, 3000, 2400, 64), True, True),
+    ((40, 2000, 3000, 64), True, False), ((40, 2000, 3200, 64), True, True), ((12, 8000, 6100, 64), True, False),
+    ((12, 6000, 1500, 128), True, True), ((12, 6000, 1400, 128), True, False), ((12, 8000, 1500, 128), True, False),
+    ((38, 1700, 1300, 128), True, True), ((24, 3000, 2200, 64), False, True), ((12, 6000, 1300, 128), False, True)])
+def test_a_last_round_of_few_tiles_is_split(shape, act16, split):
+    """A few query tiles past whole rounds of the CUs, on walks long enough, are shared out by key ranges (partial results
+    in the workspace), whatever kernel takes the walk otherwise; f32 results, which have one kernel, sooner. Past the lines
+    the split is faster by up to a seventh (24 x 3000 x 6100 x 64)."""
+    from fv_sdpa.sdpa import _FvPlan
+
+    lib, ref, need = fv_sdpa.lib(), ctypes.byref, (ctypes.c_size_t * 2)()
+    h, sq, sk, d = shape
+    q, k = _fake_tensor((1, h, sq, d), True), _fake_tensor((1, h, sk, d), True)
+    p = _FvPlan()
+    p.kv_flash = -1
+    with fv_sdpa.with_bf16_act(act16):
+        assert lib.fv_rt_sdpa_need(ref(q), ref(k), ref(k), ref(p), need) == 0
+    assert (need[1] > 0) == split, need[1]
+
+
 def test_need_is_host_arithmetic_at_any_shape():
     """fv_rt_sdpa_need answers for shapes the call itself refuses (no keys, no queries, no heads, lengths past every
     limit), for every kind of plan and either type: no division by a count of zero, and a workspace of zero or of the
