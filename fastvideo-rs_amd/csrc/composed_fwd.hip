@@ -696,7 +696,8 @@ constexpr int short_lds() {
     return tiles > merge ? tiles : merge;
 }
 
-template <int NC, int PP, int KS>
+// LOG2DOM: scale * log2(e) is one, no multiply of a score.
+template <int NC, int PP, int KS, bool LOG2DOM>
 __global__ __launch_bounds__(64 * KS, NC <= 4 ? 4 : 2) void sdpa_short_kernel(const ComposedParams p) {
     using SG = ShortGeo<NC>;
     using G = typename SG::G;
@@ -758,7 +759,7 @@ __global__ __launch_bounds__(64 * KS, NC <= 4 ? 4 : 2) void sdpa_short_kernel(co
     __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the zeros are written
     block_barrier();
     const TileReadBases rb = tile_read_bases<SG::D>(lane);
-    const float q_mul = PP == 3 ? composed_q_mul(p) : 1.f, to_log2 = composed_to_log2(p);
+    const float q_mul = PP == 3 ? composed_q_mul(p) : 1.f, to_log2 = LOG2DOM ? 1.f : composed_to_log2(p);
     bf16x8 qf[NC];
 #pragma unroll
     for (int j = 0; j < NC; j++) {
@@ -981,12 +982,13 @@ hipError_t launch_d(const ComposedParams& p, int parts, bool kv16, int ks, size_
     }
     return launch_as<D, 1, 2, true>(p, bh, st);
 }
-template <int NC, int PP, int KS>
+template <int NC, int PP, int KS, bool LOG2DOM>
 hipError_t launch_short_as(const ComposedParams& p, size_t bh, hipStream_t st) {
     constexpr int lds = short_lds<NC, KS>();
     static std::atomic<unsigned long long> attr_done;
-    const hipError_t e = fv_set_max_lds_once((const void*)sdpa_short_kernel<NC, PP, KS>, lds, attr_done);
+    const hipError_t e = fv_set_max_lds_once((const void*)sdpa_short_kernel<NC, PP, KS, LOG2DOM>, lds, attr_done);
     if (e != hipSuccess) return e;
+    if (LOG2DOM) fv_internal_count_log2_domain();
     ComposedParams a = p;
     a.nqt = (p.sq + 31) / 32;
     a.full = 0, a.splits = 1;
@@ -995,12 +997,16 @@ hipError_t launch_short_as(const ComposedParams& p, size_t bh, hipStream_t st) {
     a.total = (int)total;
     a.per_xcd = (int)((total + 7) / 8);
     a.by_head = !p.mask || p.mask_bh != 0;
-    hipLaunchKernelGGL((sdpa_short_kernel<NC, PP, KS>), dim3((unsigned)(a.per_xcd * 8)), dim3(64 * KS), lds, st, a);
+    hipLaunchKernelGGL((sdpa_short_kernel<NC, PP, KS, LOG2DOM>), dim3((unsigned)(a.per_xcd * 8)), dim3(64 * KS), lds, st, a);
     return hipGetLastError();
 }
 template <int NC, int PP>
 hipError_t launch_short_nc(const ComposedParams& p, int waves, size_t bh, hipStream_t st) {
-    return waves == 8 ? launch_short_as<NC, PP, 8>(p, bh, st) : launch_short_as<NC, PP, 4>(p, bh, st);
+    if constexpr (PP == 1) {
+        if (fv_sdpa_is_log2_domain_scale(p.scale))
+            return waves == 8 ? launch_short_as<NC, PP, 8, true>(p, bh, st) : launch_short_as<NC, PP, 4, true>(p, bh, st);
+    }
+    return waves == 8 ? launch_short_as<NC, PP, 8, false>(p, bh, st) : launch_short_as<NC, PP, 4, false>(p, bh, st);
 }
 template <int PP>
 hipError_t launch_short(const ComposedParams& p, int waves, size_t bh, hipStream_t st) {

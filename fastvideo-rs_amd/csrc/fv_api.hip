@@ -257,9 +257,7 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         c.sq = p.sq, c.sk = p.sk, c.d = (int)d, c.scale = scale, c.vec = 1;
         c.q_plane = p.q_plane, c.k_plane = p.k_plane, c.v_plane = p.v_plane;
         const hipError_t e = fv_internal_launch_short(&c, short_waves, bh, (hipStream_t)stream);
-        if (e != hipSuccess) return fail_hip(e, "sdpa_short");
-        if (p.sl2 == 1.0f) fv_internal_count_log2_domain();
-        return FV_OK;
+        return e == hipSuccess ? FV_OK : fail_hip(e, "sdpa_short");
     }
     if (mode == kMaskNone ? splits == 1 && fv_duo(bh, sq, sk, d, out_is_bf16) : duo_masked(p, bh, d)) {
         p.nqt = (int)((sq + 127) / 128);
@@ -409,7 +407,7 @@ int fv_sdpa_init(void) {
     return e == hipSuccess ? FV_OK : fail_hip(e, "fv_sdpa_init");
 }
 
-// the launcher's own test (flash_fwd.hip launch_flash): FlashParams::sl2, computed as below, equal to one
+// the launchers' own test (flash_fwd.hip: FlashParams::sl2, computed as below, equal to one)
 int fv_sdpa_is_log2_domain_scale(float scale) { return scale * 1.4426950408889634f == 1.0f ? 1 : 0; }
 
 uint64_t fv_sdpa_exact_pass_reruns(void) {

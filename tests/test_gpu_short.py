@@ -75,3 +75,22 @@ def test_row_windows_and_nan_rows(fv, sk, d):
     nan[0, 1] = True
     assert torch.equal(got.isnan().all(-1), nan) and torch.equal(got.isnan().any(-1), nan)
     assert torch.equal(got[~nan], base[~nan])
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("h,sq,sk", [(12, 320, 320), (3, 100, 700), (16, 640, 513)])   # eight waves, eight, four
+def test_the_scale_folded_into_the_queries(fv, h, sq, sk, d):
+    """scale = ln 2 takes the form without the multiply of every score, and is counted."""
+    import torch
+
+    announce(f"short log2 {h}x{sq}x{sk}x{d}")
+    ln2 = float(np.float32(np.log(2.0)))
+    q, k, v = operands(torch, sq + sk + d, 1, h, sq, sk, d)
+    q = (q.float() * (1.4426950408889634 / np.sqrt(d))).to(torch.bfloat16)
+    lib = fv.lib()
+    n0 = lib.fv_sdpa_log2_domain_launches()
+    got = fv.sdpa(q, k, v, fv.Plan.masked(ln2)).double().cpu()
+    assert lib.fv_sdpa_log2_domain_launches() == n0 + 1
+    q, k, v = (x.double().cpu() for x in (q, k, v))
+    want = ((q @ k.transpose(-1, -2)) * ln2).softmax(-1) @ v
+    assert (got - want).norm() <= 2 * 2.0 ** -9 * want.norm()

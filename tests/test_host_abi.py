@@ -270,6 +270,21 @@ def test_a_last_round_of_few_tiles_is_split(shape, act16, split):
     assert (need[1] > 0) == split, need[1]
 
 
+def test_every_fused_kernel_has_a_form_for_the_log2_domain():
+    """What fv_sdpa_log2_domain_launches counts is launches of kernels without the multiply of every score: each fused
+    kernel is built with and without it (the kernels' symbols, mangled names of their templates)."""
+    with open(fv_sdpa._lib.LIB_PATH, "rb") as f:
+        text = f.read()
+    for d in (64, 128):
+        for masked in (0, 1):
+            for form in (0, 1):
+                assert b"flash_fwd_pp2ILi2ELb%dELi%dELb%dE" % (masked, d, form) in text
+                assert b"flash_fwd_duoILb%dELi%dELb%dE" % (masked, d, form) in text
+        for waves in (4, 8):
+            for form in (0, 1):
+                assert b"sdpa_short_kernelILi%dELi1ELi%dELb%dE" % (d // 16, waves, form) in text
+
+
 def test_need_is_host_arithmetic_at_any_shape():
     """fv_rt_sdpa_need answers for shapes the call itself refuses (no keys, no queries, no heads, lengths past every
     limit), for every kind of plan and either type: no division by a count of zero, and a workspace of zero or of the
