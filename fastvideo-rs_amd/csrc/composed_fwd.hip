@@ -35,6 +35,8 @@
 // of 64 bytes (the 4 rows of a transposed read land in 4 different 64-byte bank groups).
 #include <limits.h>
 
+#include <initializer_list>
+
 #include "../../include/fv_sdpa_hip.h"
 #include "attn_core.h"
 #include "fv_internal.h"
@@ -934,14 +936,25 @@ __global__ __launch_bounds__(256) void composed_merge_kernel(const ComposedParam
     }
 }
 
+// The kernels' dynamic LDS limits, once per device.
+template <int D, int PARTS, int KS, bool KV16>
+hipError_t composed_attr() {
+    constexpr int lds = composed_lds<D, PARTS, KS>();
+    if (lds <= 64 * 1024) return hipSuccess;
+    static std::atomic<unsigned long long> attr_done;
+    return fv_set_max_lds_once((const void*)sdpa_composed_kernel<D, PARTS, KS, KV16>, lds, attr_done);
+}
+template <int NC, int PP, int KS, bool LOG2DOM>
+hipError_t short_attr() {
+    static std::atomic<unsigned long long> attr_done;
+    return fv_set_max_lds_once((const void*)sdpa_short_kernel<NC, PP, KS, LOG2DOM>, short_lds<NC, KS>(), attr_done);
+}
+
 template <int D, int PARTS, int KS, bool KV16>
 hipError_t launch_as(const ComposedParams& p, size_t bh, hipStream_t st) {
     constexpr int lds = composed_lds<D, PARTS, KS>();
-    if (lds > 64 * 1024) {
-        static std::atomic<unsigned long long> attr_done;
-        const hipError_t e = fv_set_max_lds_once((const void*)sdpa_composed_kernel<D, PARTS, KS, KV16>, lds, attr_done);
-        if (e != hipSuccess) return e;
-    }
+    const hipError_t ae = composed_attr<D, PARTS, KS, KV16>();
+    if (ae != hipSuccess) return ae;
     constexpr int rows = 32 * (composed_waves(KS) / KS);
     ComposedParams a = p;
     a.nqt = (p.sq + rows - 1) / rows;
@@ -985,8 +998,7 @@ hipError_t launch_d(const ComposedParams& p, int parts, bool kv16, int ks, size_
 template <int NC, int PP, int KS, bool LOG2DOM>
 hipError_t launch_short_as(const ComposedParams& p, size_t bh, hipStream_t st) {
     constexpr int lds = short_lds<NC, KS>();
-    static std::atomic<unsigned long long> attr_done;
-    const hipError_t e = fv_set_max_lds_once((const void*)sdpa_short_kernel<NC, PP, KS, LOG2DOM>, lds, attr_done);
+    const hipError_t e = short_attr<NC, PP, KS, LOG2DOM>();
     if (e != hipSuccess) return e;
     if (LOG2DOM) fv_internal_count_log2_domain();
     ComposedParams a = p;
@@ -1018,8 +1030,36 @@ hipError_t launch_short(const ComposedParams& p, int waves, size_t bh, hipStream
     }
     return launch_short_nc<8, PP>(p, waves, bh, st);
 }
+
+hipError_t first_error(std::initializer_list<hipError_t> all) {
+    for (const hipError_t e : all)
+        if (e != hipSuccess) return e;
+    return hipSuccess;
+}
+template <int D>
+hipError_t init_composed_d() {   // (launch_d)
+    hipError_t e = first_error({composed_attr<D, 3, 1, false>(), composed_attr<D, 3, 2, false>(), composed_attr<D, 1, 1, false>(),
+                                composed_attr<D, 1, 2, false>(), composed_attr<D, 1, 1, true>(), composed_attr<D, 1, 2, true>()});
+    if constexpr (D <= 96)
+        if (e == hipSuccess) e = first_error({composed_attr<D, 1, 4, true>(), composed_attr<D, 1, 8, true>()});
+    return e;
+}
+template <int NC, int PP>
+hipError_t init_short_nc() {
+    hipError_t e = first_error({short_attr<NC, PP, 4, false>(), short_attr<NC, PP, 8, false>()});
+    if constexpr (PP == 1)
+        if (e == hipSuccess) e = first_error({short_attr<NC, PP, 4, true>(), short_attr<NC, PP, 8, true>()});
+    return e;
+}
 }  // namespace
 }  // namespace fv
+
+extern "C" hipError_t fv_internal_init_composed(void) {
+    using namespace fv;
+    return first_error({init_composed_d<32>(), init_composed_d<64>(), init_composed_d<96>(), init_composed_d<128>(),
+                        init_short_nc<4, 1>(), init_short_nc<8, 1>(), init_short_nc<4, 3>(), init_short_nc<5, 3>(),
+                        init_short_nc<6, 3>(), init_short_nc<7, 3>(), init_short_nc<8, 3>()});
+}
 
 // Query tiles (128 queries) past a multiple of the CUs hold up the launch for a whole walk of the keys while other CUs
 // have none left: they are shared out by key ranges, in as many as fill the CUs best, where that saves more than writing

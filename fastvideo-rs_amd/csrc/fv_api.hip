@@ -402,6 +402,7 @@ const char* fv_sdpa_arch(void) { return "gfx950"; }
 int fv_sdpa_init(void) {
     hipError_t e = fv_internal_init_flash();
     if (e == hipSuccess) e = fv_internal_init_vsa();
+    if (e == hipSuccess) e = fv_internal_init_composed();
     void* p = nullptr;
     if (e == hipSuccess) e = static_scratch(&p);
     return e == hipSuccess ? FV_OK : fail_hip(e, "fv_sdpa_init");

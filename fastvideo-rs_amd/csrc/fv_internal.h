@@ -213,6 +213,7 @@ extern "C" hipError_t fv_internal_launch_splitkv_merge(const float* part_o, cons
                                                        hipStream_t st);
 extern "C" hipError_t fv_internal_init_flash(void);
 extern "C" hipError_t fv_internal_init_vsa(void);
+extern "C" hipError_t fv_internal_init_composed(void);
 extern "C" size_t fv_internal_fine_pace(fv::VsaFineParams* p);
 extern "C" hipError_t fv_internal_launch_fine(const fv::VsaFineParams* p, hipStream_t st);
 extern "C" hipError_t fv_internal_launch_combine(const float* sparse, const float* coarse,

@@ -154,3 +154,40 @@ def test_kv_cache_block_forward_replay(fv):
         torch.cuda.synchronize()
         assert cache.pointers(0) == ref.pointers(0)
         assert torch.equal(out, want), blk
+
+
+def test_first_launches_inside_a_capture_after_init():
+    """In a process of its own: fv_sdpa_init, then a capture that holds the first launch of the short kernel (its dense, its
+    masked and its wide form) and of the composed kernel on f32 operands, all with more than 64 KB of LDS. Replays give the
+    eager results."""
+    import subprocess
+    import sys
+
+    from util import PKG, ROOT
+
+    announce("graph: first launches inside a capture")
+    code = (
+        "import sys; sys.path[:0] = %r\n"
+        "import torch, fv_sdpa as fv\n"
+        "lib = fv.lib()\n"
+        "assert lib.fv_sdpa_init() == 0\n"
+        "g = torch.Generator(device='cuda').manual_seed(3)\n"
+        "mk = lambda *s: torch.randn(s, generator=g, device='cuda')\n"
+        "x, y = mk(1, 12, 320, 128), mk(1, 16, 257, 80)\n"
+        "w, m = mk(1, 12, 40, 112), mk(320, 320)\n"
+        "b = lambda t: t.to(torch.bfloat16)\n"
+        "calls = [(b(x), fv.Plan.dense()), (b(x), fv.Plan.masked(None, m)), (b(y), fv.Plan.dense()), (b(w), fv.Plan.dense()),\n"
+        "         (x, fv.Plan.composed(None, m)), (y, fv.Plan.composed())]\n"
+        "run = lambda: [fv.sdpa(t, t, t, p) for t, p in calls]\n"
+        "torch.cuda.synchronize()\n"
+        "graph = torch.cuda.CUDAGraph()\n"
+        "with torch.cuda.graph(graph):\n"
+        "    outs = run()\n"
+        "want = run()\n"
+        "for i in range(3):\n"
+        "    for o in outs: o.zero_()\n"
+        "    graph.replay()\n"
+        "    torch.cuda.synchronize()\n"
+        "    assert all(torch.equal(a, c) for a, c in zip(outs, want)), i\n" % [ROOT, PKG])
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
