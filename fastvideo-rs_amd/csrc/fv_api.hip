@@ -116,7 +116,6 @@ struct MaskArgs {
     int mode = kMaskNone;
     size_t q_rows = 0, k_rows = 0, v_rows = 0;   // rows per (batch, head) plane; 0 = contiguous (sq / sk)
     size_t splits = 1;                            // split-KV (dense only): key splits per query tile ...
-    bool split_entry = false;                     // (asked for by the caller of a split-KV entry)
     size_t full = 0;                              // ... past the first `full` ones
     size_t block_m = 0;                           // queries per workgroup (0: the kernel's own)
     int short_waves = 0;                          // > 0: the short kernel, with as many waves a workgroup
@@ -200,7 +199,7 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         p.win = (int)m.window;
         p.sink = (int)m.sink;
         // One block spanning both sequences: every key is visible to every query (tq == tk == 0
-        // for any window), so this is the dense problem and runs as the dense launch, bit for bit
+        // for any window), so this is the dense problem and runs as the launch of the kernel-level dense entry, bit for bit
         // (the reference asserts that identity for its own kernels, gpucheck kernels_wan.rs:230-261).
         if (m.block_tokens >= sq && m.block_tokens >= sk) mode = kMaskNone;
     } else if (mode == kMaskVdnWindow) {
@@ -245,12 +244,12 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         p.total = (int)((total - full) * splits);
         p.per_xcd = (p.total + 7) / 8;
     }
-    // Kernel-level calls take the short kernel up to 512 keys, and past them where a split-KV entry is asked for a bf16
-    // result with the library's own count (the result of fv_rt_sdpa on that shape, bit for bit).
+    // Kernel-level calls take the short kernel up to 512 keys. Past them fv_rt_sdpa alone asks for it (short_waves): there
+    // these calls are flash_fwd_pp2's or flash_fwd_duo's, whose bits a block-causal clip of one block then shares with the
+    // first block of a longer one, for both result types (one frame has 880 tokens and more); it costs them what the short
+    // kernel gains, 24.3 us instead of 16.8 at 12 x 1000 x 1000 x 128, 21.1 instead of 11.9 at 12 x 600 x 1000.
     int short_waves = m.short_waves;
-    if (mode == kMaskNone && !short_waves &&
-        ((splits == 1 && sk <= 512) || (m.split_entry && out_is_bf16 && m.splits == fv_sdpa_splitkv_choose(bh, sq, sk))))
-        short_waves = fv_short_waves(bh, sq, sk, d);
+    if (mode == kMaskNone && splits == 1 && !short_waves && sk <= 512) short_waves = fv_short_waves(bh, sq, sk, d);
     if (short_waves) {
         fv::ComposedParams c;
         c.q = q, c.k = k, c.v = v, c.out = out, c.q_is_bf16 = 1, c.out_is_bf16 = out_is_bf16;
@@ -475,8 +474,12 @@ int fv_sdpa_dense_bf16_splitkv(const uint16_t* q, const uint16_t* k, const uint1
     m.q_rows = q_rows;
     m.k_rows = k_rows;
     m.v_rows = v_rows;
-    m.splits = splits ? splits : 1;
-    m.split_entry = true;
+    m.splits = splits;
+    if (splits == 0) {   // the choice of fv_rt_sdpa
+        m.short_waves = out_is_bf16 ? fv_short_waves(bh, sq, sk, d) : 0;
+        m.splits = m.short_waves ? 1 : fv_sdpa_splitkv_choose(bh, sq, sk);
+        if (!workspace || workspace_bytes < fv_sdpa_splitkv_workspace_bytes(bh, sq, d, m.splits)) m.splits = 1;
+    }
     m.workspace = workspace;
     m.workspace_bytes = workspace_bytes;
     return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
@@ -516,7 +519,6 @@ int fv_sdpa_dense_bf16_splitkv_static(const uint16_t* q, const uint16_t* k, cons
     m.k_rows = k_rows;
     m.v_rows = v_rows;
     m.splits = run;
-    m.split_entry = true;
     if (run > 1) {
         void* p = nullptr;
         const hipError_t e = static_scratch(&p);

@@ -96,9 +96,12 @@ int fv_sdpa_dense_bf16_strided(const uint16_t* q, const uint16_t* k, const uint1
  * them into `out`. Same operands as fv_sdpa_dense_bf16_strided. No counterpart in the reference, whose
  * kernels run one CTA per query tile (rt/attn.rs:378-395). fv_sdpa_splitkv_choose: the split count this
  * library would pick for a shape on the current device (1 = none: use the plain entry; fv_rt_sdpa
- * applies it by itself); splits is clamped to the number of 64-key tiles and so that no split is empty. workspace: 256-byte aligned,
- * fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits) bytes. Results agree with the unsplit kernel
- * to rounding (each split normalises by its own row sum before the merge). */
+ * applies it by itself, except that its bf16 results of few query groups and up to 3072 keys, at head dim 64 4000, come from
+ * a kernel that shares the keys out inside a workgroup). splits is clamped to the number of 64-key tiles and so that no split
+ * is empty; an explicit count is the count that runs (1: the plain entry's result, bit for bit), 0 is the choice of
+ * fv_rt_sdpa, unsplit where the workspace does not hold the partials. workspace: 256-byte aligned,
+ * fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits) bytes (for 0: of fv_sdpa_splitkv_choose's count). Results agree with
+ * the unsplit kernel to rounding (each split normalises by its own row sum before the merge). */
 size_t fv_sdpa_splitkv_choose(size_t bh, size_t sq, size_t sk);
 size_t fv_sdpa_splitkv_workspace_bytes(size_t bh, size_t sq, size_t d, size_t splits);
 int fv_sdpa_dense_bf16_splitkv(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,

@@ -216,6 +216,22 @@ def test_full_size_prefix_and_block_properties(fv, bt, win, sink):
         assert delta <= min(1e-2, 0.25 * first.std().item()), delta
 
 
+@pytest.mark.parametrize("out_bf16", [False, True])
+@pytest.mark.parametrize("bh,bt,d", [(2, 513, 128), (40, 600, 64), (40, 880, 128), (12, 1560, 128)])
+def test_a_clip_of_one_block_is_the_first_block_of_a_longer_one(fv, bh, bt, d, out_bf16):
+    """One block is the dense launch, three are a masked one: the rows of the first block are the same bits, for blocks of
+    more than 512 tokens (shorter ones are dense calls that the short kernel takes)."""
+    import torch
+
+    announce(f"causal one block and three {bh}x{bt}x{d} out_bf16={out_bf16}")
+    g = torch.Generator(device="cuda").manual_seed(bh + bt)
+    q, k, v = (torch.randn((bh, 3 * bt, d), generator=g, device="cuda").to(torch.bfloat16) for _ in range(3))
+    whole = fv.sdpa_block_causal_bf16(q, k, v, bt, 0, 0, out_bf16=out_bf16)
+    one = fv.sdpa_block_causal_bf16(*(x[:, :bt].contiguous() for x in (q, k, v)), bt, 0, 0, out_bf16=out_bf16)
+    torch.cuda.synchronize()
+    assert torch.equal(one, whole[:, :bt])
+
+
 @pytest.mark.parametrize("d", [128, 64])
 def test_block_causal_pass_with_the_fixed_offset_and_its_rerun(fv, oracle, d):
     """Block-causal launches that write bf16 and in which every query sees key 0 (no window, or sink blocks) make their

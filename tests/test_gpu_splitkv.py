@@ -168,3 +168,48 @@ def test_nan_rows_stay_nan(fv, bh, sq, sk, d, act16):
         first[h, r] = True
     assert torch.equal(got.isnan(), first)
     assert torch.equal(keyed.isnan(), want)
+
+
+@pytest.mark.parametrize("d", [128, 64])
+def test_an_explicit_count_is_the_count_that_runs(fv, oracle, d):
+    """Also where it is the library's own, and where fv_rt_sdpa takes another kernel: every split of a bf16 launch checks its
+    own offset, so scores that outgrow the first 128 keys' show in the rerun counter. A count of one is the plain entry's
+    result bit for bit, for both result types; no count is the choice of fv_rt_sdpa."""
+    import torch
+
+    bh, sq, sk = 3, 600, 1100
+    announce(f"splitkv explicit counts d={d}")
+    assert fv.splitkv_choose(bh, sq, sk) == 2
+    q, k, v = (to_dev_bf16(x) for x in qkv(31 + d, bh, sq, sk, d))
+    lib = fv.lib()
+    for act16 in (True, False):
+        plain = fv.sdpa_dense_bf16(q, k, v, out_bf16=act16)
+        assert torch.equal(fv.sdpa_dense_bf16_splitkv(q, k, v, splits=1, out_bf16=act16), plain)
+        with fv.with_bf16_act(act16):
+            assert torch.equal(fv.sdpa_dense_bf16_splitkv(q, k, v, out_bf16=act16)[None], fv.sdpa(q[None], k[None], v[None], fv.Plan.dense()))
+        got = fv.sdpa_dense_bf16_splitkv(q, k, v, splits=2, out_bf16=act16)
+        assert (got.float() - plain.float()).abs().max().item() <= 2e-2
+    q[0] = q[0].abs() + 2.0
+    k[0, :128] = -0.5
+    k[0, 128:] = torch.linspace(1.0, 40.0, sk - 128, device="cuda")[:, None].to(torch.bfloat16)
+    n0 = lib.fv_sdpa_exact_pass_reruns()
+    got = fv.sdpa_dense_bf16_splitkv(q, k, v, splits=2, out_bf16=True)
+    torch.cuda.synchronize()
+    assert lib.fv_sdpa_exact_pass_reruns() >= n0 + (sq + 255) // 256
+    want = oracle.sdpa_f64(*(x.float().cpu().numpy() for x in (q, k, v)))
+    assert_parity(got.float().cpu().numpy(), want, f"splitkv_explicit_d{d}", max_abs=2e-2)
+
+
+def test_no_count_and_no_workspace_runs_unsplit(fv):
+    """The entry with splits = 0 takes what fv_rt_sdpa would, and is not refused for want of a workspace."""
+    import torch
+
+    bh, sq, sk, d = 2, 100, 5000, 128
+    announce("splitkv no count, no workspace")
+    assert fv.splitkv_choose(bh, sq, sk) > 1
+    q, k, v = (to_dev_bf16(x) for x in qkv(32, bh, sq, sk, d))
+    out = torch.full((bh, sq, d), float("nan"), device="cuda")
+    rc = fv.lib().fv_sdpa_dense_bf16_splitkv(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), 0, bh, sq, sk, d, d ** -0.5, 0,
+                                             0, 0, 0, None, 0, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0 and torch.equal(out, fv.sdpa_dense_bf16(q, k, v))
