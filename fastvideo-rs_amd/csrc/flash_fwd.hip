@@ -130,50 +130,34 @@ FV_DEV LaneMask lane_mask(const Params& p, int qi) {
     return m;
 }
 
-// A wave's 32 rows o * inv, the first of them row `row0` of the result; `rows` (and no more) are stored. `my`: 32 x 2D bytes
-// of LDS of the wave's own.
+// A wave's 32 rows o * inv in bf16, the first of them row `row0` of the result; `rows` (and no more) are stored. `my`:
+// 32 x 2D bytes of LDS of the wave's own: scattered 8-byte pieces in, whole rows out, 16 bytes per lane and 1 KB (D = 128)
+// of consecutive output per store instruction.
 template <int D>
-FV_DEV void store_rows(lds_u8* my, const f32x16 (&o)[D / 32], float inv, float* out_f32, uint16_t* out_bf16, int out_is_bf16,
-                       size_t row0, int rows, int lane) {
+FV_DEV void store_rows16(lds_u8* my, const f32x16 (&o)[D / 32], float inv, uint16_t* out, size_t row0, int rows, int lane) {
     const int h = lane >> 5, c32 = lane & 31;
-    constexpr int kNO = D / 32;
-    if (out_is_bf16) {
-        // bf16 rows: scattered 8-byte pieces in, whole rows out, 16 bytes per lane and 1 KB (D = 128) of consecutive
-        // output per store instruction
-        constexpr int kRowB = 2 * D, kCh = kRowB / 16;
+    constexpr int kRowB = 2 * D, kCh = kRowB / 16;
 #pragma unroll
-        for (int db = 0; db < kNO; db++)
+    for (int db = 0; db < D / 32; db++)
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                f32x4 r;
+        for (int g = 0; g < 4; g++) {
+            f32x4 r;
 #pragma unroll
-                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
-                const bf16x4 rb4 = __builtin_convertvector(r, bf16x4);
-                const int ch = (4 * db + g) ^ (c32 & (kCh - 1));
-                *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>(my + c32 * kRowB + (ch << 4) + 8 * h) = rb4;
-            }
-        // (same-wave LDS writes and reads complete in order; the compiler waits on the reads' data)
-        constexpr int kRowsPer = 64 / kCh;           // rows one store instruction covers
-        const int lr = lane / kCh, lc = lane % kCh;
-        uint16_t* ob = out_bf16 + row0 * D;
-#pragma unroll
-        for (int i = 0; i < 32 / kRowsPer; i++) {
-            const int rr = i * kRowsPer + lr;
-            const u32x4 val = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(
-                my + rr * kRowB + ((lc ^ (rr & (kCh - 1))) << 4));
-            if (rr < rows) global_store<u32x4>(ob + (size_t)rr * D + lc * 8, val);
+            for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
+            const bf16x4 rb4 = __builtin_convertvector(r, bf16x4);
+            const int ch = (4 * db + g) ^ (c32 & (kCh - 1));
+            *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>(my + c32 * kRowB + (ch << 4) + 8 * h) = rb4;
         }
-    } else if (c32 < rows) {
-        float* ob = out_f32 + (row0 + c32) * D;
+    // (same-wave LDS writes and reads complete in order; the compiler waits on the reads' data)
+    constexpr int kRowsPer = 64 / kCh;           // rows one store instruction covers
+    const int lr = lane / kCh, lc = lane % kCh;
+    uint16_t* ob = out + row0 * D;
 #pragma unroll
-        for (int db = 0; db < kNO; db++)
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                f32x4 r;
-#pragma unroll
-                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
-                global_store<f32x4>(ob + 32 * db + 8 * g + 4 * h, r);
-            }
+    for (int i = 0; i < 32 / kRowsPer; i++) {
+        const int rr = i * kRowsPer + lr;
+        const u32x4 val = *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(
+            my + rr * kRowB + ((lc ^ (rr & (kCh - 1))) << 4));
+        if (rr < rows) global_store<u32x4>(ob + (size_t)rr * D + lc * 8, val);
     }
 }
 
@@ -585,7 +569,7 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
             return true;
         }
     }
-    // (store_rows() written out: its call costs the long masked launches 1 %)
+    // (store_rows16() written out: its call costs the long masked launches 1 %)
     if (out_is_bf16) {
         // bf16 rows through this wave's own 32 x 2D-byte slice of the K ring (every K read is behind the last
         // barrier and no load is in flight): scattered 8-byte pieces in, whole rows out, 16 bytes per
@@ -695,7 +679,7 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
         qt = work - bh * p.nqt;
     }
     const int q0 = qt * kDuoBM, sq = p.sq, sk = p.sk, qlen = min(kDuoBM, sq - q0), nkt = (sk + kBN - 1) / kBN;
-    int a1 = 0, a2 = 0, n0 = nkt, n1 = 0, ne = nkt;   // the walk, as in flash_item
+    int a1 = 0, a2 = 0, n0 = nkt, n1 = 0, ne = nkt;   // the walk, as in flash_item (key 0 is in it)
     LaneMask lm = {0, 0x7fffffff, 0, 0};
     if constexpr (MASKED) {
         const TileWalk w = mask_tile_walk(p, q0, qlen, nkt);
@@ -703,22 +687,8 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
         lm = lane_mask(p, q0 + wave * 32 + c32);
     }
     const float sl2 = p.sl2, NEG = neg_inf();
-    float* out_f32 = p.out_f32;
-    uint16_t* out_bf16 = p.out_bf16;
-    int out_is_bf16 = p.out_is_bf16;
-    asm volatile("" : "+s"(out_f32), "+s"(out_bf16), "+s"(out_is_bf16));   // (fetched now, see flash_item)
-    if constexpr (MASKED) {
-        if (ne <= 0) {   // no key tile is visible to any query of this tile: rows of zeros (flash_item)
-            f32x16 zero[kNO];
-#pragma unroll
-            for (int db = 0; db < kNO; db++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) zero[db][i] = 0.f;
-            store_rows<D>(smem + wave * (kTileBytes / 2), zero, 0.f, out_f32, out_bf16, out_is_bf16,
-                          (size_t)bh * sq + q0 + wave * 32, qlen - wave * 32, lane);
-            return true;
-        }
-    }
+    uint16_t* out = p.out_bf16;
+    asm volatile("" : "+s"(out));   // (fetched now, see flash_item)
     // first key of walk position e; positions past the end repeat the last tile
     auto kv0_of = [&](int e) -> int {
         e = min(e, ne - 1);
@@ -909,9 +879,8 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     }
     const float l_tot = pair_sum(st.l_acc);
     // (through buffers 0 and 1 behind the vote, else 1 and 4, which the last P V does not read: half of one a wave)
-    store_rows<D>((FIXED ? smem + (wave >> 1) * kTileBytes : kbuf(1 + (wave >> 1))) + (wave & 1) * (kTileBytes / 2), o,
-                  l_tot > 0.f ? 1.f / l_tot : 0.f, out_f32, out_bf16, out_is_bf16, (size_t)bh * sq + q0 + wave * 32,
-                  qlen - wave * 32, lane);
+    store_rows16<D>((FIXED ? smem + (wave >> 1) * kTileBytes : kbuf(1 + (wave >> 1))) + (wave & 1) * (kTileBytes / 2), o,
+                    l_tot > 0.f ? 1.f / l_tot : 0.f, out, (size_t)bh * sq + q0 + wave * 32, qlen - wave * 32, lane);
     return true;
 }
 template <bool MASKED, int D, bool LOG2DOM>
