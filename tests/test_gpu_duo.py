@@ -160,3 +160,87 @@ def test_masked_bits_do_not_depend_on_heads_or_clip_length(fv, d, mask):
             n = blocks * mask[1]
             for h in (2, heads):
                 assert torch.equal(call(h, n), whole[:h, :n]), (blocks, h)
+
+
+def masked_call(fv, mask, q, k, v, **kw):
+    entry = fv.sdpa_block_causal_bf16 if mask[0] == "causal" else fv.sdpa_vdn_window_bf16
+    return entry(q, k, v, *mask[1:], out_bf16=True, **kw)
+
+
+def masked64(fv, torch, mask, q, k, v, scale=None):
+    """The f64 softmax under the mask; rows that see no key are zeros."""
+    spec = fv.BlockCausal(*mask[1:]) if mask[0] == "causal" else fv.VdnWindow(*mask[1:])
+    sq, sk = q.shape[1], k.shape[1]
+    shut = torch.from_numpy(np.asarray(spec.dense_mask(sq, sk)).reshape(sq, sk) < -1e8).cuda()
+    scale = 1.0 / np.sqrt(q.shape[-1]) if scale is None else scale
+    want = torch.empty(q.shape, dtype=torch.float64, device=q.device)
+    for b in range(q.shape[0]):
+        x = ((q[b].double() @ k[b].double().T) * scale).masked_fill(shut, float("-inf"))
+        want[b] = torch.softmax(x, -1).nan_to_num(0.0) @ v[b].double()
+    return want
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("mask", [None, ("causal", 100, 0, 0), ("causal", 100, 3, 1), ("window", 10, 70, 9, 3, 1)])
+def test_the_scale_folded_into_the_queries(fv, d, mask):
+    """scale = ln 2 takes the form without the multiply of every score, and is counted."""
+    import torch
+
+    announce(f"duo log2 d={d} {mask}")
+    ln2 = float(np.float32(np.log(2.0)))
+    g = torch.Generator(device="cuda").manual_seed(d)
+    heads, s = (60, 650) if mask else (HEADS, 140)
+    q, k, v = (torch.randn((heads, s, d), generator=g, device="cuda") for _ in range(3))
+    q, k, v = (x.to(torch.bfloat16) for x in (q * (1.4426950408889634 / np.sqrt(d)), k, v))
+    n0 = fv.lib().fv_sdpa_log2_domain_launches()
+    got = masked_call(fv, mask, q, k, v, scale=ln2) if mask else fv.sdpa_dense_bf16(q, k, v, scale=ln2, out_bf16=True)
+    assert fv.lib().fv_sdpa_log2_domain_launches() == n0 + 1
+    want = masked64(fv, torch, mask or ("causal", s, 0, 0), q, k, v, ln2)
+    assert ((got.double() - want).norm() / want.norm()).item() <= 2 * 2.0 ** -9
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("mask", [("causal", 100, 0, 0), ("causal", 100, 3, 1), ("window", 0, 70, 10, 3, 1)])
+def test_masked_reruns(fv, d, mask):
+    """One head's keys past the first 128 score hundreds of base-2 units above those: all its workgroups of 128 queries go
+    again (each sees some of them), under their masks, and no other head's."""
+    import torch
+
+    announce(f"duo masked reruns d={d} {mask}")
+    heads, s = 60, 700
+    g = torch.Generator(device="cuda").manual_seed(7 * d)
+    q, k, v = (torch.randn((heads, s, d), generator=g, device="cuda") for _ in range(3))
+    plain = masked_call(fv, mask, *(x.to(torch.bfloat16) for x in (q, k, v)))
+    q[0] = q[0].abs() + 2.0
+    k[0, :128] = -0.5
+    k[0, 128:] = torch.linspace(4.0, 40.0, s - 128, device="cuda")[:, None]
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    n0 = fv.lib().fv_sdpa_exact_pass_reruns()
+    got = masked_call(fv, mask, q, k, v)
+    torch.cuda.synchronize()
+    assert fv.lib().fv_sdpa_exact_pass_reruns() - n0 == (s + 127) // 128
+    assert torch.equal(got[1:], plain[1:])
+    want = masked64(fv, torch, mask, q[:1], k[:1], v[:1])
+    assert (got[:1].double() - want).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("sq,sk,mask", [(500, 300, (90, 0, 0)), (300, 500, (90, 0, 0)), (500, 200, (70, 2, 1)), (513, 129, (128, 1, 1)),
+                                        (500, 200, (70, 2, 0)), (513, 129, (128, 1, 0))])
+def test_more_queries_than_keys_and_fewer(fv, sq, sk, mask, d):
+    """Causal calls of many heads on rectangles, every row written; a row that sees no key (a window past the last one, no
+    sink) is zeros."""
+    import torch
+
+    announce(f"duo causal {sq}x{sk}x{d} {mask}")
+    heads = 60
+    g = torch.Generator(device="cuda").manual_seed(sq + sk + d)
+    q, k, v = (torch.randn((heads, s, d), generator=g, device="cuda").to(torch.bfloat16) for s in (sq, sk, sk))
+    out = torch.full((heads, sq, d), float("nan"), device="cuda", dtype=torch.bfloat16)
+    got = masked_call(fv, ("causal", *mask), q, k, v, out=out)
+    want = masked64(fv, torch, ("causal", *mask), q, k, v)
+    empty = ~want.abs().amax(-1).gt(0)
+    assert empty.any() == (mask[2] == 0 and mask[1] > 0)
+    assert not got[empty].any()
+    rows = (got.double() - want).norm(dim=-1)[~empty] / want.norm(dim=-1)[~empty]
+    assert rows.max().item() <= 2.0 ** -7

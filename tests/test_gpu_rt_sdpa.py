@@ -447,7 +447,8 @@ def test_first_use_of_a_kernel_on_a_shape_is_logged_once():
 
 @pytest.mark.parametrize("d", [128, 64])
 @pytest.mark.parametrize("h,sq,sk", [(1, 1, 1), (2, 127, 63), (1, 128, 64), (3, 129, 65), (2, 255, 129), (5, 257, 700),
-                                     (40, 769, 200), (128, 256, 130), (129, 130, 90), (4, 390, 2000)])
+                                     (40, 769, 200), (128, 256, 130), (129, 130, 90), (4, 390, 2000),
+                                     (3, 129, 4100), (4, 390, 4500), (200, 100, 6200), (200, 128, 6145)])   # past the short kernel
 def test_small_launches_take_half_tiles(fv, h, sq, sk, d):
     """Query tiles of 128 instead of 256 where each has a CU to itself: the same rows bit for bit, for both result
     types, ragged tiles, split keys, and a row that outgrows the fixed offset."""
