@@ -681,7 +681,7 @@ __global__ __launch_bounds__(64 * composed_waves(KS), 2) void sdpa_composed_kern
 // next K tile while the softmax runs, the next V tile behind the products. PP: parts of P, 3 for the composed plans
 // (masks, head dims in steps of 8, exact P), 1 for the fused kernels' plans (P rounded to bf16, no mask, head dims 64
 // and 128). Shader-clock stamps at 12 x 320 x 320 x 128, 13 k cycles: arguments 0.6, issue of 17 loads a wave
-// 1.6 (136 KB at 64 bytes a clock), query rows and K 2.2, two tiles 4.3, merge 3.8 (128 KB written, 128 KB read), drain
+// 1.6, query rows and K 2.2, two tiles 4.3, merge 3.8 (128 KB written, 128 KB read), drain
 // 0.5. us, in a graph, the kernels it replaces / this: 12 x 320 x 320 x 128 11.0 / 6.8 (flash_fwd_pp2, 24 k cycles in five phases),
 // 16 x 257 x 257 x 80 10.2 / 7.8, 12 x 668 x 668 x 128 17.8 / 9.7, 12 x 1200 x 1200 x 64 19.5 / 12.9.
 template <int NC>
@@ -1117,12 +1117,15 @@ extern "C" hipError_t fv_internal_launch_composed(const fv::ComposedParams* para
     p.vec = (any & 15) == 0 && d % 8 == 0;
     const int parts = kv_is_bf16 || round16 ? 1 : 3;
     // 1024 groups are one wave on every SIMD of the chip: below two waves (one with three parts, whose second share of
-    // the tiles leaves room for one workgroup per CU) the keys are shared out over a workgroup's waves. One part, bf16,
-    // us with 1 / 2 / 4 / 8 shares: 64 x 1024 x 300 x 80 (2048 groups) 33 / 39 / 56 / 83, 64 x 512 x 512 x 64 (1024)
-    // 28 / 24 / 27 / 38, 24 x 300 x 300 x 80 (240) 18.8 / 13.6 / 12.0 / 11.1, 16 x 257 x 257 x 80 (144) 15.6 / 12.4 / 11.0
-    // / 10.2, 12 x 200 x 200 x 64 (84, seven tiles) 12.2 / 10.1 / 10.0 / 10.4. Three parts, 1 / 2 shares: 64 x 3000 x 700 x
-    // 80 (6016) 284 / 331, 12 x 4096 x 4096 x 128 (1536) 606 / 1459, 24 x 1024 x 1024 x 64 (768) 71 / 62. Four and eight
-    // shares take the registers of whole tiles in flight: bf16 keys up to 96 channels only (f32 keys, 12 x 700 x 700 x
+    // the tiles leaves room for one workgroup per CU) the keys are shared out over a workgroup's waves. bf16 keys, us with 1 /
+    // 2 / 4 / 8 shares: 64 x 1024 x 300 x 80 (2048 groups) 33 / 39 / 56 / 83, 64 x 512 x 512 x 64 (1024) 28 / 24 / 27 / 38. Four and
+    // eight are left for what the short kernel (below) does not take: f32 queries on bf16 keys 16 x 257 x 257 x 80 (144) 15.9 /
+    // 12.4 / 10.4 / 9.6, 24 x 300 x 300 x 80 (240) 17.2 / 12.6 / 10.8 / 10.0, 24 x 500 x 500 x 80 (384) 24.3 / 17.3 / 16.5 / 20.5;
+    // rows that are no whole 16-byte units 16 x 257 x 257 x 76 40.0 / 32.0 / 34.5 / 28.7, 12 x 500 x 500 x 76 (192) 63.5 / 46.1 / 44.3 / 30.9,
+    // 12 x 200 x 200 x 60 (84) 21.4 / 20.0 / 18.2 / 14.5, 24 x 500 x 500 x 76 64 / 47 / 51 / 59; unaligned ones 24 x 300 x 300 x 80 46.7
+    // / 34.5 / 37.1 / 34.4, 24 x 500 x 500 x 80 67 / 49 / 57 / 69 (the line does not follow the alignment). Three parts, 1 / 2
+    // shares: 64 x 3000 x 700 x 80 (6016) 284 / 331, 12 x 4096 x 4096 x 128 (1536) 606 / 1459, 24 x 1024 x 1024 x 64 (768) 71 / 62. Four
+    // and eight shares take the registers of whole tiles in flight: bf16 keys up to 96 channels only (f32 keys, 12 x 700 x 700 x
     // 112: 39 / 29 / 61, with spills).
     // Between 1024 and 2047 groups, bf16, one / two shares: 12 x 4096 x 4096 x 64 (1536) 189 / 158, 64 x 700 x 700 x 64
     // (1408) 41.5 / 34.5, 40 x 1000 x 300 x 80 (1280) 26.4 / 23.9, 12 x 3000 x 1024 x 64 (1128) 53.2 / 43.6; but at 128

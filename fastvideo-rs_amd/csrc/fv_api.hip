@@ -337,9 +337,10 @@ FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf
     if (wgs < cus || cus % 8 != 0 || wgs > (size_t)INT_MAX / 64) {
         const size_t splits = fv_sdpa_splitkv_choose(bh, sq, sk);
         // Query tiles of 128 where each still has a CU to itself. Measured on MI355X, 256 / 128 queries a workgroup, us:
-        // 12 x 320 x 320 x 128 13.2 / 11.3, 12 x 1000 x 1000 x 128 25.6 / 23.0, 40 x 700 x 700 x 64 17.4 / 14.8, 12 x 1560 x
-        // 512 x 128 17.2 / 14.9, 24 x 390 x 2000 x 128 at 2 splits 34.2 / 29.7; past one per CU, 12 x 4000 x 512 x 128 20.3 /
-        // 29.1, 40 x 1000 x 1000 x 64 (320 tiles) 21.5 / 21.7.
+        // bf16 results past the short kernel's walks and past flash_fwd_duo's 200 x 100 x 2000 x 128 52.1 / 41.8, 200 x 100 x
+        // 8000 x 64 146 / 103, 4 x 390 x 8000 x 128 split 31.8 / 28.7, 24 x 390 x 4000 x 128 39.4 / 38.9; f32 results 12 x 1000 x
+        // 1000 x 128 split 27.2 / 25.3, 40 x 700 x 700 x 64 17.6 / 15.0, 12 x 320 x 600 x 128 18.1 / 15.9, 24 x 390 x 2000 x 128 26.8 / 27.0; past one per CU, 12 x 4000 x
+        // 512 x 128 20.3 / 29.1, 40 x 1000 x 1000 x 64 (320 tiles) 21.5 / 21.7.
         if (splits == 1 && fv_duo(bh, sq, sk, d, out_bf16)) return {bm, 0, 1, 0};
         const size_t half = bm / 2, small = bh * ((sq + half - 1) / half) * settle_splits(nkt, splits);
         return {small <= cus ? half : bm, 0, splits, fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits)};

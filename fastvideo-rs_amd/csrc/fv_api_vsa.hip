@@ -381,7 +381,7 @@ static int vsa_attention_common(const void* q, const void* k, const void* v, int
     p.slot_src = slot_src;
     p.seq = (long)seq;
     // 3. top-k tiles per query tile (rt/vsa.rs:398-400); the same launch clears the fine kernel's counters, which take the
-    //    place of the query means (fewer words than those: a line per 64 key tiles and 128 query tiles)
+    //    place of the query means (fewer words than those: 32 per 2048 key tiles and gang of workgroups; a tile has 128 means)
     const size_t words = fv_internal_fine_pace(&p);
     p.pace = words > 0 && words <= bh * num_tiles * dim ? (int*)qc : nullptr;
     e = fv_internal_launch_topk(scores, sel, (int)(bh * num_tiles), (int)num_tiles, (int)topk, p.pace, p.pace ? (int)words : 0, st);
