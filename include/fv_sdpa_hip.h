@@ -60,7 +60,7 @@ int fv_sdpa_is_log2_domain_scale(float scale);
 uint64_t fv_sdpa_log2_domain_launches(void);
 
 /* No counterpart in the reference (a diagnostic). Launches that write bf16 and in which every query sees key 0
- * (dense; block-causal without a window or with sink blocks; the VDN window) make their pass over the keys with every
+ * (dense ones but the smallest, see fv_sdpa_dense_bf16; block-causal without a window or with sink blocks; the VDN window) make their pass over the keys with every
  * query's softmax offset fixed at the largest score of its first 128 keys (no running max in the loop), check the row sums
  * and accumulators before anything is stored, and make the pass again with the running max in any workgroup where
  * a row's scores outgrew that offset by more than about 2^90: results are exact either way, the second pass only
@@ -75,8 +75,10 @@ uint64_t fv_sdpa_exact_pass_reruns(void);
  * Rounding: with out_is_bf16 == 0 every row follows its running maximum (its largest P is exactly 1); with
  * out_is_bf16 == 1 the softmax offset of a row is the largest score of its first 128 keys (see
  * fv_sdpa_exact_pass_reruns), so a row that one later key dominates carries that key's bf16-rounded P: up to 2^-8
- * relative on such a row, beside the 2^-8 of the result's own rounding. FASTVIDEO_SDPA_RUNNING_MAX=1 (read once)
- * keeps the running maximum in every launch. */
+ * relative on such a row, beside the 2^-8 of the result's own rounding. Calls of few query groups and up to 512 keys
+ * (fv_rt_sdpa: up to 3072 for a bf16 result, at head dim 64 4000) come from a kernel whose waves share the keys out, each with
+ * a running maximum over its own: no fixed offset and no second pass there, for either result type.
+ * FASTVIDEO_SDPA_RUNNING_MAX=1 (read once) keeps the running maximum in every launch. */
 int fv_sdpa_dense_bf16(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,
                        int out_is_bf16, size_t bh, size_t sq, size_t sk, size_t d, float scale,
                        void* stream);
@@ -138,7 +140,10 @@ int fv_sdpa_dense_bf16_splitkv_static(const uint16_t* q, const uint16_t* k, cons
  * stores for a row without a visible key (kernels/attn2.cu:150); its composed route with the additive -1e9 mask
  * (rt/attn.rs:455-467) would give such a row the mean of V. No reference fixture covers the case: parity unpinned.
  * Rounding of bf16 results as for fv_sdpa_dense_bf16 when every query sees key 0 (window == 0 or sink > 0); under a
- * window without a sink every row follows its running maximum. */
+ * window without a sink every row follows its running maximum. One block that spans both sequences is the call of
+ * fv_sdpa_dense_bf16, bit for bit. The first n blocks of a clip have the bits of the clip of n blocks, and a head those of a
+ * call on it alone, but for rows beside one that outgrows the fixed offset (fv_sdpa_exact_pass_reruns) and for clips of one
+ * block of up to 512 tokens (dense calls that the kernel for few query groups may take). */
 int fv_sdpa_block_causal_bf16(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,
                               int out_is_bf16, size_t bh, size_t sq, size_t sk, size_t d,
                               float scale, size_t block_tokens, size_t window, size_t sink,
