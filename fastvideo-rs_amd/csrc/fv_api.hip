@@ -258,7 +258,7 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         const hipError_t e = fv_internal_launch_short(&c, short_waves, bh, (hipStream_t)stream);
         return e == hipSuccess ? FV_OK : fail_hip(e, "sdpa_short");
     }
-    if (mode == kMaskNone ? splits == 1 && fv_duo(bh, sq, sk, d, out_is_bf16) : duo_masked(p, bh, d)) {
+    if (mode == kMaskNone ? splits == 1 && fv_duo(bh, sq, sk, d, out_is_bf16, false) : duo_masked(p, bh, d)) {
         p.nqt = (int)((sq + 127) / 128);
         p.total = (int)(bh * (size_t)p.nqt);
         p.per_xcd = (p.total + 7) / 8;
@@ -314,13 +314,15 @@ int fv_short_waves(size_t bh, size_t sq, size_t sk, size_t d) {
 // at 64 channels 16 x 4608 (32 tiles past a round) x 2000 54 / 52, x 2500 64 / 65, x 6000 129 / 147, 16 x 8704 (32 past two) x 2500
 // 103 / 102, x 6000 213 / 231, 16 x 5120 (64) x 3000 80 / 77, x 4000 99 / 101; at 128 16 x 4608 x 1300 70 / 66, x 1500 71 / 74,
 // 16 x 8960 (48) x 1350 109 / 104, x 1500 113 / 113. (Of a sixteenth or less: at any length, this kernel would pay a round for them.)
+// Where it cannot be split (no workspace, or an entry without one), flash_fwd_pp2 pays two whole rounds: 24 x 3000 x 6100 x 64
+// 176 / 149, 24 x 3000 x 1500 x 128 77 / 71, 16 x 8960 x 1500 x 128 123 / 116.
 // Few query tiles have a CU each, of 128 queries where fv_split_plan says so. f32 results follow the running max, whose
 // rescales go by pairs of tiles in flash_fwd_pp2: they stay there, and a block's result does not depend on the clip's length.
-bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16) {
+bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16, bool may_split) {
     const size_t cus = (size_t)fv_compute_units(), bm = (size_t)fv_internal_flash_block_m(), wgs = bh * ((sq + bm - 1) / bm);
     const size_t rest = wgs > cus ? wgs % cus : 0;   // tiles of the last round that flash_fwd_pp2 would split
     size_t most = d == 64 ? 6144 : 1536;
-    if (rest > 0 && rest <= cus / 4) most = d == 128 ? 1408 : rest <= cus / 8 ? 2304 : 3072;
+    if (may_split && rest > 0 && rest <= cus / 4) most = d == 128 ? 1408 : rest <= cus / 8 ? 2304 : 3072;
     if (rest > 0 && rest <= cus / 16) most = 0;
     return fv_internal_fixed_offset(out_bf16) && sk <= most && bh * ((sq + 127) / 128) > cus / 2;
 }
@@ -341,12 +343,12 @@ FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf
         // 8000 x 64 146 / 103, 4 x 390 x 8000 x 128 split 31.8 / 28.7, 24 x 390 x 4000 x 128 39.4 / 38.9; f32 results 12 x 1000 x
         // 1000 x 128 split 27.2 / 25.3, 40 x 700 x 700 x 64 17.6 / 15.0, 12 x 320 x 600 x 128 18.1 / 15.9, 24 x 390 x 2000 x 128 26.8 / 27.0; past one per CU, 12 x 4000 x
         // 512 x 128 20.3 / 29.1, 40 x 1000 x 1000 x 64 (320 tiles) 21.5 / 21.7.
-        if (splits == 1 && fv_duo(bh, sq, sk, d, out_bf16)) return {bm, 0, 1, 0};
+        if (splits == 1 && fv_duo(bh, sq, sk, d, out_bf16, false)) return {bm, 0, 1, 0};
         const size_t half = bm / 2, small = bh * ((sq + half - 1) / half) * settle_splits(nkt, splits);
         return {small <= cus ? half : bm, 0, splits, fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits)};
     }
     const size_t full = wgs / cus * cus, rest = wgs - full;
-    if (rest == 0 || fv_duo(bh, sq, sk, d, out_bf16)) return {bm, 0, 1, 0};
+    if (rest == 0 || fv_duo(bh, sq, sk, d, out_bf16, true)) return {bm, 0, 1, 0};
     const size_t rows = bh * sq - (full / nqt * sq + full % nqt * bm);
     // us, measured: a workgroup's fixed part, and a 64-key tile while `w` workgroups run (16 x 4000 x 4000 x 128, 256
     // tiles: 121 us, half of them 79); partials written and read at 4 TB/s and a launch

@@ -169,8 +169,8 @@ struct FvSplitPlan {
 FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16);
 // Waves a workgroup of the short kernel where a dense call of this shape that writes bf16 takes it, else 0.
 int fv_short_waves(size_t bh, size_t sq, size_t sk, size_t d);
-// whether an unsplit dense launch takes the kernel with two workgroups a CU
-bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16);
+// whether an unsplit dense launch takes the kernel with two workgroups a CU; may_split: where its last round could be split
+bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16, bool may_split);
 // fv_sdpa_dense_bf16_splitkv with such a plan
 int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out, int out_is_bf16, size_t bh,
                      size_t sq, size_t sk, size_t d, float scale, size_t q_rows, size_t k_rows, size_t v_rows,

@@ -244,3 +244,26 @@ def test_more_queries_than_keys_and_fewer(fv, sq, sk, mask, d):
     assert not got[empty].any()
     rows = (got.double() - want).norm(dim=-1)[~empty] / want.norm(dim=-1)[~empty]
     assert rows.max().item() <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("d,sk", [(64, 3100), (128, 1500)])
+def test_a_last_round_that_cannot_be_split(fv, d, sk):
+    """32 query tiles past a round of the CUs, on a walk long enough for their keys to be shared out: the plain entry, which
+    has no workspace for it, takes workgroups of 128 queries (a head of 200 that outgrows its offset is two of them); the bits
+    are those of fewer heads."""
+    import torch
+
+    heads, sq = 288, 200
+    announce(f"duo last round {heads}x{sq}x{sk}x{d}")
+    g = torch.Generator(device="cuda").manual_seed(d)
+    q, k, v = (torch.randn((heads, s, d), generator=g, device="cuda") for s in (sq, sk, sk))
+    q[0] = q[0].abs() + 2.0
+    k[0, 128:] = k[0, 128:].abs() + 8.0
+    k[0, :128] = -0.5
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    n0 = fv.lib().fv_sdpa_exact_pass_reruns()
+    got = fv.sdpa_dense_bf16(q, k, v, out_bf16=True)
+    torch.cuda.synchronize()
+    assert fv.lib().fv_sdpa_exact_pass_reruns() == n0 + 2
+    few = fv.sdpa_dense_bf16(*(x[200:260].contiguous() for x in (q, k, v)), out_bf16=True)
+    assert torch.equal(few, got[200:260])
