@@ -725,7 +725,7 @@ __global__ __launch_bounds__(64 * KS, NC <= 4 ? 4 : 2) void sdpa_short_kernel(co
     // One instruction's rows of a tile of `rows` valid ones (the ones past them re-read the last): whole 16-byte chunks of
     // the row, each to its swizzled place; lanes whose chunk lies past d fetch nothing. Every instruction has lanes that do.
     auto request_one = [&](lds_u8* dst, const char* base, int rows, int it_, bool is_v) {
-        const int r = it_ * G::kRowsPerDma + lr, c = lc ^ (is_v ? G::vswz(r) : G::kswz(r));
+        const int r = it_ * G::kRowsPerDma + lr, c = lc ^ (is_v ? G::vswz32(r) : G::kswz(r));
         const unsigned at = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst) + it_ * 1024;
         const unsigned off = (unsigned)(min(r, rows - 1) * rowb + (c << 4));
         if (PP == 1 || c < nch) lds_dma16_s(at, base, off);
@@ -760,7 +760,7 @@ __global__ __launch_bounds__(64 * KS, NC <= 4 ? 4 : 2) void sdpa_short_kernel(co
     else wait_vmcnt<0>();
     __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the zeros are written
     block_barrier();
-    const TileReadBases rb = tile_read_bases<SG::D>(lane);
+    const TileReadBases rb = tile_read_bases32<SG::D>(lane);
     const float q_mul = PP == 3 ? composed_q_mul(p) : 1.f, to_log2 = LOG2DOM ? 1.f : composed_to_log2(p);
     bf16x8 qf[NC];
 #pragma unroll

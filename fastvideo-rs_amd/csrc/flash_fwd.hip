@@ -9,11 +9,16 @@
 // Schedule (not a translation of the CUDA one):
 //   * one workgroup = 8 waves = 256 queries of one (batch, head); each wave
 //     owns 32 queries and walks the keys in tiles of 64;
-//   * the wave computes S^T = K Q^T with v_mfma_f32_32x32x16_bf16: K rows come
-//     from LDS as the A operand, Q^T stays in registers as the B operand for
-//     the whole kernel. In the 32x32 accumulator layout every lane then holds
-//     32 scores of ONE query, so the row max / row sum are in-lane reductions
-//     plus one exchange with lane^32;
+//   * the wave computes S^T = K Q^T with v_mfma_f32_16x16x32_bf16: K rows come
+//     from LDS as the A operand, each fragment for two MFMAs, Q^T stays in registers as the B operand for
+//     the whole kernel. In the 16x16 accumulator layout every lane then holds
+//     16 scores of each of TWO queries, so row maxima and row sums are in-lane reductions
+//     plus exchanges with lane^32 and lane^16. The shape is a matter of power, at whose limit long launches run: on
+//     random operands the chip sustains 2.01 PFLOP/s of it from registers and 1.74 with this kernel's LDS reads,
+//     1.73 and 1.52 of v_mfma_f32_32x32x16_bf16 on the same operands (on zeros both 2.45). Its MFMAs are twice as many
+//     and take the SIMD's issue port twice as long, so everything else in a phase had to shrink with it. Together, against
+//     the 32x32 form: 12 x 32760 x 32760 x 128 5.34 -> 4.76 ms, 40 x 75600 92.3 -> 84.7, block-causal 21 x 1560
+//     2.91 -> 2.67, 24 x 7800 x 7800 x 64 366 -> 344 us;
 //   * P^T (bf16, RNE) is the B operand of O^T = V^T P^T straight from those
 //     registers (the contraction index is a fixed permutation of the keys,
 //     matched on the V side); V^T fragments are read from the row-major
@@ -31,14 +36,14 @@
 //     construction. Interleaving the two instruction kinds inside one wave
 //     loses on this hardware: a wave issues in order, so its VALU work stalls
 //     behind every MFMA that waits for the matrix pipe;
-//   * K/V tiles go global -> LDS directly (global_load_lds_dwordx4) into
-//     XOR-swizzled unpadded tiles, four buffers each;
+//   * K/V tiles go global -> LDS directly (buffer_load_dwordx4 ... lds) into
+//     XOR-swizzled unpadded tiles, four buffers each; rows past the last key are the descriptor's business;
 //   * dense launches remap workgroup ids so that the workgroups resident on one
 //     XCD walk consecutive query tiles of the same head (their K/V stream hits
 //     that XCD's L2); block-causal launches run longest tiles first.
 //
 // Time is counted in slots (one phase each); a phase covers a PAIR of key tiles
-// (128 keys): a matrix phase is 64 MFMAs (PV of the previous pair, QK of the
+// (128 keys): a matrix phase is 128 MFMAs (PV of the previous pair, QK of the
 // current pair), a VALU phase the softmax of the pair with one shared max /
 // rescale decision. Barriers, the LDS-latency ramp at the head of a matrix phase
 // and the per-phase bookkeeping are thus paid once per 128 keys. Group 0 runs
@@ -46,10 +51,11 @@
 // behind. K and V tiles rotate through 4 LDS buffers each (128 KB): matrix phase
 // m reads K(2m), K(2m+1), V(2m-2), V(2m-1) and issues K(2m+2), K(2m+3), V(2m),
 // V(2m+1) into the buffers phase m-1 read last, all of them during the first tile
-// of the pair (a load needs more than a thousand cycles to land), from descriptors
-// (addresses, tail clamp) prepared in the VALU phase before, so the matrix phase
-// carries bare DMA instructions and no branches (a branch inside the unrolled phase breaks the
-// register allocation of the 16-register accumulator tuples: 59 spills measured).
+// of the pair (a load needs more than a thousand cycles to land), at offsets worked out in the VALU phase before, so the
+// matrix phase carries bare DMA instructions and no branches. The VALU phase, in turn, is kept to the softmax itself: the
+// other wave's MFMAs leave it about half the issue slots, and every scalar instruction and branch in it counts (the masks
+// are asked by position of the walk, WalkSight; with per-lane tests, clamps and 64-bit addresses block-causal launches
+// were 5 % slower than in the 32x32 form instead of 9 % faster).
 // Every wave waits for its own loads at the end of the same phase, one barrier
 // before phase m+1 of either group reads them. Phase 0 has no previous pair and runs its QK half only
 // (unrolled apart from the loop). An odd tile count is rounded up: the extra
@@ -130,23 +136,78 @@ FV_DEV LaneMask lane_mask(const Params& p, int qi) {
     return m;
 }
 
+// The walk positions at which each of a wave's 32 queries sees every key, from scalars, once per walk: e < a, w0 <= e < w1 or
+// e >= c. At the others the lanes ask key by key; those are the few that a range's ends or a frame boundary among the
+// queries cut (and the last, where the keys may end).
+struct WalkSight {
+    int a, w0, w1, c;
+    FV_DEV bool all(int from, int to) const { return (to < a) | ((from >= w0) & (to < w1)) | (from >= c); }
+};
+template <class Params>
+FV_DEV WalkSight walk_sight(const Params& p, const TileWalk& w, int first) {
+    int last = first + 31;
+    if (p.mask_mode == 2) {   // the rows of inner frames among them: the others see every key
+        first = max(first, p.vs + p.ft);
+        last = min(last, p.ve - p.ft - 1);
+        if (first > last) return {0x7fffffff, 0, 0, 0x7fffffff};
+    }
+    const LaneMask m0 = lane_mask(p, first), m1 = lane_mask(p, last);   // (both bounds of a window rise with the query)
+    const int w_lo = max(m0.w_lo, m1.w_lo), w_hi = min(m0.w_hi, m1.w_hi);
+    WalkSight s;
+    s.a = min(w.n0, m0.a_hi / kBN);
+    s.w0 = w.n0 + max(0, (w_lo + kBN - 1) / kBN - w.a1);
+    s.w1 = w.n0 + min(w.n1, w_hi / kBN - w.a1);
+    s.c = m0.c_lo == 0x7fffffff ? 0x7fffffff : w.n0 + w.n1 + max(0, (m0.c_lo + kBN - 1) / kBN - w.a2);
+    return s;
+}
+// The kernel's arguments read again from their segment, of which FlashParams is the whole: for code that runs rarely, so
+// that the loop around it keeps none of them in registers.
+using ConstParams = const __attribute__((address_space(4))) FlashParams;
+FV_DEV ConstParams* params_again() {
+    ConstParams* again = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(again));
+    return again;
+}
+// Scores of query block g that the lane's query may not see to -inf, and those of keys `left` and on; `key`: the tile's first
+// key + 4 (lane / 16), `left` counted from it.
+FV_DEV void mask_scores(ScoreTile& s, int g, const LaneMask& m, int key, int left) {
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int x = key + 16 * kb + i;
+            const bool vis = ((x < m.a_hi) | (x >= m.c_lo) | ((x >= m.w_lo) & (x < m.w_hi))) & (16 * kb + i < left);
+            s[kb][g][i] = vis ? s[kb][g][i] : neg_inf();
+        }
+}
+FV_DEV void mask_keys(ScoreTile& s, int left) {
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const bool vis = 16 * kb + i < left;
+            s[kb][0][i] = vis ? s[kb][0][i] : neg_inf();
+            s[kb][1][i] = vis ? s[kb][1][i] : neg_inf();
+        }
+}
+
 // A wave's 32 rows o * inv in bf16, the first of them row `row0` of the result; `rows` (and no more) are stored. `my`:
 // 32 x 2D bytes of LDS of the wave's own: scattered 8-byte pieces in, whole rows out, 16 bytes per lane and 1 KB (D = 128)
 // of consecutive output per store instruction.
 template <int D>
-FV_DEV void store_rows16(lds_u8* my, const f32x16 (&o)[D / 32], float inv, uint16_t* out, size_t row0, int rows, int lane) {
-    const int h = lane >> 5, c32 = lane & 31;
+FV_DEV void store_rows16(lds_u8* my, const f32x4 (&o)[D / 16][2], const float (&inv)[2], uint16_t* out, size_t row0, int rows, int lane) {
+    const int q4 = lane >> 4, i16 = lane & 15;
     constexpr int kRowB = 2 * D, kCh = kRowB / 16;
 #pragma unroll
-    for (int db = 0; db < D / 32; db++)
+    for (int db = 0; db < D / 16; db++)
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
+        for (int g = 0; g < 2; g++) {
             f32x4 r;
 #pragma unroll
-            for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
+            for (int x = 0; x < 4; x++) r[x] = o[db][g][x] * inv[g];
             const bf16x4 rb4 = __builtin_convertvector(r, bf16x4);
-            const int ch = (4 * db + g) ^ (c32 & (kCh - 1));
-            *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>(my + c32 * kRowB + (ch << 4) + 8 * h) = rb4;
+            const int ch = (2 * db + (q4 >> 1)) ^ (i16 & (kCh - 1));
+            *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>(my + (16 * g + i16) * kRowB + (ch << 4) + 8 * (q4 & 1)) = rb4;
         }
     // (same-wave LDS writes and reads complete in order; the compiler waits on the reads' data)
     constexpr int kRowsPer = 64 / kCh;           // rows one store instruction covers
@@ -172,7 +233,7 @@ FV_DEV void store_rows16(lds_u8* my, const f32x16 (&o)[D / 32], float inv, uint1
 // remains: the largest P of a row is exactly 1 under the running max and a rounded bf16 number under the fixed
 // offset, so a row that ONE late key dominates can be off by up to 2^-8 relative; the launcher therefore takes
 // this form only for results that are rounded to bf16 anyway.
-template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, class Params>
+template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, bool FAR, class Params>
 FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const int block) {
     // (masked launches: only where every query sees key 0, see launch_flash)
     using G = TileGeo<D>;
@@ -185,7 +246,7 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
 
     const int tid = wave * 64 + lane;   // (wave is scalar: branches on it stay scalar)
     const int grp = wave >> 2;
-    const int h = lane >> 5, c32 = lane & 31;
+    const int q4 = lane >> 4, i16 = lane & 15;   // this lane's queries: rows i16 and 16 + i16 of the wave's 32
     // Work order. Dense (equal tiles): workgroup i runs on XCD i % 8, and XCD x takes the
     // contiguous range [x, x+1) * per_xcd of (head, query tile) items, so its CUs stream one
     // head's K/V through its L2 together. Masked (tiles differ in length by up to the whole
@@ -240,40 +301,15 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
     // n0 + n1 + n2 = ne tiles in all. A lane's query sees key x iff
     //   x < a_hi  ||  x >= c_lo  ||  (w_lo <= x && x < w_hi).
     int a1 = 0, a2 = 0, n0 = nkt, n1 = 0, ne = nkt;
-    int a_hi = 0, c_lo = 0x7fffffff, w_lo = 0, w_hi = 0;
+    WalkSight sight = {0, 0, 0, 0};
     if constexpr (MASKED) {
-        const int qi = q0 + wave * 32 + c32;   // this lane's query (rows past sq are never stored)
         const TileWalk w = mask_tile_walk(p, q0, qlen, nkt);
         a1 = w.a1;
         a2 = w.a2;
         n0 = w.n0;
         n1 = w.n1;
         ne = w.ne;
-        // (lane_mask() written out: through the call the long masked launches took 4 % longer)
-        if (p.mask_mode == 1) {
-            // block-causal (rt/attn.rs:449-453): keys of blocks (tq - win, tq], plus the sink blocks
-            const int ft = p.ft, win = p.win;
-            const int tq = qi / ft;
-            a_hi = (int)min((long)sk, (long)p.sink * ft);
-            w_hi = (int)min((long)0x7fffffff, (long)(tq + 1) * ft);
-            w_lo = win > 0 ? max(0, tq - win + 1) * ft : 0;
-        } else {
-            // VDN window (rt/attn.rs:483-510): rows outside [vs, ve) and the frames 0 and
-            // frames-1 are dense both ways; any other frame sees the frames of its window
-            const int vs = p.vs, ve = p.ve, t = p.ft, last = p.frames - 1, c = p.chunk, r = p.radius;
-            auto lo_frame = [&](int f) { return max(0, c > 0 ? (f / c - r) * c : f - r); };
-            auto hi_frame = [&](int f) { return min(last, c > 0 ? (f / c + r + 1) * c - 1 : f + r); };
-            const bool inner_q = qi >= vs + t && qi < ve - t;
-            if (inner_q) {
-                const int qf = (qi - vs) / t;
-                a_hi = vs + t;
-                c_lo = ve - t;
-                w_lo = vs + lo_frame(qf) * t;
-                w_hi = vs + (hi_frame(qf) + 1) * t;
-            } else {
-                a_hi = 0x7fffffff;
-            }
-        }
+        sight = walk_sight(p, w, q0 + wave * 32);
     }
     if constexpr (MASKED) {
         // No key tile is visible to any query of this tile (block-causal with more queries than keys
@@ -295,32 +331,31 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         if constexpr (MASKED) return (e < n0 ? e : e < n0 + n1 ? a1 + (e - n0) : a2 + (e - n0 - n1)) * kBN;
         else return (t0 + e) * kBN;
     };
-    // tile t lives in buffer t mod 4 (t >= -2)
-    auto kbuf = [&](int t) -> lds_u8* { return smem + (t & (kRing2 - 1)) * kTileBytes; };
-    auto vbuf = [&](int t) -> lds_u8* { return smem + (kRing2 + (t & (kRing2 - 1))) * kTileBytes; };
-
-    TileDma<4 * NG, D> dma;
-    dma.init(wave, lane);
-    // tiles past the end repeat the last one
-    auto target_k = [&](int t) {
-        const int kv0 = kv0_of(t);
-        return dma.template prepare<false>(kbuf(t), Kh + (size_t)kv0 * kD, sk - kv0, wave);
-    };
-    auto target_v = [&](int t) {
-        const int kv0 = kv0_of(t);
-        return dma.template prepare<true>(vbuf(t), Vh + (size_t)kv0 * kD, sk - kv0, wave);
-    };
+    // Tile t lives in K buffer t mod 4 and V buffer t mod 4 (behind the K ring).
     using Dma = TileDma<4 * NG, D>;
-    constexpr int kIt = Dma::ITER;   // DMA instructions per wave and tile: 2 (D = 128) or 1 (D = 64); one group: twice
+    Dma dma;
+    dma.init(wave, lane);
+    constexpr int kUnits = Dma::kUnits;
+    const u32x4 kplane = plane_descriptor(Kh, FAR ? 0u : (unsigned)sk * G::kRow), vplane = plane_descriptor(Vh, FAR ? 0u : (unsigned)sk * G::kRow);
+    // (planes of 4 GB and more: a descriptor per tile)
+    auto load_k = [&](int kv0, unsigned lds, int u) {
+        if constexpr (FAR) dma.template issue<false>(plane_descriptor(Kh + (size_t)kv0 * kD, (unsigned)min(sk - kv0, kBN) * G::kRow), 0, lds, u);
+        else dma.template issue<false>(kplane, (unsigned)kv0 * G::kRow, lds, u);
+    };
+    auto load_v = [&](int kv0, unsigned lds, int u) {
+        if constexpr (FAR) dma.template issue<true>(plane_descriptor(Vh + (size_t)kv0 * kD, (unsigned)min(sk - kv0, kBN) * G::kRow), 0, lds, u);
+        else dma.template issue<true>(vplane, (unsigned)kv0 * G::kRow, lds, u);
+    };
+    const unsigned ring = (unsigned)__builtin_amdgcn_readfirstlane((int)(size_t)smem);
     {
-        const typename Dma::Prepared a0 = target_k(0), a1 = target_k(1);
+        const int k0 = kv0_of(0), k1 = kv0_of(1);
 #pragma unroll
-        for (int it = 0; it < kIt; it++) {
-            Dma::issue_prepared(a0, it);
-            Dma::issue_prepared(a1, it);
+        for (int u = 0; u < kUnits; u++) {
+            load_k(k0, ring, u);
+            load_k(k1, ring + kTileBytes, u);
         }
     }
-    bf16x8 qf[D / 16];
+    bf16x8 qf[D / 32][2];
     const TileReadBases rb = tile_read_bases<D>(lane);
     // The wave's 32 query rows come through LDS: whole rows by LDS-DMA (1 KB of consecutive global memory per
     // instruction) into the wave's own slice of the V ring (group 0: buffers 0, 1, idle until the first matrix
@@ -342,12 +377,15 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
     };
     auto q_read = [&]() {
         wait_vmcnt<0>();   // this wave's rows (and its parts of K(0), K(1)) have landed
-        const bool ok = wave * 32 + c32 < qlen;
 #pragma unroll
-        for (int dk = 0; dk < D / 16; dk++) {
-            bf16x8 t = lds_read_b128(qs + (rb.k ^ (dk << 5)));
-            if (!ok) t = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
-            qf[dk] = t;
+        for (int g = 0; g < 2; g++) {
+            const bool ok = wave * 32 + 16 * g + i16 < qlen;
+#pragma unroll
+            for (int dk = 0; dk < D / 32; dk++) {
+                bf16x8 t = lds_read_b128(qs + (rb.k ^ (dk << 6)) + 16 * g * G::kRow);
+                if (!ok) t = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+                qf[dk][g] = t;
+            }
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the slice is read before the wave passes its next barrier
     };
@@ -359,38 +397,36 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         wait_vmcnt<32 * G::kRow / 1024>();   // this wave's parts of K(0), K(1); its query rows are still in flight
     }
 
-    constexpr int kNO = D / 32;   // 32-wide d blocks of the accumulator
-    f32x16 o[kNO];
+    constexpr int kNO = D / 16;   // 16-wide d blocks of the accumulator
+    f32x4 o[kNO][2];
 #pragma unroll
     for (int db = 0; db < kNO; db++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) o[db][i] = 0.f;
+        for (int g = 0; g < 2; g++) o[db][g] = f32x4{0.f, 0.f, 0.f, 0.f};
     SoftmaxOffState st;
     st.init();
     // the C operand every S block starts from: minus the lane's softmax offset (zero until the first rescale)
-    f32x16 s_init;
+    f32x4 s_init[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    ScoreTile s0, s1;
+    ProbTile pb0, pb1;     // P of the previous pair of tiles (first read in phase 1; defined from the start)
 #pragma unroll
-    for (int i = 0; i < 16; i++) s_init[i] = 0.f;
-    f32x16 s0[2], s1[2];
-    bf16x8 pb0[4], pb1[4];     // P of the previous pair of tiles (first read in phase 1; defined from the start)
+    for (int t = 0; t < 2; t++)
 #pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-        for (int x = 0; x < 8; x++) {
-            pb0[t][x] = (__bf16)0.0f;
-            pb1[t][x] = (__bf16)0.0f;
-        }
+        for (int g = 0; g < 2; g++) pb0[t][g] = pb1[t][g] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
 
-    typename Dma::Prepared dk0 = target_k(2), dk1 = target_k(3), dv0 = target_v(0), dv1 = target_v(1);
+    // What the next matrix phase loads: V of the tiles at positions 2 m and 2 m + 1 (first keys kv[0], kv[1]), K of the two behind
+    // them (kk), and the LDS addresses of their pairs of buffers.
+    int kv[2] = {kv0_of(0), kv0_of(1)}, kk[2] = {kv0_of(2), kv0_of(3)};
+    unsigned vlds = ring + kRing2 * kTileBytes, klds = ring + 2 * kTileBytes;
     // Per-lane LDS addresses of the operand fragments of the first tile of the pair a matrix phase reads: K tiles
     // 2m, 2m+1 sit in buffers 2 (m & 1) + {0, 1}, V tiles 2m-2, 2m-1 in buffers 2 (1 - m & 1) + {0, 1}, so every
     // phase flips one bit (two tiles' worth) in each register instead of adding a buffer base to every read.
-    const lds_u8* ka[D / 16];
-    const lds_u8* va[D / 32];
+    const lds_u8* ka[D / 32];
+    const lds_u8* va[D / 16];
 #pragma unroll
-    for (int dk = 0; dk < D / 16; dk++) ka[dk] = smem + (rb.k ^ (dk << 5));
+    for (int dk = 0; dk < D / 32; dk++) ka[dk] = smem + (rb.k ^ (dk << 6));
 #pragma unroll
-    for (int db = 0; db < D / 32; db++) va[db] = smem + ((rb.v ^ (db << 6)) + (kRing2 + 2) * kTileBytes);
+    for (int db = 0; db < D / 16; db++) va[db] = smem + ((rb.v ^ (db << 5)) + (kRing2 + 2) * kTileBytes);
     // (the ring starts at LDS address 0 and spans a power of two, so flipping an address bit moves between buffers)
     auto flip = [](const lds_u8* q, unsigned bit) -> const lds_u8* {
         return (const lds_u8*)(__attribute__((address_space(3))) void*)(size_t)((unsigned)(size_t)q ^ bit);
@@ -402,36 +438,18 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         block_barrier();
     }
 
-    // scores of walk position e: keys past the end (or a position past the walk) to -inf;
-    // masked launches: keys this lane's query may not see to -inf, skipped when the whole
-    // wave sees the whole tile
-    auto mask_tile = [&](f32x16 (&s)[2], int e) {
-        const int kv0 = kv0_of(e);
-        if (e >= ne || kv0 + kBN > sk) {
-            const int lim = e >= ne ? 0 : sk;
-#pragma unroll
-            for (int b = 0; b < 2; b++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int key = kv0 + 32 * b + 8 * (i >> 2) + 4 * h + (i & 3);
-                    if (key >= lim) s[b][i] = NEG;
-                }
-        }
+    // scores of walk position e, whose first key is kv0: keys past the end (or a position past the walk) to -inf; masked
+    // launches: keys this lane's queries may not see to -inf
+    auto mask_tile = [&](ScoreTile& s, int e, int kv0) {
+        const int left = (e >= ne ? 0 : sk) - kv0 - 4 * q4;
         if constexpr (MASKED) {
-            const int kend = min(kv0 + kBN, sk);
-            const bool lane_all = kend <= a_hi || kv0 >= c_lo || (kv0 >= w_lo && kend <= w_hi);
-            if (__builtin_amdgcn_ballot_w64(!lane_all) != 0) {
 #pragma unroll
-                for (int b = 0; b < 2; b++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++) {
-                        const int key = kv0 + 32 * b + 8 * (i >> 2) + 4 * h + (i & 3);
-                        const bool vis = key < a_hi || key >= c_lo || (key >= w_lo && key < w_hi);
-                        if (!vis) s[b][i] = NEG;
-                    }
-            }
+            for (int g = 0; g < 2; g++) mask_scores(s, g, lane_mask(*params_again(), q0 + wave * 32 + 16 * g + i16), kv0 + 4 * q4, left);
+        } else {
+            mask_keys(s, left);
         }
     };
+    const bool ragged = (ne & 1) != 0 || kv0_of(ne - 1) + kBN > sk;   // keys past the end in the last phase
 
     // The first phase of a walk has no previous pair to multiply: it is unrolled apart (part 0) and runs
     // the K groups only.
@@ -444,42 +462,22 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
     for (int m = m_begin; m < m_end; m++) {
         // ---- matrix phase: group 0 in slot 2m, group 1 in slot 2m+1 ----
         __builtin_amdgcn_s_setprio(1);
-        constexpr int kAhead = MASKED ? 2 : 3;
-        const int g0 = first ? D / 16 : 0;   // the first phase starts at the K groups
-        // DMA issue slots: all of the phase's loads go out during the FIRST tile of the pair, one
-        // instruction after each of its first groups, in the order the next phase reads the tiles
-        // (V of its first tile, K of its first tile, then the second tile's). A load takes well over
+        constexpr int kAhead = 3;
+        // All of the phase's loads go out during the FIRST tile of the pair, a unit after each of its first groups, in the
+        // order the next phase reads the tiles (V of its first tile, K of its first tile, then the second tile's). A load takes well over
         // a thousand cycles to land when every CU streams K/V; issued from the second tile's groups
         // they were still in flight at the end of the phase (330 cycles of every matrix phase
         // spent in the wait below, measured with shader-clock stamps).
-        auto hook_dma = [&](int g) {
-            g -= g0;
-            // per group as many as fit all loads into the D / 16 groups of the first phase, whose walk has no PV part
-            constexpr int kPer = (4 * kIt + D / 16 - 1) / (D / 16);
-#pragma unroll
-            for (int x = g * kPer; x < g * kPer + kPer && x < 4 * kIt; x++) {
-                const int tile = x / kIt, it = x % kIt;
-                Dma::issue_prepared(tile == 0 ? dv0 : tile == 1 ? dk0 : tile == 2 ? dv1 : dk1, it);
-            }
+        auto hook_dma = [&](int i) {
+            const int x = i / kUnits, u = i % kUnits;
+            if (x >= 4) return;
+            if (x & 1) load_k(kk[x >> 1], klds + (x >> 1) * kTileBytes, u);
+            else load_v(kv[x >> 1], vlds + (x >> 1) * kTileBytes, u);
         };
-        auto hook_none = [](int) {};
-        // (dense launches address the fragments through the flipped pointers; on masked launches, whose phases
-        // read ahead less, that measured 0.6 % slower than an add per fragment, so they keep the adds)
-        if constexpr (MASKED) {
-            if (first) {
-                mfma_phase<false, kAhead, decltype(hook_dma)&, D>(vbuf(2 * m - 2), kbuf(2 * m), rb, pb0, o, qf, s0, s_init, hook_dma);
-                mfma_phase<false, kAhead, decltype(hook_none)&, D>(vbuf(2 * m - 1), kbuf(2 * m + 1), rb, pb1, o, qf, s1, s_init, hook_none);
-            } else {
-                mfma_phase<true, kAhead, decltype(hook_dma)&, D>(vbuf(2 * m - 2), kbuf(2 * m), rb, pb0, o, qf, s0, s_init, hook_dma);
-                mfma_phase<true, kAhead, decltype(hook_none)&, D>(vbuf(2 * m - 1), kbuf(2 * m + 1), rb, pb1, o, qf, s1, s_init, hook_none);
-            }
-        } else if (first) {
-            mfma_phase<false, kAhead, decltype(hook_dma)&, D>(va, ka, 0, pb0, o, qf, s0, s_init, hook_dma);
-            mfma_phase<false, kAhead, decltype(hook_none)&, D>(va, ka, kTileBytes, pb1, o, qf, s1, s_init, hook_none);
-        } else {
-            mfma_phase<true, kAhead, decltype(hook_dma)&, D>(va, ka, 0, pb0, o, qf, s0, s_init, hook_dma);
-            mfma_phase<true, kAhead, decltype(hook_none)&, D>(va, ka, kTileBytes, pb1, o, qf, s1, s_init, hook_none);
-        }
+        const ProbTile* const pbs[2] = {&pb0, &pb1};
+        ScoreTile* const ss[2] = {&s0, &s1};
+        if (first) mfma_phase<false, kAhead, 2, D>(va, ka, pbs, o, qf, ss, s_init, hook_dma);
+        else mfma_phase<true, kAhead, 2, D>(va, ka, pbs, o, qf, ss, s_init, hook_dma);
         __builtin_amdgcn_s_setprio(0);
         if constexpr (NG == 2) {
             wait_vmcnt<0>();             // this wave's loads of this phase have landed
@@ -488,24 +486,32 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         }
         __builtin_amdgcn_sched_barrier(0);
         // ---- VALU phase: group 0 in slot 2m+1, group 1 in slot 2m+2 ----
-        mask_tile(s0, 2 * m);
-        mask_tile(s1, 2 * m + 1);
+        if ((m == np - 1 && ragged) || (MASKED && !sight.all(2 * m, 2 * m + 1))) {
+            mask_tile(s0, 2 * m, kv[0]);
+            mask_tile(s1, 2 * m + 1, kv[1]);
+        }
         if (FIXED && !first) softmax_tile_pair_fixed<!LOG2DOM>(s0, s1, st, sl2, pb0, pb1);
         else softmax_tile_pair_off<!LOG2DOM, kNO>(s0, s1, st, o, s_init, sl2, pb0, pb1);
         // P and the row sum must be complete before the barrier: without this the
         // compiler sinks the exponentials past it, into the matrix phase
-        asm volatile("" ::"v"(pb0[0]), "v"(pb0[1]), "v"(pb0[2]), "v"(pb0[3]), "v"(pb1[0]), "v"(pb1[1]),
-                     "v"(pb1[2]), "v"(pb1[3]), "v"(st.l_acc));
-        if constexpr (!MASKED) {
+        asm volatile("" ::"v"(pb0[0][0]), "v"(pb0[0][1]), "v"(pb0[1][0]), "v"(pb0[1][1]), "v"(pb1[0][0]), "v"(pb1[0][1]),
+                     "v"(pb1[1][0]), "v"(pb1[1][1]), "v"(st.l_acc[0]), "v"(st.l_acc[1]));
 #pragma unroll
-            for (int dk = 0; dk < D / 16; dk++) ka[dk] = flip(ka[dk], 2 * kTileBytes);   // the other pair of K buffers
+        for (int dk = 0; dk < D / 32; dk++) ka[dk] = flip(ka[dk], 2 * kTileBytes);   // the other pair of K buffers
 #pragma unroll
-            for (int db = 0; db < D / 32; db++) va[db] = flip(va[db], 2 * kTileBytes);   // ... and of V buffers
-        }
-        dk0 = target_k(2 * m + 4);   // for matrix phase m+1
-        dk1 = target_k(2 * m + 5);
-        dv0 = target_v(2 * m + 2);
-        dv1 = target_v(2 * m + 3);
+        for (int db = 0; db < D / 16; db++) va[db] = flip(va[db], 2 * kTileBytes);   // ... and of V buffers
+        vlds ^= 2 * kTileBytes;
+        klds ^= 2 * kTileBytes;
+        kv[0] = kk[0];               // for matrix phase m + 1
+        kv[1] = kk[1];
+        kk[0] = kv0_of(2 * m + 4);
+        kk[1] = kv0_of(2 * m + 5);
+        // (here and not behind the barrier, at the head of the matrix phase, where the compiler would put them)
+#pragma unroll
+        for (int dk = 0; dk < D / 32; dk++) asm volatile("" : "+v"(ka[dk]));
+#pragma unroll
+        for (int db = 0; db < D / 16; db++) asm volatile("" : "+v"(va[db]));
+        asm volatile("" : "+s"(kk[0]), "+s"(kk[1]), "+s"(vlds), "+s"(klds));
         if (NG == 1 || grp == 0 || m + 1 < np) {
             __builtin_amdgcn_sched_barrier(0);
             // (one group: the only barrier of a phase, behind which its loads are resident and its tiles read)
@@ -516,8 +522,9 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
     }
     }
     // O += P V of the last pair (their V landed before the last barrier both groups passed)
-    pv_tile<D>(vbuf(2 * np - 2), rb.v, pb0, o);
-    pv_tile<D>(vbuf(2 * np - 1), rb.v, pb1, o);
+    lds_u8* const vlast = smem + (kRing2 + ((2 * np - 2) & (kRing2 - 1))) * kTileBytes;
+    pv_tile<D>(vlast, rb.v, pb0, o);
+    pv_tile<D>(vlast + kTileBytes, rb.v, pb1, o);
 
     if constexpr (FIXED) {
         // Did the fixed offset hold? Every row sum below 2^100 (its reciprocal a normal number with room to spare) and every accumulator finite
@@ -526,8 +533,10 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
 #pragma unroll
         for (int db = 0; db < kNO; db++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) chk = __builtin_fmaf(o[db][i], 0.f, chk);
-        const bool lane_ok = (pair_sum(st.l_acc) < 0x1p+100f) && (chk == 0.f);
+            for (int g = 0; g < 2; g++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) chk = __builtin_fmaf(o[db][g][i], 0.f, chk);
+        const bool lane_ok = quad_sum(st.l_acc[0]) < 0x1p+100f && quad_sum(st.l_acc[1]) < 0x1p+100f && chk == 0.f;
         auto* votes = (__attribute__((address_space(3))) unsigned*)(smem + 2 * kRing2 * kTileBytes);
         const bool wave_ok = __builtin_amdgcn_ballot_w64(!lane_ok) == 0;   // (of all lanes: outside the branch below)
         if (lane == 0) votes[wave] = wave_ok ? 0u : 1u;
@@ -545,26 +554,30 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         }
     }
 
-    const float l_tot = pair_sum(st.l_acc);
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    const int row = wave * 32 + c32;
+    float l_tot[2], inv[2];
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+        l_tot[g] = quad_sum(st.l_acc[g]);
+        inv[g] = l_tot[g] > 0.f ? 1.f / l_tot[g] : 0.f;
+    }
+    const int row = wave * 32 + i16;   // and row + 16
     if constexpr (!MASKED) {
         if (split) {
             // partial result of this split: O / l in f32 and log2 of the sum of 2^(s * sl2) it covers
-            if (row < qlen) {
-                const size_t prow = (size_t)sp * p.part_rows + ((size_t)bh * sq + q0 + row - p.part_row0);
+#pragma unroll
+            for (int g = 0; g < 2; g++) {
+                if (row + 16 * g >= qlen) continue;
+                const size_t prow = (size_t)sp * p.part_rows + ((size_t)bh * sq + q0 + row + 16 * g - p.part_row0);
                 float* po = p.part_o + prow * kD;
 #pragma unroll
-                for (int db = 0; db < kNO; db++)
+                for (int db = 0; db < kNO; db++) {
+                    f32x4 r;
 #pragma unroll
-                    for (int g = 0; g < 4; g++) {
-                        f32x4 r;
-#pragma unroll
-                        for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
-                        global_store<f32x4>(po + 32 * db + 8 * g + 4 * h, r);
-                    }
-                if (h == 0)
-                    p.part_lse[prow] = l_tot == 0.f ? NEG : st.template log2_offset<!LOG2DOM>(sl2) + __builtin_log2f(l_tot);   // (NaN stays)
+                    for (int x = 0; x < 4; x++) r[x] = o[db][g][x] * inv[g];
+                    global_store<f32x4>(po + 16 * db + 4 * q4, r);
+                }
+                if (q4 == 0)
+                    p.part_lse[prow] = l_tot[g] == 0.f ? NEG : st.template log2_offset<!LOG2DOM>(g, sl2) + __builtin_log2f(l_tot[g]);   // (NaN stays)
             }
             return true;
         }
@@ -579,13 +592,13 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
 #pragma unroll
         for (int db = 0; db < kNO; db++)
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
+            for (int g = 0; g < 2; g++) {
                 f32x4 r;
 #pragma unroll
-                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
+                for (int x = 0; x < 4; x++) r[x] = o[db][g][x] * inv[g];
                 const bf16x4 rb4 = __builtin_convertvector(r, bf16x4);
-                const int ch = (4 * db + g) ^ (c32 & (kCh - 1));
-                *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>(my + c32 * kRowB + (ch << 4) + 8 * h) = rb4;
+                const int ch = (2 * db + (q4 >> 1)) ^ (i16 & (kCh - 1));
+                *reinterpret_cast<__attribute__((address_space(3))) bf16x4*>(my + (16 * g + i16) * kRowB + (ch << 4) + 8 * (q4 & 1)) = rb4;
             }
         // (same-wave LDS writes and reads complete in order; the compiler waits on the reads' data)
         constexpr int kRowsPer = 64 / kCh;           // rows one store instruction covers
@@ -598,23 +611,19 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
                 my + rr * kRowB + ((lc ^ (rr & (kCh - 1))) << 4));
             if (wave * 32 + rr < qlen) global_store<u32x4>(ob + (size_t)rr * kD + lc * 8, val);
         }
-    } else if (row < qlen) {
-        const size_t base = ((size_t)bh * sq + q0 + row) * kD;
+    } else {
 #pragma unroll
-        for (int db = 0; db < kNO; db++)
+        for (int g = 0; g < 2; g++) {
+            if (row + 16 * g >= qlen) continue;
+            float* po = out_f32 + ((size_t)bh * sq + q0 + row + 16 * g) * kD;
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int d0 = 32 * db + 8 * g + 4 * h;
+            for (int db = 0; db < kNO; db++) {
                 f32x4 r;
 #pragma unroll
-                for (int x = 0; x < 4; x++) r[x] = o[db][4 * g + x] * inv;
-                if (out_is_bf16) {
-                    const bf16x4 rb4 = __builtin_convertvector(r, bf16x4);
-                    global_store<bf16x4>(out_bf16 + base + d0, rb4);
-                } else {
-                    global_store<f32x4>(out_f32 + base + d0, r);
-                }
+                for (int x = 0; x < 4; x++) r[x] = o[db][g][x] * inv[g];
+                global_store<f32x4>(po + 16 * db + 4 * q4, r);
             }
+        }
     }
     return true;
 }
@@ -627,23 +636,22 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
 // barrier a phase and no slot in which a group waits for the other's first or last phase: for launches whose query tiles
 // of 128 still have a CU each (fv_split_plan). Bit for bit the same rows. A phase takes 2.1 us instead of 2.4, a launch of
 // one phase 7.1 instead of 8.2.
-template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED>
+template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, bool FAR>
 __global__ __launch_bounds__(256 * NG, 2) void flash_fwd_pp2(const FlashParams p) {
     const int tid = threadIdx.x;
     int wave = __builtin_amdgcn_readfirstlane(tid >> 6), block = blockIdx.x;
     if constexpr (!FIXED) {
-        flash_item<NG, MASKED, D, LOG2DOM, false>(p, wave, tid & 63, block);
+        flash_item<NG, MASKED, D, LOG2DOM, false, FAR>(p, wave, tid & 63, block);
     } else {
-        if (flash_item<NG, MASKED, D, LOG2DOM, true>(p, wave, tid & 63, block)) return;
+        if (flash_item<NG, MASKED, D, LOG2DOM, true, FAR>(p, wave, tid & 63, block)) return;
         // The second pass shares nothing with the first but two scalars: its inputs are made opaque (the lane
         // index counted anew from the execution mask, the kernel arguments read again from their segment, of which
         // FlashParams is the whole), so that the compiler keeps no value of the first pass alive for it. It runs
         // once in a blue moon; the first pass is the kernel.
-        using ConstParams = const __attribute__((address_space(4))) FlashParams;
-        ConstParams* again = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
+        ConstParams* again = params_again();
         int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-        asm volatile("" : "+v"(lane), "+s"(wave), "+s"(block), "+s"(again));
-        flash_item<NG, MASKED, D, LOG2DOM, false>(*again, wave, lane, block);
+        asm volatile("" : "+v"(lane), "+s"(wave), "+s"(block));
+        flash_item<NG, MASKED, D, LOG2DOM, false, FAR>(*again, wave, lane, block);
     }
 }
 
@@ -662,10 +670,10 @@ template <bool MASKED, int D, bool LOG2DOM, bool FIXED, class Params>
 FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int block) {
     using G = TileGeo<D>;
     using Dma = TileDma<4, D>;
-    constexpr int kTileBytes = G::kTile, kNO = D / 32, kIt = Dma::ITER;
+    constexpr int kTileBytes = G::kTile, kNO = D / 16, kIt = Dma::ITER, kUnits = Dma::kUnits;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     lds_u8* smem = (lds_u8*)smem_raw;
-    const int h = lane >> 5, c32 = lane & 31;
+    const int q4 = lane >> 4, i16 = lane & 15;
     // work order as in flash_item: XCD x takes a contiguous eighth of the (head, query tile) items; masked, longest first
     const int work = MASKED ? block : (block & 7) * p.per_xcd + (block >> 3);
     if (work >= p.total) return true;
@@ -680,13 +688,13 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     }
     const int q0 = qt * kDuoBM, sq = p.sq, sk = p.sk, qlen = min(kDuoBM, sq - q0), nkt = (sk + kBN - 1) / kBN;
     int a1 = 0, a2 = 0, n0 = nkt, n1 = 0, ne = nkt;   // the walk, as in flash_item (key 0 is in it)
-    LaneMask lm = {0, 0x7fffffff, 0, 0};
+    WalkSight sight = {0, 0, 0, 0};
     if constexpr (MASKED) {
         const TileWalk w = mask_tile_walk(p, q0, qlen, nkt);
         a1 = w.a1, a2 = w.a2, n0 = w.n0, n1 = w.n1, ne = w.ne;
-        lm = lane_mask(p, q0 + wave * 32 + c32);
+        sight = walk_sight(p, w, q0 + wave * 32);
     }
-    const float sl2 = p.sl2, NEG = neg_inf();
+    const float sl2 = p.sl2;
     uint16_t* out = p.out_bf16;
     asm volatile("" : "+s"(out));   // (fetched now, see flash_item)
     // first key of walk position e; positions past the end repeat the last tile
@@ -705,15 +713,11 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     auto vbuf = [&](int t) -> lds_u8* { return smem + (t == 0 ? 2 : t & 1 ? 3 : 0) * kTileBytes; };
     Dma dma;
     dma.init(wave, lane);
-    auto target_k = [&](int t) {
-        const int kv0 = kv0_of(t);
-        return dma.template prepare<false>(kbuf(t), Kh + (size_t)kv0 * D, sk - kv0, wave);
-    };
-    auto target_v = [&](int t) {
-        const int kv0 = kv0_of(t);
-        return dma.template prepare<true>(vbuf(t), Vh + (size_t)kv0 * D, sk - kv0, wave);
-    };
-    bf16x8 qf[D / 16];
+    const u32x4 kplane = plane_descriptor(Kh, (unsigned)sk * G::kRow), vplane = plane_descriptor(Vh, (unsigned)sk * G::kRow);
+    auto lds_of = [](lds_u8* b) { return (unsigned)__builtin_amdgcn_readfirstlane((int)(size_t)b); };
+    auto load_k = [&](int t, int kv0, int u) { dma.template issue<false>(kplane, (unsigned)kv0 * G::kRow, lds_of(kbuf(t)), u); };
+    auto load_v = [&](int t, int kv0, int u) { dma.template issue<true>(vplane, (unsigned)kv0 * G::kRow, lds_of(vbuf(t)), u); };
+    bf16x8 qf[D / 32][2];
     const TileReadBases rb = tile_read_bases<D>(lane);
     {
         // the wave's query rows through its slice of buffers 2 and 3, as in flash_item; K(0) and K(1) besides
@@ -725,82 +729,65 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
             const int rg = min(wave * 32 + r, qlen - 1);   // rows past the end re-read the last one (zeroed below)
             lds_dma16_s(qlds + it * 1024, Qh, (unsigned)(rg * G::kRow + ((pch ^ G::kswz(r)) << 4)));
         }
-        const typename Dma::Prepared k0 = target_k(0), k1 = target_k(1);
+        const int k0 = kv0_of(0), k1 = kv0_of(1);
 #pragma unroll
-        for (int it = 0; it < kIt; it++) Dma::issue_prepared(k0, it);
+        for (int u = 0; u < kUnits; u++) load_k(0, k0, u);
         if (ne > 1) {
 #pragma unroll
-            for (int it = 0; it < kIt; it++) Dma::issue_prepared(k1, it);
+            for (int u = 0; u < kUnits; u++) load_k(1, k1, u);
             wait_vmcnt<2 * kIt>();
         } else {
             wait_vmcnt<kIt>();
         }
-        const bool ok = wave * 32 + c32 < qlen;
 #pragma unroll
-        for (int dk = 0; dk < D / 16; dk++) {
-            bf16x8 t = lds_read_b128(qs + (rb.k ^ (dk << 5)));
-            if (!ok) t = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
-            qf[dk] = t;
+        for (int g = 0; g < 2; g++) {
+            const bool ok = wave * 32 + 16 * g + i16 < qlen;
+#pragma unroll
+            for (int dk = 0; dk < D / 32; dk++) {
+                bf16x8 t = lds_read_b128(qs + (rb.k ^ (dk << 6)) + 16 * g * G::kRow);
+                if (!ok) t = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+                qf[dk][g] = t;
+            }
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the slice is read before the wave passes its next barrier
     }
-    auto mask_tile = [&](f32x16 (&s)[2], int e) {
-        const int kv0 = kv0_of(e);
-        if (kv0 + kBN > sk) {
-            const int left = sk - kv0 - 4 * h;
-#pragma unroll
-            for (int b = 0; b < 2; b++)
-#pragma unroll
-                for (int i = 0; i < 16; i++)
-                    if (32 * b + 8 * (i >> 2) + (i & 3) >= left) s[b][i] = NEG;
-        }
+    auto mask_tile = [&](ScoreTile& s, int e) {
+        if (e < ne - 1 && (!MASKED || sight.all(e, e))) return;
+        const int kv0 = kv0_of(e), left = sk - kv0 - 4 * q4;
         if constexpr (MASKED) {
-            const int kend = min(kv0 + kBN, sk);
-            const bool lane_all = kend <= lm.a_hi || kv0 >= lm.c_lo || (kv0 >= lm.w_lo && kend <= lm.w_hi);
-            if (__builtin_amdgcn_ballot_w64(!lane_all) != 0) {
 #pragma unroll
-                for (int b = 0; b < 2; b++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++) {
-                        const int key = kv0 + 32 * b + 8 * (i >> 2) + 4 * h + (i & 3);
-                        const bool vis = key < lm.a_hi || key >= lm.c_lo || (key >= lm.w_lo && key < lm.w_hi);
-                        if (!vis) s[b][i] = NEG;
-                    }
-            }
+            for (int g = 0; g < 2; g++) mask_scores(s, g, lane_mask(*params_again(), q0 + wave * 32 + 16 * g + i16), kv0 + 4 * q4, left);
+        } else {
+            if (kv0 + kBN > sk) mask_keys(s, left);
         }
     };
-    f32x16 o[kNO], s_init;
-#pragma unroll
-    for (int i = 0; i < 16; i++) s_init[i] = 0.f;
+    f32x4 o[kNO][2], s_init[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     SoftmaxOffState st;
-    bf16x8 pb[4];
+    ProbTile pb;
     constexpr int kAhead = 3;
-    typename Dma::Prepared dv = target_v(0), dk = target_v(1);
+    int kv = kv0_of(0), kk = kv0_of(1);   // first keys of the tiles that the next matrix part loads: V, K
     wait_vmcnt<0>();
     block_barrier();   // K(0), K(1) resident, every wave has its queries
     // The first two tiles have one offset, the largest score of their 128 keys: the one flash_fwd_pp2 gives them, and with
     // it the result's bits.
     {
         if (ne > 2) {
-            const typename Dma::Prepared k2 = target_k(2);
+            const int k2 = kv0_of(2);
 #pragma unroll
-            for (int it = 0; it < kIt; it++) Dma::issue_prepared(k2, it);
+            for (int u = 0; u < kUnits; u++) load_k(2, k2, u);
         }
-        f32x16 s0[2], s1[2];
-        constexpr int kPer = (kIt + D / 16 - 1) / (D / 16);
-        auto hook_v0 = [&](int g) {
-#pragma unroll
-            for (int x = (g - D / 16) * kPer; x < (g - D / 16 + 1) * kPer && x < kIt; x++) Dma::issue_prepared(dv, x);
+        ScoreTile s0, s1;
+        auto hook_v0 = [&](int i) {
+            if (i < kUnits) load_v(0, kv, i);
         };
-        auto hook_v1 = [&](int g) {
-#pragma unroll
-            for (int x = (g - D / 16) * kPer; x < (g - D / 16 + 1) * kPer && x < kIt; x++) Dma::issue_prepared(dk, x);
+        auto hook_v1 = [&](int i) {
+            if (i < kUnits) load_v(1, kk, i);
         };
         __builtin_amdgcn_s_setprio(1);
-        mfma_phase<false, kAhead, decltype(hook_v0)&, D>(vbuf(0), kbuf(0), rb, pb, o, qf, s0, s_init, hook_v0);
-        bf16x8 pa[4];
+        mfma_phase<false, kAhead, D>(vbuf(0), kbuf(0), rb, pb, o, qf, s0, s_init, hook_v0);
+        ProbTile pa;
         if (ne > 1) {
-            mfma_phase<false, kAhead, decltype(hook_v1)&, D>(vbuf(0), kbuf(1), rb, pb, o, qf, s1, s_init, hook_v1);
+            mfma_phase<false, kAhead, D>(vbuf(0), kbuf(1), rb, pb, o, qf, s1, s_init, hook_v1);
             __builtin_amdgcn_s_setprio(0);
             __builtin_amdgcn_sched_barrier(0);
             mask_tile(s0, 0);
@@ -812,43 +799,43 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
             mask_tile(s0, 0);
             softmax_first_off<!LOG2DOM>(s0, st, s_init, sl2, pa);
 #pragma unroll
-            for (int t = 0; t < 4; t++) pb[t] = pa[t];
+            for (int t = 0; t < 2; t++) pb[t][0] = pa[t][0], pb[t][1] = pa[t][1];
         }
-        asm volatile("" ::"v"(pa[0]), "v"(pa[1]), "v"(pa[2]), "v"(pa[3]), "v"(pb[0]), "v"(pb[1]), "v"(pb[2]), "v"(pb[3]), "v"(st.l_acc));
+        asm volatile("" ::"v"(pa[0][0]), "v"(pa[0][1]), "v"(pa[1][0]), "v"(pa[1][1]), "v"(pb[0][0]), "v"(pb[0][1]), "v"(pb[1][0]),
+                     "v"(pb[1][1]), "v"(st.l_acc[0]), "v"(st.l_acc[1]));
         __builtin_amdgcn_sched_barrier(0);
         wait_vmcnt<0>();
         block_barrier();   // V(0), V(1), K(2) resident, K(0) and K(1) read by every wave
 #pragma unroll
         for (int db = 0; db < kNO; db++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) o[db][i] = 0.f;
+            for (int g = 0; g < 2; g++) o[db][g] = f32x4{0.f, 0.f, 0.f, 0.f};
         __builtin_amdgcn_s_setprio(1);
         pv_tile<D>(vbuf(0), rb.v, pa, o);
-        dk = target_k(3);
-        dv = target_v(2);
+        kk = kv0_of(3);
+        kv = kv0_of(2);
         __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll 1
     for (int m = 2; m < ne; m++) {
-        f32x16 s[2];
-        auto hook_dma = [&](int g) {
-            if (g < kIt) Dma::issue_prepared(dv, g);
-            else if (g < 2 * kIt) Dma::issue_prepared(dk, g - kIt);
+        ScoreTile s;
+        auto hook_dma = [&](int i) {
+            if (i < kUnits) load_v(m, kv, i);
+            else if (i < 2 * kUnits) load_k(m + 1, kk, i - kUnits);
         };
         __builtin_amdgcn_s_setprio(1);
-        mfma_phase<true, kAhead, decltype(hook_dma)&, D>(vbuf(m - 1), kbuf(m), rb, pb, o, qf, s, s_init, hook_dma);
+        mfma_phase<true, kAhead, D>(vbuf(m - 1), kbuf(m), rb, pb, o, qf, s, s_init, hook_dma);
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
         mask_tile(s, m);
         if constexpr (FIXED) {
-#pragma unroll
-            for (int b = 0; b < 2; b++) softmax_off_block<!LOG2DOM>(s[b], st, sl2, pb[2 * b], pb[2 * b + 1]);
+            softmax_off_tile<!LOG2DOM>(s, st, sl2, pb);
         } else {
             softmax_tile_off<!LOG2DOM>(s, st, o, s_init, sl2, pb);
         }
-        asm volatile("" ::"v"(pb[0]), "v"(pb[1]), "v"(pb[2]), "v"(pb[3]), "v"(st.l_acc));
-        dk = target_k(m + 2);
-        dv = target_v(m + 1);
+        asm volatile("" ::"v"(pb[0][0]), "v"(pb[0][1]), "v"(pb[1][0]), "v"(pb[1][1]), "v"(st.l_acc[0]), "v"(st.l_acc[1]));
+        kv = kk;
+        kk = kv0_of(m + 2);
         __builtin_amdgcn_sched_barrier(0);
         wait_vmcnt<0>();
         block_barrier();   // K(m+1), V(m) resident; this phase's tiles read by every wave
@@ -863,8 +850,10 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
 #pragma unroll
         for (int db = 0; db < kNO; db++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) chk = __builtin_fmaf(o[db][i], 0.f, chk);
-        const bool lane_ok = (pair_sum(st.l_acc) < 0x1p+100f) && (chk == 0.f);
+            for (int g = 0; g < 2; g++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) chk = __builtin_fmaf(o[db][g][i], 0.f, chk);
+        const bool lane_ok = quad_sum(st.l_acc[0]) < 0x1p+100f && quad_sum(st.l_acc[1]) < 0x1p+100f && chk == 0.f;
         // (in buffer 4: its last K is behind the last barrier, and a second pass loads it behind its first)
         auto* votes = (__attribute__((address_space(3))) unsigned*)(smem + 4 * kTileBytes);
         const bool wave_ok = __builtin_amdgcn_ballot_w64(!lane_ok) == 0;
@@ -877,20 +866,24 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
             return false;
         }
     }
-    const float l_tot = pair_sum(st.l_acc);
+    float inv[2];
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+        const float l_tot = quad_sum(st.l_acc[g]);
+        inv[g] = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    }
     // (through buffers 0 and 1 behind the vote, else 1 and 4, which the last P V does not read: half of one a wave)
     store_rows16<D>((FIXED ? smem + (wave >> 1) * kTileBytes : kbuf(1 + (wave >> 1))) + (wave & 1) * (kTileBytes / 2), o,
-                    l_tot > 0.f ? 1.f / l_tot : 0.f, out, (size_t)bh * sq + q0 + wave * 32, qlen - wave * 32, lane);
+                    inv, out, (size_t)bh * sq + q0 + wave * 32, qlen - wave * 32, lane);
     return true;
 }
 template <bool MASKED, int D, bool LOG2DOM>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_fwd_duo(const FlashParams p) {
     int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), block = blockIdx.x;
     if (duo_item<MASKED, D, LOG2DOM, true>(p, wave, threadIdx.x & 63, block)) return;
-    using ConstParams = const __attribute__((address_space(4))) FlashParams;   // (as in flash_fwd_pp2)
-    ConstParams* again = (ConstParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    ConstParams* again = params_again();   // (as in flash_fwd_pp2)
     int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-    asm volatile("" : "+v"(lane), "+s"(wave), "+s"(block), "+s"(again));
+    asm volatile("" : "+v"(lane), "+s"(wave), "+s"(block));
     duo_item<MASKED, D, LOG2DOM, false>(*again, wave, lane, block);
 }
 
@@ -964,18 +957,18 @@ extern "C" int fv_internal_fixed_offset(int out_is_bf16) {
 
 namespace {
 // The kernel's dynamic LDS limit (128 KB at D = 128), once per device.
-template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED>
+template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, bool FAR>
 hipError_t flash_attr() {
     static std::atomic<unsigned long long> attr_done;
     constexpr int lds = 2 * fv::kRing2 * fv::TileGeo<D>::kTile + fv::kVoteBytes;
-    return fv_set_max_lds_once((const void*)fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED>, lds, attr_done);
+    return fv_set_max_lds_once((const void*)fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED, FAR>, lds, attr_done);
 }
-template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED>
+template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, bool FAR = false>
 hipError_t launch_flash_as(const fv::FlashParams* p, hipStream_t stream) {
     constexpr int lds = 2 * fv::kRing2 * fv::TileGeo<D>::kTile + fv::kVoteBytes;
-    hipError_t e = flash_attr<NG, MASKED, D, LOG2DOM, FIXED>();
+    hipError_t e = flash_attr<NG, MASKED, D, LOG2DOM, FIXED, FAR>();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED>), dim3(p->full + p->per_xcd * 8), dim3(256 * NG), lds, stream, *p);
+    hipLaunchKernelGGL((fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED, FAR>), dim3(p->full + p->per_xcd * 8), dim3(256 * NG), lds, stream, *p);
     return hipGetLastError();
 }
 template <bool MASKED, int D, bool LOG2DOM>
@@ -995,6 +988,8 @@ hipError_t launch_duo_as(const fv::FlashParams* p, hipStream_t stream) {
 std::atomic<unsigned long long> g_log2_domain_launches{0};
 template <int NG, bool MASKED, int D, bool FIXED>
 hipError_t launch_flash_fixed(const fv::FlashParams* p, hipStream_t stream) {
+    if constexpr (NG == 2 && !FIXED)
+        if (!fv::plane_fits<D>(p->sk)) return launch_flash_as<NG, MASKED, D, false, false, true>(p, stream);
     if (p->sl2 != 1.0f) return launch_flash_as<NG, MASKED, D, false, FIXED>(p, stream);
     g_log2_domain_launches.fetch_add(1, std::memory_order_relaxed);
     return launch_flash_as<NG, MASKED, D, true, FIXED>(p, stream);
@@ -1012,7 +1007,7 @@ bool takes_fixed_offset(const fv::FlashParams* p) {
 }
 template <int NG, bool MASKED, int D>
 hipError_t launch_flash(const fv::FlashParams* p, hipStream_t stream) {
-    return takes_fixed_offset<MASKED>(p) ? launch_flash_fixed<NG, MASKED, D, true>(p, stream) : launch_flash_fixed<NG, MASKED, D, false>(p, stream);
+    return takes_fixed_offset<MASKED>(p) && fv::plane_fits<D>(p->sk) ? launch_flash_fixed<NG, MASKED, D, true>(p, stream) : launch_flash_fixed<NG, MASKED, D, false>(p, stream);
 }
 template <bool MASKED, int D>
 hipError_t launch_duo(const fv::FlashParams* p, hipStream_t stream) {
@@ -1028,10 +1023,12 @@ hipError_t init_duo() {
 }
 template <int NG, bool MASKED, int D>
 hipError_t init_flash() {
-    hipError_t e = flash_attr<NG, MASKED, D, false, false>();
-    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, true, false>();
-    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, false, true>();
-    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, true, true>();
+    hipError_t e = flash_attr<NG, MASKED, D, false, false, false>();
+    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, true, false, false>();
+    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, false, true, false>();
+    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, true, true, false>();
+    if constexpr (NG == 2)
+        if (e == hipSuccess) e = flash_attr<NG, MASKED, D, false, false, true>();
     return e;
 }
 }  // namespace
@@ -1066,6 +1063,7 @@ extern "C" hipError_t fv_internal_launch_duo(const fv::FlashParams* p, int maske
 extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d, int block_m,
                                                hipStream_t stream) {
     const bool half = block_m == fv::kPpBM / 2;
+    if (half && !(d == 128 ? fv::plane_fits<128>(p->sk) : fv::plane_fits<64>(p->sk))) return hipErrorInvalidValue;
     if ((block_m != fv::kPpBM && !half) || (half && masked)) return hipErrorInvalidValue;
     if (d == 128)
         return masked ? launch_flash<2, true, 128>(p, stream)

@@ -180,7 +180,9 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
     p.q_plane = (long)(q_rows * d);
     p.k_plane = (long)(k_rows * d);
     p.v_plane = (long)(v_rows * d);
-    const size_t bm = m.block_m ? m.block_m : (size_t)fv_internal_flash_block_m();
+    // (planes of 4 GB and more have a kernel of whole tiles only; a plan of half ones has no unsplit tiles to count)
+    const bool far = sk > 0xffffffffull / (2 * d);
+    const size_t bm = m.block_m && !far ? m.block_m : (size_t)fv_internal_flash_block_m();
     p.nqt = (int)((sq + bm - 1) / bm);
     const size_t total = bh * (size_t)p.nqt;
     if (total > (size_t)INT_MAX / 2) return decline("sdpa: too many query tiles for one launch");
@@ -258,7 +260,7 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         const hipError_t e = fv_internal_launch_short(&c, short_waves, bh, (hipStream_t)stream);
         return e == hipSuccess ? FV_OK : fail_hip(e, "sdpa_short");
     }
-    if (mode == kMaskNone ? splits == 1 && fv_duo(bh, sq, sk, d, out_is_bf16, false) : duo_masked(p, bh, d)) {
+    if (!far && (mode == kMaskNone ? splits == 1 && fv_duo(bh, sq, sk, d, out_is_bf16, false) : duo_masked(p, bh, d))) {
         p.nqt = (int)((sq + 127) / 128);
         p.total = (int)(bh * (size_t)p.nqt);
         p.per_xcd = (p.total + 7) / 8;

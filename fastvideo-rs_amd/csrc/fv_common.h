@@ -48,6 +48,12 @@ FV_DEV f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// v_mfma_f32_16x16x32_bf16: A 16x32 (lane l: row l%16, k 8*(l/16)..+7), B 32x16 (lane l: column l%16, k 8*(l/16)..+7),
+// C 16x16 (lane l, reg i: column l%16, row 4*(l/16) + i).
+FV_DEV f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
 // max / sum over the pair of lanes {l, l ^ 32}, result in both.
 FV_DEV float pair_max(float x) {
     const unsigned u = __builtin_bit_cast(unsigned, x);
@@ -58,6 +64,18 @@ FV_DEV float pair_max(float x) {
 FV_DEV float pair_sum(float x) {
     const unsigned u = __builtin_bit_cast(unsigned, x);
     auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+
+// max / sum over the four lanes {l, l ^ 16, l ^ 32, l ^ 48}, result in all of them.
+FV_DEV float quad_max(float x) {
+    const unsigned u = __builtin_bit_cast(unsigned, pair_max(x));
+    auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return __builtin_fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
+}
+FV_DEV float quad_sum(float x) {
+    const unsigned u = __builtin_bit_cast(unsigned, pair_sum(x));
+    auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
     return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
 }
 

@@ -585,7 +585,7 @@ FV_DEV void fine_item(const VsaFineParams& p, lds_u8* smem, const int wave, cons
     for (int b = 0; b < NB; b++)
         load_q_frags(p.qt + ((size_t)bh * padded + (size_t)qtile * kTileElems) * 128, (NB == 2 ? wave ^ b : 0) * 32 + c32,
                      true, lane, qf[b]);
-    int krd = tile_read_bases<64>(lane).k, vrd = tile_read_bases<128>(lane).v;
+    int krd = tile_read_bases32<64>(lane).k, vrd = tile_read_bases32<128>(lane).v;
 
     f32x16 o[NB][4];
     FineState st[NB];

@@ -57,3 +57,41 @@ def test_topk_of_many_short_rows(fv):
     got = fv.vsa_topk(s, 1)
     torch.cuda.synchronize()
     assert torch.equal(got[:, 0], (s[:, 1] > s[:, 0]).to(torch.int32))
+
+
+@pytest.mark.parametrize("d", [128, 64])
+def test_planes_of_four_gigabytes(fv, d):
+    """Keys whose plane passes 4 GB, past which tile loads address by tile: dense, split by key ranges and block-causal, and
+    the longest plane below. Two far keys hold the rows, so a wrong address shows; P and the result are rounded to bf16,
+    2^-9 each."""
+    import torch
+
+    announce(f"planes of 4 GB d={d}")
+    rows = (1 << 32) // (2 * d)
+    sq, sk = 5, rows + 70
+    k = torch.zeros((1, sk, d), device="cuda", dtype=torch.bfloat16)
+    v = torch.zeros((1, sk, d), device="cuda", dtype=torch.bfloat16)
+    g = torch.Generator(device="cuda").manual_seed(d)
+    q = torch.ones((1, sq, d), device="cuda", dtype=torch.bfloat16)
+    far = [0, rows // 2 + 3, rows - 70, rows - 1, rows, rows + 5, sk - 1]
+    for i, at in enumerate(far):
+        k[0, at] = 3.0 + 0.125 * i
+        v[0, at] = torch.randn(d, generator=g, device="cuda").to(torch.bfloat16)
+
+    def want(n):
+        at = [x for x in far if x < n]
+        s = torch.full((1,), 0.0, dtype=torch.float64)
+        w = torch.exp(torch.stack([k[0, x].double().sum() / d ** 0.5 for x in at]).cpu())
+        others = (n - len(at)) * torch.exp(s)
+        return sum(wi * v[0, x].double().cpu() for wi, x in zip(w, at)) / (w.sum() + others)
+
+    def close(got, n):
+        ref = want(n)
+        assert ((got.double().cpu() - ref).norm(dim=-1) / ref.norm()).max().item() <= 2.0 ** -7
+
+    for out_bf16 in (True, False):
+        close(fv.sdpa_dense_bf16(q, k, v, out_bf16=out_bf16)[0], sk)
+    close(fv.sdpa(q[None], k[None], v[None], fv.Plan.dense())[0, 0], sk)
+    block = rows // 2 + 10
+    close(fv.sdpa_block_causal_bf16(q, k, v, block, 0, 2, out_bf16=True)[0], 2 * block)
+    close(fv.sdpa_dense_bf16(q, k[:, :rows - 1].contiguous(), v[:, :rows - 1].contiguous(), out_bf16=True)[0], rows - 1)
