@@ -168,17 +168,36 @@ FV_DEV ConstParams* params_again() {
     asm volatile("" : "+s"(again));
     return again;
 }
-// Scores of query block g that the lane's query may not see to -inf, and those of keys `left` and on; `key`: the tile's first
-// key + 4 (lane / 16), `left` counted from it.
-FV_DEV void mask_scores(ScoreTile& s, int g, const LaneMask& m, int key, int left) {
+// Scores of query block g that the lane's query may not see to -inf, and those of keys `left` (counted from the tile's first)
+// and on; `at`: the tile's first key. Most tiles that a wave cannot take whole are whole for each of its queries, seen or
+// not (a boundary of frames among its rows): those cost a select a score, the cut ones the four comparisons. Asked key by key
+// throughout, with the bounds worked out anew each time (two integer divisions), a phase of such a wave took 10 us instead of 2.9.
+FV_DEV void mask_scores(ScoreTile& s, int g, const LaneMask& m, int at, int q4, int left) {
+    const bool all = (m.a_hi - at >= kBN) | (at >= m.c_lo) | ((at >= m.w_lo) & (m.w_hi - at >= kBN));
+    const bool none = (m.a_hi <= at) & (m.c_lo - at >= kBN) & ((m.w_lo - at >= kBN) | (m.w_hi <= at));
+    if (left >= kBN && __builtin_amdgcn_ballot_w64(!(all | none)) == 0) {
+        int hidden = none;
+        asm volatile("" : "+v"(hidden));   // (a condition in scalar registers would be carried around the caller's loop)
+#pragma unroll
+        for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) s[kb][g][i] = hidden ? neg_inf() : s[kb][g][i];
+        return;
+    }
 #pragma unroll
     for (int kb = 0; kb < 4; kb++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int x = key + 16 * kb + i;
-            const bool vis = ((x < m.a_hi) | (x >= m.c_lo) | ((x >= m.w_lo) & (x < m.w_hi))) & (16 * kb + i < left);
+            const int n = 4 * q4 + 16 * kb + i, x = at + n;
+            const bool vis = ((x < m.a_hi) | (x >= m.c_lo) | ((x >= m.w_lo) & (x < m.w_hi))) & (n < left);
             s[kb][g][i] = vis ? s[kb][g][i] : neg_inf();
         }
+}
+// The scores as they are, in registers of their own: around code that runs rarely, whose merges would otherwise cost the
+// common way copies of them.
+FV_DEV void pin_scores(ScoreTile& s) {
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++) asm volatile("" : "+v"(s[kb][0]), "+v"(s[kb][1]));
 }
 FV_DEV void mask_keys(ScoreTile& s, int left) {
 #pragma unroll
@@ -302,6 +321,8 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
     //   x < a_hi  ||  x >= c_lo  ||  (w_lo <= x && x < w_hi).
     int a1 = 0, a2 = 0, n0 = nkt, n1 = 0, ne = nkt;
     WalkSight sight = {0, 0, 0, 0};
+    // (masked: the bounds of the wave's queries behind the vote, the wave's own business)
+    auto* const lane_masks = (__attribute__((address_space(3))) u32x4*)(smem + 2 * kRing2 * kTileBytes + kVoteBytes) + wave * 32;
     if constexpr (MASKED) {
         const TileWalk w = mask_tile_walk(p, q0, qlen, nkt);
         a1 = w.a1;
@@ -310,6 +331,7 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         n1 = w.n1;
         ne = w.ne;
         sight = walk_sight(p, w, q0 + wave * 32);
+        if (lane < 32) lane_masks[lane] = __builtin_bit_cast(u32x4, lane_mask(p, q0 + wave * 32 + lane));
     }
     if constexpr (MASKED) {
         // No key tile is visible to any query of this tile (block-causal with more queries than keys
@@ -441,12 +463,12 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
     // scores of walk position e, whose first key is kv0: keys past the end (or a position past the walk) to -inf; masked
     // launches: keys this lane's queries may not see to -inf
     auto mask_tile = [&](ScoreTile& s, int e, int kv0) {
-        const int left = (e >= ne ? 0 : sk) - kv0 - 4 * q4;
+        const int left = (e >= ne ? 0 : sk) - kv0;
         if constexpr (MASKED) {
 #pragma unroll
-            for (int g = 0; g < 2; g++) mask_scores(s, g, lane_mask(*params_again(), q0 + wave * 32 + 16 * g + i16), kv0 + 4 * q4, left);
+            for (int g = 0; g < 2; g++) mask_scores(s, g, __builtin_bit_cast(LaneMask, (u32x4)lane_masks[16 * g + i16]), kv0, q4, left);
         } else {
-            mask_keys(s, left);
+            mask_keys(s, left - 4 * q4);
         }
     };
     const bool ragged = (ne & 1) != 0 || kv0_of(ne - 1) + kBN > sk;   // keys past the end in the last phase
@@ -487,8 +509,10 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
         __builtin_amdgcn_sched_barrier(0);
         // ---- VALU phase: group 0 in slot 2m+1, group 1 in slot 2m+2 ----
         if ((m == np - 1 && ragged) || (MASKED && !sight.all(2 * m, 2 * m + 1))) {
+            if constexpr (MASKED) pin_scores(s0), pin_scores(s1);
             mask_tile(s0, 2 * m, kv[0]);
             mask_tile(s1, 2 * m + 1, kv[1]);
+            if constexpr (MASKED) pin_scores(s0), pin_scores(s1);
         }
         if (FIXED && !first) softmax_tile_pair_fixed<!LOG2DOM>(s0, s1, st, sl2, pb0, pb1);
         else softmax_tile_pair_off<!LOG2DOM, kNO>(s0, s1, st, o, s_init, sl2, pb0, pb1);
@@ -753,12 +777,12 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     }
     auto mask_tile = [&](ScoreTile& s, int e) {
         if (e < ne - 1 && (!MASKED || sight.all(e, e))) return;
-        const int kv0 = kv0_of(e), left = sk - kv0 - 4 * q4;
+        const int kv0 = kv0_of(e), left = sk - kv0;
         if constexpr (MASKED) {
 #pragma unroll
-            for (int g = 0; g < 2; g++) mask_scores(s, g, lane_mask(*params_again(), q0 + wave * 32 + 16 * g + i16), kv0 + 4 * q4, left);
+            for (int g = 0; g < 2; g++) mask_scores(s, g, lane_mask(*params_again(), q0 + wave * 32 + 16 * g + i16), kv0, q4, left);
         } else {
-            if (kv0 + kBN > sk) mask_keys(s, left);
+            if (kv0 + kBN > sk) mask_keys(s, left - 4 * q4);
         }
     };
     f32x4 o[kNO][2], s_init[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -956,16 +980,18 @@ extern "C" int fv_internal_fixed_offset(int out_is_bf16) {
 }
 
 namespace {
+template <bool MASKED, int D>
+constexpr int flash_lds = 2 * fv::kRing2 * fv::TileGeo<D>::kTile + fv::kVoteBytes + (MASKED ? fv::kPpBM * (int)sizeof(fv::LaneMask) : 0);
 // The kernel's dynamic LDS limit (128 KB at D = 128), once per device.
 template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, bool FAR>
 hipError_t flash_attr() {
     static std::atomic<unsigned long long> attr_done;
-    constexpr int lds = 2 * fv::kRing2 * fv::TileGeo<D>::kTile + fv::kVoteBytes;
+    constexpr int lds = flash_lds<MASKED, D>;
     return fv_set_max_lds_once((const void*)fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED, FAR>, lds, attr_done);
 }
 template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, bool FAR = false>
 hipError_t launch_flash_as(const fv::FlashParams* p, hipStream_t stream) {
-    constexpr int lds = 2 * fv::kRing2 * fv::TileGeo<D>::kTile + fv::kVoteBytes;
+    constexpr int lds = flash_lds<MASKED, D>;
     hipError_t e = flash_attr<NG, MASKED, D, LOG2DOM, FIXED, FAR>();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED, FAR>), dim3(p->full + p->per_xcd * 8), dim3(256 * NG), lds, stream, *p);
