@@ -652,6 +652,45 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
     return true;
 }
 
+// The queue of a long masked launch. A workgroup takes the next item of its XCD's list when it starts, and where that is used up
+// one of another's: XCDs differ in speed by 5 %, and an eighth more workgroups than items are launched, so that the fast ones may
+// take more (the rest find nothing and end). A list is the whole heads x * a .. one after the other and, tile by tile, a share of the
+// heads past the last multiple of eight: one head at a time goes through an L2. An item is a (head, query tile), counted as
+// `work` in flash_item.
+// us, in the order of the numbers / so: causal 40 heads 21 x 1560 8748 / 8127 (36 % of the L2 lines missed before), VDN window 40 heads
+// 18 x 880 chunk 5 radius 2 3997 / 3566, 12 heads 32 x 1560 chunk 5 radius 1 6001 / 5860, 24 heads 24 x 1560 radius 2 4849 / 4844. Launches
+// of less than eight rounds keep the order of the numbers: there a list by head ends too unevenly (12 heads, 7 frames 354 / 425),
+// and one by length is no faster (354 / 355; 24 heads, 8 frames, a window of 4 690 / 699). One workgroup a CU that walks item after
+// item needs registers that the main loop then misses: 8649 and 3863 where this form has 8345 and 3712.
+template <class Params>
+FV_DEV int queue_item(const Params& p, int x, int j) {
+    const int nqt = p.nqt, nbh = p.total / nqt, a = nbh >> 3, c = nbh & 7;
+    if (j < a * nqt) return j % nqt * nbh + x * a + j / nqt;
+    const int i = (j - a * nqt) * 8 + x;
+    return i < c * nqt ? i / c * nbh + 8 * a + i % c : -1;
+}
+constexpr int kQueueStep = 32;   // words between the XCDs' counters: a line each
+// The workgroup's item into `block`; false: there is none left.
+template <int D, class Params>
+FV_DEV bool take_item(const Params& p, const int wave, const int lane, int& block) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    auto* word = (__attribute__((address_space(3))) int*)((lds_u8*)smem_raw + 2 * kRing2 * TileGeo<D>::kTile + kVoteBytes / 2);
+    if (wave == 0) {
+        int got = -1;
+        for (int i = 0; i < 8 && got < 0; i++) {
+            const int x = (blockIdx.x + i) & 7;
+            int j = 0;
+            if (lane == 0) j = __hip_atomic_fetch_add((__attribute__((address_space(1))) int*)p.queue + x * kQueueStep, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            got = queue_item(p, x, __builtin_amdgcn_readfirstlane(j));
+        }
+        if (lane == 0) *word = got;
+        __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the word is written before the barrier
+    }
+    block_barrier();
+    block = __builtin_amdgcn_readfirstlane(*word);
+    return block >= 0;
+}
+
 // The softmax offset rides in the C operand of the K Q^T MFMAs (softmax_tile_pair_off): a score costs one multiply,
 // one exponential and one add. LOG2DOM: the call's scale * log2(e) is exactly 1 (scores are base-2 logarithms as
 // they leave the MFMAs) and the multiply is gone too. FIXED (launches that write bf16 and whose queries all see key 0): the first pass keeps
@@ -664,6 +703,8 @@ template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, bool FAR>
 __global__ __launch_bounds__(256 * NG, 2) void flash_fwd_pp2(const FlashParams p) {
     const int tid = threadIdx.x;
     int wave = __builtin_amdgcn_readfirstlane(tid >> 6), block = blockIdx.x;
+    if constexpr (MASKED)
+        if (p.queue && !take_item<D>(p, wave, tid & 63, block)) return;
     if constexpr (!FIXED) {
         flash_item<NG, MASKED, D, LOG2DOM, false, FAR>(p, wave, tid & 63, block);
     } else {
@@ -968,6 +1009,14 @@ extern "C" hipError_t fv_internal_launch_splitkv_merge(const float* part_o, cons
 
 // ---- host launchers -------------------------------------------------------------
 
+// (a kernel, not a memset: a caller may capture it into a graph)
+static __global__ void clear_queue_kernel(int* queue) { queue[threadIdx.x] = 0; }
+extern "C" hipError_t fv_internal_clear_queue(int* queue, hipStream_t stream) {
+    static_assert(8 * fv::kQueueStep * sizeof(int) == kFvQueueBytes, "a counter an XCD");
+    hipLaunchKernelGGL(clear_queue_kernel, dim3(1), dim3(8 * fv::kQueueStep), 0, stream, queue);
+    return hipGetLastError();
+}
+
 extern "C" int fv_internal_flash_block_m(void) { return fv::kPpBM; }
 
 // FASTVIDEO_SDPA_RUNNING_MAX=1: every launch keeps the running max (no fixed-offset first pass).
@@ -994,7 +1043,8 @@ hipError_t launch_flash_as(const fv::FlashParams* p, hipStream_t stream) {
     constexpr int lds = flash_lds<MASKED, D>;
     hipError_t e = flash_attr<NG, MASKED, D, LOG2DOM, FIXED, FAR>();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED, FAR>), dim3(p->full + p->per_xcd * 8), dim3(256 * NG), lds, stream, *p);
+    const int grid = p->full + (p->queue ? p->per_xcd + p->per_xcd / 8 : p->per_xcd) * 8;
+    hipLaunchKernelGGL((fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED, FAR>), dim3(grid), dim3(256 * NG), lds, stream, *p);
     return hipGetLastError();
 }
 template <bool MASKED, int D, bool LOG2DOM>

@@ -121,6 +121,7 @@ struct MaskArgs {
     int short_waves = 0;                          // > 0: the short kernel, with as many waves a workgroup
     void* workspace = nullptr;                    // ... and their partial results
     size_t workspace_bytes = 0;
+    int* queue = nullptr;                         // masked: kFvQueueBytes for the queue of its items, or none
     size_t block_tokens = 0, window = 0, sink = 0;                           // block-causal
     size_t video_start = 0, frame_tokens = 0, frames = 0, chunk = 0, radius = 0;   // VDN window
 };
@@ -226,6 +227,7 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
     p.part_row0 = p.part_rows = 0;
     p.part_o = nullptr;
     p.part_lse = nullptr;
+    p.queue = nullptr;
     const size_t nkt = (sk + 63) / 64;
     size_t splits = mode == kMaskNone ? settle_splits(nkt, m.splits) : 1;
     if (splits > 1) {
@@ -266,6 +268,11 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         p.per_xcd = (p.total + 7) / 8;
         const hipError_t e = fv_internal_launch_duo(&p, mode != kMaskNone ? 1 : 0, (int)d, (hipStream_t)stream);
         return e == hipSuccess ? FV_OK : fail_hip(e, "flash_fwd_duo");
+    }
+    if (mode != kMaskNone && m.queue && fv_masked_workspace_bytes(bh, sq)) {
+        p.queue = m.queue;
+        const hipError_t e = fv_internal_clear_queue(p.queue, (hipStream_t)stream);
+        if (e != hipSuccess) return fail_hip(e, "clear_queue");
     }
     hipError_t e = fv_internal_launch_flash(&p, mode != kMaskNone ? 1 : 0, (int)d, (int)bm, (hipStream_t)stream);
     if (e != hipSuccess) return fail_hip(e, mode != kMaskNone ? "flash_fwd_pp2<masked>" : "flash_fwd_pp2<dense>");
@@ -384,6 +391,28 @@ int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, vo
     m.short_waves = plan.short_waves;
     m.workspace = workspace;
     m.workspace_bytes = workspace_bytes;
+    return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
+}
+
+// (eight rounds of query tiles: see take_item)
+size_t fv_masked_workspace_bytes(size_t bh, size_t sq) {
+    const size_t cus = (size_t)fv_compute_units(), bm = (size_t)fv_internal_flash_block_m();
+    return cus >= 8 && bh * ((sq + bm - 1) / bm) >= 8 * cus ? kFvQueueBytes : 0;
+}
+
+int fv_masked_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out, int out_is_bf16, size_t bh,
+                      size_t sq, size_t sk, size_t d, float scale, const FvMask& mask, void* workspace, void* stream) {
+    MaskArgs m;
+    m.mode = mask.causal ? kMaskBlockCausal : kMaskVdnWindow;
+    m.block_tokens = mask.block_tokens;
+    m.window = mask.window;
+    m.sink = mask.sink;
+    m.video_start = mask.video_start;
+    m.frame_tokens = mask.frame_tokens;
+    m.frames = mask.frames;
+    m.chunk = mask.chunk;
+    m.radius = mask.radius;
+    m.queue = (int*)workspace;
     return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
 }
 
@@ -538,26 +567,16 @@ int fv_sdpa_block_causal_bf16(const uint16_t* q, const uint16_t* k, const uint16
                               int out_is_bf16, size_t bh, size_t sq, size_t sk, size_t d,
                               float scale, size_t block_tokens, size_t window, size_t sink,
                               void* stream) {
-    MaskArgs m;
-    m.mode = kMaskBlockCausal;
-    m.block_tokens = block_tokens;
-    m.window = window;
-    m.sink = sink;
-    return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
+    const FvMask mask = {true, block_tokens, window, sink, 0, 0, 0, 0, 0};
+    return fv_masked_planned(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, mask, nullptr, stream);
 }
 
 int fv_sdpa_vdn_window_bf16(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,
                             int out_is_bf16, size_t bh, size_t sq, size_t sk, size_t d, float scale,
                             size_t video_start, size_t frame_tokens, size_t frames, size_t chunk,
                             size_t radius, void* stream) {
-    MaskArgs m;
-    m.mode = kMaskVdnWindow;
-    m.video_start = video_start;
-    m.frame_tokens = frame_tokens;
-    m.frames = frames;
-    m.chunk = chunk;
-    m.radius = radius;
-    return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
+    const FvMask mask = {false, 0, 0, 0, video_start, frame_tokens, frames, chunk, radius};
+    return fv_masked_planned(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, mask, nullptr, stream);
 }
 
 // (a launch holds fewer than 2^32 work-items and the runtime does not say so: longer operands in several)

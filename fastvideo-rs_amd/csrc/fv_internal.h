@@ -34,6 +34,9 @@ struct FlashParams {
     long part_row0, part_rows;
     float* part_o;
     float* part_lse;
+    // Masked launches: eight zeroed counters (kFvQueueBytes) from which the workgroups take their items, or null: in the order of
+    // their numbers.
+    int* queue;
 };
 
 struct ComposedParams {
@@ -177,6 +180,18 @@ int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, vo
                      const FvSplitPlan& plan, void* workspace, size_t workspace_bytes, void* stream);
 
 extern "C" int fv_internal_fixed_offset(int out_is_bf16);   // whether results of that type are made with a fixed offset first
+// Masked launches of many rounds take their items from a queue where the caller has this much memory for it.
+constexpr size_t kFvQueueBytes = 1024;
+struct FvMask {
+    bool causal;
+    size_t block_tokens, window, sink;                            // block-causal
+    size_t video_start, frame_tokens, frames, chunk, radius;      // VDN window
+};
+size_t fv_masked_workspace_bytes(size_t bh, size_t sq);
+// fv_sdpa_block_causal_bf16 or fv_sdpa_vdn_window_bf16 with such a workspace, or without one (null)
+int fv_masked_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out, int out_is_bf16, size_t bh,
+                      size_t sq, size_t sk, size_t d, float scale, const FvMask& mask, void* workspace, void* stream);
+extern "C" hipError_t fv_internal_clear_queue(int* queue, hipStream_t stream);
 extern "C" int fv_internal_flash_block_m(void);   // queries per workgroup of the flash kernel in use
 extern "C" hipError_t fv_internal_launch_duo(const fv::FlashParams* p, int masked, int d, hipStream_t stream);   // total, nqt: of 128 queries
 extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d, int block_m,

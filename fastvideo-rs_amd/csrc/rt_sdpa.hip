@@ -300,13 +300,18 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
     Tensor out = std::move(std::get<Tensor>(ro));
     const uint16_t *pq = bits[0], *pk = bits[1], *pv = bits[2];
     int rc;
-    if (causal)
-        rc = fv_sdpa_block_causal_bf16(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc,
-                                       causal->block_tokens, causal->window, causal->sink, st);
-    else if (window)
-        rc = fv_sdpa_vdn_window_bf16(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc,
-                                     window->video_start, window->frame_tokens, window->frames, window->chunk,
-                                     window->radius, st);
+    if (causal || window) {
+        FvMask m{};
+        if (causal) m = {true, causal->block_tokens, causal->window, causal->sink, 0, 0, 0, 0, 0};
+        else m = {false, 0, 0, 0, window->video_start, window->frame_tokens, window->frames, window->chunk, window->radius};
+        Tensor ws;
+        const size_t need = fv_masked_workspace_bytes(s->b * s->h, s->sq);
+        if (need && st.holds(need)) {   // (in the caller's workspace only)
+            auto rw = st.temp({need / 4}, DType::F32);
+            if (is_ok(rw)) ws = std::move(std::get<Tensor>(rw));
+        }
+        rc = fv_masked_planned(pq, pk, pv, out.data, out_bf16, s->b * s->h, s->sq, s->sk, s->d, sc, m, ws.data, st);
+    }
     else {
         // query tiles that do not fill the CUs, or the last round of them: split the keys over more workgroups. The last
         // round only in the caller's workspace: a stream-ordered one costs more than the split gives after every
@@ -754,6 +759,8 @@ Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& pl
         if (t->dtype == DType::F32) n.workspace += (t->numel() * 2 + 255) & ~(size_t)255;
     if (plan.kind == Plan::Kind::Dense || plan.kind == Plan::Kind::KvWindow) {
         n.workspace += (dense_plan(s->b * s->h, s->sq, s->sk, s->d, act16).workspace_bytes + 255) & ~(size_t)255;
+    } else {
+        n.workspace += fv_masked_workspace_bytes(s->b * s->h, s->sq);
     }
     return n;
 }
