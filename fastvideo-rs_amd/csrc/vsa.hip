@@ -679,6 +679,10 @@ FV_DEV void fine_item(const VsaFineParams& p, lds_u8* smem, const int wave, cons
             bf16x8 f[8];
             auto read = [&](int dk) { f[dk] = lds_read_b128(ring + (dk < 4 ? sk0 : sk1) + (krd ^ ((dk & 3) << 5))); };
             wait_vmcnt<12>();   // the first K chunk has landed; the other three may be in flight
+            // The two waves of a SIMD come from workgroups that know nothing of each other: the one in a matrix part goes before
+            // one that waits, forms addresses or is at its softmax. us, without / so, 12 heads 21 x 30 x 52 at 0.8 1878 / 1824, 16 x 32
+            // x 64 at 0.9 1000 / 982, 24 heads 9 x 21 x 50 462 / 459. (Priority over the softmax too: 1853, 990, 461.)
+            __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int dk = 0; dk < kAhead; dk++) read(dk);
 #pragma unroll
@@ -699,6 +703,7 @@ FV_DEV void fine_item(const VsaFineParams& p, lds_u8* smem, const int wave, cons
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        __builtin_amdgcn_s_setprio(0);
         if (cur.valid_a < 16 || cur.valid_b < 16) {
             const int va = cur.valid_a - 4 * h, vb16 = cur.valid_b - 4 * h;
 #pragma unroll
@@ -752,6 +757,7 @@ FV_DEV void fine_item(const VsaFineParams& p, lds_u8* smem, const int wave, cons
             }
         }
         wait_vmcnt<16>();   // the first V chunk
+        __builtin_amdgcn_s_setprio(1);
         {
             bf16x8 f[8];
             auto read = [&](int g) {
@@ -775,6 +781,7 @@ FV_DEV void fine_item(const VsaFineParams& p, lds_u8* smem, const int wave, cons
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        __builtin_amdgcn_s_setprio(0);
         const unsigned left_slot = sv1;   // the ring moves on by four of its five slots
         sv1 = sv0, sv0 = sk1, sk1 = sk0, sk0 = spare, spare = left_slot;
         cur = nx;
