@@ -229,7 +229,8 @@ int fv_rt_free(void* p, void* stream);
  * bytes = those of the [b,h,sq,d] result in the type fv_rt_sdpa_need names (another size is refused), and the rounded
  * copies of f32 operands and the partial sums of split key ranges live in `workspace` (256-byte aligned; NULL / 0: allocated
  * stream-ordered, as what does not fit is; a dense launch's last round of query tiles is split in the workspace only, so
- * without it, and in fv_rt_sdpa, that launch is made unsplit). A result from the stream-ordered allocator costs its caller a copy or a
+ * without it, and in fv_rt_sdpa, that launch is made unsplit, and a long masked launch takes its items from a queue there only:
+ * same bits, 2 - 11 % more time without). A result from the stream-ordered allocator costs its caller a copy or a
  * wrapper and, after every synchronisation of the device, mapping its memory anew (0.2 - 0.35 ms for 100 MB).
  * fv_rt_sdpa_need: need_out = {result type (0 f32, 1 bf16), workspace bytes} of that call. Host arithmetic, except that
  * the number of compute units is asked of the current device once. */
