@@ -168,30 +168,27 @@ FV_DEV ConstParams* params_again() {
     asm volatile("" : "+s"(again));
     return again;
 }
+// The first n of 64 bits.
+FV_DEV unsigned long long first_bits(int n) {
+    const unsigned long long m = ~0ull >> ((64 - n) & 63);
+    return n <= 0 ? 0ull : n >= 64 ? ~0ull : m;
+}
 // Scores of query block g that the lane's query may not see to -inf, and those of keys `left` (counted from the tile's first)
-// and on; `at`: the tile's first key. Most tiles that a wave cannot take whole are whole for each of its queries, seen or
-// not (a boundary of frames among its rows): those cost a select a score, the cut ones the four comparisons. Asked key by key
-// throughout, with the bounds worked out anew each time (two integer divisions), a phase of such a wave took 10 us instead of 2.9.
+// and on; `at`: the tile's first key. The bounds make one word of 64 keys, and a score costs a test of its bit and a
+// select: 3 vector instructions where four comparisons and their scalar joins took 9, and no path apart for tiles that are whole
+// for each query. us, 32x32x16 form / comparisons / so: causal 12 heads 21 x 1560 2713 / 2542 / 2480, 40 heads 34 x 390 under
+// a window of one 366 / 380 / 290, VDN window 12 heads 32 x 1560 chunk 5 6421 / 5970 / 5872, 24 heads 30 x 100 radius 2 106 / 104 / 77. (The
+// bounds worked out anew a tile, two integer divisions a query, took a phase 10 us instead of 2.9: they are kept, see lane_masks and
+// duo_item.)
 FV_DEV void mask_scores(ScoreTile& s, int g, const LaneMask& m, int at, int q4, int left) {
-    const bool all = (m.a_hi - at >= kBN) | (at >= m.c_lo) | ((at >= m.w_lo) & (m.w_hi - at >= kBN));
-    const bool none = (m.a_hi <= at) & (m.c_lo - at >= kBN) & ((m.w_lo - at >= kBN) | (m.w_hi <= at));
-    if (left >= kBN && __builtin_amdgcn_ballot_w64(!(all | none)) == 0) {
-        int hidden = none;
-        asm volatile("" : "+v"(hidden));   // (a condition in scalar registers would be carried around the caller's loop)
-#pragma unroll
-        for (int kb = 0; kb < 4; kb++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) s[kb][g][i] = hidden ? neg_inf() : s[kb][g][i];
-        return;
-    }
+    const int x = at + 4 * q4;   // bit b: key x + b
+    const unsigned long long seen = (first_bits(m.a_hi - x) | ~first_bits(m.c_lo - x) | (first_bits(m.w_hi - x) & ~first_bits(m.w_lo - x))) &
+                                    first_bits(left - 4 * q4);
+    const unsigned hidden[2] = {~(unsigned)seen, ~(unsigned)(seen >> 32)};
 #pragma unroll
     for (int kb = 0; kb < 4; kb++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int n = 4 * q4 + 16 * kb + i, x = at + n;
-            const bool vis = ((x < m.a_hi) | (x >= m.c_lo) | ((x >= m.w_lo) & (x < m.w_hi))) & (n < left);
-            s[kb][g][i] = vis ? s[kb][g][i] : neg_inf();
-        }
+        for (int i = 0; i < 4; i++) s[kb][g][i] = (hidden[kb >> 1] >> (16 * (kb & 1) + i)) & 1 ? neg_inf() : s[kb][g][i];
 }
 // The scores as they are, in registers of their own: around code that runs rarely, whose merges would otherwise cost the
 // common way copies of them.
@@ -754,10 +751,15 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     const int q0 = qt * kDuoBM, sq = p.sq, sk = p.sk, qlen = min(kDuoBM, sq - q0), nkt = (sk + kBN - 1) / kBN;
     int a1 = 0, a2 = 0, n0 = nkt, n1 = 0, ne = nkt;   // the walk, as in flash_item (key 0 is in it)
     WalkSight sight = {0, 0, 0, 0};
+    // Masked: bounds of one of the wave's queries a lane, row lane % 32, which is query block q4 & 1; a tile that asks for them
+    // gets both blocks' by an exchange (mask_tile). There is no LDS left for them at D = 128, bounds of both queries a lane
+    // spilled accumulators, and worked out anew a tile they cost up to a fifth (VDN window 12 heads 8 x 390 107 / 78 us).
+    LaneMask mine = {0, 0x7fffffff, 0, 0};
     if constexpr (MASKED) {
         const TileWalk w = mask_tile_walk(p, q0, qlen, nkt);
         a1 = w.a1, a2 = w.a2, n0 = w.n0, n1 = w.n1, ne = w.ne;
         sight = walk_sight(p, w, q0 + wave * 32);
+        mine = lane_mask(p, q0 + wave * 32 + (lane & 31));
     }
     const float sl2 = p.sl2;
     uint16_t* out = p.out_bf16;
@@ -820,8 +822,16 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
         if (e < ne - 1 && (!MASKED || sight.all(e, e))) return;
         const int kv0 = kv0_of(e), left = sk - kv0;
         if constexpr (MASKED) {
+            const u32x4 m = __builtin_bit_cast(u32x4, mine);
+            u32x4 both[2];   // the even rows of 16 lanes hold block 0's, the odd ones block 1's
 #pragma unroll
-            for (int g = 0; g < 2; g++) mask_scores(s, g, lane_mask(*params_again(), q0 + wave * 32 + 16 * g + i16), kv0, q4, left);
+            for (int x = 0; x < 4; x++) {
+                const auto r = __builtin_amdgcn_permlane16_swap(m[x], m[x], false, false);
+                both[0][x] = (unsigned)r[0];
+                both[1][x] = (unsigned)r[1];
+            }
+#pragma unroll
+            for (int g = 0; g < 2; g++) mask_scores(s, g, __builtin_bit_cast(LaneMask, both[g]), kv0, q4, left);
         } else {
             if (kv0 + kBN > sk) mask_keys(s, left - 4 * q4);
         }

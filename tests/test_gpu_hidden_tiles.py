@@ -1,5 +1,5 @@
 """Masked launches: waves whose queries lie on both sides of a frame boundary, so that whole key tiles are seen by some of
-them and hidden from the others (a select a score), next to tiles that a boundary cuts (key by key)."""
+them and hidden from the others, next to tiles that a boundary cuts."""
 import pytest
 
 from util import announce, assert_parity, qkv, to_dev_bf16
@@ -50,3 +50,23 @@ def test_tiles_hidden_from_some_queries_of_a_wave(fv, oracle, mask, d, out_bf16)
         again = run(poisoned).float().cpu().numpy()
         # (not the same bits: a wave moves the offsets of all its queries when one of them asks for it)
         assert_parity(again[:, :first], want[:, :first], f"hidden_nan_{mask}_{d}")
+
+
+# bounds at every place of a tile's word of 64 keys, its ends among them; 33 heads: flash_fwd_duo where the result is bf16
+@pytest.mark.parametrize("out_bf16", [False, True])
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("frame", [1, 3, 16, 31, 32, 33, 63, 64, 65, 127, 128])
+def test_frames_of_any_length(fv, oracle, frame, d, out_bf16):
+    announce(f"frames of {frame} d={d} bf16={out_bf16}")
+    h, s = 33, 6 * frame + 130
+    q, k, v = qkv(frame + d, h, s, s, d)
+    qd, kd, vd = (to_dev_bf16(x) for x in (q, k, v))
+    # queries that see few keys have results as large as a value: P and the result are rounded to 8 bits, half a unit each, at
+    # most 2^-8 max|v| from either; f32 sums and exponentials are a hundredth of that
+    most = 1.01 * 2 * 2.0 ** -8 * float(abs(v).max())
+    for args in ((frame, 0, 0), (frame, 2, 1), (frame, 3, 0)):
+        want = oracle.sdpa_composed(q, k, v, mask=oracle.block_causal_dense_mask(*args, s, s))
+        assert_parity(fv.sdpa_block_causal_bf16(qd, kd, vd, *args, out_bf16=out_bf16).float().cpu().numpy(), want, f"causal_{args}_{d}", max_abs=most)
+    for args in ((65, frame, 6, 0, 1), (130, frame, 6, 2, 0), (7, frame, 5, 0, 0)):
+        want = oracle.sdpa_composed(q, k, v, mask=oracle.vdn_window_dense_mask(*args, s, s))
+        assert_parity(fv.sdpa_vdn_window_bf16(qd, kd, vd, *args, out_bf16=out_bf16).float().cpu().numpy(), want, f"window_{args}_{d}", max_abs=most)
