@@ -1048,7 +1048,7 @@ hipError_t flash_attr() {
     constexpr int lds = flash_lds<MASKED, D>;
     return fv_set_max_lds_once((const void*)fv::flash_fwd_pp2<NG, MASKED, D, LOG2DOM, FIXED, FAR>, lds, attr_done);
 }
-template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, bool FAR = false>
+template <int NG, bool MASKED, int D, bool LOG2DOM, bool FIXED, bool FAR>
 hipError_t launch_flash_as(const fv::FlashParams* p, hipStream_t stream) {
     constexpr int lds = flash_lds<MASKED, D>;
     hipError_t e = flash_attr<NG, MASKED, D, LOG2DOM, FIXED, FAR>();
@@ -1072,13 +1072,11 @@ hipError_t launch_duo_as(const fv::FlashParams* p, hipStream_t stream) {
 // A call whose scale * log2(e) is exactly 1 (scale = ln 2: the caller folded the softmax scale into Q) runs
 // the form without the per-score multiply.
 std::atomic<unsigned long long> g_log2_domain_launches{0};
-template <int NG, bool MASKED, int D, bool FIXED>
+template <int NG, bool MASKED, int D, bool FIXED, bool FAR>
 hipError_t launch_flash_fixed(const fv::FlashParams* p, hipStream_t stream) {
-    if constexpr (NG == 2 && !FIXED)
-        if (!fv::plane_fits<D>(p->sk)) return launch_flash_as<NG, MASKED, D, false, false, true>(p, stream);
-    if (p->sl2 != 1.0f) return launch_flash_as<NG, MASKED, D, false, FIXED>(p, stream);
+    if (p->sl2 != 1.0f) return launch_flash_as<NG, MASKED, D, false, FIXED, FAR>(p, stream);
     g_log2_domain_launches.fetch_add(1, std::memory_order_relaxed);
-    return launch_flash_as<NG, MASKED, D, true, FIXED>(p, stream);
+    return launch_flash_as<NG, MASKED, D, true, FIXED, FAR>(p, stream);
 }
 // Launches whose result is rounded to bf16 make their first pass with the fixed offset: on a row that one late
 // key dominates, that key's P is then a rounded bf16 number instead of exactly 1 (up to 2^-8 relative on the row),
@@ -1091,9 +1089,15 @@ bool takes_fixed_offset(const fv::FlashParams* p) {
     const bool offset_is_a_score = !MASKED || p->mask_mode == 2 || (p->mask_mode == 1 && (p->win == 0 || p->sink > 0));
     return fv_internal_fixed_offset(p->out_is_bf16) && offset_is_a_score;
 }
+template <int NG, bool MASKED, int D, bool FAR>
+hipError_t launch_flash_planes(const fv::FlashParams* p, hipStream_t stream) {
+    return takes_fixed_offset<MASKED>(p) ? launch_flash_fixed<NG, MASKED, D, true, FAR>(p, stream)
+                                         : launch_flash_fixed<NG, MASKED, D, false, FAR>(p, stream);
+}
 template <int NG, bool MASKED, int D>
 hipError_t launch_flash(const fv::FlashParams* p, hipStream_t stream) {
-    return takes_fixed_offset<MASKED>(p) && fv::plane_fits<D>(p->sk) ? launch_flash_fixed<NG, MASKED, D, true>(p, stream) : launch_flash_fixed<NG, MASKED, D, false>(p, stream);
+    return fv::plane_fits<D>(p->sk) ? launch_flash_planes<NG, MASKED, D, false>(p, stream)
+                                    : launch_flash_planes<NG, MASKED, D, true>(p, stream);
 }
 template <bool MASKED, int D>
 hipError_t launch_duo(const fv::FlashParams* p, hipStream_t stream) {
@@ -1107,15 +1111,18 @@ hipError_t init_duo() {
     const hipError_t e = duo_attr<MASKED, D, false>();
     return e == hipSuccess ? duo_attr<MASKED, D, true>() : e;
 }
+template <int NG, bool MASKED, int D, bool FAR>
+hipError_t init_flash_planes() {
+    hipError_t e = flash_attr<NG, MASKED, D, false, false, FAR>();
+    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, true, false, FAR>();
+    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, false, true, FAR>();
+    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, true, true, FAR>();
+    return e;
+}
 template <int NG, bool MASKED, int D>
 hipError_t init_flash() {
-    hipError_t e = flash_attr<NG, MASKED, D, false, false, false>();
-    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, true, false, false>();
-    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, false, true, false>();
-    if (e == hipSuccess) e = flash_attr<NG, MASKED, D, true, true, false>();
-    if constexpr (NG == 2)
-        if (e == hipSuccess) e = flash_attr<NG, MASKED, D, false, false, true>();
-    return e;
+    const hipError_t e = init_flash_planes<NG, MASKED, D, false>();
+    return e == hipSuccess ? init_flash_planes<NG, MASKED, D, true>() : e;
 }
 }  // namespace
 
@@ -1149,7 +1156,6 @@ extern "C" hipError_t fv_internal_launch_duo(const fv::FlashParams* p, int maske
 extern "C" hipError_t fv_internal_launch_flash(const fv::FlashParams* p, int masked, int d, int block_m,
                                                hipStream_t stream) {
     const bool half = block_m == fv::kPpBM / 2;
-    if (half && !(d == 128 ? fv::plane_fits<128>(p->sk) : fv::plane_fits<64>(p->sk))) return hipErrorInvalidValue;
     if ((block_m != fv::kPpBM && !half) || (half && masked)) return hipErrorInvalidValue;
     if (d == 128)
         return masked ? launch_flash<2, true, 128>(p, stream)

@@ -181,9 +181,8 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
     p.q_plane = (long)(q_rows * d);
     p.k_plane = (long)(k_rows * d);
     p.v_plane = (long)(v_rows * d);
-    // (planes of 4 GB and more have a kernel of whole tiles only; a plan of half ones has no unsplit tiles to count)
-    const bool far = sk > 0xffffffffull / (2 * d);
-    const size_t bm = m.block_m && !far ? m.block_m : (size_t)fv_internal_flash_block_m();
+    const bool far = sk > 0xffffffffull / (2 * d);   // planes of 4 GB and more: flash_fwd_pp2 alone
+    const size_t bm = m.block_m ? m.block_m : (size_t)fv_internal_flash_block_m();
     p.nqt = (int)((sq + bm - 1) / bm);
     const size_t total = bh * (size_t)p.nqt;
     if (total > (size_t)INT_MAX / 2) return decline("sdpa: too many query tiles for one launch");

@@ -1,10 +1,14 @@
 """Operands longer than one launch holds (2^32 work-items in a grid dimension; past it the runtime cuts the size off
 without an error): every element, in its place."""
+import math
+
 import pytest
 
 from util import announce
 
 pytestmark = pytest.mark.gpu
+
+LN2 = math.log(2.0)
 
 
 @pytest.fixture(scope="module")
@@ -95,3 +99,61 @@ def test_planes_of_four_gigabytes(fv, d):
     block = rows // 2 + 10
     close(fv.sdpa_block_causal_bf16(q, k, v, block, 0, 2, out_bf16=True)[0], 2 * block)
     close(fv.sdpa_dense_bf16(q, k[:, :rows - 1].contiguous(), v[:, :rows - 1].contiguous(), out_bf16=True)[0], rows - 1)
+
+
+@pytest.mark.parametrize("d", [128, 64])
+def test_planes_of_four_gigabytes_keep_every_form(fv, d):
+    """Past 4 GB a call has the forms that it has below: scale * log2(e) = 1 without the multiply (counted), a bf16 result
+    with a fixed offset (a late key that outgrows it makes the second pass, counted), query tiles of 128."""
+    import torch
+
+    announce(f"forms of planes of 4 GB d={d}")
+    lib, rows, sq = fv.lib(), (1 << 32) // (2 * d), 130
+    sk = rows + 70
+    k = torch.zeros((1, sk, d), device="cuda", dtype=torch.bfloat16)
+    v = torch.zeros((1, sk, d), device="cuda", dtype=torch.bfloat16)
+    q = torch.ones((1, sq, d), device="cuda", dtype=torch.bfloat16)
+    v[0, rows + 5] = torch.randn(d, generator=torch.Generator(device="cuda").manual_seed(d), device="cuda").to(torch.bfloat16)
+    k[0, rows + 5] = 0.5   # d / 2 bits above the others, which are 2^24 and 2^25: the row is its value
+    want = v[0, rows + 5].double()
+    n0, r0 = lib.fv_sdpa_log2_domain_launches(), lib.fv_sdpa_exact_pass_reruns()
+    near = [fv.sdpa_dense_bf16(q, k, v, scale=LN2, out_bf16=True)[0],
+            fv.sdpa_dense_bf16(q, k, v, scale=LN2)[0],
+            fv.sdpa_block_causal_bf16(q, k, v, rows, 0, 2, scale=LN2, out_bf16=True)[0],
+            fv.sdpa(q[None], k[None], v[None], fv.Plan.dense(LN2))[0, 0]]
+    torch.cuda.synchronize()
+    assert lib.fv_sdpa_log2_domain_launches() == n0 + 4 and lib.fv_sdpa_exact_pass_reruns() == r0
+    for got in near:   # the others' share of the sum is below 2^(25 - 32); P and the result are rounded to bf16
+        assert float((got.double() - want).abs().max()) <= 2.0 ** -6 * float(want.abs().max())
+    k[0, rows + 5] = 16.0   # 184 and 261 bits: past the range of the fixed offset
+    for fn in (lambda: fv.sdpa_dense_bf16(q, k, v, out_bf16=True), lambda: fv.sdpa_block_causal_bf16(q, k, v, rows, 0, 2, out_bf16=True)):
+        r0 = lib.fv_sdpa_exact_pass_reruns()
+        far = fn()[0]
+        torch.cuda.synchronize()
+        assert lib.fv_sdpa_exact_pass_reruns() == r0 + 1
+        assert float((far.double() - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("d", [128, 64])
+def test_vdn_window_on_planes_of_four_gigabytes(fv, d):
+    import torch
+
+    announce(f"VDN window on planes of 4 GB d={d}")
+    t, rows = 64, (1 << 32) // (2 * d)
+    frames = rows // t + 1
+    s, vs = t * frames + 90, 40
+    g = torch.Generator(device="cuda").manual_seed(d)
+    q, k, v = (torch.randn((1, s, d), generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    for out_bf16 in (True, False):
+        got = fv.sdpa_vdn_window_bf16(q, k, v, vs, t, frames, 0, 1, out_bf16=out_bf16)[0]
+        for i in (vs + t, vs + 5 * t - 1, rows // 2, rows - 1, rows, s - 50 - t - 1):
+            f = (i - vs) // t
+            seen = torch.zeros(s, dtype=torch.bool, device="cuda")
+            for a, b in ((0, vs + t), (vs + (f - 1) * t, vs + (f + 2) * t), (vs + (frames - 1) * t, s)):
+                seen[a:b] = True
+            at = seen.nonzero()[:, 0]
+            p = torch.softmax(k[0, at].double() @ q[0, i].double() / d ** 0.5, 0)
+            ref = p @ v[0, at].double()
+            # P and the result rounded to 8 bits, half a unit of each
+            bound = 2.0 ** -8 * (p @ v[0, at].double().abs() + ref.abs()) + 1e-5
+            assert bool(((got[i].double() - ref).abs() <= bound).all()), (out_bf16, i)
