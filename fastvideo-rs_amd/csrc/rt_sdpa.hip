@@ -306,7 +306,7 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
         else m = {false, 0, 0, 0, window->video_start, window->frame_tokens, window->frames, window->chunk, window->radius};
         Tensor ws;
         const size_t need = fv_masked_workspace_bytes(s->b * s->h, s->sq);
-        if (need && st.holds(need)) {   // (in the caller's workspace only)
+        if (need && st.own && st.holds(need)) {   // (counters that two launches shared would leave rows of both unwritten)
             auto rw = st.temp({need / 4}, DType::F32);
             if (is_ok(rw)) ws = std::move(std::get<Tensor>(rw));
         }
@@ -759,7 +759,7 @@ Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& pl
         if (t->dtype == DType::F32) n.workspace += (t->numel() * 2 + 255) & ~(size_t)255;
     if (plan.kind == Plan::Kind::Dense || plan.kind == Plan::Kind::KvWindow) {
         n.workspace += (dense_plan(s->b * s->h, s->sq, s->sk, s->d, act16).workspace_bytes + 255) & ~(size_t)255;
-    } else {
+    } else if (plan.own_workspace) {
         n.workspace += fv_masked_workspace_bytes(s->b * s->h, s->sq);
     }
     return n;
@@ -829,6 +829,14 @@ struct FlatCall {
         const Tensor* pm = p->mask ? &mask : nullptr;
         const std::optional<float> scale = p->has_scale ? std::optional<float>(p->scale) : std::nullopt;
         switch (p->kind) {
+            case FV_PLAN_BLOCK_CAUSAL | FV_PLAN_OWN_WORKSPACE:
+            case FV_PLAN_BLOCK_CAUSAL:
+                plan = Plan::block_causal(scale, BlockCausal{p->block_tokens, p->window, p->sink});
+                break;
+            case FV_PLAN_VDN_WINDOW | FV_PLAN_OWN_WORKSPACE:
+            case FV_PLAN_VDN_WINDOW:
+                plan = Plan::vdn_window(scale, VdnWindow{p->video_start, p->frame_tokens, p->frames, p->chunk, p->radius});
+                break;
             case FV_PLAN_DENSE:
                 plan = Plan::masked(scale, pm);
                 if (p->fp8_first) plan = plan.fp8_first();
@@ -836,18 +844,13 @@ struct FlatCall {
             case FV_PLAN_COMPOSED:
                 plan = Plan::composed(scale, pm);
                 break;
-            case FV_PLAN_BLOCK_CAUSAL:
-                plan = Plan::block_causal(scale, BlockCausal{p->block_tokens, p->window, p->sink});
-                break;
-            case FV_PLAN_VDN_WINDOW:
-                plan = Plan::vdn_window(scale, VdnWindow{p->video_start, p->frame_tokens, p->frames, p->chunk, p->radius});
-                break;
             case FV_PLAN_KV_WINDOW:
                 plan = p->kv_flash < 0 ? Plan::kv_window() : Plan::kv_window_with(p->kv_flash != 0);
                 break;
             default:
                 return fv_invalid("fv_rt_sdpa: unknown plan kind");
         }
+        plan.own_workspace = (p->kind & FV_PLAN_OWN_WORKSPACE) != 0;
         return FV_OK;
     }
 };
@@ -896,7 +899,9 @@ int fv_rt_sdpa_into(const fv_tensor* q, const fv_tensor* k, const fv_tensor* v, 
     if (const int rc = c.open(q, k, v, plan); rc != FV_OK) return rc;
     // (an empty result is written nowhere, but its buffer must still be the caller's)
     static char nothing;
-    auto r = sdpa(c.q, c.k, c.v, c.plan, Mem((hipStream_t)stream, out ? out : &nothing, out_bytes, workspace, workspace_bytes));
+    Mem mem((hipStream_t)stream, out ? out : &nothing, out_bytes, workspace, workspace_bytes);
+    mem.own = c.plan.own_workspace;
+    auto r = sdpa(c.q, c.k, c.v, c.plan, mem);
     return is_ok(r) ? FV_OK : flat_error(std::get<TensorError>(r));
 }
 

@@ -80,6 +80,7 @@ class Mem {
     operator hipStream_t() const { return stream; }
     Result<Tensor> temp(std::vector<size_t> shape, DType dtype);
     bool holds(size_t bytes) const;   // does the rest of the caller's workspace have room for this?
+    bool own = false;                 // Plan::own_workspace
     Result<Tensor> result(std::vector<size_t> shape, DType dtype);
     hipStream_t stream;
 
@@ -125,6 +126,7 @@ class Plan {
     BlockCausal causal;
     VdnWindow window;
     std::optional<bool> kv_flash;
+    bool own_workspace = false;   // block-causal, VDN window: no other call in flight uses the caller's workspace
 };
 
 // rt/tensor.rs:61-76 `bf16_activations` / `with_bf16_act`: FASTVIDEO_BF16_ACT

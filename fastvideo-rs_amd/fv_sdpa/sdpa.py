@@ -135,6 +135,7 @@ _TENSOR_BYTES = struct.Struct("@Pii9N")
 _PLAN_BYTES = struct.Struct("@iifPi8Ni0P")
 assert _TENSOR_BYTES.size == C.sizeof(_FvTensor) and _PLAN_BYTES.size == C.sizeof(_FvPlan)
 _NO_SHAPE = (0,) * 8
+_OWN_WORKSPACE = 256   # FV_PLAN_OWN_WORKSPACE
 _BF16, _F32 = torch.bfloat16, torch.float32
 
 
@@ -167,19 +168,20 @@ def _desc(t, name):
     return _FvTensor.from_buffer_copy(_desc_bytes(t, name))
 
 
-def _plan_bytes(plan, mask):
-    """`plan` as the bytes of a struct fv_plan; `mask`: the address of its mask's struct fv_tensor, or 0."""
-    scale, causal, window = plan.scale, plan.causal, plan.window
+def _plan_bytes(plan, mask, flags=0):
+    """`plan` as the bytes of a struct fv_plan; `mask`: the address of its mask's struct fv_tensor, or 0;
+    `flags`: or'ed into its kind."""
+    scale, causal, window, kind = plan.scale, plan.causal, plan.window, plan.kind | flags
     causal = (causal.block_tokens, causal.window, causal.sink) if causal is not None else (0, 0, 0)
     window = window._args() if window is not None else (0, 0, 0, 0, 0)
     kv_flash = -1 if plan.kv_flash is None else int(plan.kv_flash)
     try:
-        return _PLAN_BYTES.pack(plan.kind, 0 if scale is None else 1, 0.0 if scale is None else scale, mask,
+        return _PLAN_BYTES.pack(kind, 0 if scale is None else 1, 0.0 if scale is None else scale, mask,
                                 1 if plan.fp8 else 0, *causal, *window, kv_flash)
     except (struct.error, OverflowError):
         # numbers that do not fit their fields (negative, a scale past f32): what C makes of them, for the library to judge
         p = _FvPlan()
-        p.kind, p.fp8_first, p.kv_flash = plan.kind, 1 if plan.fp8 else 0, kv_flash
+        p.kind, p.fp8_first, p.kv_flash = kind, 1 if plan.fp8 else 0, kv_flash
         p.has_scale, p.scale = (0, 0.0) if scale is None else (1, float(scale))
         p.mask = C.cast(C.c_void_p(mask), C.POINTER(_FvTensor))
         p.block_tokens, p.window, p.sink = causal
@@ -194,7 +196,9 @@ def sdpa(q, k, v, plan):
     mask = None
     if plan.mask is not None:
         mask = C.create_string_buffer(_desc_bytes(plan.mask, "mask"), _TENSOR_BYTES.size)   # alive until the call is made
-    p = _plan_bytes(plan, 0 if mask is None else C.addressof(mask))
+    kind = plan.kind   # (the workspace of a block-causal or window call is allocated below, for it alone)
+    p = _plan_bytes(plan, 0 if mask is None else C.addressof(mask),
+                    _OWN_WORKSPACE if kind == Plan.BLOCK_CAUSAL or kind == Plan.VDN_WINDOW else 0)
     need = (C.c_size_t * 2)()
     rc = lib.fv_rt_sdpa_need(dq, dk, dv, p, need)
     if rc != 0:

@@ -205,6 +205,9 @@ enum {
     FV_PLAN_VDN_WINDOW = 3,   /* Plan::vdn_window (rt/sdpa.rs:111-119) */
     FV_PLAN_KV_WINDOW = 4     /* Plan::kv_window / kv_window_with (rt/sdpa.rs:125-137) */
 };
+/* or'ed into BLOCK_CAUSAL or VDN_WINDOW (no counterpart in the reference): the workspace of fv_rt_sdpa_into is this call's
+ * alone until the call's work on its stream is done, see there */
+#define FV_PLAN_OWN_WORKSPACE 256
 
 typedef struct fv_plan {
     int kind;
@@ -229,8 +232,10 @@ int fv_rt_free(void* p, void* stream);
  * bytes = those of the [b,h,sq,d] result in the type fv_rt_sdpa_need names (another size is refused), and the rounded
  * copies of f32 operands and the partial sums of split key ranges live in `workspace` (256-byte aligned; NULL / 0: allocated
  * stream-ordered, as what does not fit is; a dense launch's last round of query tiles is split in the workspace only, so
- * without it, and in fv_rt_sdpa, that launch is made unsplit, and a long masked launch takes its items from a queue there only:
- * same bits, 2 - 11 % more time without). A result from the stream-ordered allocator costs its caller a copy or a
+ * without it, and in fv_rt_sdpa, that launch is made unsplit). Calls that keep anything in one workspace and overlap on
+ * several streams race. A long masked call on bf16 operands keeps nothing there, unless its plan says FV_PLAN_OWN_WORKSPACE: then
+ * it takes its items from a queue in the workspace (1 KB more of fv_rt_sdpa_need; same bits, up to an eighth less time).
+ * A result from the stream-ordered allocator costs its caller a copy or a
  * wrapper and, after every synchronisation of the device, mapping its memory anew (0.2 - 0.35 ms for 100 MB).
  * fv_rt_sdpa_need: need_out = {result type (0 f32, 1 bf16), workspace bytes} of that call. Host arithmetic, except that
  * the number of compute units is asked of the current device once. */

@@ -71,3 +71,71 @@ def test_the_queue_in_a_graph(fv):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want), i
+
+
+def call_into(fv, q, k, v, plan, work, own):
+    """fv_rt_sdpa_into with the test's own workspace on the current stream -> the result (bf16)."""
+    import ctypes
+
+    import torch
+    from fv_sdpa import _lib
+    from fv_sdpa.sdpa import _desc_bytes, _plan_bytes
+
+    out = torch.empty_like(q)
+    rc = fv.lib().fv_rt_sdpa_into(*(_desc_bytes(x, "x") for x in (q, k, v)), _plan_bytes(plan, 0, 256 if own else 0),
+                                  out.data_ptr(), out.numel() * 2, work.data_ptr(), work.numel(), _lib.stream())
+    assert rc == 0, ctypes.string_at(fv.lib().fv_sdpa_last_error())
+    return out
+
+
+# lists of shared heads only, of whole and shared ones, with one shared head: 128 channels, where a bf16 result takes the queue
+@pytest.mark.parametrize("h,s", [(3, 175200), (12, 44000), (41, 13000)])
+def test_the_items_come_from_the_queue(fv, h, s):
+    """A call with a workspace of its own draws every item from the eight counters (32 words apart), one that shares its
+    workspace leaves it alone; the bits are the same, also where a late key makes items go again with the running max."""
+    import torch
+
+    announce(f"queue counters h={h} s={s}")
+    g = torch.Generator(device="cuda").manual_seed(h)
+    q, k, v = (torch.randn((1, h, s, 128), generator=g, device="cuda").to(torch.bfloat16) for _ in range(3))
+    t = s // 11
+    plan = fv.Plan.block_causal(None, fv.BlockCausal(t, 0, 0))
+    items = h * ((s + 255) // 256)
+    for late in (False, True):
+        if late:
+            k[:, 0, s // 2:] *= 40.0
+        n0 = fv.lib().fv_sdpa_exact_pass_reruns()
+        want = fv.sdpa_block_causal_bf16(q[0], k[0], v[0], t, 0, 0, out_bf16=True)
+        torch.cuda.synchronize()
+        n1 = fv.lib().fv_sdpa_exact_pass_reruns()
+        assert (n1 > n0) == late
+        work = torch.full((1024,), 0x55, device="cuda", dtype=torch.uint8)
+        assert torch.equal(call_into(fv, q, k, v, plan, work, own=False)[0], want)
+        assert bool((work == 0x55).all())
+        n2 = fv.lib().fv_sdpa_exact_pass_reruns()
+        assert torch.equal(call_into(fv, q, k, v, plan, work, own=True)[0], want)
+        torch.cuda.synchronize()
+        assert fv.lib().fv_sdpa_exact_pass_reruns() - n2 == n1 - n0
+        drawn = work.view(torch.int32)
+        assert int(drawn[::32].sum()) >= items and int(drawn.count_nonzero()) == 8
+
+
+def test_two_streams_share_a_workspace(fv):
+    """Two long masked calls on bf16 operands in flight with one workspace, as they may be: neither has it for its own."""
+    import torch
+
+    announce("two streams, one workspace")
+    g = torch.Generator(device="cuda").manual_seed(9)
+    sets = [[torch.randn((1, 12, 44000, 128), generator=g, device="cuda").to(torch.bfloat16) for _ in range(3)] for _ in range(2)]
+    plan = fv.Plan.block_causal(None, fv.BlockCausal(4400, 0, 0))
+    want = [fv.sdpa(*x, plan) for x in sets]
+    work = torch.zeros(1 << 20, device="cuda", dtype=torch.uint8)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in sets]
+    got = []
+    for x, s in zip(sets, streams):
+        with torch.cuda.stream(s):
+            got.append(call_into(fv, *x, plan, work, own=False))
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

@@ -285,6 +285,27 @@ def test_every_fused_kernel_has_a_form_for_the_log2_domain():
                 assert b"sdpa_short_kernelILi%dELi1ELi%dELb%dE" % (d // 16, waves, form) in text
 
 
+@pytest.mark.parametrize("kind", [2, 3])
+def test_a_masked_call_keeps_nothing_in_a_workspace_that_is_not_its_own(kind):
+    """Two long masked calls on bf16 operands may share a workspace on two streams: only a plan that says that the
+    workspace is its own (256) asks for the queue's memory. The flag belongs to these two kinds."""
+    from fv_sdpa.sdpa import _FvPlan
+
+    lib, ref, need = fv_sdpa.lib(), ctypes.byref, (ctypes.c_size_t * 2)()
+    q, k = _fake_tensor((1, 40, 32760, 128), True), _fake_tensor((1, 40, 32760, 128), True)
+    p = _FvPlan()
+    p.kv_flash = -1
+    p.block_tokens = p.frame_tokens = 1560
+    p.frames = 21
+    for flag, bytes_ in ((0, 0), (256, 1024)):
+        p.kind = kind | flag
+        assert lib.fv_rt_sdpa_need(ref(q), ref(k), ref(k), ref(p), need) == 0
+        assert need[1] == bytes_, (flag, need[1])
+    for other in (0, 1, 4):
+        p.kind = other | 256
+        assert lib.fv_rt_sdpa_need(ref(q), ref(k), ref(k), ref(p), need) == -1
+
+
 def test_need_is_host_arithmetic_at_any_shape():
     """fv_rt_sdpa_need answers for shapes the call itself refuses (no keys, no queries, no heads, lengths past every
     limit), for every kind of plan and either type: no division by a count of zero, and a workspace of zero or of the
