@@ -103,63 +103,6 @@ FV_DEV int vdn_tile_order(const Params& p, int r) {
     return back - 1 - r;   // r counts on from back - start: start - 1 down to front
 }
 
-// The keys query qi of a masked launch sees: x < a_hi || x >= c_lo || (w_lo <= x && x < w_hi).
-struct LaneMask {
-    int a_hi, c_lo, w_lo, w_hi;
-};
-template <class Params>
-FV_DEV LaneMask lane_mask(const Params& p, int qi) {
-    LaneMask m = {0, 0x7fffffff, 0, 0};
-    if (p.mask_mode == 1) {
-        // block-causal (rt/attn.rs:449-453): keys of blocks (tq - win, tq], plus the sink blocks
-        const int ft = p.ft, win = p.win;
-        const int tq = qi / ft;
-        m.a_hi = (int)min((long)p.sk, (long)p.sink * ft);
-        m.w_hi = (int)min((long)0x7fffffff, (long)(tq + 1) * ft);
-        m.w_lo = win > 0 ? max(0, tq - win + 1) * ft : 0;
-    } else {
-        // VDN window (rt/attn.rs:483-510): rows outside [vs, ve) and the frames 0 and
-        // frames-1 are dense both ways; any other frame sees the frames of its window
-        const int vs = p.vs, ve = p.ve, t = p.ft, last = p.frames - 1, c = p.chunk, r = p.radius;
-        auto lo_frame = [&](int f) { return max(0, c > 0 ? (f / c - r) * c : f - r); };
-        auto hi_frame = [&](int f) { return min(last, c > 0 ? (f / c + r + 1) * c - 1 : f + r); };
-        if (qi >= vs + t && qi < ve - t) {
-            const int qf = (qi - vs) / t;
-            m.a_hi = vs + t;
-            m.c_lo = ve - t;
-            m.w_lo = vs + lo_frame(qf) * t;
-            m.w_hi = vs + (hi_frame(qf) + 1) * t;
-        } else {
-            m.a_hi = 0x7fffffff;
-        }
-    }
-    return m;
-}
-
-// The walk positions at which each of a wave's 32 queries sees every key, from scalars, once per walk: e < a, w0 <= e < w1 or
-// e >= c. At the others the lanes ask key by key; those are the few that a range's ends or a frame boundary among the
-// queries cut (and the last, where the keys may end).
-struct WalkSight {
-    int a, w0, w1, c;
-    FV_DEV bool all(int from, int to) const { return (to < a) | ((from >= w0) & (to < w1)) | (from >= c); }
-};
-template <class Params>
-FV_DEV WalkSight walk_sight(const Params& p, const TileWalk& w, int first) {
-    int last = first + 31;
-    if (p.mask_mode == 2) {   // the rows of inner frames among them: the others see every key
-        first = max(first, p.vs + p.ft);
-        last = min(last, p.ve - p.ft - 1);
-        if (first > last) return {0x7fffffff, 0, 0, 0x7fffffff};
-    }
-    const LaneMask m0 = lane_mask(p, first), m1 = lane_mask(p, last);   // (both bounds of a window rise with the query)
-    const int w_lo = max(m0.w_lo, m1.w_lo), w_hi = min(m0.w_hi, m1.w_hi);
-    WalkSight s;
-    s.a = min(w.n0, m0.a_hi / kBN);
-    s.w0 = w.n0 + max(0, (w_lo + kBN - 1) / kBN - w.a1);
-    s.w1 = w.n0 + min(w.n1, w_hi / kBN - w.a1);
-    s.c = m0.c_lo == 0x7fffffff ? 0x7fffffff : w.n0 + w.n1 + max(0, (m0.c_lo + kBN - 1) / kBN - w.a2);
-    return s;
-}
 // The kernel's arguments read again from their segment, of which FlashParams is the whole: for code that runs rarely, so
 // that the loop around it keeps none of them in registers.
 using ConstParams = const __attribute__((address_space(4))) FlashParams;

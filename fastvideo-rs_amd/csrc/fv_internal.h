@@ -150,6 +150,79 @@ __host__ __device__ inline TileWalk mask_tile_walk(const Params& p, int q0, int 
     return w;
 }
 
+// The keys query qi of a masked launch sees: x < a_hi || x >= c_lo || (w_lo <= x && x < w_hi).
+struct LaneMask {
+    int a_hi, c_lo, w_lo, w_hi;
+};
+template <class Params>
+__host__ __device__ inline LaneMask lane_mask(const Params& p, int qi) {
+    auto imin = [](int a, int b) { return a < b ? a : b; };
+    auto imax = [](int a, int b) { return a > b ? a : b; };
+    LaneMask m = {0, 0x7fffffff, 0, 0};
+    if (p.mask_mode == 1) {
+        // block-causal (rt/attn.rs:449-453): keys of blocks (tq - win, tq], plus the sink blocks
+        const int ft = p.ft, win = p.win;
+        const int tq = qi / ft;
+        const long sink_l = (long)p.sink * ft, hi_l = (long)(tq + 1) * ft;
+        m.a_hi = (int)(sink_l < (long)p.sk ? sink_l : (long)p.sk);
+        m.w_hi = (int)(hi_l < 0x7fffffffL ? hi_l : 0x7fffffffL);
+        m.w_lo = win > 0 ? imax(0, tq - win + 1) * ft : 0;
+    } else {
+        // VDN window (rt/attn.rs:483-510): rows outside [vs, ve) and the frames 0 and
+        // frames-1 are dense both ways; any other frame sees the frames of its window
+        const int vs = p.vs, ve = p.ve, t = p.ft, last = p.frames - 1, c = p.chunk, r = p.radius;
+        auto lo_frame = [&](int f) { return imax(0, c > 0 ? (f / c - r) * c : f - r); };
+        auto hi_frame = [&](int f) { return imin(last, c > 0 ? (f / c + r + 1) * c - 1 : f + r); };
+        if (qi >= vs + t && qi < ve - t) {
+            const int qf = (qi - vs) / t;
+            m.a_hi = vs + t;
+            m.c_lo = ve - t;
+            m.w_lo = vs + lo_frame(qf) * t;
+            m.w_hi = vs + (hi_frame(qf) + 1) * t;
+        } else {
+            m.a_hi = 0x7fffffff;
+        }
+    }
+    return m;
+}
+
+// The walk positions at which each of a wave's 32 queries sees every key, from scalars, once per walk: e < a, w0 <= e < w1 or
+// e >= c. At the others the lanes ask key by key; those are the few that a range's ends or a frame boundary among the
+// queries cut (and the last, where the keys may end). Every visible range counts in every range of the walk: a query tile
+// with a row of an anchor frame walks everything in one. (With ranges matched to ranges its tiles past the first frame were
+// taken for cut: VDN windows that cover the clip, 12 heads 12 x 390 174 us instead of 110, 12 x 880 645 instead of 510; 12 heads 32 x
+// 1560 chunk 5 5872 instead of 5626.)
+struct WalkSight {
+    int a, w0, w1, c;
+    __host__ __device__ inline bool all(int from, int to) const { return (to < a) | ((from >= w0) & (to < w1)) | (from >= c); }
+};
+template <class Params>
+__host__ __device__ inline WalkSight walk_sight(const Params& p, const TileWalk& w, int first) {
+    constexpr int kNone = 0x7fffffff;
+    auto imin = [](int a, int b) { return a < b ? a : b; };
+    auto imax = [](int a, int b) { return a > b ? a : b; };
+    int last = first + 31;
+    if (p.mask_mode == 2) {   // the rows of inner frames among them: the others see every key
+        first = imax(first, p.vs + p.ft);
+        last = imin(last, p.ve - p.ft - 1);
+        if (first > last) return {kNone, 0, 0, kNone};
+    }
+    const LaneMask m0 = lane_mask(p, first), m1 = lane_mask(p, last);   // (both bounds of a window rise with the query)
+    const int w_lo = imax(m0.w_lo, m1.w_lo), w_hi = imin(m0.w_hi, m1.w_hi);
+    int a = m0.a_hi, c = m0.c_lo;
+    if (w_lo < w_hi) {   // a window that touches its neighbours is one range with them
+        if (w_lo <= a) a = imax(a, w_hi);
+        if (w_hi >= c) c = imin(c, w_lo);
+        if (a >= c) a = kNone;
+    }
+    // positions of the walk whose tile lies before tile t
+    auto before = [&](int t) {
+        return imin(t, w.n0) + imin(imax(t - w.a1, 0), w.n1) + imin(imax(t - w.a2, 0), w.ne - w.n0 - w.n1);
+    };
+    auto up = [](int x) { return (x >> 6) + ((x & 63) != 0); };
+    return {before(a >> 6), before(up(w_lo)), before(w_hi >> 6), c == kNone ? kNone : before(up(c))};
+}
+
 }  // namespace fv
 
 // y = bf16(x * mul), RNE, for up to three operands in one launch

@@ -72,3 +72,13 @@ def test_oracle_c_functions_are_clean_under_address_and_undefined_sanitizers(tmp
     env["ASAN_OPTIONS"] = "detect_leaks=1:verify_asan_link_order=0"
     out = subprocess.run([exe], capture_output=True, text=True, timeout=120, env=env)
     assert out.returncode == 0 and "oracle sanitizer run: ok" in out.stdout, (out.returncode, out.stdout[-500:], out.stderr[-3000:])
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="no hipcc")
+def test_walk_positions_that_a_wave_sees_whole(tmp_path):
+    """walk_sight (host code of the kernels' header) against the masks key by key."""
+    exe = str(tmp_path / "walk_sight")
+    subprocess.check_call(["hipcc", "--offload-host-only", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "fastvideo-rs_amd", "csrc"),
+                           os.path.join(ROOT, "tests", "c_abi", "walk_sight.hip"), "-o", exe])
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0 and int(out.stdout) > 50000, out.stdout
