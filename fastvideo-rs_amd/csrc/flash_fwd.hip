@@ -597,11 +597,9 @@ FV_DEV bool flash_item(const Params& p, const int wave, const int lane, const in
 // take more (the rest find nothing and end). A list is the whole heads x * a .. one after the other and, tile by tile, a share of the
 // heads past the last multiple of eight: one head at a time goes through an L2. An item is a (head, query tile), counted as
 // `work` in flash_item.
-// us, in the order of the numbers / so: causal 40 heads 21 x 1560 8748 / 8127 (36 % of the L2 lines missed before), VDN window 40 heads
-// 18 x 880 chunk 5 radius 2 3997 / 3566, 12 heads 32 x 1560 chunk 5 radius 1 6001 / 5860, 24 heads 24 x 1560 radius 2 4849 / 4844. Launches
-// of less than eight rounds keep the order of the numbers: there a list by head ends too unevenly (12 heads, 7 frames 354 / 425),
-// and one by length is no faster (354 / 355; 24 heads, 8 frames, a window of 4 690 / 699). One workgroup a CU that walks item after
-// item needs registers that the main loop then misses: 8649 and 3863 where this form has 8345 and 3712.
+// Which launches gain by it: fv_masked_workspace_bytes (causal 40 heads 21 x 1560 8624 us in the order of the numbers, where 36 % of the
+// L2 lines missed, 7979 so). One workgroup a CU that walks item after item needs registers that the main loop then misses: 8649 and 3863
+// where this form had 8345 and 3712 (those two: before a tile's bounds were one word of bits).
 template <class Params>
 FV_DEV int queue_item(const Params& p, int x, int j) {
     const int nqt = p.nqt, nbh = p.total / nqt, a = nbh >> 3, c = nbh & 7;

@@ -121,7 +121,7 @@ struct MaskArgs {
     int short_waves = 0;                          // > 0: the short kernel, with as many waves a workgroup
     void* workspace = nullptr;                    // ... and their partial results
     size_t workspace_bytes = 0;
-    int* queue = nullptr;                         // masked: kFvQueueBytes for the queue of its items, or none
+    int* queue = nullptr;                         // masked: kFvQueueBytes for the queue of its items, or in the order of their numbers
     size_t block_tokens = 0, window = 0, sink = 0;                           // block-causal
     size_t video_start = 0, frame_tokens = 0, frames = 0, chunk = 0, radius = 0;   // VDN window
 };
@@ -268,7 +268,7 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
         const hipError_t e = fv_internal_launch_duo(&p, mode != kMaskNone ? 1 : 0, (int)d, (hipStream_t)stream);
         return e == hipSuccess ? FV_OK : fail_hip(e, "flash_fwd_duo");
     }
-    if (mode != kMaskNone && m.queue && fv_masked_workspace_bytes(bh, sq)) {
+    if (mode != kMaskNone && m.queue) {
         p.queue = m.queue;
         const hipError_t e = fv_internal_clear_queue(p.queue, (hipStream_t)stream);
         if (e != hipSuccess) return fail_hip(e, "clear_queue");
@@ -393,10 +393,32 @@ int fv_dense_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, vo
     return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
 }
 
-// (eight rounds of query tiles: see take_item)
-size_t fv_masked_workspace_bytes(size_t bh, size_t sq) {
+// The queue (take_item in flash_fwd.hip) saves L2 misses where walks are long, and goes through its lists head by head: the last
+// head's longest walk may begin near the end. So it takes launches of eight rounds and more at 128 channels whose walks are
+// 4096 keys long on average and whose work is four times a CU's longest walk. us, in the order of the numbers / from the queue, with
+// that ratio: causal 40 x 21 x 1560 (10) 8624 / 7979, 12 x 32 x 1560 (4.6) 5795 / 5535, 40 x 21 x 1560 under a window of four with a sink 3863
+// / 3747; VDN window 40 x 18 x 880 chunk 5 radius 2 (9.7) 3781 / 3524, 40 x 21 x 1560 radius 2 (7.9) 6917 / 6787, 12 x 32 x 1560 chunk 5
+// (5.1) 6033 / 5911, 24 x 24 x 1560 radius 2 (4.8) 4787 / 4782 and f32 results 5310 / 5084. Past the lines: 24 x 40 x 1560 radius 1 (3.9) 6735 /
+// 6887, 12 x 60 x 1560 radius 2 (2.5) 6564 / 8292, 40 x 40 x 390 radius 0 (1.2) 766 / 961; causal under a window of one 12 x 32 x 1560
+// (1535 keys) 601 / 616, 40 x 34 x 390 267 / 292; f32 results at 64 channels causal 24 x 21 x 1560 3567 / 3634, VDN 12 x 32 x 1560 chunk 5
+// 4382 / 4424. (Numbers as they come: the bounds of a mask are judged by the launch.)
+size_t fv_masked_workspace_bytes(size_t bh, size_t sq, size_t sk, size_t d, const FvMask& m) {
     const size_t cus = (size_t)fv_compute_units(), bm = (size_t)fv_internal_flash_block_m();
-    return cus >= 8 && bh * ((sq + bm - 1) / bm) >= 8 * cus ? kFvQueueBytes : 0;
+    const double tiles = (double)bh * (double)((sq + bm - 1) / bm), nq = (double)sq, nk = (double)sk;
+    if (d != 128 || cus < 8 || tiles < 8.0 * (double)cus) return 0;
+    double mean, longest;   // keys of a walk
+    if (m.causal) {
+        const double seen = ((double)m.window + (double)m.sink) * (double)m.block_tokens;
+        longest = std::min(m.window > 0 ? std::min(seen, nk) : nk, nq);
+        mean = longest * (1.0 - longest / (2.0 * nq));   // (the first queries see less)
+    } else {
+        const double frames = (double)m.frames, ft = (double)m.frame_tokens;
+        const double seen = std::min(frames, 2.0 + (2.0 * (double)m.radius + 1.0) * std::max(1.0, (double)m.chunk));
+        const double inner = std::min(std::max(0.0, frames - 2.0) * ft, nq);
+        longest = nk;
+        mean = ((nq - inner) * nk + inner * std::max(0.0, nk - (frames - seen) * ft)) / nq;
+    }
+    return mean >= 4096.0 && tiles * mean >= 4.0 * (double)cus * longest ? kFvQueueBytes : 0;
 }
 
 int fv_masked_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out, int out_is_bf16, size_t bh,
@@ -411,7 +433,7 @@ int fv_masked_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, v
     m.frames = mask.frames;
     m.chunk = mask.chunk;
     m.radius = mask.radius;
-    m.queue = (int*)workspace;
+    if (fv_masked_workspace_bytes(bh, sq, sk, d, mask)) m.queue = (int*)workspace;
     return flash_common(q, k, v, out, out_is_bf16, bh, sq, sk, d, scale, m, stream);
 }
 

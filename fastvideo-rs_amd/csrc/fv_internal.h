@@ -260,7 +260,7 @@ struct FvMask {
     size_t block_tokens, window, sink;                            // block-causal
     size_t video_start, frame_tokens, frames, chunk, radius;      // VDN window
 };
-size_t fv_masked_workspace_bytes(size_t bh, size_t sq);
+size_t fv_masked_workspace_bytes(size_t bh, size_t sq, size_t sk, size_t d, const FvMask& mask);
 // fv_sdpa_block_causal_bf16 or fv_sdpa_vdn_window_bf16 with such a workspace, or without one (null)
 int fv_masked_planned(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out, int out_is_bf16, size_t bh,
                       size_t sq, size_t sk, size_t d, float scale, const FvMask& mask, void* workspace, void* stream);

@@ -256,6 +256,9 @@ FvSplitPlan dense_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16)
     return p;
 }
 
+FvMask mask_of(const BlockCausal& c) { return {true, c.block_tokens, c.window, c.sink, 0, 0, 0, 0, 0}; }
+FvMask mask_of(const VdnWindow& w) { return {false, 0, 0, 0, w.video_start, w.frame_tokens, w.frames, w.chunk, w.radius}; }
+
 // One fused launch (dense, block-causal or VDN window); nullopt = the kernel declined.
 Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tensor& v,
                                     std::optional<float> scale, bool out_bf16,
@@ -301,11 +304,9 @@ Result<std::optional<Tensor>> fused(const Tensor& q, const Tensor& k, const Tens
     const uint16_t *pq = bits[0], *pk = bits[1], *pv = bits[2];
     int rc;
     if (causal || window) {
-        FvMask m{};
-        if (causal) m = {true, causal->block_tokens, causal->window, causal->sink, 0, 0, 0, 0, 0};
-        else m = {false, 0, 0, 0, window->video_start, window->frame_tokens, window->frames, window->chunk, window->radius};
+        const FvMask m = causal ? mask_of(*causal) : mask_of(*window);
         Tensor ws;
-        const size_t need = fv_masked_workspace_bytes(s->b * s->h, s->sq);
+        const size_t need = fv_masked_workspace_bytes(s->b * s->h, s->sq, s->sk, s->d, m);
         if (need && st.own && st.holds(need)) {   // (counters that two launches shared would leave rows of both unwritten)
             auto rw = st.temp({need / 4}, DType::F32);
             if (is_ok(rw)) ws = std::move(std::get<Tensor>(rw));
@@ -760,7 +761,8 @@ Need sdpa_need(const Tensor& q, const Tensor& k, const Tensor& v, const Plan& pl
     if (plan.kind == Plan::Kind::Dense || plan.kind == Plan::Kind::KvWindow) {
         n.workspace += (dense_plan(s->b * s->h, s->sq, s->sk, s->d, act16).workspace_bytes + 255) & ~(size_t)255;
     } else if (plan.own_workspace) {
-        n.workspace += fv_masked_workspace_bytes(s->b * s->h, s->sq);
+        n.workspace += fv_masked_workspace_bytes(s->b * s->h, s->sq, s->sk, s->d,
+                                                 plan.kind == Plan::Kind::BlockCausalK ? mask_of(plan.causal) : mask_of(plan.window));
     }
     return n;
 }

@@ -306,6 +306,40 @@ def test_a_masked_call_keeps_nothing_in_a_workspace_that_is_not_its_own(kind):
         assert lib.fv_rt_sdpa_need(ref(q), ref(k), ref(k), ref(p), need) == -1
 
 
+# (kind, heads, frame, frames, window or chunk, sink or radius, channels, whether its items come from the queue)
+QUEUED = [
+    (2, 40, 1560, 21, 0, 0, 128, True),      # causal, the mean walk half the longest
+    (2, 12, 1560, 21, 0, 0, 128, False),     # six rounds
+    (2, 40, 1560, 21, 0, 0, 64, False),
+    (2, 40, 1560, 21, 4, 1, 128, True),      # a window: walks of one length, long ...
+    (2, 12, 1560, 32, 1, 0, 128, False),     # ... and short
+    (2, 12, 1560, 32, 1 << 62, 1 << 62, 128, True),
+    (3, 12, 1560, 32, 5, 1, 128, True),
+    (3, 40, 880, 18, 5, 2, 128, True),       # the window covers the clip
+    (3, 12, 1560, 60, 0, 2, 128, False),     # the first and last frame's walks are much longer than the others
+    (3, 40, 390, 40, 0, 0, 128, False),
+    (3, 12, 1560, 32, 1 << 62, 1 << 62, 128, True),
+]
+
+
+@pytest.mark.parametrize("kind,h,frame,frames,a,b,d,queued", QUEUED)
+def test_which_masked_calls_ask_for_the_queue(kind, h, frame, frames, a, b, d, queued):
+    """Eight rounds of query tiles are not enough: walks of very unequal length end late where the queue's lists go head by
+    head (12 heads 60 x 1560, radius 2: 8.3 ms instead of 6.6), short ones do not gain."""
+    from fv_sdpa.sdpa import _FvPlan
+
+    need = (ctypes.c_size_t * 2)()
+    q = _fake_tensor((1, h, frame * frames, d), True)
+    p = _FvPlan()
+    p.kv_flash, p.kind = -1, kind | 256
+    if kind == 2:
+        p.block_tokens, p.window, p.sink = frame, a, b
+    else:
+        p.frame_tokens, p.frames, p.chunk, p.radius = frame, frames, a, b
+    assert fv_sdpa.lib().fv_rt_sdpa_need(*[ctypes.byref(q)] * 3, ctypes.byref(p), need) == 0
+    assert need[1] == (1024 if queued else 0)
+
+
 def test_need_is_host_arithmetic_at_any_shape():
     """fv_rt_sdpa_need answers for shapes the call itself refuses (no keys, no queries, no heads, lengths past every
     limit), for every kind of plan and either type: no division by a count of zero, and a workspace of zero or of the
