@@ -780,7 +780,15 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
     f32x4 o[kNO][2], s_init[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     SoftmaxOffState st;
     ProbTile pb;
-    constexpr int kAhead = 3;
+    // Two waves of a SIMD that are in step halve its rate: both multiply, then both are at their softmax. Where walks are of one
+    // length and the launch is one round they start so, and the softmax, the longer part, goes first: whoever reaches it
+    // gets its issue slots while the other multiplies. With the matrix part first, which served the 32x32x16 form well, waves stayed
+    // in step. At 64 channels four groups of operands are read ahead, whose MFMAs leave the port to the other wave's softmax.
+    // us, 32x32x16 form / matrix part first, three ahead / now, at 64 channels: 9 x 4000 x 512 12.3 / 13.0 / 12.5, x 1024 18.2 / 20.4 / 18.6,
+    // x 4096 54.4 / 63.0 / 54.6, 16 x 2560 x 2048 30.9 / 34.9 / 30.8, 16 x 4000 x 4096 70.9 / 72.6 / 66.6, 16 x 7680 x 3000 103.5 / 101.0 / 98.1; at
+    // 128: 9 x 4000 x 512 16.5 / 17.6 / 17.1, 16 x 4000 x 700 26.8 / 25.8 / 25.2, 12 x 32760 x 512 108.6 / 103.4 / 103.3. (Masked walks,
+    // which differ in length, lose by it: causal 24 x 8 x 880 at 64 channels 183.5 / 187.5.)
+    constexpr int kAhead = D == 64 && !MASKED ? 4 : 3, kMatrixPrio = MASKED ? 1 : 0, kSoftmaxPrio = 1 - kMatrixPrio;
     int kv = kv0_of(0), kk = kv0_of(1);   // first keys of the tiles that the next matrix part loads: V, K
     wait_vmcnt<0>();
     block_barrier();   // K(0), K(1) resident, every wave has its queries
@@ -799,18 +807,18 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
         auto hook_v1 = [&](int i) {
             if (i < kUnits) load_v(1, kk, i);
         };
-        __builtin_amdgcn_s_setprio(1);
+        __builtin_amdgcn_s_setprio(kMatrixPrio);
         mfma_phase<false, kAhead, D>(vbuf(0), kbuf(0), rb, pb, o, qf, s0, s_init, hook_v0);
         ProbTile pa;
         if (ne > 1) {
             mfma_phase<false, kAhead, D>(vbuf(0), kbuf(1), rb, pb, o, qf, s1, s_init, hook_v1);
-            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_s_setprio(kSoftmaxPrio);
             __builtin_amdgcn_sched_barrier(0);
             mask_tile(s0, 0);
             mask_tile(s1, 1);
             softmax_first_off<!LOG2DOM>(s0, s1, st, s_init, sl2, pa, pb);
         } else {
-            __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_s_setprio(kSoftmaxPrio);
             __builtin_amdgcn_sched_barrier(0);
             mask_tile(s0, 0);
             softmax_first_off<!LOG2DOM>(s0, st, s_init, sl2, pa);
@@ -826,7 +834,7 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
         for (int db = 0; db < kNO; db++)
 #pragma unroll
             for (int g = 0; g < 2; g++) o[db][g] = f32x4{0.f, 0.f, 0.f, 0.f};
-        __builtin_amdgcn_s_setprio(1);
+        __builtin_amdgcn_s_setprio(kMatrixPrio);
         pv_tile<D>(vbuf(0), rb.v, pa, o);
         kk = kv0_of(3);
         kv = kv0_of(2);
@@ -839,9 +847,9 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
             if (i < kUnits) load_v(m, kv, i);
             else if (i < 2 * kUnits) load_k(m + 1, kk, i - kUnits);
         };
-        __builtin_amdgcn_s_setprio(1);
+        __builtin_amdgcn_s_setprio(kMatrixPrio);
         mfma_phase<true, kAhead, D>(vbuf(m - 1), kbuf(m), rb, pb, o, qf, s, s_init, hook_dma);
-        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_s_setprio(kSoftmaxPrio);
         __builtin_amdgcn_sched_barrier(0);
         mask_tile(s, m);
         if constexpr (FIXED) {
@@ -857,9 +865,9 @@ FV_DEV bool duo_item(const Params& p, const int wave, const int lane, const int 
         block_barrier();   // K(m+1), V(m) resident; this phase's tiles read by every wave
         __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_s_setprio(1);
+    __builtin_amdgcn_s_setprio(kMatrixPrio);
     if (ne > 1) pv_tile<D>(vbuf(ne - 1), rb.v, pb, o);
-    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_s_setprio(kSoftmaxPrio);
 
     if constexpr (FIXED) {   // did the fixed offset hold (flash_item)?
         float chk = 0.f;
