@@ -135,7 +135,8 @@ _TENSOR_BYTES = struct.Struct("@Pii9N")
 _PLAN_BYTES = struct.Struct("@iifPi8Ni0P")
 assert _TENSOR_BYTES.size == C.sizeof(_FvTensor) and _PLAN_BYTES.size == C.sizeof(_FvPlan)
 _NO_SHAPE = (0,) * 8
-_OWN_WORKSPACE = 256   # FV_PLAN_OWN_WORKSPACE
+_OWN_WORKSPACE = 256   # FV_PLAN_OWN_WORKSPACE, of these kinds
+_OWN_KINDS = (Plan.BLOCK_CAUSAL, Plan.VDN_WINDOW)
 _BF16, _F32 = torch.bfloat16, torch.float32
 
 
@@ -171,7 +172,9 @@ def _desc(t, name):
 def _plan_bytes(plan, mask, flags=0):
     """`plan` as the bytes of a struct fv_plan; `mask`: the address of its mask's struct fv_tensor, or 0;
     `flags`: or'ed into its kind."""
-    scale, causal, window, kind = plan.scale, plan.causal, plan.window, plan.kind | flags
+    scale, causal, window, kind = plan.scale, plan.causal, plan.window, plan.kind
+    if flags:
+        kind |= flags
     causal = (causal.block_tokens, causal.window, causal.sink) if causal is not None else (0, 0, 0)
     window = window._args() if window is not None else (0, 0, 0, 0, 0)
     kv_flash = -1 if plan.kv_flash is None else int(plan.kv_flash)
@@ -196,9 +199,8 @@ def sdpa(q, k, v, plan):
     mask = None
     if plan.mask is not None:
         mask = C.create_string_buffer(_desc_bytes(plan.mask, "mask"), _TENSOR_BYTES.size)   # alive until the call is made
-    kind = plan.kind   # (the workspace of a block-causal or window call is allocated below, for it alone)
-    p = _plan_bytes(plan, 0 if mask is None else C.addressof(mask),
-                    _OWN_WORKSPACE if kind == Plan.BLOCK_CAUSAL or kind == Plan.VDN_WINDOW else 0)
+    # (the workspace of a block-causal or window call is allocated below, for it alone)
+    p = _plan_bytes(plan, 0 if mask is None else C.addressof(mask), _OWN_WORKSPACE if plan.kind in _OWN_KINDS else 0)
     need = (C.c_size_t * 2)()
     rc = lib.fv_rt_sdpa_need(dq, dk, dv, p, need)
     if rc != 0:
