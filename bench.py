@@ -27,7 +27,7 @@ PEAK_HBM_GBS = 8000.0
 # HBM bytes per launch of the flash kernel at the headline workload. NOT measured by this script: the figure
 # comes from two rocprofv3 --pmc runs of this same command (FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 KiB, the
 # factors from a plain 1 GiB copy in the same runs), whose summary is the file named beside it.
-MEASURED_TRAFFIC_BYTES = {"self": (1.0069e9, "profiles/flash_fwd_pp2_wan13b_self_attention.md")}
+MEASURED_TRAFFIC_BYTES = {"self": (1.0067e9, "profiles/flash_fwd_pp2_wan13b_self_attention.md")}
 
 WORKLOADS = {
     # name: (H, Sq, Sk, causal block_tokens or 0, description)
@@ -125,7 +125,7 @@ def bench_vsa(args):
         "whole_op_tile_ordered_inputs_ms": {"avg": round(avg_t, 4), "median": round(med_t, 4), "wall": round(wall_t, 4)},
         "stages_median_ms": {k2: round(v2, 4) for k2, v2 in stages.items()},
         "roofline": {"bound": "mfma", "achieved": round(fine_tflops, 3), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(fine_tflops / PEAK_BF16_TFLOPS, 4), "traffic": None, "kernel": "fv::vsa_fine_kernel<false>",
+                     "frac": round(fine_tflops / PEAK_BF16_TFLOPS, 4), "traffic": None, "kernel": "fv::vsa_fine_kernel",
                      "avg_kernel_ms": round(stages["fine"], 4),
                      "banded_selection_tflops": round(flops / (stages["fine_banded_selection"] * 1e-3) / 1e12, 3)},
     }
@@ -220,7 +220,7 @@ def bench_kvcache(args, fpb=3):
         "ms_per_step_with_window_copies_no_split": round(copied, 4), "ms_per_step_in_place_no_split": round(unsplit, 4),
         "ms_per_step_eager_python_loop": round(eager, 4),
         "roofline": {"bound": "mfma", "achieved": round(tf, 3), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(tf / PEAK_BF16_TFLOPS, 4), "traffic": None, "kernel": "fv::flash_fwd_pp2<2, false, 128, false, true>"},
+                     "frac": round(tf / PEAK_BF16_TFLOPS, 4), "traffic": None, "kernel": "fv::flash_fwd_pp2<2, false, 128, false, true, false>"},
     }
     print(json.dumps(rec), flush=True)
 
@@ -655,6 +655,16 @@ def main():
     traffic, traffic_source = MEASURED_TRAFFIC_BYTES.get(args.workload, (None, None)) if args.out_bf16 else (None, None)
     if traffic_source:
         traffic_source += " (rocprofv3 --pmc runs of this command; not measured in this run)"
+    fixed = args.out_bf16 and os.environ.get("FASTVIDEO_SDPA_RUNNING_MAX", "0") in ("", "0")
+    fold = "true" if args.fold_scale else "false"
+    if args.workload == "tiny":
+        kernel = f"fv::sdpa_short_kernel<8, 1, 8, {fold}>"
+    elif sk == 512 and fixed:   # cross-attention: few keys
+        kernel = f"fv::flash_fwd_duo<false, {d}, {fold}>"
+    else:
+        # template arguments: groups of four waves, masked, head dim, scale folded into Q, fixed-offset first pass (launches
+        # that write bf16 and whose queries all see key 0: every workload here), planes of 4 GB and more
+        kernel = f"fv::flash_fwd_pp2<2, {'true' if bt else 'false'}, {d}, {fold}, {'true' if fixed else 'false'}, false>"
     rec = {
         "metric": "SDPA TFLOP/s + % bf16 MFMA peak, Wan-1.3B 480p self-attn (S=32760,H=12,d=128)"
         if args.workload == "self" and not args.fold_scale else
@@ -678,10 +688,7 @@ def main():
         "roofline": {"bound": "mfma", "achieved": round(achieved, 3), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_BF16_TFLOPS, 4),
                      "traffic": traffic, "traffic_source": traffic_source,
-                     # template arguments: groups of four waves, masked, head dim, scale folded into Q, fixed-offset first pass (launches
-                     # that write bf16 and whose queries all see key 0: every workload here)
-                     "kernel": f"fv::flash_fwd_pp2<2, {'true' if bt else 'false'}, {d}, {'true' if args.fold_scale else 'false'}, "
-                               f"{'true' if args.out_bf16 and os.environ.get('FASTVIDEO_SDPA_RUNNING_MAX', '0') in ('', '0') else 'false'}>",
+                     "kernel": kernel,
                      "avg_kernel_ms": round(avg_kernel_ms, 4), "median_kernel_ms": round(kern_ms[len(kern_ms) // 2], 4),
                      "min_hbm_bytes": bytes_min,
                      "hbm_frac_at_min_traffic": round(bytes_min / (avg_kernel_ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4)},

@@ -34,8 +34,8 @@ struct TileGeo {
     static constexpr int kChunks = kRow / 16;            // 16-byte chunks per row
     static constexpr int kRowsPerDma = 1024 / kRow;      // rows one wave-wide DMA instruction covers
     static constexpr int kDmaPerTile = kTile / 1024;
-    static constexpr int kVGroups = D / 16;              // PV groups per tile (2 MFMAs each)
-    static constexpr int kKGroups = D / 16;              // QK groups per tile
+    static constexpr int kVGroups = D / 16;              // PV groups per tile (two operand fragments, 4 MFMAs each)
+    static constexpr int kKGroups = D / 16;              // QK groups per tile (the same)
     static constexpr int kGroups = kVGroups + kKGroups;
     static FV_DEV int kswz(int r) { return D == 128 ? (r & 15) : ((r >> 1) & 7); }
     static FV_DEV int vswz(int r) { return D == 128 ? ((r & 7) << 1) : (((r >> 1) & 3) << 1); }
@@ -371,7 +371,7 @@ FV_DEV void pv_tile(const lds_u8* vb, int v_base, const ProbTile& pb, f32x4 (&o)
 // One MFMA phase over NT key tiles with a deep, explicit LDS prefetch: for each of them O^T += V^T P^T of the
 // tile NT before it (if DO_PV), then S^T = K Q^T. A group is 2 operand fragments (8 VGPRs), each feeding the MFMAs of both
 // query blocks; the first K MFMAs of a key block take `s_init` as their C operand (zeros, or minus the
-// softmax offset of the lane's queries). kAhead (2-3, bounded by the 256-VGPR budget) groups are always in flight ahead of the group
+// softmax offset of the lane's queries). kAhead (3, or 4 where the registers allow it) groups are always in flight ahead of the group
 // being multiplied, so an MFMA waits on a read issued kAhead x 64 cycles of
 // matrix-pipe time earlier instead of on LDS latency plus the 64 B/clk per-SIMD
 // LDS return path. sched_barrier keeps the compiler from re-serialising reads

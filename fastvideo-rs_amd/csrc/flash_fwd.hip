@@ -17,8 +17,9 @@
 //     random operands the chip sustains 2.01 PFLOP/s of it from registers and 1.74 with this kernel's LDS reads,
 //     1.73 and 1.52 of v_mfma_f32_32x32x16_bf16 on the same operands (on zeros both 2.45). Its MFMAs are twice as many
 //     and take the SIMD's issue port twice as long, so everything else in a phase had to shrink with it. Together, against
-//     the 32x32 form: 12 x 32760 x 32760 x 128 5.34 -> 4.76 ms, 40 x 75600 92.3 -> 84.7, block-causal 21 x 1560
-//     2.91 -> 2.67, 24 x 7800 x 7800 x 64 366 -> 344 us;
+//     the 32x32 form: 12 x 32760 x 32760 x 128 4.92 -> 4.40 ms, block-causal 21 x 1560 2.69 -> 2.55, 24 x 7800 x 7800 x 64
+//     363 -> 344 us. Launches that the power limit does not hold, of one round, lose by it where the softmax is the longer
+//     part: f32 results 12 x 4000 x 4096 x 64 66.2 -> 70.2 us;
 //   * P^T (bf16, RNE) is the B operand of O^T = V^T P^T straight from those
 //     registers (the contraction index is a fixed permutation of the keys,
 //     matched on the V side); V^T fragments are read from the row-major
@@ -40,7 +41,7 @@
 //     XOR-swizzled unpadded tiles, four buffers each; rows past the last key are the descriptor's business;
 //   * dense launches remap workgroup ids so that the workgroups resident on one
 //     XCD walk consecutive query tiles of the same head (their K/V stream hits
-//     that XCD's L2); block-causal launches run longest tiles first.
+//     that XCD's L2); masked launches run longest tiles first, long ones from a queue head by head (take_item).
 //
 // Time is counted in slots (one phase each); a phase covers a PAIR of key tiles
 // (128 keys): a matrix phase is 128 MFMAs (PV of the previous pair, QK of the

@@ -131,14 +131,16 @@ struct MaskArgs {
 // the first two tiles of every walk are keys 0 to 127 whatever the query tile's size. Its tiles of 128 queries cross fewer frame boundaries and leave a shorter
 // last round, which counts where a query reaches few keys; long walks run at the chip's power limit, where 256 queries to a
 // K and V stream cost less. Causal launches without a window, whose walks are half their reach on average, and windows that
-// are part of their clip take it up to 8192 keys reached, walks of one length up to 4096. us, flash_fwd_pp2 / flash_fwd_duo,
-// heads x frame x frames (keys reached): causal 12 x 880 x 2 (1760) 59 / 56, 12 x 390 x 6 in blocks of 3 (2340) 97 / 68, 24 x 390 x 8
-// (3120) 94 / 82, 40 x 390 x 12 in blocks of 3 (4680) 303 / 270, 24 x 880 x 8 (7040) 341 / 318, 12 x 1560 x 4 (6240) 180 / 181;
-// under a window 12 x 880 x 8 (3520) 172 / 164, 24 x 880 x 8 with a sink (3520) 266 / 255, 12 x 1560 x 6 (6240) 304 / 314, x 8 438 / 425,
-// 12 x 1560 x 12 (18720) 1211 / 1250; VDN window 40 x 390 x 16 (2730) 452 / 410, 12 x 880 x 10 (4400) 390 / 317, 24 x 390 x 20 (6630)
-// 518 / 508, 12 x 1560 x 24 (7800) 2383 / 2102, 40 x 1560 x 12 (7800) 3199 / 3213, 24 x 880 x 12 (9680) 930 / 945, 12 x 1560 x 32 (26520)
-// 6478 / 6623, over the whole clip 12 x 390 x 8 (3120) 97 / 82, 12 x 390 x 12 (4680) 120 / 125. At head dim 64 causal 24 x 880 x 4
-// 92 / 83, 12 x 1560 x 21 (32760) 1817 / 1674.
+// are part of their clip take it up to 8192 keys reached, walks of one length up to 4096; near those lines the two are within
+// 7 %. us, flash_fwd_pp2 / flash_fwd_duo, heads x frame x frames (keys reached): causal 12 x 880 x 2 (1760) 46 / 40, 12 x 390 x 6 in
+// blocks of 3 (2340) 66 / 51, 24 x 390 x 8 (3120) 78 / 71, 40 x 390 x 12 in blocks of 3 (4680) 257 / 241, 24 x 880 x 8 (7040) 291 / 284,
+// 12 x 1560 x 4 (6240) 141 / 140, x 5 (7800) 190 / 200, 24 x 1560 x 6 (9360) 490 / 506; under a window with a sink 12 x 880 x 8 (2640)
+// 130 / 113, 24 x 880 x 8 (3520) 245 / 224, 12 x 1560 x 6 (6240) 245 / 261, x 8 343 / 337, 12 x 1560 x 12 (18720) 882 / 893; VDN window
+// 40 x 390 x 16 (2730) 415 / 381, 12 x 880 x 10 (4400) 276 / 266, 24 x 390 x 20 (6630) 484 / 448, 12 x 1560 x 24 (7800) 1999 / 2005, 40 x
+// 1560 x 12 (7800) 2983 / 3116, 24 x 880 x 12 (9680) 881 / 834, 12 x 1560 x 24 (10920) 2389 / 2464, x 32 (26520) 5962 / 6335, over the whole
+// clip 12 x 390 x 8 (3120) 67.8 / 67.2, 12 x 390 x 12 (4680) 109 / 113. At head dim 64 causal 24 x 880 x 4 71 / 68, 12 x 1560 x 21 (32760)
+// 1743 / 1617, 40 x 1560 x 21 5543 / 5590, 40 x 1560 x 12 under a window of 3 with a sink 1312 / 1106, VDN window 12 x 1560 x 32 chunk 5
+// 4129 / 3800.
 bool duo_masked(const fv::FlashParams& p, size_t bh, size_t d) {
     const long ft = p.ft;
     const bool causal = p.mask_mode == kMaskBlockCausal;
@@ -250,7 +252,7 @@ int flash_common(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* 
     // Kernel-level calls take the short kernel up to 512 keys. Past them fv_rt_sdpa alone asks for it (short_waves): there
     // these calls are flash_fwd_pp2's or flash_fwd_duo's, whose bits a block-causal clip of one block then shares with the
     // first block of a longer one, for both result types (one frame has 880 tokens and more); it costs them what the short
-    // kernel gains, 24.3 us instead of 16.8 at 12 x 1000 x 1000 x 128, 21.1 instead of 11.9 at 12 x 600 x 1000.
+    // kernel gains, 22.8 us instead of 16.7 at 12 x 1000 x 1000 x 128, 19.2 instead of 10.8 at 12 x 600 x 1000.
     int short_waves = m.short_waves;
     if (mode == kMaskNone && splits == 1 && !short_waves && sk <= 512) short_waves = fv_short_waves(bh, sq, sk, d);
     if (short_waves) {
@@ -300,11 +302,12 @@ int fv_compute_units() {
 // The short kernel (composed_fwd.hip) takes calls whose 32-query groups are one round of resident workgroups: of eight
 // waves where each has a CU to itself, of four up to two a CU (three at head dim 64, which has room for four), while the walk of the keys is
 // short enough that sharing it out over the chip (split-KV) or reading K and V once for 128 or 256 queries gains less. us in a
-// graph, flash_fwd_pp2 / short: at 128 channels 12 x 320 x 320 11.0 / 6.8, 3 x 390 x 200 9.6 / 6.4, 12 x 600 x 1000 21.1 / 11.9,
-// x 3000 30.9 / 23.7, x 5000 (12 x 320) 33.6 / 31.7, (3 x 390) 25.5 / 30.7; 264 to 512 groups 12 x 680 x 500 13.8 / 11.4,
-// 12 x 1000 x 1000 24.3 / 16.8, x 2000 31.1 / 28.4, x 3000 35.9 / 38.7; 516 groups 12 x 1360 x 500 14.4 / 16.8, x 2000 37 / 43.
-// At 64 channels 12 x 320 x 320 8.0 / 4.9, 3 x 390 x 3000 16.6 / 13.5, x 5000 19.6 / 19.4, 12 x 1000 x 3000 27.5 / 23.0 (four
-// waves 24.5), 12 x 1560 x 1500 24.9 / 19.5, 40 x 560 x 500 10.6 / 9.9, x 3000 36.9 / 35.2; 880 groups 40 x 700 x 700 14.3 / 14.4.
+// graph, without it / short: at 128 channels 12 x 320 x 320 10.4 / 6.8, 3 x 390 x 200 8.7 / 6.0, 12 x 600 x 1000 19.2 / 10.8,
+// x 3000 29.0 / 23.2, 12 x 320 x 4000 25.2 / 24.1, x 5000 32.1 / 30.2, 3 x 390 x 3000 20.2 / 19.2, x 5000 24.1 / 30.1; 264 to 512 groups
+// 12 x 680 x 500 12.0 / 10.5, 12 x 1000 x 1000 22.8 / 16.7, x 2000 29.7 / 26.1, x 3000 31.9 / 36.0; 516 groups 12 x 1360 x 500 12.1 / 16.0,
+// x 2000 34 / 41. At 64 channels 12 x 320 x 320 7.6 / 5.0, 3 x 390 x 3000 15.0 / 13.0, x 4000 16.7 / 15.9, x 5000 18.2 / 19.0, 12 x 1000 x 3000
+// 26.5 / 23.8 (eight waves 22.3), 12 x 1560 x 1500 24.3 / 18.8, x 3000 32.1 / 32.6, 40 x 560 x 500 9.1 / 9.5, x 3000 35.3 / 34.7; 880 groups
+// 40 x 700 x 700 11.6 / 14.6.
 // (Query tiles of 256 that have a CU each already, of few rows: flash_fwd_pp2 as before.)
 int fv_short_waves(size_t bh, size_t sq, size_t sk, size_t d) {
     const size_t cus = (size_t)fv_compute_units(), nq = (sq + 31) / 32, bm = (size_t)fv_internal_flash_block_m();
@@ -315,15 +318,16 @@ int fv_short_waves(size_t bh, size_t sq, size_t sk, size_t d) {
 
 // flash_fwd_duo (two or, at head dim 64, three workgroups a CU) against flash_fwd_pp2, for walks so short that an item's
 // ends count. Past them the chip runs at its power limit in either form, and 256 queries to a K and V stream cost less. us,
-// flash_fwd_pp2 / flash_fwd_duo: at 128 channels 12 x 32760 x 64 57 / 39, x 200 77 / 69, x 512 116 / 111, x 800 168 / 157, x 1000
-// 187 / 188, x 1500 264 / 267; 16 x 2560 x 700 25.2 / 23.1, 16 x 6144 x 1500 84.9 / 80.0, 24 x 10000 x 1000 126 / 124. At 64: 24 x
-// 4001 x 50 14.3 / 8.4, 16 x 4096 x 3000 55 / 53, 16 x 6144 x 4000 119 / 109, 16 x 12288 x 6000 311 / 299, 16 x 7680 x 6000 202 / 198.
+// flash_fwd_pp2 / flash_fwd_duo: at 128 channels 12 x 32760 x 64 61 / 38, x 200 77 / 64, x 512 109 / 100, x 800 160 / 144, x 1000
+// 177 / 171, x 1500 243 / 242; one round 12 x 4000 x 512 17.3 / 17.3, x 700 22.2 / 20.9, x 1024 26.0 / 26.9, x 1500 35.8 / 36.7; 16 x 2560 x 700
+// 21.6 / 20.2, 16 x 6144 x 1500 72.9 / 68.5, 24 x 10000 x 1000 115 / 111. At 64: 24 x 4001 x 50 14.2 / 7.6, 12 x 4000 x 4096 58.5 / 55.5,
+// 16 x 4096 x 3000 50 / 48, 16 x 6144 x 4000 105 / 99, 16 x 12288 x 6000 270 / 268, x 8000 357 / 355, 16 x 7680 x 6000 178 / 177.
 // A last round of a quarter of the CUs or less is shared out by key ranges (fv_split_plan), the sooner the fewer its tiles:
-// at 64 channels 16 x 4608 (32 tiles past a round) x 2000 54 / 52, x 2500 64 / 65, x 6000 129 / 147, 16 x 8704 (32 past two) x 2500
-// 103 / 102, x 6000 213 / 231, 16 x 5120 (64) x 3000 80 / 77, x 4000 99 / 101; at 128 16 x 4608 x 1300 70 / 66, x 1500 71 / 74,
-// 16 x 8960 (48) x 1350 109 / 104, x 1500 113 / 113. (Of a sixteenth or less: at any length, this kernel would pay a round for them.)
+// at 64 channels 16 x 4608 (32 tiles past a round) x 2000 52 / 49, x 2500 61 / 60, x 6000 120 / 136, 16 x 8704 (32 past two) x 2500
+// 100 / 96, x 6000 213 / 218, 16 x 5120 (64) x 3000 75 / 71, x 4000 93 / 94; at 128 16 x 4608 x 1300 63 / 58, x 1500 64 / 66,
+// 16 x 8960 (48) x 1350 102 / 97, x 1500 106 / 105. (Of a sixteenth or less: at any length, this kernel would pay a round for them.)
 // Where it cannot be split (no workspace, or an entry without one), flash_fwd_pp2 pays two whole rounds: 24 x 3000 x 6100 x 64
-// 176 / 149, 24 x 3000 x 1500 x 128 77 / 71, 16 x 8960 x 1500 x 128 123 / 116.
+// 172 / 139, 24 x 3000 x 1500 x 128 72 / 66, 16 x 8960 x 1500 x 128 114 / 105.
 // Few query tiles have a CU each, of 128 queries where fv_split_plan says so. f32 results follow the running max, whose
 // rescales go by pairs of tiles in flash_fwd_pp2: they stay there, and a block's result does not depend on the clip's length.
 bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16, bool may_split) {
@@ -338,19 +342,19 @@ bool fv_duo(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16, bool may_s
 // Fewer query tiles than CUs: fv_sdpa_splitkv_choose. More: they run in rounds of one per CU, and the last round costs a
 // whole walk of the keys however few tiles are left for it. Where they are few, they are shared out over the chip by key
 // ranges instead; where they are many it does not pay, because a chip that is half busy runs at a higher clock.
-// Measured on MI355X, unsplit and so, us: 24 x 3000 x 3000 x 128 (288 tiles: 256 + 32 x 5) 145 / 120, 40 x 2000 x 2000
-// x 64 (320: 256 + 64 x 4) 69 / 61, 40 x 75600 x 75600 x 128 (11840: 11776 + 64 x 4) 94470 / 92960 on one MI355X, where runs
-// of one side differ by 0.2 %, and inside the spread on another.
+// Measured on MI355X, unsplit and so, us: 24 x 3000 x 3000 x 128 (288 tiles: 256 + 32 x 4) 130 / 102, 40 x 2000 x 2000
+// x 64 (320: 256 + 64 x 4) 64 / 55, 40 x 5000 x 5000 x 128 (800: 768 + 32 x 5) 441 / 391, 40 x 75600 x 75600 x 128 (11840: 11776 + 64 x 4)
+// 80900 / 80200.
 FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16) {
     const size_t cus = (size_t)fv_compute_units(), bm = (size_t)fv_internal_flash_block_m();
     const size_t nqt = (sq + bm - 1) / bm, wgs = bh * nqt, nkt = (sk + 63) / 64;
     if (wgs < cus || cus % 8 != 0 || wgs > (size_t)INT_MAX / 64) {
         const size_t splits = fv_sdpa_splitkv_choose(bh, sq, sk);
         // Query tiles of 128 where each still has a CU to itself. Measured on MI355X, 256 / 128 queries a workgroup, us:
-        // bf16 results past the short kernel's walks and past flash_fwd_duo's 200 x 100 x 2000 x 128 52.1 / 41.8, 200 x 100 x
-        // 8000 x 64 146 / 103, 4 x 390 x 8000 x 128 split 31.8 / 28.7, 24 x 390 x 4000 x 128 39.4 / 38.9; f32 results 12 x 1000 x
-        // 1000 x 128 split 27.2 / 25.3, 40 x 700 x 700 x 64 17.6 / 15.0, 12 x 320 x 600 x 128 18.1 / 15.9, 24 x 390 x 2000 x 128 26.8 / 27.0; past one per CU, 12 x 4000 x
-        // 512 x 128 20.3 / 29.1, 40 x 1000 x 1000 x 64 (320 tiles) 21.5 / 21.7.
+        // bf16 results past the short kernel's walks and past flash_fwd_duo's 200 x 100 x 2000 x 128 45.9 / 37.1, 200 x 100 x
+        // 8000 x 64 123 / 90, 4 x 390 x 8000 x 128 split 32.5 / 27.7; f32 results 12 x 1000 x 1000 x 128 split 26.8 / 23.5, 40 x 700 x
+        // 700 x 64 17.5 / 13.4, 12 x 320 x 600 x 128 19.4 / 15.6; past one per CU, 24 x 390 x 4000 x 128 36.7 / 45.5, 24 x 390 x 2000 x
+        // 128 f32 26.8 / 33.8, 12 x 4000 x 512 x 128 19.8 / 27.2, 40 x 1000 x 1000 x 64 (320 tiles) 22.1 / 23.1.
         if (splits == 1 && fv_duo(bh, sq, sk, d, out_bf16, false)) return {bm, 0, 1, 0};
         const size_t half = bm / 2, small = bh * ((sq + half - 1) / half) * settle_splits(nkt, splits);
         return {small <= cus ? half : bm, 0, splits, fv_sdpa_splitkv_workspace_bytes(bh, sq, d, splits)};
@@ -358,8 +362,11 @@ FvSplitPlan fv_split_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf
     const size_t full = wgs / cus * cus, rest = wgs - full;
     if (rest == 0 || fv_duo(bh, sq, sk, d, out_bf16, true)) return {bm, 0, 1, 0};
     const size_t rows = bh * sq - (full / nqt * sq + full % nqt * bm);
-    // us, measured: a workgroup's fixed part, and a 64-key tile while `w` workgroups run (16 x 4000 x 4000 x 128, 256
-    // tiles: 121 us, half of them 79); partials written and read at 4 TB/s and a launch
+    // us: a workgroup's fixed part, and a 64-key tile while `w` workgroups run; partials written and read at 4 TB/s and a launch.
+    // Fitted to the kernel on 32x32x16 MFMAs (16 x 4000 x 4000 x 128, 256 tiles: 121 us, half of them 79). Now it
+    // takes 104 and 79, at 64 channels 70 and 59: the last tiles of a full chip cost less than this says, so it splits later than it could.
+    // 16 x 6144 x 4000 x 128 (128 tiles past a round) 174 as planned, unsplit, 160 in two; elsewhere the plan is within 6 % of the best
+    // count: 24 x 3000 x 6000 x 64 125 / 119, 40 x 2000 x 8000 x 64 167 / 159, 24 x 3000 x 3000 x 128 102 / 101, 12 x 8000 x 8000 290 / 290.
     const double fixed = d == 64 ? 5.0 : 8.0;
     auto run = [&](size_t w, size_t tiles) {
         const double x = w <= cus / 2 ? 0.0 : ((double)w / (double)cus - 0.5) * 2.0;
@@ -503,9 +510,9 @@ size_t fv_sdpa_splitkv_choose(size_t bh, size_t sq, size_t sk) {
     const size_t bm = (size_t)fv_internal_flash_block_m();
     const size_t wgs = bh * ((sq + bm - 1) / bm), nkt = (sk + 63) / 64;
     if (wgs == 0 || wgs >= (size_t)cus) return 1;               // the query tiles alone fill the CUs
-    // Cost model (microseconds, measured on MI355X): a workgroup costs about 10 fixed + 1.7 per 64-key
-    // tile, workgroups run in rounds of one per CU, and the merge reads `s` f32 partials at about
-    // 4 TB/s. Take the cheapest split count, if it wins by more than 10 %.
+    // Cost model (microseconds): a workgroup costs about 10 fixed + 1.7 per 64-key tile (an early form of the kernel; now 7
+    // and 1.1 on a chip that is half full, 1.5 on a full one, so it splits a little early: f32 results 12 x 1000 x 1000 x 128 23.2
+    // as it chooses, 21.6 unsplit; 24 x 390 x 4000 36 / 60, 12 x 1560 x 32760 270 / 470), workgroups run in rounds of one per CU, and the merge reads `s` f32 partials at about 4 TB/s. Take the cheapest split count, if it wins by more than 10 %.
     auto cost = [&](size_t sp) {
         const size_t per = (nkt + sp - 1) / sp, real = (nkt + per - 1) / per;
         const double rounds = (double)((wgs * real + cus - 1) / cus);

@@ -247,7 +247,7 @@ Result<Tensor> compact(const Tensor& x, Mem& st) {
 
 // The short kernel takes bf16 results of every length it is the faster for, f32 ones as a kernel-level call does (up to 512
 // keys): past those an f32 result keeps to one kernel's sums, alone or merged, which the block-causal launches share
-// (12 x 1000 x 1000 x 128 25 us; a bf16 result 17).
+// (12 x 1000 x 1000 x 128 23 us; a bf16 result 17).
 FvSplitPlan dense_plan(size_t bh, size_t sq, size_t sk, size_t d, bool out_bf16) {
     const int waves = out_bf16 ? fv_short_waves(bh, sq, sk, d) : 0;
     if (!waves) return fv_split_plan(bh, sq, sk, d, out_bf16);
