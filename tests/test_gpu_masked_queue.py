@@ -1,5 +1,5 @@
-"""The queue that masked launches of eight rounds and more take their items from through `sdpa`: the bits of the
-launch in the order of the workgroups' numbers, which the kernel-level entries make."""
+"""The queue that long masked launches at 128 channels take their items from through `sdpa` (fv_masked_workspace_bytes): the
+bits of the launch in the order of the workgroups' numbers, which the kernel-level entries make."""
 import pytest
 
 from util import announce
@@ -18,8 +18,19 @@ def fv():
     return fv_sdpa
 
 
+def queue_bytes(fv, q, plan):
+    import ctypes
+
+    from fv_sdpa.sdpa import _desc_bytes, _plan_bytes
+
+    need = (ctypes.c_size_t * 2)()
+    assert fv.lib().fv_rt_sdpa_need(*[_desc_bytes(q, "q")] * 3, _plan_bytes(plan, 0, 256), need) == 0
+    return need[1]
+
+
 # eight rounds of query tiles: lists of shared heads only, of whole and shared ones, of whole ones, with one shared head
-QUEUE = [(3, 175200, 64), (12, 44000, 128), (16, 33000, 128), (41, 13000, 64)]
+# (at 64 channels such launches go without it)
+QUEUE = [(3, 175200, 64), (12, 44000, 128), (16, 33000, 128), (41, 13000, 64), (3, 175200, 128), (41, 13000, 128)]
 
 
 @pytest.mark.parametrize("kind", ["causal", "sink", "window"])
@@ -38,6 +49,7 @@ def test_the_queue_gives_the_bits_of_the_launch_without_it(fv, h, s, d, kind):
         args = (t, 0, 0) if kind == "causal" else (t, 5, 1)
         plan = fv.Plan.block_causal(None, fv.BlockCausal(*args))
     fn = fv.sdpa_vdn_window_bf16 if kind == "window" else fv.sdpa_block_causal_bf16
+    assert queue_bytes(fv, q, plan) == (1024 if d == 128 else 0)
     for bf16 in (True, False):
         want = fn(q[0], k[0], v[0], *args, out_bf16=bf16)
         with fv.with_bf16_act(bf16):
